@@ -233,9 +233,19 @@ def _empty(nbytes):
     return _Buf(torch.empty(nbytes, dtype=torch.int8, device="cuda"))
 
 
+_streams = []
+
+
+def _stream():
+    """The program's processing stream: blocks are taken one after the other, as a pipeline takes them."""
+    if not _streams:
+        _streams.append(capi.Stream())
+    return _streams[0]
+
+
 def prepare(case, seed):
     gen, kind = _gen(seed), case["kind"]
-    st = {"kind": kind, "case": case, "stream": capi.Stream()}
+    st = {"kind": kind, "case": case, "stream": _stream()}
     if kind in ("block", "taftp", "ftpa"):
         A, F, B, ts, fs, T = case["antennas"], case["chans"], case["beams"], case["ts"], case["fs"], _samples(case)
         total = case.get("total", A)
