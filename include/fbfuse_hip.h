@@ -196,10 +196,11 @@ int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_block, size_t b
  * copy is written; otherwise the call split-transposes into an FTPA buffer
  * that the plan owns (grown on demand, as the staging buffer) first.  As
  * with fbf_cb_beamform, calls with one plan on different streams must not
- * overlap (they share the plan's buffers).  With
- * the automatic variant and more than 48 antennas it picks the transposed
- * kernel with 128 beams per wave where that applies (half the transposed
- * LDS reads per MFMA of 64 beams per wave). */
+ * overlap (they share the plan's buffers).  The automatic variant picks the
+ * transposed kernel with 128 beams per wave up to 64 antennas and with 64
+ * above, and the split-transpose where few beams would leave such waves
+ * empty (up to 48 antennas with at most 96 beams, above 64 with at most
+ * 32). */
 int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes,
                           int nantennas_total, int start_antenna, int nsamples_per_heap,
                           const void* fba_weights, size_t weights_bytes,
@@ -207,7 +208,8 @@ int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_byt
 /* *direct = 1 when fbf_cb_beamform_taftp reads a block of this geometry
  * without the FTPA copy: the plan's kernel is the transposed one with 64 or
  * 128 beams per wave, fscrunch 1, nsamples_per_heap a power of two >= 16,
- * and one heap group under 2 GiB.  No counterpart in the reference. */
+ * one heap group under 2 GiB and the block under 4 GiB.  No counterpart in
+ * the reference. */
 int fbf_cb_taftp_direct(const fbf_cb_plan* plan, int nantennas_total, int nsamples_per_heap,
                         long long nsamples, int* direct);
 /* Timing of the coherent kernel alone: every later beamform call with this
@@ -272,9 +274,9 @@ int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void
                              int nsamples_per_heap, const void* fba_weights, size_t weights_bytes,
                              void* tbtf, size_t tbtf_bytes, void* tf, size_t tf_bytes, fbf_stream_t stream);
 /* *fused = 1 when fbf_cb_ib_beamform_taftp forms the incoherent beam inside
- * the coherent kernel: the direct TAFTP path with 128 beams per wave, and
- * an incoherent-beam plan of the same antennas, channels and heap size.  No
- * counterpart in the reference. */
+ * the coherent kernel: the direct TAFTP path with 128 beams per wave (or 64
+ * above 64 antennas), and an incoherent-beam plan of the same antennas,
+ * channels and heap size.  No counterpart in the reference. */
 int fbf_cb_ib_fused(const fbf_cb_plan* plan, const fbf_ib_plan* ib_plan, int nsamples_per_heap,
                     long long nsamples, int* fused);
 

@@ -1,0 +1,968 @@
+// Coherent beamformer: the transposed-tile kernel (cb_tr_k), its detection and
+// its quantiser.
+#pragma once
+
+#include "cb_common.hpp"
+
+namespace fbf {
+namespace {
+
+// ---------------------------------------------------------------------------
+// Transposed tiles: voltages as the A operand, weights as the B operand.
+//
+//   D[m][n] = sum_k V[m][k] W'[n][k]
+//
+// Rows m are 32 consecutive input columns (t, p) of one channel, columns n
+// are 16 beams x (Re, Im) embedding rows.  Lane l holds column n = l % 32
+// and rows 8*(i/4) + 4*(l/32) + i%4 (i = 0..15).  For an integration window
+// of W = 2*tscrunch = 8, 16 or 32 columns, or a multiple of 32, every window
+// a lane touches is a fixed group of its 16 values, so the squares sum into
+// one int64 per (beam tile, window) in the lane.  The four lanes holding
+// {Re, Im} x {row halves} of a beam are combined once per pass of windows by
+// a reduce-scatter (exchange with lane ^ 1, then lane ^ 32) that leaves each
+// lane a distinct (beam, window) total to quantise.
+//
+// A wave keeps RT beam tiles (16 RT beams) of weights in registers for its
+// channel and reads each voltage tile once from LDS for all of them: LDS
+// traffic is 1/RT of a tile per MFMA.  With fscrunch FS = 2 or 4 the waves of
+// a work-group take different channels of the fscrunch group (each with its
+// own weights) and add their window totals through LDS before quantising.
+//
+// Voltage staging is a ring of NB tile sets in LDS (one tile per channel of
+// the fscrunch group per set) filled by direct global->LDS loads issued
+// NB - 1 tiles ahead.  Every step issues one set (past the work-group's last
+// tile the loads repeat the last tile into a slot nobody reads), so the
+// number of loads in flight after a wave's loads of the current set is the
+// constant (NB - 2) * M and the wait is a fixed s_waitcnt.
+// ---------------------------------------------------------------------------
+
+// s_waitcnt vmcnt(N) lgkmcnt(0).
+template <int N>
+__device__ __forceinline__ void wait_vm_lgkm0()
+{
+    static_assert(N >= 0 && N <= 63, "vmcnt");
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+// One 16-byte global->LDS load per lane: lane i's 16 bytes land at
+// lds_run + 16 * i (lds_run is wave-uniform).
+__device__ __forceinline__ void dma16(const int8_t* src, int8_t* lds_run)
+{
+    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_run, 16, 0, 0);
+}
+
+// A wave-uniform pointer as scalar registers, so that a load from it plus a
+// 32-bit lane offset takes the scalar-base address form (no 64-bit vector
+// address arithmetic per load).
+template <typename T>
+__device__ __forceinline__ T* uniform_ptr(T* ptr)
+{
+    const unsigned long long v = reinterpret_cast<unsigned long long>(ptr);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return reinterpret_cast<T*>(((unsigned long long)hi << 32) | lo);
+}
+
+// A pointer known to address global memory, so that stores through it are
+// global (not flat: a flat store also counts against the LDS wait counter).
+__device__ __forceinline__ __attribute__((address_space(1))) int8_t* global_ptr(int8_t* ptr)
+{
+    return (__attribute__((address_space(1))) int8_t*)ptr;
+}
+
+// Work-group barrier without the memory fence of __syncthreads (which would
+// wait for every outstanding global load, including the LDS prefetches).
+// Callers wait for their own LDS and global->LDS traffic first; the empty
+// asm statements keep the compiler from moving memory accesses across.
+__device__ __forceinline__ void block_barrier()
+{
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+}
+
+// The incoherent-beam partials of tiles [t0, t1) of channel f straight from
+// the TAFTP block, for the work-groups on the exact path (which leave the
+// tile loop): per sample the power over all antennas and both pols in
+// column 2j of half 0, zeros in its other three places.
+__device__ __forceinline__ void cb_exact_ib_partials(const CbArgs& p, int* ibp, int ntiles, int f, int t0, int t1,
+                                                  int tid, int nt)
+{
+    const size_t astep = (size_t)p.F * p.S * 4;
+    for (int i = tid; i < (t1 - t0) * 16; i += nt) {
+        const int tile = t0 + i / 16, j = i % 16;
+        const long long t = (long long)tile * 16 + j;
+        const int8_t* v = p.ftpa + (((size_t)(t / p.S) * p.Atot + p.a0) * p.F + f) * p.S * 4 + (size_t)(t % p.S) * 4;
+        int sum = 0;
+        for (int a = 0; a < p.A; ++a) {
+            const int w = *reinterpret_cast<const int*>(v + a * astep);
+            sum = __builtin_amdgcn_sdot4(w, w, sum, false);
+        }
+        int* dst = ibp + ((size_t)f * ntiles + tile) * 64 + 2 * j;
+        dst[0] = sum;
+        dst[1] = 0;
+        dst[32] = 0;
+        dst[33] = 0;
+    }
+}
+
+// The 16-byte A operands of one step's K slices (8 antennas x char2 of one
+// column each) from an LDS tile laid out [antenna][32 columns] int16, 64
+// bytes a row: two ds_read_b64_tr_b16 of 4 antenna rows each per slice.
+// Within every 16-lane group G the instruction gives lane i, as its element
+// r, element i % 4 of the 8 bytes read by lane 16 G + 4 r + i / 4.  So when
+// lane L reads the 4 columns 16 (G % 2) + 4 (L % 4) .. + 3 of antenna row
+// base + (L / 4) % 4, lane c + 32 h (c < 32) receives column c of rows
+// base .. base + 3, in row order.  `src` is that row piece of slice 0 for
+// this lane; slice s is 8 rows (512 bytes) further on, its second read 4
+// rows (256 bytes) after its first.
+//
+// The reads of up to four slices are issued in one asm block that ends with
+// their LDS wait.
+// Issued through the builtin, every transposed read is preceded by a wait
+// for all outstanding global->LDS loads (the compiler cannot tell that they
+// fill other ring slots), which cost the kernel a memory round trip per
+// step; the ring's own vmcnt wait and barrier already order them.  The
+// outputs are complete when the block ends (lgkmcnt(0) inside it).
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+// 2 * N transposed reads of N slices from `addr` on, and their LDS wait.
+template <int N>
+__device__ __forceinline__ void tr_reads(uint32_t addr, v2i* r)
+{
+    static_assert(N >= 1 && N <= 4, "slices per block");
+    if constexpr (N == 1) {
+        __asm__ volatile(
+            "ds_read_b64_tr_b16 %0, %2\n\t"
+            "ds_read_b64_tr_b16 %1, %2 offset:256\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0]), "=&v"(r[1])
+            : "v"(addr)
+            : "memory");
+    } else if constexpr (N == 2) {
+        __asm__ volatile(
+            "ds_read_b64_tr_b16 %0, %4\n\t"
+            "ds_read_b64_tr_b16 %1, %4 offset:256\n\t"
+            "ds_read_b64_tr_b16 %2, %4 offset:512\n\t"
+            "ds_read_b64_tr_b16 %3, %4 offset:768\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+            : "v"(addr)
+            : "memory");
+    } else if constexpr (N == 3) {
+        __asm__ volatile(
+            "ds_read_b64_tr_b16 %0, %6\n\t"
+            "ds_read_b64_tr_b16 %1, %6 offset:256\n\t"
+            "ds_read_b64_tr_b16 %2, %6 offset:512\n\t"
+            "ds_read_b64_tr_b16 %3, %6 offset:768\n\t"
+            "ds_read_b64_tr_b16 %4, %6 offset:1024\n\t"
+            "ds_read_b64_tr_b16 %5, %6 offset:1280\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5])
+            : "v"(addr)
+            : "memory");
+    } else {
+        __asm__ volatile(
+            "ds_read_b64_tr_b16 %0, %8\n\t"
+            "ds_read_b64_tr_b16 %1, %8 offset:256\n\t"
+            "ds_read_b64_tr_b16 %2, %8 offset:512\n\t"
+            "ds_read_b64_tr_b16 %3, %8 offset:768\n\t"
+            "ds_read_b64_tr_b16 %4, %8 offset:1024\n\t"
+            "ds_read_b64_tr_b16 %5, %8 offset:1280\n\t"
+            "ds_read_b64_tr_b16 %6, %8 offset:1536\n\t"
+            "ds_read_b64_tr_b16 %7, %8 offset:1792\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]),
+              "=&v"(r[7])
+            : "v"(addr)
+            : "memory");
+    }
+}
+
+template <int KSTEPS>
+__device__ __forceinline__ void tr_operands(const int8_t* src, v4i (&a)[KSTEPS])
+{
+    const uint32_t addr = (uint32_t)(size_t)(const __attribute__((address_space(3))) int8_t*)src;
+    v2i r[2 * KSTEPS];
+    static_assert(KSTEPS >= 1 && KSTEPS <= 8, "K steps");
+    constexpr int N0 = KSTEPS < 4 ? KSTEPS : 4;
+    tr_reads<N0>(addr, r);
+    if constexpr (KSTEPS > 4) tr_reads<KSTEPS - 4>(addr + 2048, r + 8);
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) a[s] = v4i{r[2 * s].x, r[2 * s].y, r[2 * s + 1].x, r[2 * s + 1].y};
+}
+
+// A tile's incoherent-beam partials from the operands tr_operands gave this
+// wave (every K slice): per lane the power of its column over the 8 * KSTEPS
+// antennas of its row half, each word (two antennas' re, im) squared with
+// v_dot4, antenna groups of 4 past A left out (they re-read antenna 0); the
+// 64 lanes store their sums as the tile's [2 halves][32 columns] record.
+template <int KSTEPS>
+__device__ __forceinline__ void ib_tile(const v4i (&a)[KSTEPS], int* ibp, int ntiles, int A, int f, int tile,
+                                        int lane)
+{
+    int v = 0;
+    if (A == 16 * KSTEPS) {   // uniform: no padded rows, one dot chain
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v = __builtin_amdgcn_sdot4(a[s][q], a[s][q], v, false);
+    } else {
+        const int h = lane >> 5;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int q = 0; q < 4; q += 2) {
+                int t = __builtin_amdgcn_sdot4(a[s][q], a[s][q], 0, false);
+                t = __builtin_amdgcn_sdot4(a[s][q + 1], a[s][q + 1], t, false);
+                v += 8 * (h * KSTEPS + s) + 2 * q < A ? t : 0;
+            }
+    }
+    if (tile < ntiles) ibp[((size_t)f * ntiles + tile) * 64 + lane] = v;
+}
+
+// a + b' where lanes below 32 keep a and take b' = (a of lane + 32), and
+// lanes from 32 keep b and take (b of lane - 32): the halves' exchange of a
+// reduce-scatter in one v_permlane32_swap per dword.  With a = value for the
+// lower half and b = value for the upper half, every lane gets its own sum.
+__device__ __forceinline__ long long swap32_sum(long long a, long long b)
+{
+    const unsigned alo = (uint32_t)(unsigned long long)a, ahi = (uint32_t)((unsigned long long)a >> 32);
+    const unsigned blo = (uint32_t)(unsigned long long)b, bhi = (uint32_t)((unsigned long long)b >> 32);
+    const auto lo = __builtin_amdgcn_permlane32_swap(alo, blo, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(ahi, bhi, false, false);
+    // 64-bit sum as one add and one add-with-carry of the halves.
+    const unsigned slo = lo[0] + lo[1];
+    const unsigned shi = hi[0] + hi[1] + (slo < lo[0] ? 1u : 0u);
+    return (long long)(((unsigned long long)shi << 32) | slo);
+}
+
+// Constants of the threshold quantiser's estimates: FP64 (P - offset) * inv
+// with inv = RN(1 / scale), and FP32 P * inv_f + c_f with inv_f = RN(1 /
+// scale), c_f = RN(-offset * inv_f).
+struct QuantConst {
+    double off_d, inv;
+    float inv_f, c_f;
+};
+
+__device__ __forceinline__ QuantConst quant_const(float off, float sc)
+{
+    const float inv_f = 1.0f / sc;
+    return QuantConst{(double)off, 1.0 / (double)sc, inv_f, -off * inv_f};
+}
+
+// Quantiser thresholds.  For a positive, normal, finite scale and a finite
+// offset, quantise((double)P, offset, scale, mode) is a non-decreasing step
+// function of the integer power P: thr[j] is the least P >= 0 that quantises
+// to at least j - 128 (thr[0] = INT64_MIN, thr[256] = INT64_MAX, and
+// INT64_MAX where no P < 2^62 gets there).  The kernel needs only an
+// estimate e within one step of the result q: the two thresholds around e
+// then settle q without a division or a branch (P >= thr[e + 129] means
+// q = e + 1, P < thr[e + 128] means q = e - 1).  The estimate is
+// e = trunc(clamp(y, -128, 127)) for an approximation y of the quotient Y
+// that the exact quantiser rounds: whenever |y - Y| < 0.5, truncation moves
+// y by less than 1 and the mode's rounding moves Y by at most 0.5 (truncation
+// by less than 1, and then |y - Y| < 1 suffices), so |e - q| < 2 in either
+// mode (the clamp keeps this), i.e. e is q or a neighbour.
+constexpr int kThr = 257;
+constexpr int kThrBytes = 2304;   // kThr int64, padded to a multiple of 256 bytes
+static_assert(kThrBytes >= kThr * 8, "threshold table");
+
+__device__ __forceinline__ bool thr_applies(float off, float sc)
+{
+    return isfinite(off) && sc >= 1.17549435e-38f && sc <= 3.40282347e+38f;
+}
+
+// Threshold correction of an estimate e in [-128, 127]; thr_mid = thr + 128
+// (so thr_mid[e] and thr_mid[e + 1] are one ds_read2_b64).
+__device__ __forceinline__ int8_t thr_settle(long long P, int e, const long long* thr_mid)
+{
+    const long long lo = thr_mid[e], hi = thr_mid[e + 1];
+    return (int8_t)(e + (int)(P >= hi) - (int)(P < lo));
+}
+
+// FP64 estimate RN(RN((double)P - offset) * RN(1 / scale)): it rounds the
+// same difference as the exact quantiser, so it is within 2^-43 of Y for
+// |Y| <= 256 at any offset and scale; beyond, both saturate alike.
+__device__ __forceinline__ int thr_estimate(long long P, const QuantConst& q)
+{
+    const double y = ((double)P - q.off_d) * q.inv;
+    return (int)fmin(fmax(y, -128.0), 127.0);
+}
+
+__device__ __forceinline__ int8_t quantise_thr(long long P, const QuantConst& q, const long long* thr_mid)
+{
+    return thr_settle(P, thr_estimate(P, q), thr_mid);
+}
+
+// FP32 estimate (about a third of the VALU time of the FP64 one).  For
+// P >= 0, RN(RN(hi) * 2^32 + RN(lo)) is within 3 * 2^-24 of P relative;
+// RN(1 / scale) and c = RN(-offset * inv) are within 2^-24 and 2^-23
+// relative, and the fma rounds once, so for |Y| <= 130 the estimate is
+// within 2^-24 * (4 |P / scale| + 2 |offset / scale| + 131) <=
+// 2^-24 * (651 + 6 |offset / scale|) of Y: below 0.38 when
+// |offset / scale| < 2^20 (thr_f32_applies); beyond |Y| = 130 both
+// saturate alike.
+__device__ __forceinline__ bool thr_f32_applies(float off, float sc)
+{
+    return fabsf(off / sc) < 1048576.0f;
+}
+
+__device__ __forceinline__ int thr_estimate_f32(long long P, const QuantConst& q)
+{
+    const float pf = (float)(int)(P >> 32) * 4294967296.0f + (float)(uint32_t)P;
+    const float y = __builtin_fmaf(pf, q.inv_f, q.c_f);
+    return (int)__builtin_amdgcn_fmed3f(y, -128.0f, 127.0f);
+}
+
+// One tile step of the transposed kernels: the RT tiles' MFMA chains and the
+// detection of their values into the pass accumulators pw[RT / 2][NSLOT]
+// (tile r adds to beam group r / 2; values of window q of the tile go to
+// slot g * SPT + q), one v_mad_i64_i32 per value.  (Splitting the
+// dependent chains into independent partial sums measured 0.7 % slower:
+// the other waves of the SIMD already cover their latency.)
+template <int RT, int KSTEPS, int SPT, int NSLOT>
+__device__ __forceinline__ void detect_step(const v4i (&a)[KSTEPS], const v4i (&w)[RT][KSTEPS],
+                                            long long (&pw)[RT / 2][NSLOT], int g)
+{
+    constexpr int n = 16 / SPT;   // values per window per tile
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        v16i acc = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s], w[r][s], acc, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < SPT; ++q)
+#pragma unroll
+            for (int i = 0; i < n; ++i) pw[r >> 1][g * SPT + q] += (long long)acc[q * n + i] * acc[q * n + i];
+    }
+}
+
+// Staging constants of cb_tr_k for FS channels x KSTEPS 32-byte K steps.
+template <int FS, int KSTEPS, int NTS>
+struct TrStage {
+    static constexpr int NW = 4 * NTS;                     // waves per work-group
+    static constexpr int NI = NTS * FS * KSTEPS;           // 1 KiB loads per set
+    static constexpr int M = (NI + NW - 1) / NW;           // per wave (the rest load into a dummy run)
+    static constexpr int SET = NI * 1024;                  // bytes per set
+    static constexpr int NB = 60 / NI < 2 ? 2 : (60 / NI > 8 ? 8 : 60 / NI);
+    static constexpr int G = NB >= 4 ? 2 : 1;             // steps per barrier
+    static constexpr int WAIT = (NB - 2 * G) * M;
+    static constexpr int DUMMY = (NI % NW) ? NW * 1024 : 0;
+};
+
+template <int RT, int NSLOT>
+struct TrRed {
+    // totals per lane after the reduce-scatter
+    static constexpr int VALS = RT == 2 ? NSLOT / 2 : (RT / 4) * NSLOT;
+};
+
+// RT: beam tiles per wave (RT / 2 groups of 32 beams, a Re and an Im tile
+// each); SPT: windows per tile (1, 2, 4); NSLOT: windows
+// per pass held in registers; FS: fscrunch; NTS: time slots per work-group;
+// TA: the voltages are a TAFTP block (CbArgs::S > 0), staged straight into
+// [antenna][column] tiles and read with transposed LDS loads (tr_operands),
+// else FTPA columns; IBF (with TA, FS = 1, all antennas of the block): the
+// work-groups of beam group 0 also leave the incoherent beam's per-sample
+// partials (CbTrArgs::ibp) from the same operands.
+//
+// A work-group has 4 * NTS waves: NTS time slots (contiguous runs of passes
+// of the same channel group and beams) x 4 waves ((4 / FS) beam groups x FS
+// channels).  With 64 beams per wave a work-group holds every wave of its
+// compute unit (NTS = tr_nts waves per SIMD: 3 or 4), so the per-step
+// barrier keeps them in lockstep: waves of separate work-groups sharing a
+// SIMD progress at different rates (the issue arbiter prefers older waves),
+// which leaves SIMDs with one wave at the end.  With 128 beams per wave
+// (two waves per SIMD) a work-group is one time slot, two share a compute
+// unit, and they take turns at a raised wave priority instead.
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, bool TA, bool IBF>
+__global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs ta)
+{
+    using St = TrStage<FS, KSTEPS, NTS>;
+    constexpr int KPAD = 32 * KSTEPS;
+    constexpr int PR = 2 * KSTEPS;                 // 16-byte pieces per LDS column
+    constexpr int VALS = TrRed<RT, NSLOT>::VALS;
+    constexpr int NB = St::NB;
+    constexpr int NG = RT / 2;                     // groups of 32 beams per wave
+    static_assert(RT == 2 || RT == 4 || RT == 8, "RT");
+    static_assert(NSLOT % SPT == 0 && (RT != 2 || NSLOT % 2 == 0), "slots");
+    static_assert(St::M <= 2, "at most two staging loads per wave per set");
+    static_assert(!IBF || (TA && FS == 1 && NTS <= 2), "incoherent-beam partials");
+    extern __shared__ __align__(16) int8_t lds[];
+    const CbArgs& p = ta.p;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const int h = lane >> 5;
+    const int c = lane & 31;
+    const int tsl = wv >> 2;         // time slot
+    const int wc = (wv & 3) % FS;    // channel of the fscrunch group
+    const int wb = (wv & 3) / FS;    // beam group within the work-group
+    constexpr int NWB = 4 / FS;
+
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int bgroup = logical % ta.n_bgroups;
+    const int rest = logical / ta.n_bgroups;
+    const int tgroup = rest % ta.n_tgroups;
+    const int fo = rest / ta.n_tgroups;
+    if (fo >= p.Fo) return;   // uniform over the work-group
+
+    const int K = 2 * p.A;
+    const int f = fo * FS + wc;
+    const int beam_base = (bgroup * NWB + wb) * 16 * RT;
+    const size_t TP = (size_t)2 * p.nsamples;
+    const int slot_tiles = ta.npasses * ta.ntp;
+    const int tile0 = (tgroup * NTS + tsl) * slot_tiles;
+
+    // Start-up loads first, all in flight together: the channel's quantiser
+    // thresholds (to LDS below), the weights, then the first staged tiles.
+    // One threshold per thread, two for the first threads of a one-slot
+    // work-group (256 threads, kThr = 257).
+    static_assert(512 * NTS >= kThr, "at most two thresholds per thread");
+    const long long thr_v = tid < kThr ? p.thr[(size_t)fo * kThr + tid] : 0;
+    const long long thr_v2 = tid + 256 * NTS < kThr ? p.thr[(size_t)fo * kThr + tid + 256 * NTS] : 0;
+
+    // Weights (B operand).  Tile r holds the Re (r even) or Im (r odd)
+    // embedding rows of the 32 beams beam_base + 32 (r / 2) + n, n = lane %
+    // 32, so a lane's Re and Im outputs belong to one beam and its power
+    // sums in-lane.
+    v4i w[RT][KSTEPS];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int b = beam_base + 32 * g + c;
+        const bool bvalid = b < p.B;
+        const int8_t* wcol = p.fba + ((size_t)f * p.B + (bvalid ? b : p.B - 1)) * K;
+        // K % 16 == 8 (antennas a multiple of 4 only) is a TAFTP form: FTPA
+        // staging moves whole 16-byte pieces of a column.
+        if (TA && (K & 15)) {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) w[2 * g][s] = load_wslice<false>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+        } else {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) w[2 * g][s] = load_wslice<true>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+        }
+    }
+
+    // Staging.  A wave's 16-byte load lands at LDS offset 16 * lane of a
+    // 1 KiB run.  FTPA: the bank swizzle is chosen on the global side:
+    // physical piece pp of column col holds K piece (pp + rot(col)) % PR with
+    // rot(col) = col * KPAD / 256.  K pieces past the column (k >= K) re-read
+    // piece 0: the weights there are zero.  TAFTP: a tile is 16 * KSTEPS
+    // antenna rows of 64 bytes (its 32 columns, contiguous in TAFTP), and a
+    // load fills 16 rows, 4 lanes a row; rows past A re-read antenna 0.
+    const int kpieces = K / 16;
+    // LDS: the channel's thresholds first (at address 0, so that a
+    // threshold read takes the table's offset as its immediate), then the
+    // ring, the dummy run and the fscrunch reduction.
+    long long* thr = reinterpret_cast<long long*>(lds);                   // [kThr] of channel fo
+    int8_t* const ring = lds + kThrBytes;
+    int8_t* dummy = ring + NB * St::SET;
+    long long* red = reinterpret_cast<long long*>(dummy + St::DUMMY);   // [waves][VALS][64]
+    // A set holds one tile per (time slot, channel): tile index
+    // tsl * FS + ch.  Load m of this wave fills 1 KiB of tile ti = u / KSTEPS
+    // (u = wave + NW * m, the same tile for the whole wave): the channel's
+    // base is wave-uniform (scalar), and each lane adds its column and
+    // swizzled K piece as a 32-bit offset.
+    const int8_t* cbase[St::M];
+    uint32_t goff[St::M];
+    int gtile[St::M];
+    int ldst[St::M];
+#pragma unroll
+    for (int m = 0; m < St::M; ++m) {
+        const int u = wv + St::NW * m;
+        if (u < St::NI) {
+            const int ti = u / KSTEPS;
+            if constexpr (TA) {
+                const int kp = u - ti * KSTEPS;
+                int an = 16 * kp + (lane >> 2);
+                if (an >= p.A) an = 0;
+                cbase[m] = p.ftpa + (size_t)(fo * FS + ti % FS) * p.S * 4;
+                goff[m] = (uint32_t)(p.a0 + an) * (uint32_t)(p.F * p.S * 4) + 16 * (lane & 3);
+            } else {
+                const int rem = (u - ti * KSTEPS) * 1024 + lane * 16;
+                const int col = rem / KPAD;
+                const int pp = (rem - col * KPAD) >> 4;
+                const int j = (pp + ((col * KPAD) >> 8)) % PR;
+                const int jj = j < kpieces ? j : 0;
+                cbase[m] = p.ftpa + (size_t)(fo * FS + ti % FS) * TP * p.vstride + p.voff;
+                goff[m] = (uint32_t)(col * p.vstride + 16 * jj);
+            }
+            gtile[m] = (tgroup * NTS + ti / FS) * slot_tiles;
+            ldst[m] = u * 1024;
+        } else {
+            cbase[m] = TA ? p.ftpa : p.ftpa + (size_t)(fo * FS) * TP * p.vstride + p.voff;
+            goff[m] = 0;
+            gtile[m] = 0;
+            ldst[m] = -1;
+        }
+    }
+    const size_t tile_stride = (size_t)32 * p.vstride;
+    const int tmask = (1 << ta.lgtph) - 1;
+    // TAFTP: each load keeps a running 32-bit offset of its next tile (the
+    // block is below 4 GiB, fbf_cb_beamform_taftp's condition), since the
+    // issues take consecutive tiles: 64 bytes on within a heap, the next
+    // heap's first tile at a heap boundary; loads past the last tile keep
+    // re-reading it.  A handful of scalar instructions per load instead of a
+    // 64-bit tile address (every wave of a compute unit shares one scalar
+    // unit, and the loads are issued right after a barrier).
+    uint32_t toff_run[St::M];
+    int tile_run[St::M];
+    if constexpr (TA) {
+#pragma unroll
+        for (int m = 0; m < St::M; ++m) {
+            const int t = gtile[m] < ta.ntiles ? gtile[m] : ta.ntiles - 1;
+            tile_run[m] = gtile[m];
+            toff_run[m] = (uint32_t)(t >> ta.lgtph) * (uint32_t)ta.hstride + ((uint32_t)(t & tmask) << 6);
+            cbase[m] = uniform_ptr(cbase[m]);
+        }
+    }
+    const uint32_t heap_jump = (uint32_t)ta.hstride - (uint32_t)tmask * 64u;
+    auto issue = [&](int q, int slot) {
+        int8_t* set = ring + slot * St::SET;
+#pragma unroll
+        for (int m = 0; m < St::M; ++m) {
+            int8_t* dst = ldst[m] >= 0 ? set + ldst[m] : dummy + wv * 1024;
+            if constexpr (TA) {
+                dma16(cbase[m] + toff_run[m] + goff[m], dst);
+                ++tile_run[m];
+                if (tile_run[m] < ta.ntiles) toff_run[m] += (tile_run[m] & tmask) ? 64u : heap_jump;
+            } else {
+                const int tt = gtile[m] + q < ta.ntiles ? gtile[m] + q : ta.ntiles - 1;
+                dma16(uniform_ptr(cbase[m] + (size_t)tt * tile_stride) + goff[m], dst);
+            }
+        }
+    };
+    // Physical offsets of this lane's K pieces in its column (FTPA), or of
+    // the row piece this lane reads for K slice s (TAFTP, tr_operands): rows
+    // 8 (h KSTEPS + s) + (lane / 4) % 4, columns 16 ((lane / 16) % 2) +
+    // 4 (lane % 4), so lane c + 32 h gets the antennas of K piece
+    // h KSTEPS + s, as FTPA's column holds them.
+    int aoff[KSTEPS];
+    if constexpr (TA) {
+        const int rr = (lane >> 2) & 3, xx = lane & 3, gh = (lane >> 4) & 1;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+            aoff[s] = (tsl * FS + wc) * KSTEPS * 1024 + (8 * (h * KSTEPS + s) + rr) * 64 + 32 * gh + 8 * xx;
+    } else {
+        const int rot = (c * KPAD) >> 8;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+            aoff[s] = ((tsl * FS + wc) * 32 + c) * KPAD + 16 * ((h * KSTEPS + s - rot + 32 * PR) % PR);
+    }
+
+    const bool wave_active = beam_base < p.B;
+#pragma unroll
+    for (int q = 0; q < NB - St::G; ++q) issue(q, q);
+    int step = 0;
+    int rs = 0;              // ring slot read this step
+    int is = NB - St::G;     // next ring slot to fill
+
+    bool m128 = false;
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            m128 |= raw_has_m128(w[2 * g][s]);
+            w[2 * g + 1][s] = embed_slice(w[2 * g][s], true);
+            w[2 * g][s] = embed_slice(w[2 * g][s], false);
+        }
+    // A work-group any of whose waves holds a weight wi = -128 computes its
+    // outputs on the exact path instead.  The flags pass through the
+    // thresholds' LDS before the thresholds are written there: written, a
+    // barrier, read by every wave, a barrier.
+    {
+        int* const flags = reinterpret_cast<int*>(thr);
+        const bool wave_m128 = wave_any(m128);   // every lane votes (not inside the lane-0 branch)
+        if (lane == 0) flags[wv] = wave_m128 ? 1 : 0;
+        wait_vm_lgkm0<63>();
+        block_barrier();
+        int any = 0;
+#pragma unroll
+        for (int i = 0; i < St::NW; ++i) any |= flags[i];
+        any = __builtin_amdgcn_readfirstlane(any);
+        wait_vm_lgkm0<63>();
+        block_barrier();
+        if (any) {
+            wait_vm_lgkm0<0>();   // the staging loads land before LDS is released
+            const int tend = (tgroup + 1) * NTS * slot_tiles;
+            cb_exact_outputs<MODE_INT8>(p, fo, bgroup * NWB * 16 * RT, NWB * 16 * RT,
+                                        (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
+                                        (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps, tid,
+                                        (int)blockDim.x);
+            if constexpr (IBF) {
+                if (bgroup == 0)
+                    cb_exact_ib_partials(p, ta.ibp, ta.ntiles, fo, tgroup * NTS * slot_tiles,
+                                         tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
+            }
+            return;
+        }
+    }
+
+    // Quantiser: the thresholds are visible after the tile loop's first
+    // barrier.
+    const float q_off = p.offsets[fo], q_sc = p.scales[fo];
+    const bool q_thr = thr_applies(q_off, q_sc);
+    const bool q_f32 = q_thr && thr_f32_applies(q_off, q_sc);
+    const QuantConst qz = quant_const(q_off, q_sc);
+    if (tid < kThr) thr[tid] = thr_v;
+    if (tid + 256 * NTS < kThr) thr[tid + 256 * NTS] = thr_v2;
+    const long long* const thr_mid = thr + 128;
+    // Quantise and store one pass's totals (staged [fo][to][b] int8); with
+    // FS > 1 the waves of a beam group share the totals out.
+    // Value v of a lane: slot 2v + h of beam c (RT = 2), else slot
+    // v % NSLOT of beam 64 (v / NSLOT) + 32 h + c.  The row of slot 2v
+    // (RT = 2) or v % NSLOT is wave-uniform, so its address is scalar and
+    // each lane adds a 32-bit offset (the next row for the upper half when
+    // RT = 2).
+    int8_t* const out_f = static_cast<int8_t*>(p.out) + (size_t)fo * p.nsamples_out * p.B;
+    const int b_lane = RT == 2 ? beam_base + c : beam_base + 32 * h + c;
+    const int lane_off = (RT == 2 ? h * p.B : 0) + b_lane;
+    // Output windows number below 2^31 (cb_tr_applies), so window indices
+    // compare as int: a scalar compare for the wave-uniform rows.
+    const int nout = (int)p.nsamples_out;
+    const bool all_beams = wave_active && beam_base + 16 * RT <= p.B;
+    // All of a pass's values are estimated first, then their thresholds
+    // read (the LDS reads in flight together, one wait), then stored.
+    auto store_pass = [&](const long long (&t)[VALS], int w0) {
+        int q[VALS];   // (ints: no packing into dwords before the byte stores)
+        if (q_thr) {
+            int e[VALS];
+            if (q_f32) {
+#pragma unroll
+                for (int v = 0; v < VALS; ++v) e[v] = thr_estimate_f32(t[v], qz);
+            } else {
+#pragma unroll
+                for (int v = 0; v < VALS; ++v) e[v] = thr_estimate(t[v], qz);
+            }
+#pragma unroll
+            for (int v = 0; v < VALS; ++v) q[v] = thr_settle(t[v], e[v], thr_mid);
+        } else {
+#pragma unroll
+            for (int v = 0; v < VALS; ++v) q[v] = quantise((double)t[v], q_off, q_sc, p.quant);
+        }
+        // Every beam of the wave and every window of the pass in range (the
+        // usual case, uniform over the wave): the four rows' bases are
+        // scalar and the stores need no per-store checks.
+        if constexpr (RT != 2 && FS == 1) {
+            if (all_beams && w0 + NSLOT <= nout) {
+                int8_t* const base = out_f + (size_t)w0 * p.B;
+#pragma unroll
+                for (int v = 0; v < VALS; ++v)
+                    global_ptr(uniform_ptr(base + (size_t)(v % NSLOT) * p.B + 64 * (v / NSLOT)))[(unsigned)lane_off] =
+                        q[v];
+                return;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < VALS; ++v) {
+            if (FS > 1 && v % FS != wc) continue;
+            const int row = w0 + (RT == 2 ? 2 * v : v % NSLOT);
+            const int bsh = RT == 2 ? 0 : 64 * (v / NSLOT);
+            // Uniform bounds first (a scalar branch), then the lane's.
+            if (!wave_active || row >= nout) continue;
+            if (b_lane + bsh < p.B && (RT != 2 || row + h < nout))
+                global_ptr(uniform_ptr(out_f + (size_t)row * p.B + bsh))[(unsigned)lane_off] = q[v];
+        }
+    };
+    const int prio_phase = blockIdx.x >= gridDim.x / 2 ? 1 : 0;
+    // First window of the pass; tile0 is a multiple of the slot's tiles, so
+    // the division is exact.
+    int w0_pass = tile0 * SPT / ta.tps;
+    for (int pass = 0; pass < ta.npasses; ++pass) {
+        long long pw[NG][NSLOT];
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int sl = 0; sl < NSLOT; ++sl) pw[g][sl] = 0;
+        // Passes past the end of the channel (the last slots of a one-round
+        // grid) still take part in the staging and the barriers but leave
+        // the MFMA pipe to the other waves of the SIMD.
+        const bool tiles_live = tile0 + pass * ta.ntp < ta.ntiles;
+        const bool live = wave_active && tiles_live;
+        // Incoherent-beam partials: in beam group 0, one wave of each time
+        // slot per step (whether it holds beams or not) forms the tile's.
+        // The role rotates with the step (and, with two time slots, the
+        // slot), so that a wave issues one partials store per four steps
+        // (stores count against the staging loads' vmcnt wait) and the
+        // SIMDs take turns.
+        const bool ib_live = IBF && bgroup == 0 && tiles_live;
+
+        // Tiles of the pass: NSLOT/SPT groups of tps tiles (tps = 1 unless
+        // a window spans several tiles).
+#pragma unroll
+        for (int g = 0; g < NSLOT / SPT; ++g) {
+            for (int x = 0; x < ta.tps; ++x) {
+                // Every G steps: this wave's loads of the next G sets are
+                // done once WAIT later loads remain; the barrier makes every
+                // wave's loads visible and frees the G slots read since the
+                // last barrier, which are refilled NB - G steps ahead.
+                // One-slot work-groups (two per compute unit, one wave each
+                // per SIMD): the issue arbiter favours the older wave of a
+                // SIMD, so the two work-groups take turns at a raised
+                // priority, every 16 steps in opposite phase (the halves of
+                // the grid), instead of the older one finishing first and
+                // leaving its SIMDs one wave for the rest.
+                if constexpr (NTS == 1) {
+                    if (step % 16 == 0) {
+                        if (((step >> 4) + prio_phase) & 1) __builtin_amdgcn_s_setprio(2);
+                        else __builtin_amdgcn_s_setprio(0);
+                    }
+                }
+                if (step % St::G == 0) {
+                    wait_vm_lgkm0<St::WAIT>();
+                    block_barrier();
+#pragma unroll
+                    for (int j = 0; j < St::G; ++j) {
+                        issue(step + NB - St::G + j, is);
+                        is = is + 1 == NB ? 0 : is + 1;
+                    }
+                }
+                const bool ib_now = ib_live && ((step + 2 * tsl) & 3) == (wv & 3);
+                if (live || ib_now) {
+                    const int8_t* src = ring + rs * St::SET;
+                    v4i a[KSTEPS];
+                    if constexpr (TA) {
+                        tr_operands<KSTEPS>(src + aoff[0], a);
+                    } else {
+#pragma unroll
+                        for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const v4i*>(src + aoff[s]);
+                    }
+                    if (live) detect_step<RT, KSTEPS, SPT, NSLOT>(a, w, pw, g);
+                    if constexpr (IBF) {
+                        if (ib_now) ib_tile<KSTEPS>(a, ta.ibp, ta.ntiles, p.A, fo, tile0 + pass * ta.ntp + g * ta.tps + x,
+                                                    lane);
+                    }
+                }
+                rs = rs + 1 == NB ? 0 : rs + 1;
+                ++step;
+            }
+        }
+
+        // A window's power is split over the row halves (lane and lane ^ 32):
+        // one v_permlane32_swap reduce-scatter per value, lanes below 32
+        // keeping the even beam group of each pair (RT >= 4) or the even
+        // slots (RT = 2).
+        long long tot[VALS];
+        if constexpr (RT == 2) {
+#pragma unroll
+            for (int v = 0; v < VALS; ++v) tot[v] = swap32_sum(pw[0][2 * v], pw[0][2 * v + 1]);
+        } else {
+#pragma unroll
+            for (int gp = 0; gp < NG / 2; ++gp)
+#pragma unroll
+                for (int sl = 0; sl < NSLOT; ++sl)
+                    tot[gp * NSLOT + sl] = swap32_sum(pw[2 * gp][sl], pw[2 * gp + 1][sl]);
+        }
+
+        // Sum over the fscrunch channels (one per wave of a beam group).
+        if constexpr (FS > 1) {
+#pragma unroll
+            for (int v = 0; v < VALS; ++v) red[(wv * VALS + v) * 64 + lane] = tot[v];
+            wait_vm_lgkm0<63>();
+            block_barrier();
+#pragma unroll
+            for (int v = 0; v < VALS; ++v) {
+                long long sum = 0;
+#pragma unroll
+                for (int ch = 0; ch < FS; ++ch) sum += red[((tsl * 4 + wb * FS + ch) * VALS + v) * 64 + lane];
+                tot[v] = sum;
+            }
+            wait_vm_lgkm0<63>();
+            block_barrier();
+        }
+
+        store_pass(tot, w0_pass);
+        w0_pass += NSLOT;   // a pass holds NSLOT windows (ta.ntp = NSLOT / SPT * tps tiles)
+    }
+    // The loads past the last tile are still in flight: LDS must not be
+    // released before they land.
+    wait_vm_lgkm0<0>();
+}
+
+// Launch of cb_tr_k.  Supports 8 | A (16-byte K slices; 4 | A from TAFTP,
+// whose staged rows are antennas), A <= 128, tscrunch a power of two >= 4
+// (window 8, 16, 32 or a multiple of 32 columns), fscrunch 1, 2 or 4 with
+// fscrunch * ceil(A / 16) <= 8, int8 output.
+// Windows per pass.  With 64 beams per wave and windows of 16 or more
+// columns, two windows per pass keep a wave within 128 VGPRs, so four waves
+// share a SIMD (tr_nts).  Windows of 8 columns fill a tile four times, so a
+// pass holds at least 4.
+inline int cb_tr_nslot(int rt, int W)
+{
+    if (W == 16 && rt == 4) return 2;
+    if (W <= 16) return rt == 2 ? 8 : 4;
+    return W == 32 && rt != 4 ? 4 : 2;
+}
+
+inline int cb_tr_nb(int ni) { return 60 / ni < 2 ? 2 : (60 / ni > 8 ? 8 : 60 / ni); }
+
+// Time slots per work-group of the transposed kernel: four with 64 beams
+// per wave and two windows per pass (at most 128 VGPRs a wave, four waves per
+// SIMD), one with 128 beams per wave (256 VGPRs, two work-groups and so two
+// waves per SIMD), else three.  With four waves a SIMD overlaps one wave's
+// MFMAs with the others' detection better: at 64 antennas the VALU work per
+// step outweighs the MFMA work.  With 128 beams per wave, one work-group of
+// two time slots kept its two waves of a SIMD in lockstep, and the older one
+// waited at every barrier for the younger; two one-slot work-groups with
+// alternating priority measured 2.0-2.4 % faster.
+// 64 beams per wave over more than four K steps (65 to 128 antennas) hold as
+// many weights (up to 128 VGPRs; the wave stays within 256) and take the same
+// one-slot form: at 128 antennas, 1024 beams, 64 channels, 8192 samples the
+// one-pass block took 494 us against 643 us with 32 beams per wave in
+// three-slot work-groups from a split-transposed copy.
+constexpr int tr_nts(int rt, int ksteps, int nslot)
+{
+    return rt == 8 || (rt == 4 && ksteps > 4) ? 1 : (rt == 4 && nslot == 2 ? 4 : 3);
+}
+
+inline size_t cb_tr_shm(int fs, int ksteps, int vals, int nts)
+{
+    const int nw = 4 * nts;
+    const int ni = nts * fs * ksteps;
+    return (size_t)cb_tr_nb(ni) * ni * 1024 + ((ni % nw) ? (size_t)nw * 1024 : 0) +
+           (fs > 1 ? (size_t)nw * vals * 64 * sizeof(long long) : 0) + kThrBytes;
+}
+
+inline bool cb_tr_supported(int A, int ts, int fs, int rt, bool taftp)
+{
+    if (A % (taftp ? 4 : 8) != 0 || A > 128) return false;
+    if (ts < 4 || (ts & (ts - 1)) != 0) return false;
+    if (!(fs == 1 || fs == 2 || fs == 4)) return false;
+    const int ksteps = (2 * A + 31) / 32;
+    if (rt == 8 ? (fs != 1 || ksteps > 4) : rt * ksteps > 16 && (rt != 4 || fs != 1)) return false;
+    if (fs * ksteps > 8) return false;
+    const int nslot = cb_tr_nslot(rt, 2 * ts);
+    const int vals = rt == 2 ? nslot / 2 : (rt / 4) * nslot;
+    return cb_tr_shm(fs, ksteps, vals, tr_nts(rt, ksteps, nslot)) <= 65536;
+}
+
+// Compute units of the current device (cached per device).
+inline int device_cu_count()
+{
+    static int cus[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cus[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        cus[dev] = n;
+    }
+    return cus[dev];
+}
+
+// One round of resident work-groups: every (channel group, beam group) gets
+// (resident work-groups) / (channel groups x beam groups) work-groups, each a
+// contiguous run of passes, so the per-work-group start-up (weights, the
+// first staged tiles) is paid once per resident slot and all work-groups end
+// together.
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, bool TA, bool IBF = false>
+hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
+{
+    constexpr int NTS = tr_nts(RT, KSTEPS, NSLOT);
+    const size_t shm = cb_tr_shm(FS, KSTEPS, TrRed<RT, NSLOT>::VALS, NTS);
+    static int occ = 0;
+    if (occ == 0) {
+        int o = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, TA, IBF>, 256 * NTS,
+                                                         shm) != hipSuccess ||
+            o < 1)
+            o = 1;
+        occ = o;
+    }
+    // Work-groups per (channel group, beam group): one round of resident
+    // work-groups where the problem allows; each covers NTS slots of
+    // npasses passes.
+    const long long units = (long long)a.p.Fo * a.n_bgroups;
+    long long per_unit = (long long)occ * device_cu_count() / units;
+    if (per_unit < 1) per_unit = 1;
+    const long long max_groups = (passes + NTS - 1) / NTS;
+    if (per_unit > max_groups) per_unit = max_groups;
+    a.npasses = (int)((passes + per_unit * NTS - 1) / (per_unit * NTS));
+    a.n_tgroups = (int)((passes + (long long)a.npasses * NTS - 1) / ((long long)a.npasses * NTS));
+    const long long nblocks = units * a.n_tgroups;
+    if (nblocks <= 0 || nblocks >= (1ll << 31)) return hipErrorInvalidConfiguration;
+    cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, TA, IBF><<<dim3((unsigned)nblocks), 256 * NTS, shm, s>>>(a);
+    return hipGetLastError();
+}
+
+// TAFTP staging (a.p.S > 0) is built for 64 and 128 beams per wave and
+// fscrunch 1 only (cb_taftp_direct): with 64 beams per wave no fscrunch above
+// 1 fits the kernel's LDS (cb_tr_supported).  The incoherent-beam partials
+// (a.ibp) are built for the one-slot work-groups (cb_ib_fused).
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS>
+hipError_t launch_tr_k(CbTrArgs a, int passes, hipStream_t s)
+{
+    if (a.p.S > 0) {
+        if constexpr (RT != 2 && FS == 1) {
+            if (a.ibp) {
+                if constexpr (RT == 8 || KSTEPS > 4)
+                    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, true, true>(a, passes, s);
+                return hipErrorInvalidValue;
+            }
+            return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, true>(a, passes, s);
+        }
+        return hipErrorInvalidValue;
+    }
+    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, false>(a, passes, s);
+}
+
+template <int RT, int SPT, int NSLOT, int FS>
+hipError_t launch_tr_ks(const CbTrArgs& a, int ksteps, int passes, hipStream_t s)
+{
+    if constexpr (FS * 2 <= 8) {
+        if (ksteps == 1) return launch_tr_k<RT, 1, SPT, NSLOT, FS>(a, passes, s);
+        if (ksteps == 2) return launch_tr_k<RT, 2, SPT, NSLOT, FS>(a, passes, s);
+    }
+    if constexpr (FS * 4 <= 8) {
+        if (ksteps == 3) return launch_tr_k<RT, 3, SPT, NSLOT, FS>(a, passes, s);
+        if (ksteps == 4) return launch_tr_k<RT, 4, SPT, NSLOT, FS>(a, passes, s);
+    }
+    if constexpr (FS == 1 && RT != 8) {
+        switch (ksteps) {
+        case 5: return launch_tr_k<RT, 5, SPT, NSLOT, FS>(a, passes, s);
+        case 6: return launch_tr_k<RT, 6, SPT, NSLOT, FS>(a, passes, s);
+        case 7: return launch_tr_k<RT, 7, SPT, NSLOT, FS>(a, passes, s);
+        case 8: return launch_tr_k<RT, 8, SPT, NSLOT, FS>(a, passes, s);
+        default: break;
+        }
+    }
+    return hipErrorInvalidValue;
+}
+
+template <int RT, int FS>
+hipError_t launch_tr_w(const CbTrArgs& a, int W, int ksteps, int passes, hipStream_t s)
+{
+    // Windows per pass as cb_tr_nslot
+    constexpr int small = RT == 2 ? 8 : 4;
+    if (W == 8) return launch_tr_ks<RT, 4, small, FS>(a, ksteps, passes, s);
+    if (W == 16) return launch_tr_ks<RT, 2, RT == 4 ? 2 : small, FS>(a, ksteps, passes, s);
+    if (W == 32) return launch_tr_ks<RT, 1, RT == 4 ? 2 : 4, FS>(a, ksteps, passes, s);
+    return launch_tr_ks<RT, 1, 2, FS>(a, ksteps, passes, s);
+}
+
+template <int RT>
+hipError_t launch_tr(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s)
+{
+    if constexpr (RT == 8) {
+        if (fs != 1 || ksteps > 4) return hipErrorInvalidValue;
+        return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
+    } else {
+        if (fs == 1) return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
+        if (fs == 2) return launch_tr_w<RT, 2>(a, W, ksteps, passes, s);
+        return launch_tr_w<RT, 4>(a, W, ksteps, passes, s);
+    }
+}
+
+// Windows per pass of cb_ws_k.
+inline int cb_ws_nslot(int W) { return W <= 32 ? 4 : 2; }
+
+// cb_ws_k serves 8 | A <= 64, fscrunch 1, tscrunch a power of two >= 4.
+inline bool cb_ws_supported(int A, int ts, int fs)
+{
+    return A % 8 == 0 && A <= 64 && fs == 1 && ts >= 4 && (ts & (ts - 1)) == 0;
+}
+
+}  // namespace
+}  // namespace fbf

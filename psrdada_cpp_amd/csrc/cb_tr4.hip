@@ -1,0 +1,7 @@
+// Instances of the transposed kernel (cb_tr_k) with 64 beams per wave.
+#include "cb_tr.hpp"
+
+hipError_t fbf::cb_launch_tr4(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s)
+{
+    return launch_tr<4>(a, fs, W, ksteps, passes, s);
+}

@@ -362,3 +362,24 @@ def test_cb_ib_next_weights_rejects_other_geometry(gpu, oracle):
     d_cb, d_tf = capi.DeviceBuffer(F * (S // ts) * B), capi.DeviceBuffer(ib.output_bytes(d_t.nbytes))
     with pytest.raises(capi.FbfError):
         plan.ib_beamform_taftp_next(ib, d_t, d_w, d_cb, d_tf, wp_other, d_d, 1.0, d_w)
+
+
+@pytest.mark.parametrize("A,F,nhg,B,ts,ib_ts,ib_fs", [
+    (12, 4, 2, 104, 16, 16, 1),     # one K step, half a slice padded, beams just past the direct path's line
+    (20, 4, 2, 136, 4, 4, 1),       # two K steps, four windows a tile
+    (44, 4, 2, 128, 64, 1, 1),      # three K steps
+    (60, 8, 2, 400, 16, 16, 1),     # four K steps, a partial group of beams
+    (68, 4, 3, 264, 16, 256, 1),    # five K steps: 64 beams per wave, the last wave with 8
+    (92, 4, 1, 40, 8, 16, 4),       # six K steps, one partly filled wave
+    (108, 4, 2, 256, 64, 64, 1),    # seven K steps
+    (124, 4, 2, 72, 4, 8, 1),       # eight K steps, four windows a tile
+    (128, 4, 2, 512, 32, 16, 2),    # eight whole K steps, two beam groups
+])
+def test_cb_one_pass_any_antennas(gpu, oracle, A, F, nhg, B, ts, ib_ts, ib_fs):
+    """Antennas a multiple of 4 only and above 64 on the one-pass path, the
+    automatic pick; and as a subset of a wider block from an antenna that is
+    no multiple of 4, with a few weight components of -128."""
+    _check_cb_ib(gpu, oracle, A, F, nhg, B, ts, ib_ts, ib_fs, 256, 0, True, 3100 + A + B)
+    w = unit_weights(3201 + A, F * B * A).reshape(F, B, A, 2).copy()
+    w[0, B - 1, A - 1, 1] = -128
+    _check_taftp(gpu, oracle, A + 12, A, 5, F, nhg, B, ts, 1, 128, 0, True, 3200 + A, weights=w.reshape(-1))
