@@ -638,3 +638,31 @@ def test_cb_set_levels_waits_for_work_in_flight(gpu, oracle):
     for k in range(3):
         np.testing.assert_array_equal(outs[k].download(), ref1, err_msg=f"call {k} (old levels)")
     np.testing.assert_array_equal(outs[3].download(), oracle.cb_tbtf(p, off2, sc2, ohs))
+
+
+def test_weights_equal_64_bits_off_the_half_integers(gpu):
+    """Every component whose FP64 value 127 cos, 127 sin of the reduced phase
+    lies further than 1e-4 from a half-integer equals its rounding (sincospif
+    is within a few FP32 ulp of it: below 3e-5 at amplitude 127), over phases
+    of thousands of cycles, exact eighths of a cycle, zero and NaN delays
+    (NaN: both components as sincospif's NaN gives them, 0)."""
+    capi = gpu
+    from psrdada_cpp_amd import workloads as wl
+    A, B, F = 61, 33, 21
+    d = wl.synth_delays(B, A, 4711, 2e-6, rate_max=1e-9).reshape(B, A, 2)
+    d[0, :, 0] = 0.0
+    d[0, :16, 1] = np.arange(16) / 8.0       # seconds at 1 Hz steps of frequency below
+    d[1, 3] = np.nan
+    fr = capi.channel_frequencies_f64(wl.L_BAND_CENTRE_HZ, F * wl.CHANNEL_BW_HZ, F)
+    fr[:4] = np.arange(1, 5)
+    w, ph = _weights_gpu(capi, d.reshape(-1), fr, 321.5, A, B, F)
+    ph = ph.astype(np.float64).reshape(F, B, A)
+    w = w.reshape(F, B, A, 2)
+    nan = np.isnan(ph)
+    assert nan[:, 1, 3].all() and nan.sum() == F and not w[nan].any()
+    for k, fn in enumerate((np.cos, np.sin)):
+        v = 127.0 * fn(2 * np.pi * ph[~nan])
+        off_half = np.abs(np.abs(v - np.floor(v)) - 0.5) > 1e-4
+        assert off_half.mean() > 0.99
+        np.testing.assert_array_equal(w[..., k][~nan][off_half], np.rint(v[off_half]).astype(np.int8))
+        assert np.abs(w[..., k][~nan] - np.rint(v)).max() <= 1
