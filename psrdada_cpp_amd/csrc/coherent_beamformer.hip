@@ -562,8 +562,14 @@ struct TaftpView {
     int S, Atot, a0;
     int variant;   // the kernel variant to pick from (cb_taftp_variant)
     int* ibp;      // incoherent-beam partials to leave (cb_ib_fused), or null
-    IbFinishJob ibj;   // their finish, run in the reorder's launch
-    WeightsJob wj;     // weights generated in the reorder's launch (the next block's)
+};
+
+// Work for the reorder's launch beside the reorder: the finish of the
+// incoherent-beam partials, and weights generated there (the next block's:
+// the coherent kernel has read this block's by then).
+struct TailJobs {
+    IbFinishJob ib;
+    WeightsJob weights;
 };
 
 // Validates and launches one coherent-beam kernel over T samples of voltage
@@ -572,7 +578,8 @@ struct TaftpView {
 // (the caller has checked cb_taftp_direct).
 static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T, int vstride, int voff,
                      const void* fba, size_t weights_bytes, void* out, size_t out_bytes, fbf_stream_t stream,
-                     void* workspace = nullptr, size_t workspace_bytes = 0, const TaftpView* tv = nullptr)
+                     void* workspace = nullptr, size_t workspace_bytes = 0, const TaftpView* tv = nullptr,
+                     const TailJobs& tail = TailJobs{})
 {
     FBF_REQUIRE(plan, FBF_ERR_ARG, "fbf_cb: null plan");
     FBF_REQUIRE(ftpa && fba && out, FBF_ERR_ARG, "fbf_cb: null buffer");
@@ -656,7 +663,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         if (e != hipSuccess) return hip_status(e, "cb_ws_k launch");
         e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
                                   plan->ohs),
-                        s);
+                        s, tail.ib, tail.weights);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
         return FBF_OK;
     }
@@ -709,7 +716,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         if (e != hipSuccess) return hip_status(e, "cb_tr_k launch");
         e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
                                   plan->ohs),
-                        s, tv ? tv->ibj : IbFinishJob{}, tv ? tv->wj : WeightsJob{});
+                        s, tail.ib, tail.weights);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
         return FBF_OK;
     }
@@ -774,7 +781,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
     if (mode == MODE_INT8) {
         e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
                                   plan->ohs),
-                        s);
+                        s, tail.ib, tail.weights);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
     }
     return FBF_OK;
@@ -840,9 +847,20 @@ static bool cb_taftp_direct(const fbf_cb_plan* plan, long long T, int nantennas_
            (long long)4 * nantennas_total * d.nchans * T < (1ll << 32);   // 32-bit tile offsets
 }
 
-extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes, int nantennas_total,
-                                     int start_antenna, int nsamples_per_heap, const void* fba_weights,
-                                     size_t weights_bytes, void* tbtf, size_t tbtf_bytes, fbf_stream_t stream)
+// The incoherent beam of the block formed in the split-transpose's pass.
+struct SplitIb {
+    fbf_ib_plan* plan;
+    void* tf;
+    size_t tf_bytes;
+};
+
+// fbf_cb_beamform_taftp, with work for the reorder's launch and, when the
+// block is split-transposed (all its antennas), the incoherent beam in that
+// pass.
+static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes, int nantennas_total,
+                        int start_antenna, int nsamples_per_heap, const void* fba_weights, size_t weights_bytes,
+                        void* tbtf, size_t tbtf_bytes, fbf_stream_t stream, const TailJobs& tail,
+                        const SplitIb* split_ib)
 {
     FBF_REQUIRE(plan, FBF_ERR_ARG, "fbf_cb_beamform_taftp: null plan");
     FBF_REQUIRE(taftp && fba_weights && tbtf, FBF_ERR_ARG, "fbf_cb_beamform_taftp: null buffer");
@@ -857,10 +875,9 @@ extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_
     FBF_REQUIRE((reinterpret_cast<uintptr_t>(taftp) & 15) == 0, FBF_ERR_ARG,
                 "fbf_cb_beamform_taftp: buffers must be 16-byte aligned");
     if (T == 0 || cb_taftp_direct(plan, T, nantennas_total, nsamples_per_heap)) {
-        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna, cb_taftp_variant(plan, T), nullptr,
-                           IbFinishJob{}, WeightsJob{}};
+        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna, cb_taftp_variant(plan, T), nullptr};
         return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf,
-                         tbtf_bytes, stream, nullptr, 0, T ? &tv : nullptr);
+                         tbtf_bytes, stream, nullptr, 0, T ? &tv : nullptr, tail);
     }
     // Otherwise the plan's antennas are split-transposed into the plan's FTPA
     // buffer for the FTPA kernels.  Sizes are checked before any launch.
@@ -877,11 +894,21 @@ extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_
     void* ftpa = nullptr;
     st = cb_grow(&plan->ftpa, &plan->ftpa_bytes, fbytes, static_cast<hipStream_t>(stream), &ftpa);
     if (st) return st;
-    st = fbf_split_transpose(taftp, taftp_bytes, ftpa, fbytes, nantennas_total, d.nantennas, start_antenna,
-                             d.nchans, nsamples_per_heap, stream);
+    st = split_ib ? fbf_split_transpose_ib(taftp, taftp_bytes, ftpa, fbytes, d.nchans, nsamples_per_heap,
+                                           split_ib->plan, split_ib->tf, split_ib->tf_bytes, stream)
+                  : fbf_split_transpose(taftp, taftp_bytes, ftpa, fbytes, nantennas_total, d.nantennas,
+                                        start_antenna, d.nchans, nsamples_per_heap, stream);
     if (st) return st;
     return cb_launch(plan, MODE_INT8, ftpa, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
-                     stream);
+                     stream, nullptr, 0, nullptr, tail);
+}
+
+extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes, int nantennas_total,
+                                     int start_antenna, int nsamples_per_heap, const void* fba_weights,
+                                     size_t weights_bytes, void* tbtf, size_t tbtf_bytes, fbf_stream_t stream)
+{
+    return cb_taftp_run(plan, taftp, taftp_bytes, nantennas_total, start_antenna, nsamples_per_heap, fba_weights,
+                        weights_bytes, tbtf, tbtf_bytes, stream, TailJobs{}, nullptr);
 }
 
 // Whether fbf_cb_ib_beamform_taftp forms the incoherent beam inside the
@@ -897,10 +924,9 @@ static bool cb_ib_fused(const fbf_cb_plan* plan, const IbFuseParams& ibp, long l
            ibp.nchans == d.nchans && ibp.nsamples_per_heap == S;
 }
 
-// Both beams of a TAFTP block in one pass (or one after the other where the
-// plans do not allow it); `wjob`, when it has work-groups, generates weights
-// in the reorder's launch, else `next` (a fbf_weights_generate call) runs
-// after the beams.
+// Both beams of a TAFTP block in one pass, or where the plans do not allow it
+// the incoherent beam in the split-transpose's pass or on its own; `next` (a
+// fbf_weights_generate call) runs in the reorder's launch.
 struct NextWeights {
     fbf_weights_plan* plan;
     const void* delays;
@@ -940,12 +966,30 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
         wj.nblocks = (int)(wj.w.gx * wj.w.gy);
     }
     if (T == 0 || !cb_ib_fused(plan, ibp, T, nsamples_per_heap)) {
-        // The two beamformers one after the other, then the next weights.
-        st = fbf_ib_beamform(ib_plan, taftp, taftp_bytes, tf, tf_bytes, stream);
-        if (st) return st;
-        st = fbf_cb_beamform_taftp(plan, taftp, taftp_bytes, d.nantennas, 0, nsamples_per_heap, fba_weights,
-                                   weights_bytes, tbtf, tbtf_bytes, stream);
-        if (st || !next) return st;
+        // The incoherent beam comes out of the split-transpose's pass where
+        // there is one and the plan's scrunch allows it (one read of the
+        // block and one launch less: a block of 16 antennas, 16 channels,
+        // 2048 spectra and 32 beams, which is launches and latency, took
+        // 21.4 us in five launches and takes 17.2 us in three); else it runs
+        // first.
+        const bool split_ib = T > 0 && !cb_taftp_direct(plan, T, d.nantennas, nsamples_per_heap) &&
+                              ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
+                              ibp.nsamples_per_heap == nsamples_per_heap && split_ib_applies(ibp);
+        if (split_ib) {
+            size_t tf_expect = 0;
+            st = fbf_ib_output_bytes(ib_plan, taftp_bytes, &tf_expect);
+            if (st) return st;
+            FBF_REQUIRE(tf_bytes == tf_expect, FBF_ERR_SIZE,
+                        "fbf_cb_ib_beamform_taftp: incoherent-beam output size " + std::to_string(tf_bytes) +
+                            " != expected " + std::to_string(tf_expect));
+        } else {
+            st = fbf_ib_beamform(ib_plan, taftp, taftp_bytes, tf, tf_bytes, stream);
+            if (st) return st;
+        }
+        const SplitIb sib{ib_plan, tf, tf_bytes};
+        st = cb_taftp_run(plan, taftp, taftp_bytes, d.nantennas, 0, nsamples_per_heap, fba_weights, weights_bytes,
+                          tbtf, tbtf_bytes, stream, TailJobs{IbFinishJob{}, wj}, split_ib ? &sib : nullptr);
+        if (st || !next || T > 0) return st;
         return fbf_weights_generate(next->plan, next->delays, next->delays_bytes, next->epoch, next->weights,
                                     next->weights_bytes, nullptr, stream);
     }
@@ -964,10 +1008,9 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
     IbFinishJob ibj{};
     st = ib_finish_job(ib_plan, static_cast<const int*>(part), T, tf, tf_bytes, &ibj);
     if (st) return st;
-    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_variant(plan, T), static_cast<int*>(part), ibj,
-                       wj};
+    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_variant(plan, T), static_cast<int*>(part)};
     return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
-                     stream, nullptr, 0, &tv);
+                     stream, nullptr, 0, &tv, TailJobs{ibj, wj});
 }
 
 extern "C" int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,

@@ -383,3 +383,42 @@ def test_cb_one_pass_any_antennas(gpu, oracle, A, F, nhg, B, ts, ib_ts, ib_fs):
     w = unit_weights(3201 + A, F * B * A).reshape(F, B, A, 2).copy()
     w[0, B - 1, A - 1, 1] = -128
     _check_taftp(gpu, oracle, A + 12, A, 5, F, nhg, B, ts, 1, 128, 0, True, 3200 + A, weights=w.reshape(-1))
+
+
+@pytest.mark.parametrize("A,B,ib_ts,ib_fs", [
+    (16, 32, 16, 1),     # the incoherent beam in the split-transpose's pass
+    (20, 64, 32, 1),     # antennas in fours: the LDS-staged kernel
+    (128, 32, 1, 1),     # 32 beams per wave
+    (40, 96, 64, 1),     # windows longer than the split-transpose's tiles: a pass of its own
+    (24, 40, 16, 2),     # two channels to an output channel: likewise
+])
+def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs):
+    """Blocks that are split-transposed: the coherent beams, the incoherent
+    beam and the next block's weights, written over this block's, of one call
+    equal the oracle's beams and fbf_weights_generate."""
+    capi = gpu
+    from psrdada_cpp_amd import workloads as wl
+    F, nhg, ts, S = 8, 2, 16, 256
+    T = nhg * S
+    taftp = gaussian_int8(3300 + A, nhg * A * F * S * 4, 16.0)
+    off, sc = _levels(oracle, A, ts, 1, F)
+    _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, A, ts, 1, A, ib_ts, ib_fs)
+    ioff, isc = np.full(F // ib_fs, ibo, np.float32), np.full(F // ib_fs, ibs, np.float32)
+    plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=T // ts)
+    ib = capi.IbPlan(A, F, ib_ts, ib_fs, ioff, isc)
+    assert not plan.ib_fused(ib, T, S)
+    wp = capi.WeightsPlan(A, B, F, capi.channel_frequencies_f64(wl.L_BAND_CENTRE_HZ, F * wl.CHANNEL_BW_HZ, F))
+    d_d = _dev(capi, wl.synth_delays(B, A, 3301, 1e-6, rate_max=1e-9))
+    d_w, d_next = capi.DeviceBuffer(F * B * A * 2), capi.DeviceBuffer(F * B * A * 2)
+    wp.generate(d_d, 7.5, d_w)
+    wp.generate(d_d, 8.25, d_next)
+    w = d_w.download()
+    ftpa = oracle.split_transpose(taftp, nhg, A, A, 0, F)
+    ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, T // ts)
+    ib_ref = oracle.ib_tf(oracle.ib_power(taftp, F, ib_ts, ib_fs, nhg, A), ioff, isc)
+    d_t, d_o = _dev(capi, taftp), capi.DeviceBuffer(F * (T // ts) * B)
+    d_tf = capi.DeviceBuffer(ib.output_bytes(d_t.nbytes))
+    plan.ib_beamform_taftp_next(ib, d_t, d_w, d_o, d_tf, wp, d_d, 8.25, d_w)
+    np.testing.assert_array_equal(d_o.download(), ref)
+    np.testing.assert_array_equal(d_tf.download(), ib_ref.reshape(-1))
+    np.testing.assert_array_equal(d_w.download(), d_next.download())
