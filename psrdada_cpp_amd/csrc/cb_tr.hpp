@@ -338,6 +338,19 @@ __device__ __forceinline__ void detect_step(const v4i (&a)[KSTEPS], const v4i (&
     }
 }
 
+// Tile sets in the staging ring for ni 1 KiB loads a set: within 60 KiB, or
+// 48 KiB where a one-slot work-group (two per compute unit) also holds the
+// fscrunch reduction.
+constexpr int tr_nb(int ni, int fs, int nts)
+{
+    const int n = (fs > 1 && nts == 1 ? 48 : 60) / ni;
+    return n < 2 ? 2 : (n > 8 ? 8 : n);
+}
+
+// Totals per lane that one round of the fscrunch reduction passes through
+// LDS: as many as leave a one-slot work-group's ring its 48 KiB.
+constexpr int tr_red_vals(int vals) { return vals < 4 ? vals : 4; }
+
 // Staging constants of cb_tr_k for FS channels x KSTEPS 32-byte K steps.
 template <int FS, int KSTEPS, int NTS>
 struct TrStage {
@@ -345,7 +358,7 @@ struct TrStage {
     static constexpr int NI = NTS * FS * KSTEPS;           // 1 KiB loads per set
     static constexpr int M = (NI + NW - 1) / NW;           // per wave (the rest load into a dummy run)
     static constexpr int SET = NI * 1024;                  // bytes per set
-    static constexpr int NB = 60 / NI < 2 ? 2 : (60 / NI > 8 ? 8 : 60 / NI);
+    static constexpr int NB = tr_nb(NI, FS, NTS);
     static constexpr int G = NB >= 4 ? 2 : 1;             // steps per barrier
     static constexpr int WAIT = (NB - 2 * G) * M;
     static constexpr int DUMMY = (NI % NW) ? NW * 1024 : 0;
@@ -386,7 +399,12 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     constexpr int NG = RT / 2;                     // groups of 32 beams per wave
     static_assert(RT == 2 || RT == 4 || RT == 8, "RT");
     static_assert(NSLOT % SPT == 0 && (RT != 2 || NSLOT % 2 == 0), "slots");
-    static_assert(St::M <= 2, "at most two staging loads per wave per set");
+    static_assert(St::M <= 4, "staging loads per wave per set");
+    constexpr int RV = tr_red_vals(VALS);          // totals per round of the fscrunch reduction
+    // Waves of a beam group share its totals out: value v goes to the wave of
+    // channel v % FS.
+    constexpr bool SHARE = FS > 1 && RV % FS == 0;
+    constexpr int NV = SHARE ? VALS / FS : VALS;   // values a wave quantises
     static_assert(!IBF || (TA && FS == 1 && NTS <= 2), "incoherent-beam partials");
     extern __shared__ __align__(16) int8_t lds[];
     const CbArgs& p = ta.p;
@@ -434,9 +452,7 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
         const int b = beam_base + 32 * g + c;
         const bool bvalid = b < p.B;
         const int8_t* wcol = p.fba + ((size_t)f * p.B + (bvalid ? b : p.B - 1)) * K;
-        // K % 16 == 8 (antennas a multiple of 4 only) is a TAFTP form: FTPA
-        // staging moves whole 16-byte pieces of a column.
-        if (TA && (K & 15)) {
+        if (K & 15) {   // antennas a multiple of 4 only: rows of 8-byte alignment
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) w[2 * g][s] = load_wslice<false>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
         } else {
@@ -449,17 +465,20 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     // 1 KiB run.  FTPA: the bank swizzle is chosen on the global side:
     // physical piece pp of column col holds K piece (pp + rot(col)) % PR with
     // rot(col) = col * KPAD / 256.  K pieces past the column (k >= K) re-read
-    // piece 0: the weights there are zero.  TAFTP: a tile is 16 * KSTEPS
+    // piece 0: the weights there are zero.  Where K % 16 == 8 the last piece
+    // runs 8 bytes into the next column (zero weights again), and past the
+    // block's end in its very last column: there the load starts 8 bytes
+    // early (`early`) and the operand is moved down (`tail_s`).  TAFTP: a tile is 16 * KSTEPS
     // antenna rows of 64 bytes (its 32 columns, contiguous in TAFTP), and a
     // load fills 16 rows, 4 lanes a row; rows past A re-read antenna 0.
-    const int kpieces = K / 16;
+    const int kpieces = (K + 15) / 16;
     // LDS: the channel's thresholds first (at address 0, so that a
     // threshold read takes the table's offset as its immediate), then the
     // ring, the dummy run and the fscrunch reduction.
     long long* thr = reinterpret_cast<long long*>(lds);                   // [kThr] of channel fo
     int8_t* const ring = lds + kThrBytes;
     int8_t* dummy = ring + NB * St::SET;
-    long long* red = reinterpret_cast<long long*>(dummy + St::DUMMY);   // [waves][VALS][64]
+    long long* red = reinterpret_cast<long long*>(dummy + St::DUMMY);   // [waves][RV][64]
     // A set holds one tile per (time slot, channel): tile index
     // tsl * FS + ch.  Load m of this wave fills 1 KiB of tile ti = u / KSTEPS
     // (u = wave + NW * m, the same tile for the whole wave): the channel's
@@ -467,11 +486,13 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     // swizzled K piece as a 32-bit offset.
     const int8_t* cbase[St::M];
     uint32_t goff[St::M];
+    uint32_t early[St::M];
     int gtile[St::M];
     int ldst[St::M];
 #pragma unroll
     for (int m = 0; m < St::M; ++m) {
         const int u = wv + St::NW * m;
+        early[m] = 0;
         if (u < St::NI) {
             const int ti = u / KSTEPS;
             if constexpr (TA) {
@@ -488,6 +509,7 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                 const int jj = j < kpieces ? j : 0;
                 cbase[m] = p.ftpa + (size_t)(fo * FS + ti % FS) * TP * p.vstride + p.voff;
                 goff[m] = (uint32_t)(col * p.vstride + 16 * jj);
+                early[m] = (K & 15) && fo * FS + ti % FS == p.F - 1 && col == 31 && jj == kpieces - 1 ? 8 : 0;
             }
             gtile[m] = (tgroup * NTS + ti / FS) * slot_tiles;
             ldst[m] = u * 1024;
@@ -529,8 +551,9 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                 ++tile_run[m];
                 if (tile_run[m] < ta.ntiles) toff_run[m] += (tile_run[m] & tmask) ? 64u : heap_jump;
             } else {
-                const int tt = gtile[m] + q < ta.ntiles ? gtile[m] + q : ta.ntiles - 1;
-                dma16(uniform_ptr(cbase[m] + (size_t)tt * tile_stride) + goff[m], dst);
+                const int tt = gtile[m] + q < ta.ntiles - 1 ? gtile[m] + q : ta.ntiles - 1;
+                const uint32_t off = tt == ta.ntiles - 1 ? goff[m] - early[m] : goff[m];
+                dma16(uniform_ptr(cbase[m] + (size_t)tt * tile_stride) + off, dst);
             }
         }
     };
@@ -551,6 +574,11 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
         for (int s = 0; s < KSTEPS; ++s)
             aoff[s] = ((tsl * FS + wc) * 32 + c) * KPAD + 16 * ((h * KSTEPS + s - rot + 32 * PR) % PR);
     }
+
+    // The block's last tile (FTPA, K % 16 == 8) and the slice of this lane's
+    // operands that was loaded 8 bytes early there.
+    const int tail_tile = !TA && (K & 15) && f == p.F - 1 ? ta.ntiles - 1 : -1;
+    const int tail_s = c == 31 ? K / 16 - h * KSTEPS : -1;
 
     const bool wave_active = beam_base < p.B;
 #pragma unroll
@@ -625,22 +653,22 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     const bool all_beams = wave_active && beam_base + 16 * RT <= p.B;
     // All of a pass's values are estimated first, then their thresholds
     // read (the LDS reads in flight together, one wait), then stored.
-    auto store_pass = [&](const long long (&t)[VALS], int w0) {
-        int q[VALS];   // (ints: no packing into dwords before the byte stores)
+    auto store_pass = [&](const long long (&t)[NV], int w0) {
+        int q[NV];   // (ints: no packing into dwords before the byte stores)
         if (q_thr) {
-            int e[VALS];
+            int e[NV];
             if (q_f32) {
 #pragma unroll
-                for (int v = 0; v < VALS; ++v) e[v] = thr_estimate_f32(t[v], qz);
+                for (int v = 0; v < NV; ++v) e[v] = thr_estimate_f32(t[v], qz);
             } else {
 #pragma unroll
-                for (int v = 0; v < VALS; ++v) e[v] = thr_estimate(t[v], qz);
+                for (int v = 0; v < NV; ++v) e[v] = thr_estimate(t[v], qz);
             }
 #pragma unroll
-            for (int v = 0; v < VALS; ++v) q[v] = thr_settle(t[v], e[v], thr_mid);
+            for (int v = 0; v < NV; ++v) q[v] = thr_settle(t[v], e[v], thr_mid);
         } else {
 #pragma unroll
-            for (int v = 0; v < VALS; ++v) q[v] = quantise((double)t[v], q_off, q_sc, p.quant);
+            for (int v = 0; v < NV; ++v) q[v] = quantise((double)t[v], q_off, q_sc, p.quant);
         }
         // Every beam of the wave and every window of the pass in range (the
         // usual case, uniform over the wave): the four rows' bases are
@@ -649,21 +677,22 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
             if (all_beams && w0 + NSLOT <= nout) {
                 int8_t* const base = out_f + (size_t)w0 * p.B;
 #pragma unroll
-                for (int v = 0; v < VALS; ++v)
+                for (int v = 0; v < NV; ++v)
                     global_ptr(uniform_ptr(base + (size_t)(v % NSLOT) * p.B + 64 * (v / NSLOT)))[(unsigned)lane_off] =
                         q[v];
                 return;
             }
         }
 #pragma unroll
-        for (int v = 0; v < VALS; ++v) {
-            if (FS > 1 && v % FS != wc) continue;
+        for (int k = 0; k < NV; ++k) {
+            const int v = SHARE ? k * FS + wc : k;
+            if (FS > 1 && !SHARE && v % FS != wc) continue;
             const int row = w0 + (RT == 2 ? 2 * v : v % NSLOT);
             const int bsh = RT == 2 ? 0 : 64 * (v / NSLOT);
             // Uniform bounds first (a scalar branch), then the lane's.
             if (!wave_active || row >= nout) continue;
             if (b_lane + bsh < p.B && (RT != 2 || row + h < nout))
-                global_ptr(uniform_ptr(out_f + (size_t)row * p.B + bsh))[(unsigned)lane_off] = q[v];
+                global_ptr(uniform_ptr(out_f + (size_t)row * p.B + bsh))[(unsigned)lane_off] = q[k];
         }
     };
     const int prio_phase = blockIdx.x >= gridDim.x / 2 ? 1 : 0;
@@ -728,6 +757,11 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                     } else {
 #pragma unroll
                         for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const v4i*>(src + aoff[s]);
+                        if (tile0 + pass * ta.ntp + g * ta.tps + x == tail_tile) {
+#pragma unroll
+                            for (int s = 0; s < KSTEPS; ++s)
+                                if (s == tail_s) a[s] = v4i{a[s].z, a[s].w, a[s].z, a[s].w};
+                        }
                     }
                     if (live) detect_step<RT, KSTEPS, SPT, NSLOT>(a, w, pw, g);
                     if constexpr (IBF) {
@@ -756,24 +790,32 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                     tot[gp * NSLOT + sl] = swap32_sum(pw[2 * gp][sl], pw[2 * gp + 1][sl]);
         }
 
-        // Sum over the fscrunch channels (one per wave of a beam group).
+        // Sum over the fscrunch channels (one per wave of a beam group), RV
+        // totals at a time through LDS; each wave of the group reads back
+        // the sums of the values it quantises.
         if constexpr (FS > 1) {
+            long long sum[NV];
 #pragma unroll
-            for (int v = 0; v < VALS; ++v) red[(wv * VALS + v) * 64 + lane] = tot[v];
-            wait_vm_lgkm0<63>();
-            block_barrier();
+            for (int r = 0; r < VALS; r += RV) {
 #pragma unroll
-            for (int v = 0; v < VALS; ++v) {
-                long long sum = 0;
+                for (int v = 0; v < RV; ++v) red[(wv * RV + v) * 64 + lane] = tot[r + v];
+                wait_vm_lgkm0<63>();
+                block_barrier();
 #pragma unroll
-                for (int ch = 0; ch < FS; ++ch) sum += red[((tsl * 4 + wb * FS + ch) * VALS + v) * 64 + lane];
-                tot[v] = sum;
+                for (int k = 0; k < (SHARE ? RV / FS : RV); ++k) {
+                    const int v = SHARE ? k * FS + wc : k;
+                    long long t = 0;
+#pragma unroll
+                    for (int ch = 0; ch < FS; ++ch) t += red[((tsl * 4 + wb * FS + ch) * RV + v) * 64 + lane];
+                    sum[SHARE ? r / FS + k : r + k] = t;
+                }
+                wait_vm_lgkm0<63>();
+                block_barrier();
             }
-            wait_vm_lgkm0<63>();
-            block_barrier();
+            store_pass(sum, w0_pass);
+        } else {
+            store_pass(tot, w0_pass);
         }
-
-        store_pass(tot, w0_pass);
         w0_pass += NSLOT;   // a pass holds NSLOT windows (ta.ntp = NSLOT / SPT * tps tiles)
     }
     // The loads past the last tile are still in flight: LDS must not be
@@ -781,10 +823,10 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     wait_vm_lgkm0<0>();
 }
 
-// Launch of cb_tr_k.  Supports 8 | A (16-byte K slices; 4 | A from TAFTP,
-// whose staged rows are antennas), A <= 128, tscrunch a power of two >= 4
-// (window 8, 16, 32 or a multiple of 32 columns), fscrunch 1, 2 or 4 with
-// fscrunch * ceil(A / 16) <= 8, int8 output.
+// Launch of cb_tr_k.  Supports 4 | A <= 128, tscrunch a power of two >= 4
+// (window 8, 16, 32 or a multiple of 32 columns), fscrunch 1, 2 or 4 (with
+// work-groups of several time slots fscrunch * ceil(A / 16) <= 8), int8
+// output.
 // Windows per pass.  With 64 beams per wave and windows of 16 or more
 // columns, two windows per pass keep a wave within 128 VGPRs, so four waves
 // share a SIMD (tr_nts).  Windows of 8 columns fill a tile four times, so a
@@ -795,8 +837,6 @@ inline int cb_tr_nslot(int rt, int W)
     if (W <= 16) return rt == 2 ? 8 : 4;
     return W == 32 && rt != 4 ? 4 : 2;
 }
-
-inline int cb_tr_nb(int ni) { return 60 / ni < 2 ? 2 : (60 / ni > 8 ? 8 : 60 / ni); }
 
 // Time slots per work-group of the transposed kernel: four with 64 beams
 // per wave and two windows per pass (at most 128 VGPRs a wave, four waves per
@@ -821,21 +861,22 @@ inline size_t cb_tr_shm(int fs, int ksteps, int vals, int nts)
 {
     const int nw = 4 * nts;
     const int ni = nts * fs * ksteps;
-    return (size_t)cb_tr_nb(ni) * ni * 1024 + ((ni % nw) ? (size_t)nw * 1024 : 0) +
-           (fs > 1 ? (size_t)nw * vals * 64 * sizeof(long long) : 0) + kThrBytes;
+    return (size_t)tr_nb(ni, fs, nts) * ni * 1024 + ((ni % nw) ? (size_t)nw * 1024 : 0) +
+           (fs > 1 ? (size_t)nw * tr_red_vals(vals) * 64 * sizeof(long long) : 0) + kThrBytes;
 }
 
-inline bool cb_tr_supported(int A, int ts, int fs, int rt, bool taftp)
+inline bool cb_tr_supported(int A, int ts, int fs, int rt)
 {
-    if (A % (taftp ? 4 : 8) != 0 || A > 128) return false;
+    if (A % 4 != 0 || A > 128) return false;
     if (ts < 4 || (ts & (ts - 1)) != 0) return false;
     if (!(fs == 1 || fs == 2 || fs == 4)) return false;
     const int ksteps = (2 * A + 31) / 32;
-    if (rt == 8 ? (fs != 1 || ksteps > 4) : rt * ksteps > 16 && (rt != 4 || fs != 1)) return false;
-    if (fs * ksteps > 8) return false;
+    if (rt == 8 ? ksteps > 4 : rt * ksteps > 16 && (rt != 4 || fs > 2)) return false;
     const int nslot = cb_tr_nslot(rt, 2 * ts);
+    const int nts = tr_nts(rt, ksteps, nslot);
+    if (nts > 1 && fs * ksteps > 8) return false;
     const int vals = rt == 2 ? nslot / 2 : (rt / 4) * nslot;
-    return cb_tr_shm(fs, ksteps, vals, tr_nts(rt, ksteps, nslot)) <= 65536;
+    return cb_tr_shm(fs, ksteps, vals, nts) <= 65536;
 }
 
 // Compute units of the current device (cached per device).
@@ -887,17 +928,16 @@ hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
     return hipGetLastError();
 }
 
-// TAFTP staging (a.p.S > 0) is built for 64 and 128 beams per wave and
-// fscrunch 1 only (cb_taftp_direct): with 64 beams per wave no fscrunch above
-// 1 fits the kernel's LDS (cb_tr_supported).  The incoherent-beam partials
-// (a.ibp) are built for the one-slot work-groups (cb_ib_fused).
+// TAFTP staging (a.p.S > 0) is built for 64 beams per wave at fscrunch 1 and
+// for 128 (cb_taftp_variant).  The incoherent-beam partials (a.ibp) are built
+// for the one-slot work-groups at fscrunch 1 (cb_ib_fused).
 template <int RT, int KSTEPS, int SPT, int NSLOT, int FS>
 hipError_t launch_tr_k(CbTrArgs a, int passes, hipStream_t s)
 {
     if (a.p.S > 0) {
-        if constexpr (RT != 2 && FS == 1) {
+        if constexpr (RT == 8 || (RT == 4 && FS == 1)) {
             if (a.ibp) {
-                if constexpr (RT == 8 || KSTEPS > 4)
+                if constexpr (FS == 1 && (RT == 8 || KSTEPS > 4))
                     return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, true, true>(a, passes, s);
                 return hipErrorInvalidValue;
             }
@@ -915,11 +955,11 @@ hipError_t launch_tr_ks(const CbTrArgs& a, int ksteps, int passes, hipStream_t s
         if (ksteps == 1) return launch_tr_k<RT, 1, SPT, NSLOT, FS>(a, passes, s);
         if (ksteps == 2) return launch_tr_k<RT, 2, SPT, NSLOT, FS>(a, passes, s);
     }
-    if constexpr (FS * 4 <= 8) {
+    if constexpr (RT == 8 || FS * 4 <= 8) {
         if (ksteps == 3) return launch_tr_k<RT, 3, SPT, NSLOT, FS>(a, passes, s);
         if (ksteps == 4) return launch_tr_k<RT, 4, SPT, NSLOT, FS>(a, passes, s);
     }
-    if constexpr (FS == 1 && RT != 8) {
+    if constexpr ((FS == 1 && RT == 2) || (FS <= 2 && RT == 4)) {
         switch (ksteps) {
         case 5: return launch_tr_k<RT, 5, SPT, NSLOT, FS>(a, passes, s);
         case 6: return launch_tr_k<RT, 6, SPT, NSLOT, FS>(a, passes, s);
@@ -945,23 +985,18 @@ hipError_t launch_tr_w(const CbTrArgs& a, int W, int ksteps, int passes, hipStre
 template <int RT>
 hipError_t launch_tr(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s)
 {
-    if constexpr (RT == 8) {
-        if (fs != 1 || ksteps > 4) return hipErrorInvalidValue;
-        return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
-    } else {
-        if (fs == 1) return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
-        if (fs == 2) return launch_tr_w<RT, 2>(a, W, ksteps, passes, s);
-        return launch_tr_w<RT, 4>(a, W, ksteps, passes, s);
-    }
+    if (fs == 1) return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
+    if (fs == 2) return launch_tr_w<RT, 2>(a, W, ksteps, passes, s);
+    return launch_tr_w<RT, 4>(a, W, ksteps, passes, s);
 }
 
 // Windows per pass of cb_ws_k.
 inline int cb_ws_nslot(int W) { return W <= 32 ? 4 : 2; }
 
-// cb_ws_k serves 8 | A <= 64, fscrunch 1, tscrunch a power of two >= 4.
+// cb_ws_k serves 4 | A <= 64, fscrunch 1, tscrunch a power of two >= 4.
 inline bool cb_ws_supported(int A, int ts, int fs)
 {
-    return A % 8 == 0 && A <= 64 && fs == 1 && ts >= 4 && (ts & (ts - 1)) == 0;
+    return A % 4 == 0 && A <= 64 && fs == 1 && ts >= 4 && (ts & (ts - 1)) == 0;
 }
 
 }  // namespace

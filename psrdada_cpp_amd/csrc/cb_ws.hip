@@ -54,7 +54,8 @@ struct WsStage {
     static constexpr int WAIT = (NB - 1) * LPT;
 };
 
-template <int KSTEPS, int SPT, int NSLOT>
+// AL16: K = 2A is a multiple of 16 (else of 8: antennas in fours).
+template <int KSTEPS, int SPT, int NSLOT, bool AL16>
 __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
 {
     using St = WsStage<KSTEPS>;
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
     // the work-group to the exact path (before any staging load is issued).
     const int K = 2 * p.A;
     {
-        const int kp = K / 16;
+        const int kp = (K + 15) / 16;
         const int per_unit = 64 * kp;
         bool m128 = false;
         for (int i = tid; i < U * per_unit; i += 64 * kWsWaves) {
@@ -98,8 +99,8 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
             const int r = i % per_unit;
             const int b = (gu % wa.nbg) * 64 + r / kp;
             if (gu < wa.nunits && b < p.B)
-                m128 |= raw_has_m128(
-                    *reinterpret_cast<const v4i*>(p.fba + ((size_t)unit_fo(gu) * p.B + b) * K + 16 * (r % kp)));
+                m128 |= raw_has_m128(load_wslice<AL16>(p.fba + ((size_t)unit_fo(gu) * p.B + b) * K, 16 * (r % kp), K,
+                                                        true));
         }
         const bool wave_m128 = wave_any(m128);   // every lane votes (not inside the lane-0 branch)
         if (lane == 0) m128_flags[wv] = wave_m128 ? 1 : 0;
@@ -125,14 +126,16 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
     }
 
     const size_t TP = (size_t)2 * p.nsamples;
-    const int kpieces = K / 16;
+    const int kpieces = (K + 15) / 16;
     const int chunk_tiles = wa.ct;
 
     // This lane's part of a tile load m: column and K piece (swizzled as in
     // cb_tr_k: physical piece pp of column col holds K piece
     // (pp + col * KPAD / 256) % PR; pieces past K re-read piece 0, whose
-    // weights there are zero).
+    // weights there are zero; the block's last piece is loaded 8 bytes early
+    // where K % 16 == 8).
     int goff[St::LPT];
+    int early[St::LPT];
 #pragma unroll
     for (int m = 0; m < St::LPT; ++m) {
         const int off = m * 1024 + lane * 16;
@@ -140,6 +143,7 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
         const int pp = (off - col * KPAD) >> 4;
         const int j = (pp + ((col * KPAD) >> 8)) % PR;
         goff[m] = col * p.vstride + 16 * (j < kpieces ? j : 0);
+        early[m] = !AL16 && col == 31 && j == kpieces - 1 ? 8 : 0;
     }
     int aoff[KSTEPS];
     {
@@ -177,19 +181,24 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
     const size_t tile_bytes = (size_t)32 * p.vstride;
     const int8_t* isrc = p.ftpa + p.voff;
     int ilast = 0;
+    int itail = -1;   // the block's last tile within the chunk, if it is there
     auto set_issue_chunk = [&](int d) {
         isrc = p.ftpa + p.voff;
         ilast = 0;
+        itail = p.F == 1 && wa.ntiles == 1 ? 0 : -1;
         if (d >= 0) {
             const int t0 = chunk_tile0(d);
             isrc += (size_t)unit_fo(unit0 + (d >> 24)) * TP * p.vstride + (size_t)t0 * tile_bytes;
             ilast = (wa.ntiles - t0 < chunk_tiles ? wa.ntiles - t0 : chunk_tiles) - 1;
+            itail = unit_fo(unit0 + (d >> 24)) == p.F - 1 && t0 + ilast == wa.ntiles - 1 ? ilast : -1;
         }
     };
     auto issue = [&](int off, int slot) {
-        const int8_t* src = isrc + (size_t)(off < ilast ? off : ilast) * tile_bytes;
+        const int o = off < ilast ? off : ilast;
+        const int8_t* src = isrc + (size_t)o * tile_bytes;
 #pragma unroll
-        for (int m = 0; m < St::LPT; ++m) dma16(src + (uint32_t)goff[m], ring + slot * St::TILE + m * 1024);
+        for (int m = 0; m < St::LPT; ++m)
+            dma16(src + (uint32_t)(!AL16 && o == itail ? goff[m] - early[m] : goff[m]), ring + slot * St::TILE + m * 1024);
     };
 
     int cdesc = grab();          // chunk of the compute cursor
@@ -226,7 +235,7 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
                 const int8_t* wcol = p.fba + ((size_t)fo * p.B + (bvalid ? b : p.B - 1)) * K;
 #pragma unroll
                 for (int s = 0; s < KSTEPS; ++s)
-                    w[2 * g][s] = load_wslice<true>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+                    w[2 * g][s] = load_wslice<AL16>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
             }
 #pragma unroll
             for (int g = 0; g < NG; ++g)
@@ -260,6 +269,11 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
                     v4i a[KSTEPS];
 #pragma unroll
                     for (int s = 0; s < KSTEPS; ++s) a[s] = *reinterpret_cast<const v4i*>(src + aoff[s]);
+                    if (!AL16 && fo == p.F - 1 && ctile0 + pc + g * wa.tps + x == wa.ntiles - 1) {
+#pragma unroll
+                        for (int s = 0; s < KSTEPS; ++s)
+                            if (c == 31 && h * KSTEPS + s == K / 16) a[s] = v4i{a[s].z, a[s].w, a[s].z, a[s].w};
+                    }
                     wait_vm_lgkm0<63>();
                     // The slot is free again: refill it NB positions ahead.
                     if (ioff == chunk_tiles) {
@@ -322,7 +336,10 @@ hipError_t launch_ws_k(CbWsArgs a, hipStream_t s)
     const long long nblocks = (nunits + a.U - 1) / a.U;
     const size_t shm = (size_t)kWsWaves * nb * WsStage<KSTEPS>::TILE + (size_t)a.U * (kThr * sizeof(long long) + 4) +
                        kWsWaves * sizeof(int);
-    cb_ws_k<KSTEPS, SPT, NSLOT><<<dim3((unsigned)nblocks), 64 * kWsWaves, shm, s>>>(a);
+    if (a.p.A % 8 == 0)
+        cb_ws_k<KSTEPS, SPT, NSLOT, true><<<dim3((unsigned)nblocks), 64 * kWsWaves, shm, s>>>(a);
+    else
+        cb_ws_k<KSTEPS, SPT, NSLOT, false><<<dim3((unsigned)nblocks), 64 * kWsWaves, shm, s>>>(a);
     return hipGetLastError();
 }
 

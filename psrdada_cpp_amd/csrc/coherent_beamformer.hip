@@ -481,11 +481,10 @@ constexpr int kCbVariantTr4 = 9;
 constexpr int kCbVariantWs = 10;
 constexpr int kCbVariantTr8 = 11;
 
-// `taftp`: the voltages are a TAFTP block that the kernel stages itself.
-static bool cb_tr_applies(const fbf_cb_desc& d, int rt, int mode, long long T, bool taftp)
+static bool cb_tr_applies(const fbf_cb_desc& d, int rt, int mode, long long T)
 {
     return mode == MODE_INT8 && T % 16 == 0 && 2 * T / 32 < (1ll << 31) && T / d.tscrunch < (1ll << 31) &&
-           cb_tr_supported(d.nantennas, d.tscrunch, d.fscrunch, rt, taftp);
+           cb_tr_supported(d.nantennas, d.tscrunch, d.fscrunch, rt);
 }
 
 static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
@@ -494,28 +493,33 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
            cb_ws_supported(d.nantennas, d.tscrunch, d.fscrunch);
 }
 
-// Automatic choice: up to three 32-byte K steps (48 antennas) the
-// wave-private kernel, which measured 20-85 % faster there (8 to 48
-// antennas, tscrunch 4 to 64; one exception, 32 antennas at tscrunch 4, 8 %
-// slower); else the transposed kernel with 128 beams per wave (fscrunch 1:
-// 3.2 % faster than 64 beams per wave at 64 antennas, 64 channels, 512
-// beams), else with 64 (above 64 antennas only with more than 32 beams: a
-// 64-beam wave would be half empty), else with 32 beams per wave, else the
-// LDS-staged kernel (which also serves int32 sums, power output and the geometries the
-// transposed kernels do not).
-static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, long long T, bool taftp)
+// Automatic choice.  fscrunch 1, up to three 32-byte K steps (48 antennas):
+// the wave-private kernel, which measured 20-85 % faster there than the
+// transposed kernel with 64 beams per wave (8 to 48 antennas, tscrunch 4 to
+// 64; one exception, 32 antennas at tscrunch 4, 8 % slower).  Else the
+// transposed kernel with 128 beams per wave (fscrunch 1: 3.2 % faster than 64
+// beams per wave at 64 antennas, 64 channels, 512 beams; fscrunch 2 and 4,
+// where the forms with several time slots per work-group stop at two K steps
+// of four channels: 241 us against 348 us of the LDS-staged kernel at 44
+// antennas, 1024 beams, 64 channels, 8192 samples, fscrunch 4) unless few
+// beams leave its waves empty, else with 64 (above 64 antennas only with more
+// than 32 beams: a 64-beam wave would be half empty), else with 32 beams per
+// wave, else the LDS-staged kernel (which also serves int32 sums, power output
+// and the geometries the transposed kernels do not).
+static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, long long T)
 {
     if (variant <= 0) {
         const int ksteps = (2 * d.nantennas + 31) / 32;
-        if (!taftp && ksteps <= 3 && cb_ws_applies(d, mode, T)) return kCbVariants[kCbVariantWs];
-        if (ksteps > 3 && cb_tr_applies(d, 8, mode, T, taftp)) return kCbVariants[kCbVariantTr8];
-        if ((ksteps <= 4 || d.nbeams > 32) && cb_tr_applies(d, 4, mode, T, taftp)) return kCbVariants[kCbVariantTr4];
-        if (cb_tr_applies(d, 2, mode, T, taftp)) return kCbVariants[kCbVariantTr2];
+        if (ksteps <= 3 && cb_ws_applies(d, mode, T)) return kCbVariants[kCbVariantWs];
+        if ((d.fscrunch > 1 ? d.nbeams > 96 : ksteps > 3) && cb_tr_applies(d, 8, mode, T))
+            return kCbVariants[kCbVariantTr8];
+        if ((ksteps <= 4 || d.nbeams > 32) && cb_tr_applies(d, 4, mode, T)) return kCbVariants[kCbVariantTr4];
+        if (cb_tr_applies(d, 2, mode, T)) return kCbVariants[kCbVariantTr2];
         return kCbVariants[kCbVariantLds];
     }
     const CbVariant v = kCbVariants[variant];
-    if (v.ws && !cb_ws_applies(d, mode, T)) return cb_pick_variant(d, 0, mode, T, taftp);
-    if (v.tr && !v.ws && !cb_tr_applies(d, v.rows, mode, T, taftp)) return kCbVariants[kCbVariantLds];
+    if (v.ws && !cb_ws_applies(d, mode, T)) return cb_pick_variant(d, 0, mode, T);
+    if (v.tr && !v.ws && !cb_tr_applies(d, v.rows, mode, T)) return kCbVariants[kCbVariantLds];
     return v;
 }
 
@@ -624,11 +628,11 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         }
     }
 
-    const CbVariant var = cb_pick_variant(d, tv ? tv->variant : plan->variant, mode, T, tv != nullptr);
+    const CbVariant var = cb_pick_variant(d, tv ? tv->variant : plan->variant, mode, T);
     // The timing events (fbf_cb_plan_set_timing), around the coherent kernel only.
     auto mark = [&](hipEvent_t ev) { return ev ? hipEventRecord(ev, s) : hipSuccess; };
-    FBF_REQUIRE(!tv || (var.tr && !var.ws && var.rows != 2 && d.fscrunch == 1), FBF_ERR_STATE,
-                "fbf_cb: the TAFTP input needs the transposed kernel with 64 or 128 beams per wave, fscrunch 1");
+    FBF_REQUIRE(!tv || (var.tr && !var.ws && (var.rows == 8 || (var.rows == 4 && d.fscrunch == 1))), FBF_ERR_STATE,
+                "fbf_cb: the TAFTP input needs the transposed kernel with 128 beams per wave, or 64 at fscrunch 1");
     if (var.ws) {
         CbWsArgs wa{};
         CbArgs& a = wa.p;
@@ -825,15 +829,15 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 static int cb_taftp_variant(const fbf_cb_plan* plan, long long T)
 {
     const fbf_cb_desc& d = plan->d;
-    if (d.fscrunch != 1) return 0;
     if (plan->variant > 0) {
-        const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T, true);
-        return v.tr && !v.ws && v.rows != 2 ? plan->variant : 0;
+        const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T);
+        return v.tr && !v.ws && (v.rows == 8 || (v.rows == 4 && d.fscrunch == 1)) ? plan->variant : 0;
     }
     const int ksteps = (2 * d.nantennas + 31) / 32;
-    if (ksteps > 4) return d.nbeams > 32 && cb_tr_applies(d, 4, MODE_INT8, T, true) ? kCbVariantTr4 : 0;
-    if (ksteps <= 3 && d.nbeams <= 96) return 0;
-    return cb_tr_applies(d, 8, MODE_INT8, T, true) ? kCbVariantTr8 : 0;
+    if (ksteps > 4)
+        return d.fscrunch == 1 && d.nbeams > 32 && cb_tr_applies(d, 4, MODE_INT8, T) ? kCbVariantTr4 : 0;
+    if ((ksteps <= 3 || d.fscrunch > 1) && d.nbeams <= 96) return 0;
+    return cb_tr_applies(d, 8, MODE_INT8, T) ? kCbVariantTr8 : 0;
 }
 
 // Whether fbf_cb_beamform_taftp stages the TAFTP block itself: such a
@@ -920,7 +924,7 @@ static bool cb_ib_fused(const fbf_cb_plan* plan, const IbFuseParams& ibp, long l
     const fbf_cb_desc& d = plan->d;
     if (!cb_taftp_direct(plan, T, d.nantennas, S)) return false;
     const int rows = kCbVariants[cb_taftp_variant(plan, T)].rows;
-    return (rows == 8 || (2 * d.nantennas + 31) / 32 > 4) && ibp.nantennas == d.nantennas &&
+    return d.fscrunch == 1 && (rows == 8 || (2 * d.nantennas + 31) / 32 > 4) && ibp.nantennas == d.nantennas &&
            ibp.nchans == d.nchans && ibp.nsamples_per_heap == S;
 }
 

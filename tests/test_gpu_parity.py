@@ -666,3 +666,38 @@ def test_weights_equal_64_bits_off_the_half_integers(gpu):
         assert off_half.mean() > 0.99
         np.testing.assert_array_equal(w[..., k][~nan][off_half], np.rint(v[off_half]).astype(np.int8))
         assert np.abs(w[..., k][~nan] - np.rint(v)).max() <= 1
+
+
+@pytest.mark.parametrize("variant", [0, 8, 9, 10, 11])
+@pytest.mark.parametrize("F,T,A,B,ts,fs", [
+    (1, 16, 4, 8, 16, 1),          # one tile of one channel: its last piece ends the block
+    (2, 144, 36, 24, 16, 1),       # nine tiles, half a slice in the last K step
+    (3, 1040, 20, 72, 4, 1),       # two K steps, four windows a tile
+    (4, 1024, 44, 264, 16, 4),     # four channels an output channel, antennas in fours
+    (8, 512, 12, 104, 32, 2), (4, 512, 60, 136, 64, 2), (4, 512, 64, 128, 8, 4),
+    (2, 256, 100, 72, 8, 1),       # seven K steps, 64 beams per wave
+    (4, 256, 124, 200, 4, 2),      # eight K steps at fscrunch 2
+])
+def test_cb_antennas_in_fours_bit_exact(gpu, oracle, variant, F, T, A, B, ts, fs):
+    """FTPA columns of 8-byte granularity and fscrunch 2 and 4 on the
+    transposed and wave-private kernels, from a block that ends with the last
+    column and in place from a wider block."""
+    capi = gpu
+    rng = np.random.default_rng(6100 + A + F)
+    ftpa = gaussian_int8(6100 + A + F, F * T * 2 * A * 2, 24.0)
+    w = rng.integers(-127, 128, F * B * A * 2).astype(np.int8)
+    off, sc = _levels(oracle, A, ts, fs, F)
+    ohs = T // ts
+    plan = capi.CbPlan(A, B, F, ts, fs, off, sc, nsamples_per_heap_out=ohs)
+    plan.set_variant(variant)
+    ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, fs), off, sc, ohs)
+    d_w, d_o = _dev(capi, w), capi.DeviceBuffer((F // fs) * ohs * B)
+    d_o.fill(0x5A)
+    plan.beamform(_dev(capi, ftpa), d_w, d_o)
+    np.testing.assert_array_equal(d_o.download(), ref)
+    a0 = 4 if A % 8 else 8
+    blk = rng.integers(-127, 128, F * T * 2 * (A + a0) * 2).astype(np.int8).reshape(F, T * 2, (A + a0) * 2)
+    blk[:, :, 2 * a0:] = ftpa.reshape(F, T * 2, A * 2)
+    d_o.fill(0x5A)
+    plan.beamform_subarray(_dev(capi, blk.reshape(-1)), A + a0, a0, d_w, d_o)
+    np.testing.assert_array_equal(d_o.download(), ref)
