@@ -196,20 +196,21 @@ int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_block, size_t b
  * copy is written; otherwise the call split-transposes into an FTPA buffer
  * that the plan owns (grown on demand, as the staging buffer) first.  As
  * with fbf_cb_beamform, calls with one plan on different streams must not
- * overlap (they share the plan's buffers).  The automatic variant picks the
- * transposed kernel with 128 beams per wave up to 64 antennas and with 64
- * above, and the split-transpose where few beams would leave such waves
- * empty (up to 48 antennas with at most 96 beams, above 64 with at most
- * 32). */
+ * overlap (they share the plan's buffers).  The automatic variant stages the
+ * block itself with 128 beams per wave up to 64 antennas (32 or 64 for at
+ * most so many beams) and with 64 above; a subset of at most 48 antennas with
+ * at most 96 beams, and more than 64 antennas with at most 32, are
+ * split-transposed. */
 int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes,
                           int nantennas_total, int start_antenna, int nsamples_per_heap,
                           const void* fba_weights, size_t weights_bytes,
                           void* tbtf, size_t tbtf_bytes, fbf_stream_t stream);
 /* *direct = 1 when fbf_cb_beamform_taftp reads a block of this geometry
- * without the FTPA copy: the plan's kernel is the transposed one with 64 or
- * 128 beams per wave, fscrunch 1, nsamples_per_heap a power of two >= 16,
- * one heap group under 2 GiB and the block under 4 GiB.  No counterpart in
- * the reference. */
+ * without the FTPA copy: the plan's kernel is a transposed one that stages
+ * TAFTP (64 beams per wave at fscrunch 1, 128 also at 2 and 4; automatic:
+ * see fbf_cb_beamform_taftp), nsamples_per_heap a power of two >= 16, one
+ * heap group under 2 GiB and the block under 4 GiB.  No counterpart in the
+ * reference. */
 int fbf_cb_taftp_direct(const fbf_cb_plan* plan, int nantennas_total, int nsamples_per_heap,
                         long long nsamples, int* direct);
 /* Timing of the coherent kernel alone: every later beamform call with this
@@ -274,9 +275,11 @@ int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void
                              int nsamples_per_heap, const void* fba_weights, size_t weights_bytes,
                              void* tbtf, size_t tbtf_bytes, void* tf, size_t tf_bytes, fbf_stream_t stream);
 /* *fused = 1 when fbf_cb_ib_beamform_taftp forms the incoherent beam inside
- * the coherent kernel: the direct TAFTP path with 128 beams per wave (or 64
- * above 64 antennas), and an incoherent-beam plan of the same antennas,
- * channels and heap size.  No counterpart in the reference. */
+ * the coherent kernel: fscrunch 1, the block staged by that kernel (every
+ * automatic pick; 128 beams per wave, or 64 above 64 antennas) and an
+ * incoherent-beam plan of the same antennas, channels and heap size (up to
+ * 48 antennas with at most 96 beams one of fscrunch 1).  No counterpart in
+ * the reference. */
 int fbf_cb_ib_fused(const fbf_cb_plan* plan, const fbf_ib_plan* ib_plan, int nsamples_per_heap,
                     long long nsamples, int* fused);
 

@@ -66,10 +66,12 @@ struct CbWsArgs {
 };
 
 // The kernels' launchers, one translation unit each (the template instances
-// compile side by side): cb_tr2/4/8.hip, cb_ws.hip and cb_lds.hip.
+// compile side by side): cb_tr2, cb_tr4, cb_tr8, cb_tr8_fs, cb_tr_few, cb_ws and cb_lds.
 hipError_t cb_launch_tr2(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s);
 hipError_t cb_launch_tr4(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s);
-hipError_t cb_launch_tr8(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s);
+hipError_t cb_launch_tr8(const CbTrArgs& a, int W, int ksteps, int passes, hipStream_t s);
+hipError_t cb_launch_tr8_fs(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s);
+hipError_t cb_launch_tr_few(const CbTrArgs& a, int rt, int W, int ksteps, int passes, hipStream_t s);
 hipError_t cb_launch_ws(const CbWsArgs& a, int W, int ksteps, hipStream_t s);
 hipError_t cb_launch_lds(const CbArgs& a, int mode, int rt, int ksteps, int jc, dim3 grid, hipStream_t s);
 hipError_t cb_launch_mfma32(const CbArgs& a, int mode, int rt, int ksteps, dim3 grid, hipStream_t s);

@@ -338,27 +338,34 @@ __device__ __forceinline__ void detect_step(const v4i (&a)[KSTEPS], const v4i (&
     }
 }
 
-// Tile sets in the staging ring for ni 1 KiB loads a set: within 60 KiB, or
-// 48 KiB where a one-slot work-group (two per compute unit) also holds the
-// fscrunch reduction.
-constexpr int tr_nb(int ni, int fs, int nts)
+// Four-wave work-groups per compute unit (waves per SIMD): two with 128 beams
+// per wave or more than four K steps (256 VGPRs a wave), else three.
+constexpr int tr_wgs(int rt, int ksteps) { return rt == 8 || ksteps > 4 ? 2 : 3; }
+
+// Tile sets in the staging ring for ni 1 KiB loads a set: within 60 KiB; in a
+// four-wave work-group less the dummy run and, with fscrunch, the 8 KiB of
+// its reduction (48 KiB keep whole sets of 16), and within 48 KiB where three
+// share a compute unit.
+constexpr int tr_nb(int rt, int ksteps, int ni, int fs, int nw)
 {
-    const int n = (fs > 1 && nts == 1 ? 48 : 60) / ni;
+    const int kib = nw > 4 ? 60 : (fs > 1 || tr_wgs(rt, ksteps) > 2 ? 48 : 60) - (ni % nw ? nw : 0);
+    const int n = kib / ni;
     return n < 2 ? 2 : (n > 8 ? 8 : n);
 }
 
 // Totals per lane that one round of the fscrunch reduction passes through
-// LDS: as many as leave a one-slot work-group's ring its 48 KiB.
+// LDS: as many as leave a four-wave work-group's ring its 48 KiB.
 constexpr int tr_red_vals(int vals) { return vals < 4 ? vals : 4; }
 
-// Staging constants of cb_tr_k for FS channels x KSTEPS 32-byte K steps.
-template <int FS, int KSTEPS, int NTS>
+// Staging constants of cb_tr_k for NTS time slots x FS channels x KSTEPS
+// 32-byte K steps and NWB beam groups.
+template <int RT, int FS, int KSTEPS, int NTS, int NWB>
 struct TrStage {
-    static constexpr int NW = 4 * NTS;                     // waves per work-group
+    static constexpr int NW = NTS * NWB * FS;              // waves per work-group
     static constexpr int NI = NTS * FS * KSTEPS;           // 1 KiB loads per set
     static constexpr int M = (NI + NW - 1) / NW;           // per wave (the rest load into a dummy run)
     static constexpr int SET = NI * 1024;                  // bytes per set
-    static constexpr int NB = tr_nb(NI, FS, NTS);
+    static constexpr int NB = tr_nb(RT, KSTEPS, NI, FS, NW);
     static constexpr int G = NB >= 4 ? 2 : 1;             // steps per barrier
     static constexpr int WAIT = (NB - 2 * G) * M;
     static constexpr int DUMMY = (NI % NW) ? NW * 1024 : 0;
@@ -372,26 +379,27 @@ struct TrRed {
 
 // RT: beam tiles per wave (RT / 2 groups of 32 beams, a Re and an Im tile
 // each); SPT: windows per tile (1, 2, 4); NSLOT: windows
-// per pass held in registers; FS: fscrunch; NTS: time slots per work-group;
+// per pass held in registers; FS: fscrunch; NTS: time slots and NWB: beam
+// groups (of 16 RT beams) per work-group;
 // TA: the voltages are a TAFTP block (CbArgs::S > 0), staged straight into
 // [antenna][column] tiles and read with transposed LDS loads (tr_operands),
 // else FTPA columns; IBF (with TA, FS = 1, all antennas of the block): the
 // work-groups of beam group 0 also leave the incoherent beam's per-sample
 // partials (CbTrArgs::ibp) from the same operands.
 //
-// A work-group has 4 * NTS waves: NTS time slots (contiguous runs of passes
-// of the same channel group and beams) x 4 waves ((4 / FS) beam groups x FS
-// channels).  With 64 beams per wave a work-group holds every wave of its
-// compute unit (NTS = tr_nts waves per SIMD: 3 or 4), so the per-step
+// A work-group has NTS x NWB x FS waves: NTS time slots (contiguous runs of
+// passes of the same channel group and beams) of NWB beam groups x FS
+// channels.  With 64 beams per wave a work-group holds every wave of its
+// compute unit (4 NTS = 12 or 16), so the per-step
 // barrier keeps them in lockstep: waves of separate work-groups sharing a
 // SIMD progress at different rates (the issue arbiter prefers older waves),
 // which leaves SIMDs with one wave at the end.  With 128 beams per wave
-// (two waves per SIMD) a work-group is one time slot, two share a compute
+// (two waves per SIMD) a work-group is four waves, two share a compute
 // unit, and they take turns at a raised wave priority instead.
-template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, bool TA, bool IBF>
-__global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs ta)
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF>
+__global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(RT, KSTEPS) : 1) void cb_tr_k(CbTrArgs ta)
 {
-    using St = TrStage<FS, KSTEPS, NTS>;
+    using St = TrStage<RT, FS, KSTEPS, NTS, NWB>;
     constexpr int KPAD = 32 * KSTEPS;
     constexpr int PR = 2 * KSTEPS;                 // 16-byte pieces per LDS column
     constexpr int VALS = TrRed<RT, NSLOT>::VALS;
@@ -399,13 +407,13 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     constexpr int NG = RT / 2;                     // groups of 32 beams per wave
     static_assert(RT == 2 || RT == 4 || RT == 8, "RT");
     static_assert(NSLOT % SPT == 0 && (RT != 2 || NSLOT % 2 == 0), "slots");
-    static_assert(St::M <= 4, "staging loads per wave per set");
+    static_assert(St::M <= 4 && St::WAIT >= 0, "staging loads per wave per set");
     constexpr int RV = tr_red_vals(VALS);          // totals per round of the fscrunch reduction
     // Waves of a beam group share its totals out: value v goes to the wave of
     // channel v % FS.
     constexpr bool SHARE = FS > 1 && RV % FS == 0;
     constexpr int NV = SHARE ? VALS / FS : VALS;   // values a wave quantises
-    static_assert(!IBF || (TA && FS == 1 && NTS <= 2), "incoherent-beam partials");
+    static_assert(!IBF || (TA && FS == 1), "incoherent-beam partials");
     extern __shared__ __align__(16) int8_t lds[];
     const CbArgs& p = ta.p;
 
@@ -415,10 +423,11 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     const int wv = __builtin_amdgcn_readfirstlane(wave);
     const int h = lane >> 5;
     const int c = lane & 31;
-    const int tsl = wv >> 2;         // time slot
-    const int wc = (wv & 3) % FS;    // channel of the fscrunch group
-    const int wb = (wv & 3) / FS;    // beam group within the work-group
-    constexpr int NWB = 4 / FS;
+    constexpr int WPS = NWB * FS;                 // waves per time slot
+    constexpr int NTHR = 64 * St::NW;
+    const int tsl = wv / WPS;                     // time slot
+    const int wc = (wv - tsl * WPS) % FS;         // channel of the fscrunch group
+    const int wb = (wv - tsl * WPS) / FS;         // beam group within the work-group
 
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int bgroup = logical % ta.n_bgroups;
@@ -436,11 +445,11 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
 
     // Start-up loads first, all in flight together: the channel's quantiser
     // thresholds (to LDS below), the weights, then the first staged tiles.
-    // One threshold per thread, two for the first threads of a one-slot
+    // One threshold per thread, two for the first threads of a four-wave
     // work-group (256 threads, kThr = 257).
-    static_assert(512 * NTS >= kThr, "at most two thresholds per thread");
+    static_assert(2 * NTHR >= kThr, "at most two thresholds per thread");
     const long long thr_v = tid < kThr ? p.thr[(size_t)fo * kThr + tid] : 0;
-    const long long thr_v2 = tid + 256 * NTS < kThr ? p.thr[(size_t)fo * kThr + tid + 256 * NTS] : 0;
+    const long long thr_v2 = tid + NTHR < kThr ? p.thr[(size_t)fo * kThr + tid + NTHR] : 0;
 
     // Weights (B operand).  Tile r holds the Re (r even) or Im (r odd)
     // embedding rows of the 32 beams beam_base + 32 (r / 2) + n, n = lane %
@@ -635,7 +644,7 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
     const bool q_f32 = q_thr && thr_f32_applies(q_off, q_sc);
     const QuantConst qz = quant_const(q_off, q_sc);
     if (tid < kThr) thr[tid] = thr_v;
-    if (tid + 256 * NTS < kThr) thr[tid + 256 * NTS] = thr_v2;
+    if (tid + NTHR < kThr) thr[tid + NTHR] = thr_v2;
     const long long* const thr_mid = thr + 128;
     // Quantise and store one pass's totals (staged [fo][to][b] int8); with
     // FS > 1 the waves of a beam group share the totals out.
@@ -727,13 +736,13 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                 // done once WAIT later loads remain; the barrier makes every
                 // wave's loads visible and frees the G slots read since the
                 // last barrier, which are refilled NB - G steps ahead.
-                // One-slot work-groups (two per compute unit, one wave each
+                // Four-wave work-groups (two per compute unit, one wave each
                 // per SIMD): the issue arbiter favours the older wave of a
                 // SIMD, so the two work-groups take turns at a raised
                 // priority, every 16 steps in opposite phase (the halves of
                 // the grid), instead of the older one finishing first and
                 // leaving its SIMDs one wave for the rest.
-                if constexpr (NTS == 1) {
+                if constexpr (St::NW == 4) {
                     if (step % 16 == 0) {
                         if (((step >> 4) + prio_phase) & 1) __builtin_amdgcn_s_setprio(2);
                         else __builtin_amdgcn_s_setprio(0);
@@ -748,7 +757,7 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                         is = is + 1 == NB ? 0 : is + 1;
                     }
                 }
-                const bool ib_now = ib_live && ((step + 2 * tsl) & 3) == (wv & 3);
+                const bool ib_now = ib_live && (step + 2 * tsl) % WPS == wv - tsl * WPS;
                 if (live || ib_now) {
                     const int8_t* src = ring + rs * St::SET;
                     v4i a[KSTEPS];
@@ -806,7 +815,7 @@ __global__ __launch_bounds__(256 * NTS, NTS == 1 ? 2 : 1) void cb_tr_k(CbTrArgs 
                     const int v = SHARE ? k * FS + wc : k;
                     long long t = 0;
 #pragma unroll
-                    for (int ch = 0; ch < FS; ++ch) t += red[((tsl * 4 + wb * FS + ch) * RV + v) * 64 + lane];
+                    for (int ch = 0; ch < FS; ++ch) t += red[((tsl * WPS + wb * FS + ch) * RV + v) * 64 + lane];
                     sum[SHARE ? r / FS + k : r + k] = t;
                 }
                 wait_vm_lgkm0<63>();
@@ -838,30 +847,55 @@ inline int cb_tr_nslot(int rt, int W)
     return W == 32 && rt != 4 ? 4 : 2;
 }
 
-// Time slots per work-group of the transposed kernel: four with 64 beams
-// per wave and two windows per pass (at most 128 VGPRs a wave, four waves per
-// SIMD), one with 128 beams per wave (256 VGPRs, two work-groups and so two
+// Whether a form of the transposed kernel has four-wave work-groups, two per
+// compute unit: 128 beams per wave (256 VGPRs, two waves per SIMD), and 64
+// beams per wave over more than four K steps (65 to 128 antennas), which
+// holds as many weights (up to 128 VGPRs; the wave stays within 256).  With
+// 128 beams per wave, one work-group of two time slots kept its two waves of a
+// SIMD in lockstep, and the older one waited at every barrier for the
+// younger; two work-groups with alternating priority measured 2.0-2.4 %
+// faster.  At 128 antennas, 1024 beams, 64 channels, 8192 samples the one-pass
+// block took 494 us with 64 beams per wave against 643 us with 32 in
+// three-slot work-groups from a split-transposed copy.
+//
+// The other forms have one work-group per compute unit: four time slots with
+// 64 beams per wave and two windows per pass (at most 128 VGPRs a wave, four
 // waves per SIMD), else three.  With four waves a SIMD overlaps one wave's
 // MFMAs with the others' detection better: at 64 antennas the VALU work per
-// step outweighs the MFMA work.  With 128 beams per wave, one work-group of
-// two time slots kept its two waves of a SIMD in lockstep, and the older one
-// waited at every barrier for the younger; two one-slot work-groups with
-// alternating priority measured 2.0-2.4 % faster.
-// 64 beams per wave over more than four K steps (65 to 128 antennas) hold as
-// many weights (up to 128 VGPRs; the wave stays within 256) and take the same
-// one-slot form: at 128 antennas, 1024 beams, 64 channels, 8192 samples the
-// one-pass block took 494 us against 643 us with 32 beams per wave in
-// three-slot work-groups from a split-transposed copy.
-constexpr int tr_nts(int rt, int ksteps, int nslot)
+// step outweighs the MFMA work.
+constexpr bool tr_four_waves(int rt, int ksteps) { return rt == 8 || (rt == 4 && ksteps > 4); }
+
+// Beam groups per four-wave work-group: 4 / fs, or fewer (and as many more
+// time slots) where that many would leave waves without beams.  Fewer beam
+// groups stage each tile for fewer waves, so they have to win a tenth, and
+// over more than four K steps the ring holds two time slots at most.
+constexpr int tr_nwb_min(int ksteps) { return ksteps > 4 ? 2 : 1; }
+
+inline int tr_nwb(int rt, int ksteps, int fs, int B)
 {
-    return rt == 8 || (rt == 4 && ksteps > 4) ? 1 : (rt == 4 && nslot == 2 ? 4 : 3);
+    const int groups = (B + 16 * rt - 1) / (16 * rt);
+    int best = 4 / fs, cost = (groups + best - 1) / best * best;   // wave slots taken
+    for (int n = best / 2; n >= tr_nwb_min(ksteps); n /= 2) {
+        const int c = (groups + n - 1) / n * n;
+        if (10 * c <= 9 * cost) {
+            best = n;
+            cost = c;
+        }
+    }
+    return best;
 }
 
-inline size_t cb_tr_shm(int fs, int ksteps, int vals, int nts)
+// Time slots per work-group.
+constexpr int tr_nts(int rt, int ksteps, int nslot, int fs, int nwb)
 {
-    const int nw = 4 * nts;
+    return tr_four_waves(rt, ksteps) ? 4 / (fs * nwb) : (rt == 4 && nslot == 2 ? 4 : 3);
+}
+
+inline size_t cb_tr_shm(int rt, int fs, int ksteps, int vals, int nts, int nwb)
+{
+    const int nw = nts * nwb * fs;
     const int ni = nts * fs * ksteps;
-    return (size_t)tr_nb(ni, fs, nts) * ni * 1024 + ((ni % nw) ? (size_t)nw * 1024 : 0) +
+    return (size_t)tr_nb(rt, ksteps, ni, fs, nw) * ni * 1024 + ((ni % nw) ? (size_t)nw * 1024 : 0) +
            (fs > 1 ? (size_t)nw * tr_red_vals(vals) * 64 * sizeof(long long) : 0) + kThrBytes;
 }
 
@@ -872,11 +906,11 @@ inline bool cb_tr_supported(int A, int ts, int fs, int rt)
     if (!(fs == 1 || fs == 2 || fs == 4)) return false;
     const int ksteps = (2 * A + 31) / 32;
     if (rt == 8 ? ksteps > 4 : rt * ksteps > 16 && (rt != 4 || fs > 2)) return false;
+    if (tr_four_waves(rt, ksteps)) return true;   // their rings are sized to fit
+    if (fs * ksteps > 8) return false;
     const int nslot = cb_tr_nslot(rt, 2 * ts);
-    const int nts = tr_nts(rt, ksteps, nslot);
-    if (nts > 1 && fs * ksteps > 8) return false;
     const int vals = rt == 2 ? nslot / 2 : (rt / 4) * nslot;
-    return cb_tr_shm(fs, ksteps, vals, nts) <= 65536;
+    return cb_tr_shm(rt, fs, ksteps, vals, tr_nts(rt, ksteps, nslot, fs, 4 / fs), 4 / fs) <= 65536;
 }
 
 // Compute units of the current device (cached per device).
@@ -898,17 +932,19 @@ inline int device_cu_count()
 // contiguous run of passes, so the per-work-group start-up (weights, the
 // first staged tiles) is paid once per resident slot and all work-groups end
 // together.
-template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, bool TA, bool IBF = false>
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF = false>
 hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
 {
-    constexpr int NTS = tr_nts(RT, KSTEPS, NSLOT);
-    const size_t shm = cb_tr_shm(FS, KSTEPS, TrRed<RT, NSLOT>::VALS, NTS);
+    constexpr int NTHR = 64 * NTS * NWB * FS;
+    constexpr auto kernel = cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, TA, IBF>;
+    const size_t shm = cb_tr_shm(RT, FS, KSTEPS, TrRed<RT, NSLOT>::VALS, NTS, NWB);
+    if (shm > 65536) return hipErrorInvalidConfiguration;
+    constexpr int beams_per_wg = 16 * RT * NWB;
+    a.n_bgroups = (a.p.B + beams_per_wg - 1) / beams_per_wg;
     static int occ = 0;
     if (occ == 0) {
         int o = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, TA, IBF>, 256 * NTS,
-                                                         shm) != hipSuccess ||
-            o < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel, NTHR, shm) != hipSuccess || o < 1)
             o = 1;
         occ = o;
     }
@@ -924,28 +960,42 @@ hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
     a.n_tgroups = (int)((passes + (long long)a.npasses * NTS - 1) / ((long long)a.npasses * NTS));
     const long long nblocks = units * a.n_tgroups;
     if (nblocks <= 0 || nblocks >= (1ll << 31)) return hipErrorInvalidConfiguration;
-    cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, TA, IBF><<<dim3((unsigned)nblocks), 256 * NTS, shm, s>>>(a);
+    kernel<<<dim3((unsigned)nblocks), NTHR, shm, s>>>(a);
     return hipGetLastError();
 }
 
 // TAFTP staging (a.p.S > 0) is built for 64 beams per wave at fscrunch 1 and
-// for 128 (cb_taftp_variant).  The incoherent-beam partials (a.ibp) are built
-// for the one-slot work-groups at fscrunch 1 (cb_ib_fused).
-template <int RT, int KSTEPS, int SPT, int NSLOT, int FS>
-hipError_t launch_tr_k(CbTrArgs a, int passes, hipStream_t s)
+// for 128 (cb_taftp_form).  The incoherent-beam partials (a.ibp) are built
+// for the four-wave work-groups at fscrunch 1 (cb_ib_fused).
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NWB>
+hipError_t launch_tr_kn(const CbTrArgs& a, int passes, hipStream_t s)
 {
+    constexpr int NTS = tr_nts(RT, KSTEPS, NSLOT, FS, NWB);
     if (a.p.S > 0) {
         if constexpr (RT == 8 || (RT == 4 && FS == 1)) {
             if (a.ibp) {
-                if constexpr (FS == 1 && (RT == 8 || KSTEPS > 4))
-                    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, true, true>(a, passes, s);
+                if constexpr (FS == 1 && tr_four_waves(RT, KSTEPS))
+                    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, true, true>(a, passes, s);
                 return hipErrorInvalidValue;
             }
-            return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, true>(a, passes, s);
+            return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, true>(a, passes, s);
         }
         return hipErrorInvalidValue;
     }
-    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, false>(a, passes, s);
+    return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, false>(a, passes, s);
+}
+
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS>
+hipError_t launch_tr_k(const CbTrArgs& a, int passes, hipStream_t s)
+{
+    if constexpr (tr_four_waves(RT, KSTEPS)) {
+        const int nwb = tr_nwb(RT, KSTEPS, FS, a.p.B);
+        if constexpr (FS <= 2 && tr_nwb_min(KSTEPS) == 1)
+            if (nwb == 1) return launch_tr_kn<RT, KSTEPS, SPT, NSLOT, FS, 1>(a, passes, s);
+        if constexpr (FS == 1)
+            if (nwb == 2) return launch_tr_kn<RT, KSTEPS, SPT, NSLOT, FS, 2>(a, passes, s);
+    }
+    return launch_tr_kn<RT, KSTEPS, SPT, NSLOT, FS, 4 / FS>(a, passes, s);
 }
 
 template <int RT, int SPT, int NSLOT, int FS>
@@ -980,14 +1030,6 @@ hipError_t launch_tr_w(const CbTrArgs& a, int W, int ksteps, int passes, hipStre
     if (W == 16) return launch_tr_ks<RT, 2, RT == 4 ? 2 : small, FS>(a, ksteps, passes, s);
     if (W == 32) return launch_tr_ks<RT, 1, RT == 4 ? 2 : 4, FS>(a, ksteps, passes, s);
     return launch_tr_ks<RT, 1, 2, FS>(a, ksteps, passes, s);
-}
-
-template <int RT>
-hipError_t launch_tr(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s)
-{
-    if (fs == 1) return launch_tr_w<RT, 1>(a, W, ksteps, passes, s);
-    if (fs == 2) return launch_tr_w<RT, 2>(a, W, ksteps, passes, s);
-    return launch_tr_w<RT, 4>(a, W, ksteps, passes, s);
 }
 
 // Windows per pass of cb_ws_k.

@@ -3,5 +3,7 @@
 
 hipError_t fbf::cb_launch_tr4(const CbTrArgs& a, int fs, int W, int ksteps, int passes, hipStream_t s)
 {
-    return launch_tr<4>(a, fs, W, ksteps, passes, s);
+    if (fs == 1) return launch_tr_w<4, 1>(a, W, ksteps, passes, s);
+    if (fs == 2) return launch_tr_w<4, 2>(a, W, ksteps, passes, s);
+    return launch_tr_w<4, 4>(a, W, ksteps, passes, s);
 }

@@ -562,9 +562,17 @@ extern "C" int fbf_cb_output_bytes(const fbf_cb_plan* plan, size_t ftpa_bytes, s
 
 // A TAFTP block read directly by the coherent beamformer: S samples per
 // heap, Atot antennas, the beamformer's antennas from antenna a0.
+// The transposed kernel that stages a TAFTP block itself: RT beam tiles (16
+// RT beams) per wave, 0 where none does; `few`: the form with one wave per
+// time slot for at most 64 beams (cb_tr_few.hip).
+struct TaftpForm {
+    int rt;
+    bool few;
+};
+
 struct TaftpView {
     int S, Atot, a0;
-    int variant;   // the kernel variant to pick from (cb_taftp_variant)
+    TaftpForm form;   // the kernel (cb_taftp_form)
     int* ibp;      // incoherent-beam partials to leave (cb_ib_fused), or null
 };
 
@@ -628,11 +636,10 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         }
     }
 
-    const CbVariant var = cb_pick_variant(d, tv ? tv->variant : plan->variant, mode, T);
+    const CbVariant var =
+        tv ? CbVariant{32, tv->form.rt, true, true, false} : cb_pick_variant(d, plan->variant, mode, T);
     // The timing events (fbf_cb_plan_set_timing), around the coherent kernel only.
     auto mark = [&](hipEvent_t ev) { return ev ? hipEventRecord(ev, s) : hipSuccess; };
-    FBF_REQUIRE(!tv || (var.tr && !var.ws && (var.rows == 8 || (var.rows == 4 && d.fscrunch == 1))), FBF_ERR_STATE,
-                "fbf_cb: the TAFTP input needs the transposed kernel with 128 beams per wave, or 64 at fscrunch 1");
     if (var.ws) {
         CbWsArgs wa{};
         CbArgs& a = wa.p;
@@ -708,14 +715,14 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         ta.ntp = (nslot / spt) * ta.tps;
         ta.ntiles = (int)(2 * T / 32);
         const int passes = (ta.ntiles + ta.ntp - 1) / ta.ntp;
-        const int beams_per_wg = 16 * rt * (4 / d.fscrunch);
-        ta.n_bgroups = (d.nbeams + beams_per_wg - 1) / beams_per_wg;
         const int ksteps = (2 * d.nantennas + 31) / 32;
         hipError_t e = mark(plan->t_before);
         if (e == hipSuccess)
-            e = rt == 2   ? cb_launch_tr2(ta, d.fscrunch, W, ksteps, passes, s)
-                : rt == 4 ? cb_launch_tr4(ta, d.fscrunch, W, ksteps, passes, s)
-                          : cb_launch_tr8(ta, d.fscrunch, W, ksteps, passes, s);
+            e = tv && tv->form.few ? cb_launch_tr_few(ta, rt, W, ksteps, passes, s)
+                : rt == 2           ? cb_launch_tr2(ta, d.fscrunch, W, ksteps, passes, s)
+                : rt == 4           ? cb_launch_tr4(ta, d.fscrunch, W, ksteps, passes, s)
+                : d.fscrunch == 1   ? cb_launch_tr8(ta, W, ksteps, passes, s)
+                                    : cb_launch_tr8_fs(ta, d.fscrunch, W, ksteps, passes, s);
         if (e == hipSuccess) e = mark(plan->t_after);
         if (e != hipSuccess) return hip_status(e, "cb_tr_k launch");
         e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
@@ -817,38 +824,54 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
                      weights_bytes, tbtf, tbtf_bytes, stream);
 }
 
-// The kernel variant with which fbf_cb_beamform_taftp stages the TAFTP block
-// itself, 0 where the plan's kernel does not: the plan's variant, or when
+// The kernel that stages a TAFTP block itself for the plan's coherent beams
+// (rt 0: none, the block is split-transposed): the plan's variant, or when
 // that is automatic 128 beams per wave up to 64 antennas and 64 beams per
-// wave above.  Up to 48 antennas with at most 96 beams a 128-beam wave is
-// too empty: those blocks keep the split-transpose and the wave-private
-// kernel.  Measured, direct against split-transposed (us; antennas / beams /
-// channels / samples / tscrunch): 40/768/64/8192/64 157 against 178, 48/512/
-// 64/8192/16 107 against 156, 32/256/64/8192/16 61 against 75,
-// 24/256/32/4096/16 24.9 against 26.7, 8/64/64/8192/16 39 against 34.
-static int cb_taftp_variant(const fbf_cb_plan* plan, long long T)
+// wave above, with 32 or 64 per wave where at most so many are asked for.
+// `one_pass`: the incoherent beam of the whole block is formed as well.
+//
+// Staging the block itself was the faster at every size measured.  Blocks of
+// both beams, direct against split-transposed (us; antennas / beams / channels
+// / heaps, tscrunch 16): 16/32/16/8 8.6 against 17.1, 48/64/64/8 13.0 against
+// 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
+// of 32 or 64 beams for so few took 8.6 and 33.7 us where 128-beam waves took
+// 10.8 and 41.0.
+// Without the incoherent beam, a subset of at most 48 antennas with at most
+// 96 beams and more than 64 antennas with at most 32 keep the
+// split-transpose, as fbf_cb_taftp_direct has always answered for them.
+static TaftpForm cb_taftp_form(const fbf_cb_plan* plan, long long T, int nantennas_total, bool one_pass)
 {
     const fbf_cb_desc& d = plan->d;
+    const TaftpForm none{0, false};
     if (plan->variant > 0) {
         const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T);
-        return v.tr && !v.ws && (v.rows == 8 || (v.rows == 4 && d.fscrunch == 1)) ? plan->variant : 0;
+        return v.tr && !v.ws && (v.rows == 8 || (v.rows == 4 && d.fscrunch == 1)) ? TaftpForm{v.rows, false} : none;
     }
     const int ksteps = (2 * d.nantennas + 31) / 32;
-    if (ksteps > 4)
-        return d.fscrunch == 1 && d.nbeams > 32 && cb_tr_applies(d, 4, MODE_INT8, T) ? kCbVariantTr4 : 0;
-    if ((ksteps <= 3 || d.fscrunch > 1) && d.nbeams <= 96) return 0;
-    return cb_tr_applies(d, 8, MODE_INT8, T) ? kCbVariantTr8 : 0;
+    if (ksteps > 4) {
+        if (d.fscrunch != 1 || (d.nbeams <= 32 && !one_pass) || !cb_tr_applies(d, 4, MODE_INT8, T)) return none;
+        return TaftpForm{4, false};
+    }
+    const bool whole = d.fscrunch == 1 && nantennas_total == d.nantennas;
+    if ((ksteps <= 3 || d.fscrunch > 1) && d.nbeams <= 96 && !whole) return none;
+    if (!cb_tr_applies(d, 8, MODE_INT8, T)) return none;
+    if (d.fscrunch == 1 && d.nbeams <= 64) return TaftpForm{d.nbeams <= 32 ? 2 : 4, true};
+    return TaftpForm{8, false};
 }
 
-// Whether fbf_cb_beamform_taftp stages the TAFTP block itself: such a
-// variant, a heap of a power-of-two number of samples, at least one tile
-// (16 samples), and a heap group's bytes within a 31-bit offset.
+// Whether the block's geometry lets cb_tr_k stage it: a heap of a power-of-two
+// number of samples, at least one tile (16 samples), a heap group's bytes
+// within a 31-bit offset and 32-bit tile offsets.
+static bool cb_taftp_stages(const fbf_cb_desc& d, long long T, int nantennas_total, int S)
+{
+    return S >= 16 && (S & (S - 1)) == 0 && (long long)4 * nantennas_total * d.nchans * S < (1ll << 31) &&
+           (long long)4 * nantennas_total * d.nchans * T < (1ll << 32);
+}
+
+// Whether fbf_cb_beamform_taftp stages the TAFTP block itself.
 static bool cb_taftp_direct(const fbf_cb_plan* plan, long long T, int nantennas_total, int S)
 {
-    const fbf_cb_desc& d = plan->d;
-    return cb_taftp_variant(plan, T) > 0 && S >= 16 && (S & (S - 1)) == 0 &&
-           (long long)4 * nantennas_total * d.nchans * S < (1ll << 31) &&
-           (long long)4 * nantennas_total * d.nchans * T < (1ll << 32);   // 32-bit tile offsets
+    return cb_taftp_form(plan, T, nantennas_total, false).rt > 0 && cb_taftp_stages(plan->d, T, nantennas_total, S);
 }
 
 // The incoherent beam of the block formed in the split-transpose's pass.
@@ -879,7 +902,8 @@ static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes
     FBF_REQUIRE((reinterpret_cast<uintptr_t>(taftp) & 15) == 0, FBF_ERR_ARG,
                 "fbf_cb_beamform_taftp: buffers must be 16-byte aligned");
     if (T == 0 || cb_taftp_direct(plan, T, nantennas_total, nsamples_per_heap)) {
-        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna, cb_taftp_variant(plan, T), nullptr};
+        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna,
+                           cb_taftp_form(plan, T, nantennas_total, false), nullptr};
         return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf,
                          tbtf_bytes, stream, nullptr, 0, T ? &tv : nullptr, tail);
     }
@@ -916,16 +940,20 @@ extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_
 }
 
 // Whether fbf_cb_ib_beamform_taftp forms the incoherent beam inside the
-// coherent beamformer: the direct TAFTP path with one-slot work-groups (128
-// beams per wave, or 64 above 64 antennas) over all the block's antennas, and
-// an incoherent-beam plan of the same block (antennas, channels, heap size).
+// coherent beamformer: the block staged by four-wave work-groups (every
+// automatic form at fscrunch 1; 128 beams per wave, or 64 above 64 antennas),
+// and an incoherent-beam plan of the same block (antennas, channels, heap
+// size).  Up to 48 antennas with at most 96 beams an incoherent beam of several
+// channels keeps its own pass, as fbf_cb_ib_fused has always answered.
 static bool cb_ib_fused(const fbf_cb_plan* plan, const IbFuseParams& ibp, long long T, int S)
 {
     const fbf_cb_desc& d = plan->d;
-    if (!cb_taftp_direct(plan, T, d.nantennas, S)) return false;
-    const int rows = kCbVariants[cb_taftp_variant(plan, T)].rows;
-    return d.fscrunch == 1 && (rows == 8 || (2 * d.nantennas + 31) / 32 > 4) && ibp.nantennas == d.nantennas &&
-           ibp.nchans == d.nchans && ibp.nsamples_per_heap == S;
+    const TaftpForm form = cb_taftp_form(plan, T, d.nantennas, true);
+    const int ksteps = (2 * d.nantennas + 31) / 32;
+    if (form.rt == 0 || d.fscrunch != 1 || !(form.few || tr_four_waves(form.rt, ksteps))) return false;
+    if (ksteps <= 3 && d.nbeams <= 96 && ibp.fscrunch > 1 && plan->variant <= 0) return false;
+    return cb_taftp_stages(d, T, d.nantennas, S) && ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
+           ibp.nsamples_per_heap == S;
 }
 
 // Both beams of a TAFTP block in one pass, or where the plans do not allow it
@@ -1012,7 +1040,8 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
     IbFinishJob ibj{};
     st = ib_finish_job(ib_plan, static_cast<const int*>(part), T, tf, tf_bytes, &ibj);
     if (st) return st;
-    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_variant(plan, T), static_cast<int*>(part)};
+    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_form(plan, T, d.nantennas, true),
+                       static_cast<int*>(part)};
     return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
                      stream, nullptr, 0, &tv, TailJobs{ibj, wj});
 }

@@ -385,14 +385,32 @@ def test_cb_one_pass_any_antennas(gpu, oracle, A, F, nhg, B, ts, ib_ts, ib_fs):
     _check_taftp(gpu, oracle, A + 12, A, 5, F, nhg, B, ts, 1, 128, 0, True, 3200 + A, weights=w.reshape(-1))
 
 
-@pytest.mark.parametrize("A,B,ib_ts,ib_fs", [
-    (16, 32, 16, 1),     # the incoherent beam in the split-transpose's pass
-    (20, 64, 32, 1),     # antennas in fours: the LDS-staged kernel
-    (128, 32, 1, 1),     # 32 beams per wave
-    (40, 96, 64, 1),     # windows longer than the split-transpose's tiles: a pass of its own
-    (24, 40, 16, 2),     # two channels to an output channel: likewise
+@pytest.mark.parametrize("A,F,nhg,B,ts,ib_ts", [
+    (16, 16, 3, 32, 16, 16),    # 32 beams per wave, one K step
+    (40, 4, 2, 24, 4, 1),       # three K steps, four windows a tile, a wave with unused beams
+    (64, 4, 2, 8, 64, 256),     # four K steps, one window over four tiles
+    (20, 4, 2, 64, 8, 4),       # 64 beams per wave, antennas in fours
+    (60, 4, 1, 40, 16, 16),
+    (48, 8, 2, 96, 32, 64),     # 128 beams per wave, four time slots
+    (64, 4, 2, 200, 16, 16),    # two beam groups, two time slots
+    (32, 4, 2, 640, 16, 16),    # five beam groups: one to a work-group
+    (128, 4, 2, 32, 16, 16),    # 64 beams per wave over eight K steps, half empty
+    (76, 4, 1, 136, 4, 1),      # three beam groups in pairs
 ])
-def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs):
+def test_cb_one_pass_few_beams(gpu, oracle, A, F, nhg, B, ts, ib_ts):
+    """The one-pass path where few beams share their waves out over time
+    slots, against the oracle."""
+    _check_cb_ib(gpu, oracle, A, F, nhg, B, ts, ib_ts, 1, 256, 0, True, 3400 + A + B)
+
+
+@pytest.mark.parametrize("A,B,ib_ts,ib_fs,variant", [
+    (16, 32, 16, 1, 10),    # the incoherent beam in the split-transpose's pass
+    (20, 64, 32, 1, 5),     # antennas in fours: the LDS-staged kernel
+    (128, 32, 1, 1, 8),     # 32 beams per wave
+    (40, 96, 64, 1, 10),    # windows longer than the split-transpose's tiles: a pass of its own
+    (24, 40, 16, 2, 0),     # two channels to an output channel: likewise
+])
+def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs, variant):
     """Blocks that are split-transposed: the coherent beams, the incoherent
     beam and the next block's weights, written over this block's, of one call
     equal the oracle's beams and fbf_weights_generate."""
@@ -405,6 +423,7 @@ def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs):
     _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, A, ts, 1, A, ib_ts, ib_fs)
     ioff, isc = np.full(F // ib_fs, ibo, np.float32), np.full(F // ib_fs, ibs, np.float32)
     plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=T // ts)
+    plan.set_variant(variant)
     ib = capi.IbPlan(A, F, ib_ts, ib_fs, ioff, isc)
     assert not plan.ib_fused(ib, T, S)
     wp = capi.WeightsPlan(A, B, F, capi.channel_frequencies_f64(wl.L_BAND_CENTRE_HZ, F * wl.CHANNEL_BW_HZ, F))
