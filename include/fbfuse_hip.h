@@ -417,10 +417,14 @@ int fbf_batch_autotune(fbf_batch* batch, int reps);
  * pipeline). */
 int fbf_batch_set_serial(fbf_batch* batch, int serial);
 int fbf_batch_get_serial(const fbf_batch* batch, int* serial);
-/* Split-transposes the block once into a full-antenna FTPA workspace and
- * runs every subarray's coherent beamformer on it (and the incoherent beam
- * on the TAFTP block), as independent branches forked from `stream` and
- * joined back into it.  use_graph != 0 captures this once into a hipGraph and
+/* Beamforms every subarray straight from the TAFTP block, in turn, where all
+ * their kernels stage it (the incoherent beam then comes out of the same
+ * kernels when the subarrays share all of the block's antennas out, else from
+ * a pass of its own).  Otherwise, and with the subarrays side by side
+ * (fbf_batch_set_serial), split-transposes the block once into a full-antenna
+ * FTPA workspace and runs every subarray's coherent beamformer on it, in turn
+ * or as independent branches forked from `stream` and joined back into it.
+ * use_graph != 0 captures this once into a hipGraph and
  * replays it; the graph is captured again whenever a buffer pointer
  * changes.  weights[i]: device FBA weights of subarray i; outputs: device
  * outputs (TBTF per subarray, then TF if the incoherent beam is enabled). */

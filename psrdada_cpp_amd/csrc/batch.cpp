@@ -1,11 +1,18 @@
 // Batched subarrays on one DADA block.
 //
-// One split transpose of the whole block into a full-antenna FTPA workspace,
-// then every subarray's coherent beamformer reads its antenna range straight
-// from that workspace (fbf_cb_beamform_subarray), and the incoherent beam
-// reads the TAFTP block.  The beamformers are independent branches forked
-// from the caller's stream and joined back, so uneven subarrays share the
-// device; with use_graph the whole block is one hipGraph launch.
+// Where every subarray's kernel stages the TAFTP block itself (batch_direct),
+// each beamforms its antennas straight from the block; when the subarrays
+// share all of the block's antennas out, they also leave the incoherent beam's
+// partials, which the last one's reorder launch adds up, else the incoherent
+// beam reads the block on its own.  Otherwise one split transpose of the whole
+// block into a full-antenna FTPA workspace (with the incoherent beam where its
+// scrunch allows it), then every subarray's coherent beamformer reads its
+// antenna range from that workspace (fbf_cb_beamform_subarray).  A block of 64
+// antennas, 64 channels, 8192 spectra as 40/16/8 antennas with 768/256/64
+// beams took 315 us split-transposed and takes 249 us straight from TAFTP.
+// The subarrays run in turn on the caller's stream,
+// or as independent branches forked from it and joined back; with use_graph
+// the whole block is one hipGraph launch.
 #include <cstring>
 #include <string>
 #include <vector>
@@ -22,6 +29,7 @@ struct fbf_batch {
     bool ib_fused = false;         // incoherent beam computed by the split-transpose pass
     void* ftpa = nullptr;          // full-antenna FTPA workspace
     size_t ftpa_bytes = 0;
+    void* ibp = nullptr;           // incoherent-beam partials of each subarray, where they share the antennas out
     std::vector<hipStream_t> streams;
     std::vector<hipEvent_t> join;
     hipEvent_t fork_ib = nullptr;   // block available: incoherent beam may start
@@ -45,6 +53,26 @@ static size_t sub_out_bytes(const fbf_batch* b, const fbf_subarray_desc& d)
     return T / d.tscrunch * d.nbeams * (b->F / d.fscrunch);
 }
 
+// Whether every subarray's kernel stages the TAFTP block itself.
+static bool batch_direct(const fbf_batch* b, bool partials)
+{
+    if (b->S % 32 != 0 || b->nhg >= 1 << 20) return false;   // (as the split-transpose)
+    for (auto* p : b->plans)
+        if (!cb_batch_stages(p, (long long)b->nhg * b->S, b->A, b->S, partials)) return false;
+    return true;
+}
+
+// Whether the subarrays share the block's antennas out: each in exactly one.
+static bool batch_shares_antennas(const fbf_batch* b)
+{
+    std::vector<int> seen(b->A, 0);
+    for (const auto& s : b->subs)
+        for (int a = s.start_antenna; a < s.start_antenna + s.nantennas; ++a) ++seen[a];
+    for (int n : seen)
+        if (n != 1) return false;
+    return true;
+}
+
 static void batch_release(fbf_batch* b)
 {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -52,6 +80,7 @@ static void batch_release(fbf_batch* b)
     for (auto* p : b->plans) fbf_cb_plan_destroy(p);
     if (b->ib) fbf_ib_plan_destroy(b->ib);
     if (b->ftpa) (void)hipFree(b->ftpa);
+    if (b->ibp) (void)hipFree(b->ibp);
     for (auto s : b->streams) (void)hipStreamDestroy(s);
     for (auto e : b->join) (void)hipEventDestroy(e);
     if (b->fork_ib) (void)hipEventDestroy(b->fork_ib);
@@ -136,6 +165,14 @@ extern "C" int fbf_batch_enable_ib(fbf_batch* b, int tscrunch, int fscrunch, int
     fbf_ib_plan* p = nullptr;
     int st = fbf_ib_plan_create(&d, offsets, scales, &p);
     if (st) return st;
+    if (!b->ibp && batch_shares_antennas(b)) {
+        // (16 bytes per channel and sample for each subarray.)
+        const hipError_t e = hipMalloc(&b->ibp, (size_t)16 * b->F * b->nhg * b->S * b->subs.size());
+        if (e != hipSuccess) {
+            fbf_ib_plan_destroy(p);
+            return hip_status(e, "hipMalloc(incoherent-beam partials)");
+        }
+    }
     if (b->ib) fbf_ib_plan_destroy(b->ib);
     b->ib = p;
     b->ib_fused = fscrunch == 1 && tscrunch > 0 && 32 % tscrunch == 0 && b->S % 32 == 0;
@@ -190,8 +227,9 @@ extern "C" int fbf_batch_get_serial(const fbf_batch* b, int* serial)
 }
 
 // Tunes every subarray's kernel (fbf_cb_autotune), then times whole blocks
-// as graph launches with the subarrays in turn and side by side, on
-// synthetic data of the batch's geometry.  In turn is kept unless side by
+// as graph launches with the subarrays in turn and side by side, and in turn
+// with the automatic kernels where those stage the TAFTP block themselves but
+// the tuned ones do not, on synthetic data of the batch's geometry.  In turn is kept unless side by
 // side is faster by more than 3 %: the synthetic bytes run at a higher
 // clock than real voltages, and on real data in turn was the faster at
 // every tscrunch measured.
@@ -249,9 +287,24 @@ extern "C" int fbf_batch_autotune(fbf_batch* b, int reps)
         return hip_status(e, "fbf_batch_autotune setup");
     }
     const int nrep = reps < 8 ? 8 : reps;
-    float mode_ms[2] = {0.0f, 0.0f};   // [0] in turn, [1] side by side
-    for (int mode = 0; mode < 2; ++mode) {
-        b->serial = mode == 0;
+    std::vector<std::pair<int, int>> tuned, automatic(n, {0, 0});   // (variant, chunk) of each subarray
+    for (auto* p : b->plans) tuned.push_back(cb_plan_tuning(p));
+    auto use = [&](const std::vector<std::pair<int, int>>& t) {
+        for (int i = 0; i < n; ++i) {
+            (void)fbf_cb_plan_set_variant(b->plans[i], t[i].first);
+            (void)fbf_cb_plan_set_chunk(b->plans[i], t[i].second);
+        }
+    };
+    int modes = 2;
+    if (!batch_direct(b, false)) {
+        use(automatic);
+        if (batch_direct(b, false)) modes = 3;
+        use(tuned);
+    }
+    float mode_ms[3] = {0.0f, 0.0f, 0.0f};   // [0] in turn, [1] side by side, [2] in turn straight from TAFTP
+    for (int mode = 0; mode < modes; ++mode) {
+        b->serial = mode != 1;
+        if (mode == 2) use(automatic);
         b->graph_ptrs.clear();
         int st = FBF_OK;
         for (int r = 0; r < 2 && st == FBF_OK; ++r) st = fbf_batch_run(b, taftp, b->ftpa_bytes, w.data(), o.data(), 1, s);
@@ -263,13 +316,51 @@ extern "C" int fbf_batch_autotune(fbf_batch* b, int reps)
         if (st != FBF_OK || e != hipSuccess) {
             (void)hipStreamSynchronize(s);
             b->serial = serial0;
+            use(tuned);
             cleanup();
             return st != FBF_OK ? st : hip_status(e, "fbf_batch_autotune timing");
         }
         (void)hipEventElapsedTime(&mode_ms[mode], e0, e1);
     }
-    b->serial = !(mode_ms[1] < 0.97f * mode_ms[0]);
+    const bool direct = modes == 3 && mode_ms[2] < mode_ms[0];
+    if (!direct) use(tuned);
+    b->serial = !(mode_ms[1] < 0.97f * (direct ? mode_ms[2] : mode_ms[0]));
+    if (!b->serial) use(tuned);
     cleanup();
+    return FBF_OK;
+}
+
+// Enqueues one block in turn on `stream` straight from TAFTP (batch_direct).
+static int batch_enqueue_direct(fbf_batch* b, const void* taftp, size_t taftp_bytes, const void* const* weights,
+                                void* const* outputs, hipStream_t stream)
+{
+    const int n = (int)b->subs.size();
+    const long long T = (long long)b->nhg * b->S;
+    int st = FBF_OK;
+    size_t ob = 0;
+    if (b->ib) {
+        st = fbf_ib_output_bytes(b->ib, taftp_bytes, &ob);
+        if (st) return st;
+    }
+    const bool partials = b->ib && b->ibp && batch_direct(b, true);
+    if (b->ib && !partials) {
+        st = fbf_ib_beamform(b->ib, taftp, taftp_bytes, outputs[n], ob, stream);
+        if (st) return st;
+    }
+    int* const part = static_cast<int*>(b->ibp);
+    const size_t step = (size_t)4 * b->F * T;   // ints per subarray
+    for (int i = 0; i < n; ++i) {
+        IbFinishJob job{};
+        if (partials && i == n - 1) {
+            st = ib_finish_job(b->ib, part, n, T, outputs[n], ob, &job);
+            if (st) return st;
+        }
+        size_t wb = 0;
+        fbf_batch_weights_bytes(b, i, &wb);
+        st = cb_batch_beamform(b->plans[i], taftp, T, b->A, b->subs[i].start_antenna, b->S, weights[i], wb, outputs[i],
+                               sub_out_bytes(b, b->subs[i]), stream, partials ? part + i * step : nullptr, job);
+        if (st) return st;
+    }
     return FBF_OK;
 }
 
@@ -307,6 +398,9 @@ static int batch_enqueue_serial(fbf_batch* b, const void* taftp, size_t taftp_by
 static int batch_enqueue(fbf_batch* b, const void* taftp, size_t taftp_bytes, const void* const* weights,
                          void* const* outputs, hipStream_t stream)
 {
+    const bool aligned = (reinterpret_cast<uintptr_t>(taftp) & 15) == 0;   // (else the calls below refuse it)
+    if (b->serial && aligned && batch_direct(b, false))
+        return batch_enqueue_direct(b, taftp, taftp_bytes, weights, outputs, stream);
     if (b->serial) return batch_enqueue_serial(b, taftp, taftp_bytes, weights, outputs, stream);
     const int n = (int)b->subs.size();
     // The incoherent beam comes out of the split-transpose pass when its

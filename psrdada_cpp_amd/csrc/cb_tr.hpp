@@ -927,11 +927,33 @@ inline int device_cu_count()
     return cus[dev];
 }
 
-// One round of resident work-groups: every (channel group, beam group) gets
-// (resident work-groups) / (channel groups x beam groups) work-groups, each a
-// contiguous run of passes, so the per-work-group start-up (weights, the
-// first staged tiles) is paid once per resident slot and all work-groups end
-// together.
+// Work-groups per (channel group, beam group), each a contiguous run of
+// passes on every time slot: `slots` resident work-groups run at a time.  The
+// fewest tile steps in a row over the rounds, where a work-group's start-up
+// (weights, the first staged tiles) is about five steps long.  That is one
+// round wherever it fills the slots; 192 units on 512 slots (40 antennas, 768
+// beams, 64 channels) left a quarter of them empty: 185 us in one round, 165 us
+// in three (8192 samples, tscrunch 16).
+inline long long tr_groups_per_unit(long long units, long long slots, int passes, int nts, int ntp)
+{
+    constexpr int kStart = 5;
+    const long long most = (passes + nts - 1) / nts;
+    long long best = 1, best_cost = 0;
+    for (int round = 1; round <= 8; ++round) {   // the most work-groups of each number of rounds
+        long long n = round * slots / units;
+        n = n < 1 ? 1 : n > most ? most : n;
+        const long long np = (passes + n * nts - 1) / (n * nts);   // passes per slot
+        const long long groups = (passes + np * nts - 1) / (np * nts);
+        const long long cost = (units * groups + slots - 1) / slots * (np * ntp + kStart);
+        if (best_cost == 0 || cost < best_cost) {
+            best = n;
+            best_cost = cost;
+        }
+        if (n == most) break;
+    }
+    return best;
+}
+
 template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF = false>
 hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
 {
@@ -948,14 +970,8 @@ hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
             o = 1;
         occ = o;
     }
-    // Work-groups per (channel group, beam group): one round of resident
-    // work-groups where the problem allows; each covers NTS slots of
-    // npasses passes.
     const long long units = (long long)a.p.Fo * a.n_bgroups;
-    long long per_unit = (long long)occ * device_cu_count() / units;
-    if (per_unit < 1) per_unit = 1;
-    const long long max_groups = (passes + NTS - 1) / NTS;
-    if (per_unit > max_groups) per_unit = max_groups;
+    const long long per_unit = tr_groups_per_unit(units, (long long)occ * device_cu_count(), passes, NTS, a.ntp);
     a.npasses = (int)((passes + per_unit * NTS - 1) / (per_unit * NTS));
     a.n_tgroups = (int)((passes + (long long)a.npasses * NTS - 1) / ((long long)a.npasses * NTS));
     const long long nblocks = units * a.n_tgroups;

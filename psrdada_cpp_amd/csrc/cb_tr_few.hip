@@ -1,5 +1,5 @@
-// Instances of the transposed kernel (cb_tr_k) for at most 64 beams of a TAFTP
-// block of up to 64 antennas: one wave of 32 or 64 beams per time slot, four
+// Instances of the transposed kernel (cb_tr_k) for at most 64 beams of up to 64
+// antennas: one wave of 32 or 64 beams per time slot, four
 // time slots to a work-group.
 #include "cb_tr.hpp"
 
@@ -9,6 +9,7 @@ namespace {
 template <int RT, int KSTEPS, int SPT, int NSLOT>
 hipError_t launch_few(const CbTrArgs& a, int passes, hipStream_t s)
 {
+    if (a.p.S == 0) return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, 1, 4, 1, false>(a, passes, s);
     return a.ibp ? launch_tr_kt<RT, KSTEPS, SPT, NSLOT, 1, 4, 1, true, true>(a, passes, s)
                  : launch_tr_kt<RT, KSTEPS, SPT, NSLOT, 1, 4, 1, true, false>(a, passes, s);
 }

@@ -460,6 +460,7 @@ struct CbVariant {
     bool lds;        // voltage tile staged through LDS and shared by the work-group
     bool tr;         // transposed tiles (cb_tr_k): voltages as the A operand
     bool ws;         // transposed tiles with wave-private staging (cb_ws_k)
+    bool few = false;   // transposed: one wave per time slot, for at most 64 beams (cb_tr_few.hip)
 };
 static const CbVariant kCbVariants[] = {
     {0, 0, false, false, false},   // auto
@@ -478,7 +479,6 @@ static const CbVariant kCbVariants[] = {
 constexpr int kCbVariantLds = 5;
 constexpr int kCbVariantTr2 = 8;
 constexpr int kCbVariantTr4 = 9;
-constexpr int kCbVariantWs = 10;
 constexpr int kCbVariantTr8 = 11;
 
 static bool cb_tr_applies(const fbf_cb_desc& d, int rt, int mode, long long T)
@@ -493,26 +493,26 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
            cb_ws_supported(d.nantennas, d.tscrunch, d.fscrunch);
 }
 
-// Automatic choice.  fscrunch 1, up to three 32-byte K steps (48 antennas):
-// the wave-private kernel, which measured 20-85 % faster there than the
-// transposed kernel with 64 beams per wave (8 to 48 antennas, tscrunch 4 to
-// 64; one exception, 32 antennas at tscrunch 4, 8 % slower).  Else the
-// transposed kernel with 128 beams per wave (fscrunch 1: 3.2 % faster than 64
-// beams per wave at 64 antennas, 64 channels, 512 beams; fscrunch 2 and 4,
-// where the forms with several time slots per work-group stop at two K steps
-// of four channels: 241 us against 348 us of the LDS-staged kernel at 44
-// antennas, 1024 beams, 64 channels, 8192 samples, fscrunch 4) unless few
-// beams leave its waves empty, else with 64 (above 64 antennas only with more
-// than 32 beams: a 64-beam wave would be half empty), else with 32 beams per
-// wave, else the LDS-staged kernel (which also serves int32 sums, power output
-// and the geometries the transposed kernels do not).
+// Automatic choice from FTPA: the transposed kernel, up to 64 antennas with
+// 128 beams per wave or with 32 or 64 for so few beams, above with 64 (32 for
+// at most 32: a 64-beam wave would be half empty); the LDS-staged kernel for
+// the rest (tscrunch below 4 or no power of two, fscrunch above 4, also int32
+// sums and power output).  Measured against the wave-private kernel and the
+// earlier picks (us; antennas / beams / channels / samples / tscrunch):
+// 16/256/64/8192/16 40.6 against 44.7, 48/512/64/8192/16 111 against 128,
+// 40/768/64/8192/4 250 against 272, 8/64/64/8192/16 16.4 against 17.4,
+// 16/32/16/2048/16 8.3 against 9.4.  fscrunch 2 and 4: 128 beams per wave
+// above 96 beams, or where the forms with several time slots per work-group
+// end (two K steps of four channels); 44/1024/64/8192/16 at fscrunch 4 took
+// 205 against 348 of the LDS-staged kernel, 44/64 32 against 50, but 24/64 26.7
+// against 24.5 with 32 beams per wave.
 static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, long long T)
 {
     if (variant <= 0) {
         const int ksteps = (2 * d.nantennas + 31) / 32;
-        if (ksteps <= 3 && cb_ws_applies(d, mode, T)) return kCbVariants[kCbVariantWs];
-        if ((d.fscrunch > 1 ? d.nbeams > 96 : ksteps > 3) && cb_tr_applies(d, 8, mode, T))
-            return kCbVariants[kCbVariantTr8];
+        const bool tr8 = cb_tr_applies(d, 8, mode, T);
+        if (tr8 && d.fscrunch == 1 && d.nbeams <= 64) return {32, d.nbeams <= 32 ? 2 : 4, true, true, false, true};
+        if (tr8 && (d.fscrunch == 1 || d.nbeams > 96 || d.fscrunch * ksteps > 8)) return kCbVariants[kCbVariantTr8];
         if ((ksteps <= 4 || d.nbeams > 32) && cb_tr_applies(d, 4, mode, T)) return kCbVariants[kCbVariantTr4];
         if (cb_tr_applies(d, 2, mode, T)) return kCbVariants[kCbVariantTr2];
         return kCbVariants[kCbVariantLds];
@@ -563,8 +563,7 @@ extern "C" int fbf_cb_output_bytes(const fbf_cb_plan* plan, size_t ftpa_bytes, s
 // A TAFTP block read directly by the coherent beamformer: S samples per
 // heap, Atot antennas, the beamformer's antennas from antenna a0.
 // The transposed kernel that stages a TAFTP block itself: RT beam tiles (16
-// RT beams) per wave, 0 where none does; `few`: the form with one wave per
-// time slot for at most 64 beams (cb_tr_few.hip).
+// RT beams) per wave, 0 where none does; `few` as in CbVariant.
 struct TaftpForm {
     int rt;
     bool few;
@@ -637,7 +636,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
     }
 
     const CbVariant var =
-        tv ? CbVariant{32, tv->form.rt, true, true, false} : cb_pick_variant(d, plan->variant, mode, T);
+        tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_variant(d, plan->variant, mode, T);
     // The timing events (fbf_cb_plan_set_timing), around the coherent kernel only.
     auto mark = [&](hipEvent_t ev) { return ev ? hipEventRecord(ev, s) : hipSuccess; };
     if (var.ws) {
@@ -718,7 +717,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         const int ksteps = (2 * d.nantennas + 31) / 32;
         hipError_t e = mark(plan->t_before);
         if (e == hipSuccess)
-            e = tv && tv->form.few ? cb_launch_tr_few(ta, rt, W, ksteps, passes, s)
+            e = var.few             ? cb_launch_tr_few(ta, rt, W, ksteps, passes, s)
                 : rt == 2           ? cb_launch_tr2(ta, d.fscrunch, W, ksteps, passes, s)
                 : rt == 4           ? cb_launch_tr4(ta, d.fscrunch, W, ksteps, passes, s)
                 : d.fscrunch == 1   ? cb_launch_tr8(ta, W, ksteps, passes, s)
@@ -828,7 +827,6 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 // (rt 0: none, the block is split-transposed): the plan's variant, or when
 // that is automatic 128 beams per wave up to 64 antennas and 64 beams per
 // wave above, with 32 or 64 per wave where at most so many are asked for.
-// `one_pass`: the incoherent beam of the whole block is formed as well.
 //
 // Staging the block itself was the faster at every size measured.  Blocks of
 // both beams, direct against split-transposed (us; antennas / beams / channels
@@ -836,42 +834,50 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 // 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
 // of 32 or 64 beams for so few took 8.6 and 33.7 us where 128-beam waves took
 // 10.8 and 41.0.
-// Without the incoherent beam, a subset of at most 48 antennas with at most
-// 96 beams and more than 64 antennas with at most 32 keep the
-// split-transpose, as fbf_cb_taftp_direct has always answered for them.
-static TaftpForm cb_taftp_form(const fbf_cb_plan* plan, long long T, int nantennas_total, bool one_pass)
+// On their own (kTaftpAlone), a subset of at most 48 antennas with at most 96
+// beams and more than 64 antennas with at most 32 keep the split-transpose,
+// as fbf_cb_taftp_direct has always answered for them.
+enum TaftpUse {
+    kTaftpAlone,     // fbf_cb_beamform_taftp
+    kTaftpOnePass,   // with the incoherent beam of the whole block
+    kTaftpBatch      // one of a batch's subarrays
+};
+
+static TaftpForm cb_taftp_form(const fbf_cb_plan* plan, long long T, int nantennas_total, TaftpUse use)
 {
     const fbf_cb_desc& d = plan->d;
     const TaftpForm none{0, false};
-    if (plan->variant > 0) {
-        const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T);
-        return v.tr && !v.ws && (v.rows == 8 || (v.rows == 4 && d.fscrunch == 1)) ? TaftpForm{v.rows, false} : none;
-    }
+    const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T);
     const int ksteps = (2 * d.nantennas + 31) / 32;
-    if (ksteps > 4) {
-        if (d.fscrunch != 1 || (d.nbeams <= 32 && !one_pass) || !cb_tr_applies(d, 4, MODE_INT8, T)) return none;
-        return TaftpForm{4, false};
+    if (plan->variant <= 0 && use != kTaftpBatch) {
+        if (ksteps > 4 && d.nbeams <= 32 && use == kTaftpAlone) return none;
+        const bool whole = d.fscrunch == 1 && nantennas_total == d.nantennas;
+        if ((ksteps <= 3 || (ksteps == 4 && d.fscrunch > 1)) && d.nbeams <= 96 && !whole) return none;
     }
-    const bool whole = d.fscrunch == 1 && nantennas_total == d.nantennas;
-    if ((ksteps <= 3 || d.fscrunch > 1) && d.nbeams <= 96 && !whole) return none;
-    if (!cb_tr_applies(d, 8, MODE_INT8, T)) return none;
-    if (d.fscrunch == 1 && d.nbeams <= 64) return TaftpForm{d.nbeams <= 32 ? 2 : 4, true};
-    return TaftpForm{8, false};
+    // Above 64 antennas no other form stages TAFTP.
+    if (plan->variant <= 0 && ksteps > 4 && d.fscrunch == 1 && cb_tr_applies(d, 4, MODE_INT8, T))
+        return TaftpForm{4, false};
+    return v.tr && !v.ws && (v.rows == 8 || v.few || (v.rows == 4 && d.fscrunch == 1)) ? TaftpForm{v.rows, v.few}
+                                                                                        : none;
 }
 
 // Whether the block's geometry lets cb_tr_k stage it: a heap of a power-of-two
-// number of samples, at least one tile (16 samples), a heap group's bytes
-// within a 31-bit offset and 32-bit tile offsets.
-static bool cb_taftp_stages(const fbf_cb_desc& d, long long T, int nantennas_total, int S)
+// number of samples, at least one tile (16 samples; two where other heaps were
+// refused by the split-transpose), a heap group's bytes within a 31-bit offset
+// and 32-bit tile offsets.
+static bool cb_taftp_stages(const fbf_cb_plan* plan, long long T, int nantennas_total, int S)
 {
-    return S >= 16 && (S & (S - 1)) == 0 && (long long)4 * nantennas_total * d.nchans * S < (1ll << 31) &&
+    const fbf_cb_desc& d = plan->d;
+    const bool one_tile = d.nantennas % 8 == 0 && d.nantennas <= 64 && d.fscrunch == 1 &&
+                          (plan->variant > 0 || d.nantennas > 48);
+    return S >= (one_tile ? 16 : 32) && (S & (S - 1)) == 0 && (long long)4 * nantennas_total * d.nchans * S < (1ll << 31) &&
            (long long)4 * nantennas_total * d.nchans * T < (1ll << 32);
 }
 
 // Whether fbf_cb_beamform_taftp stages the TAFTP block itself.
 static bool cb_taftp_direct(const fbf_cb_plan* plan, long long T, int nantennas_total, int S)
 {
-    return cb_taftp_form(plan, T, nantennas_total, false).rt > 0 && cb_taftp_stages(plan->d, T, nantennas_total, S);
+    return cb_taftp_form(plan, T, nantennas_total, kTaftpAlone).rt > 0 && cb_taftp_stages(plan, T, nantennas_total, S);
 }
 
 // The incoherent beam of the block formed in the split-transpose's pass.
@@ -903,7 +909,7 @@ static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes
                 "fbf_cb_beamform_taftp: buffers must be 16-byte aligned");
     if (T == 0 || cb_taftp_direct(plan, T, nantennas_total, nsamples_per_heap)) {
         const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna,
-                           cb_taftp_form(plan, T, nantennas_total, false), nullptr};
+                           cb_taftp_form(plan, T, nantennas_total, kTaftpAlone), nullptr};
         return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf,
                          tbtf_bytes, stream, nullptr, 0, T ? &tv : nullptr, tail);
     }
@@ -948,11 +954,11 @@ extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_
 static bool cb_ib_fused(const fbf_cb_plan* plan, const IbFuseParams& ibp, long long T, int S)
 {
     const fbf_cb_desc& d = plan->d;
-    const TaftpForm form = cb_taftp_form(plan, T, d.nantennas, true);
+    const TaftpForm form = cb_taftp_form(plan, T, d.nantennas, kTaftpOnePass);
     const int ksteps = (2 * d.nantennas + 31) / 32;
     if (form.rt == 0 || d.fscrunch != 1 || !(form.few || tr_four_waves(form.rt, ksteps))) return false;
     if (ksteps <= 3 && d.nbeams <= 96 && ibp.fscrunch > 1 && plan->variant <= 0) return false;
-    return cb_taftp_stages(d, T, d.nantennas, S) && ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
+    return cb_taftp_stages(plan, T, d.nantennas, S) && ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
            ibp.nsamples_per_heap == S;
 }
 
@@ -1038,12 +1044,32 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
     st = cb_grow(&plan->ibp, &plan->ibp_bytes, (size_t)d.nchans * T * 4 * sizeof(int), s, &part);
     if (st) return st;
     IbFinishJob ibj{};
-    st = ib_finish_job(ib_plan, static_cast<const int*>(part), T, tf, tf_bytes, &ibj);
+    st = ib_finish_job(ib_plan, static_cast<const int*>(part), 1, T, tf, tf_bytes, &ibj);
     if (st) return st;
-    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_form(plan, T, d.nantennas, true),
+    const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_form(plan, T, d.nantennas, kTaftpOnePass),
                        static_cast<int*>(part)};
     return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
                      stream, nullptr, 0, &tv, TailJobs{ibj, wj});
+}
+
+std::pair<int, int> fbf::cb_plan_tuning(const fbf_cb_plan* plan) { return {plan->variant, plan->chunk}; }
+
+bool fbf::cb_batch_stages(const fbf_cb_plan* plan, long long T, int nantennas_total, int S, bool partials)
+{
+    const fbf_cb_desc& d = plan->d;
+    const TaftpForm form = cb_taftp_form(plan, T, nantennas_total, kTaftpBatch);
+    if (form.rt == 0 || T % d.tscrunch != 0 || !cb_taftp_stages(plan, T, nantennas_total, S)) return false;
+    return !partials || (d.fscrunch == 1 && (form.few || tr_four_waves(form.rt, (2 * d.nantennas + 31) / 32)));
+}
+
+int fbf::cb_batch_beamform(fbf_cb_plan* plan, const void* taftp, long long T, int nantennas_total, int start_antenna,
+                           int S, const void* fba_weights, size_t weights_bytes, void* tbtf, size_t tbtf_bytes,
+                           hipStream_t s, int* partials, const IbFinishJob& ib)
+{
+    const TaftpView tv{S, nantennas_total, start_antenna, cb_taftp_form(plan, T, nantennas_total, kTaftpBatch),
+                       partials};
+    return cb_launch(plan, MODE_INT8, taftp, T, 2 * plan->d.nantennas, 0, fba_weights, weights_bytes, tbtf,
+                     tbtf_bytes, s, nullptr, 0, &tv, TailJobs{ib, WeightsJob{}});
 }
 
 extern "C" int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
@@ -1194,7 +1220,8 @@ extern "C" int fbf_cb_autotune(fbf_cb_plan* plan, long long nsamples, int reps, 
     const int saved_variant = plan->variant, saved_chunk = plan->chunk;
     int bv = saved_variant, bc = saved_chunk;
     float bms = 1e30f;
-    for (int var = 1; var < nvar; ++var) {
+    float auto_ms = 1e30f;   // the automatic pick (variant 0)
+    for (int var = 0; var < nvar; ++var) {
         std::vector<int> chunks{0};
         if (kCbVariants[var].lds && !kCbVariants[var].tr)
             for (int jc = jc_max / 2; jc >= 1; jc >>= 1) chunks.push_back(jc);
@@ -1217,18 +1244,30 @@ extern "C" int fbf_cb_autotune(fbf_cb_plan* plan, long long nsamples, int reps, 
             float ms = 0.0f;
             (void)hipEventElapsedTime(&ms, e0, e1);
             ms /= (float)reps;
-            if (ms < bms) {
+            if (var == 0) {
+                auto_ms = ms;
+            } else if (ms < bms) {
                 bms = ms;
                 bv = var;
                 bc = jc;
             }
         }
     }
-    plan->variant = bv;
+    // The automatic pick stays unless a variant beats it: it may be a form that
+    // no variant names (few beams), and leaves fbf_cb_beamform_taftp its own
+    // choice.  It is reported as the variant of its kernel.
+    const bool keep_auto = auto_ms <= 1.01f * bms;
+    if (keep_auto) {
+        const CbVariant v = cb_pick_variant(d, 0, MODE_INT8, nsamples);
+        bv = !v.tr ? kCbVariantLds : v.rows == 2 ? kCbVariantTr2 : v.rows == 4 ? kCbVariantTr4 : kCbVariantTr8;
+        bc = 0;
+        bms = auto_ms;
+    }
+    plan->variant = keep_auto ? 0 : bv;
     plan->chunk = bc;
     {
         std::lock_guard<std::mutex> lock(g_tune_mutex);
-        g_tune_table[tune_key(d)] = {bv, bc};
+        g_tune_table[tune_key(d)] = {plan->variant, bc};
     }
     cleanup();
     if (best_variant) *best_variant = bv;

@@ -6,6 +6,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <string>
+#include <utility>
 
 #include "../../include/fbfuse_hip.h"
 
@@ -59,7 +60,8 @@ inline bool split_ib_applies(const IbFuseParams& p)
 // ([F][T / 16][2 halves][32 columns] int32; sample j of a tile is the sum of
 // columns 2j, 2j + 1 of both halves), int8 TF of T samples with the IB
 // plan's scrunch and quantiser, as a job for nblocks work-groups of 256
-// threads of another launch (ib_finish_run).
+// threads of another launch (ib_finish_run).  nparts partials one after the
+// other (the subarrays that share the block's antennas out) are added up.
 struct IbFinishJob {
     const int* part;
     int8_t* out;
@@ -67,10 +69,23 @@ struct IbFinishJob {
     const float* scales;
     long long nwin;   // output windows (T / tscrunch)
     int ntiles, Fo, ts, fs, quant;
+    int nparts;
     int nblocks;      // 0: none
 };
-int ib_finish_job(const fbf_ib_plan* plan, const int* partials, long long T, void* tf, size_t tf_bytes,
+int ib_finish_job(const fbf_ib_plan* plan, const int* partials, int nparts, long long T, void* tf, size_t tf_bytes,
                   IbFinishJob* out);
+
+// A coherent plan's kernel variant and chunk length.
+std::pair<int, int> cb_plan_tuning(const fbf_cb_plan* plan);
+
+// A batch's subarray beamformed from the TAFTP block itself: whether the
+// plan's kernel stages such a block (with `partials`: and leaves the
+// incoherent beam's partials of its antennas), and the call, whose reorder
+// launch also runs the `ib` job.
+bool cb_batch_stages(const fbf_cb_plan* plan, long long T, int nantennas_total, int S, bool partials);
+int cb_batch_beamform(fbf_cb_plan* plan, const void* taftp, long long T, int nantennas_total, int start_antenna,
+                      int S, const void* fba_weights, size_t weights_bytes, void* tbtf, size_t tbtf_bytes,
+                      hipStream_t s, int* partials, const IbFinishJob& ib);
 
 // Weights generation (weights.hip), shared by weights_k and by launches that
 // generate the weights beside other work.  A thread takes one (beam,
@@ -195,23 +210,26 @@ __device__ __forceinline__ void ib_finish_run(const IbFinishJob& j, long long gi
     const long long w = valid ? i - (long long)fo * j.nwin : 0;
     long long P = 0;
     if (valid) {
-        for (int fc = 0; fc < j.fs; ++fc) {
-            const int* pf = j.part + (size_t)(fo * j.fs + fc) * j.ntiles * 64;
-            if (j.ts >= 16) {
-                // Whole tiles: the ts / 16 records, ts 16-byte pieces.
-                const int4* r = reinterpret_cast<const int4*>(pf + (size_t)(w * (j.ts / 16)) * 64);
-                for (int k = q; k < j.ts; k += 4) {
-                    const int4 v = r[k];
-                    P += (long long)v.x + v.y + v.z + v.w;
-                }
-            } else {
-                // Samples j0 .. j0 + ts - 1 of one tile: the column pairs
-                // j0 .. j0 + ts - 1 of both halves (8 bytes each).
-                const long long t0 = w * j.ts;
-                const int2* r = reinterpret_cast<const int2*>(pf + (size_t)(t0 >> 4) * 64) + (t0 & 15);
-                for (int k = q; k < 2 * j.ts; k += 4) {
-                    const int2 v = r[(k & 1) * 16 + (k >> 1)];
-                    P += (long long)v.x + v.y;
+        const int* base = j.part;
+        for (int k = 0; k < j.nparts; ++k, base += (size_t)j.Fo * j.fs * j.ntiles * 64) {
+            for (int fc = 0; fc < j.fs; ++fc) {
+                const int* pf = base + (size_t)(fo * j.fs + fc) * j.ntiles * 64;
+                if (j.ts >= 16) {
+                    // Whole tiles: the ts / 16 records, ts 16-byte pieces.
+                    const int4* r = reinterpret_cast<const int4*>(pf + (size_t)(w * (j.ts / 16)) * 64);
+                    for (int q4 = q; q4 < j.ts; q4 += 4) {
+                        const int4 v = r[q4];
+                        P += (long long)v.x + v.y + v.z + v.w;
+                    }
+                } else {
+                    // Samples j0 .. j0 + ts - 1 of one tile: the column pairs
+                    // j0 .. j0 + ts - 1 of both halves (8 bytes each).
+                    const long long t0 = w * j.ts;
+                    const int2* r = reinterpret_cast<const int2*>(pf + (size_t)(t0 >> 4) * 64) + (t0 & 15);
+                    for (int q4 = q; q4 < 2 * j.ts; q4 += 4) {
+                        const int2 v = r[(q4 & 1) * 16 + (q4 >> 1)];
+                        P += (long long)v.x + v.y;
+                    }
                 }
             }
         }

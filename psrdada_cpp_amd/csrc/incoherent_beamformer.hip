@@ -250,8 +250,8 @@ static int ib_run(fbf_ib_plan* plan, int mode, const void* taftp, size_t taftp_b
     return FBF_OK;
 }
 
-int fbf::ib_finish_job(const fbf_ib_plan* plan, const int* partials, long long T, void* tf, size_t tf_bytes,
-                       IbFinishJob* out)
+int fbf::ib_finish_job(const fbf_ib_plan* plan, const int* partials, int nparts, long long T, void* tf,
+                       size_t tf_bytes, IbFinishJob* out)
 {
     FBF_REQUIRE(plan && partials && tf && out, FBF_ERR_ARG, "fbf_ib: null argument");
     const fbf_ib_desc& d = plan->d;
@@ -266,7 +266,7 @@ int fbf::ib_finish_job(const fbf_ib_plan* plan, const int* partials, long long T
     const long long nblocks = (4 * nout + 255) / 256;
     FBF_REQUIRE(nblocks < (1ll << 30) && T / 16 < (1ll << 31), FBF_ERR_UNSUPPORTED, "fbf_ib: grid too large");
     *out = IbFinishJob{partials, static_cast<int8_t*>(tf), plan->d_levels, plan->d_levels + Fo, nwin, (int)(T / 16),
-                       Fo, d.tscrunch, d.fscrunch, d.quant_mode, (int)nblocks};
+                       Fo, d.tscrunch, d.fscrunch, d.quant_mode, nparts, (int)nblocks};
     return FBF_OK;
 }
 

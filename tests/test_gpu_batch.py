@@ -113,3 +113,46 @@ def test_autotune_picks_a_variant_that_is_bit_exact(gpu, oracle):
         d_o.fill(0)
         plan.beamform(d_v, d_w, d_o)
         np.testing.assert_array_equal(d_o.download(), oracle.cb_tbtf(p, off, sc, T // ts))
+
+
+@pytest.mark.parametrize("split,ts,fs,ib", [
+    ([(0, 24, 104), (24, 8, 8), (32, 32, 40)], 8, 1, (16, 1)),     # all antennas, the partials of three forms
+    ([(0, 40, 136), (40, 24, 64)], 64, 1, (64, 2)),                # two channels to an incoherent channel
+    ([(0, 16, 32), (16, 32, 32)], 16, 1, (16, 1)),                 # antennas 48..63 in no subarray: a pass of its own
+    ([(0, 40, 104), (32, 32, 104)], 16, 1, (16, 1)),               # antennas shared by two subarrays: likewise
+    ([(0, 32, 128), (32, 32, 104)], 16, 2, (1, 1)),                # fscrunch 2 leaves no partials
+    ([(0, 60, 40), (60, 4, 8)], 4, 1, (256, 1)),                   # antennas in fours
+    ([(0, 56, 40), (56, 8, 8)], 24, 1, (16, 1)),                   # tscrunch 24: the split-transposed block
+])
+def test_batch_straight_from_taftp(gpu, oracle, split, ts, fs, ib):
+    """Subarrays in turn from the TAFTP block itself, and the batch's
+    incoherent beam from their partials or from a pass of its own, against the
+    oracle; eagerly, captured and replayed on new voltages."""
+    capi = gpu
+    F, nhg = 4, 3
+    T = nhg * 256
+    subs = [dict(start_antenna=a0, nantennas=A, nbeams=B, tscrunch=ts, fscrunch=fs, nsamples_per_heap_out=T // ts)
+            for a0, A, B in split]
+    levels = [_levels(oracle, sd["nantennas"], ts, fs, F) for sd in subs]
+    batch = capi.Batch(A_TOT, F, nhg, subs, levels)
+    _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, 8, 16, 1, A_TOT, *ib)
+    ioff, isc = np.full(F // ib[1], ibo, np.float32), np.full(F // ib[1], ibs, np.float32)
+    batch.enable_ib(*ib, ioff, isc)
+    ws = [unit_weights(3500 + k, F * sd["nbeams"] * sd["nantennas"]) for k, sd in enumerate(subs)]
+    d_ws = [capi.DeviceBuffer.from_array(w) for w in ws]
+    outs = [capi.DeviceBuffer(batch.output_bytes(i)) for i in range(len(subs) + 1)]
+    s = capi.Stream()
+    for rep, use_graph in enumerate((False, True, True)):
+        taftp = gaussian_int8(3600 + rep, nhg * A_TOT * F * 256 * 4, 16.0)
+        d_taftp = capi.DeviceBuffer.from_array(taftp) if rep == 0 else d_taftp
+        if rep:
+            d_taftp.upload(taftp, s)
+        for o in outs:
+            o.fill(0x55, s)
+        batch.run(d_taftp, d_ws, outs, use_graph=use_graph, stream=s)
+        s.sync()
+        for k, sd in enumerate(subs):
+            ref = _reference(oracle, taftp, nhg, F, sd, ts, fs, levels[k][0], levels[k][1], T // ts, ws[k])
+            np.testing.assert_array_equal(outs[k].download(), ref, err_msg=f"run {rep} subarray {k}")
+        np.testing.assert_array_equal(outs[-1].download(),
+                                      oracle.ib_tf(oracle.ib_power(taftp, F, *ib, nhg, A_TOT), ioff, isc))
