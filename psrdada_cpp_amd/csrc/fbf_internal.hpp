@@ -183,6 +183,14 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks)
     return (bid % kNumXcd) * per + bid / kNumXcd;
 }
 
+// A 16-byte load of data that is read once, and the matching store.
+__device__ __forceinline__ int4 load_stream(const void* p)
+{
+    typedef int v4 __attribute__((ext_vector_type(4)));
+    const v4 v = __builtin_nontemporal_load(static_cast<const v4*>(p));
+    return int4{v.x, v.y, v.z, v.w};
+}
+
 // Quantiser shared by every output path: (P - offset) / scale in IEEE double,
 // round half away from zero (mode 0) or truncate (mode 1), saturate to int8.
 __device__ __forceinline__ int8_t quantise(double power, float offset, float scale, int mode)

@@ -7,12 +7,16 @@
 //               pols of re^2 + im^2,  out = quantise(P, offset[fo], scale[fo])
 // written TF: [heap_group * S / ts + window][fo].
 //
-// MI355X design: HBM-bound read of the whole TAFTP block.  A 256-thread block
-// owns one heap group and `cpb` channels; each 64-thread row reads one
-// 1 KiB (channel, antenna) row as 16-byte vectors (4 samples x 2 pols), so
-// every load instruction is fully coalesced, and squares with v_dot4_i32_i8
-// (exact int32).  tscrunch is reduced in-lane and across lanes with
-// shuffles, fscrunch across rows through LDS, in int64 (exact).
+// MI355X design: HBM-bound read of the whole TAFTP block.  A work-group owns
+// one heap group and output channel; its waves share the rows (channel,
+// antenna) out in contiguous runs, and each reads whole 1 KiB (channel, antenna) rows as
+// 16-byte vectors (4 samples x 2 pols a lane) and squares with v_dot4_i32_i8
+// (exact int32).  tscrunch is reduced in-lane and across lanes with shuffles,
+// the waves' sums through LDS, in int64 (exact).  Blocks of 16 MiB or more are
+// read past the cache (once), and work-groups that follow each other in a heap
+// group stay on one XCD.  64 antennas, 64 channels, 32 heaps, fscrunch 2:
+// 26.0 us with cached loads and a wave to each of four channels, 21.5 us now
+// (6.2 TB/s).
 //
 // fbf_ib_beamform_weights also generates the block's beamforming weights in
 // the same launch (its first work-groups), as the split-transpose launch can.
@@ -28,7 +32,7 @@ struct IbArgs {
     void* out;
     const float* offsets;
     const float* scales;
-    int nhg, A, F, Fo, ts, fs, quant, cpb, nfb;
+    int nhg, A, F, Fo, ts, fs, quant;
 };
 
 __device__ __forceinline__ int sq4(int x, int acc)
@@ -36,54 +40,71 @@ __device__ __forceinline__ int sq4(int x, int acc)
     return __builtin_amdgcn_sdot4(x, x, acc, false);
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256) void ib_k(IbArgs p, WeightsJob wj)
+// NW waves per work-group: 4, or 16 where the grid is small; PAST: the block
+// is read past the cache (ib_run).
+template <int MODE, int NW, bool PAST>
+__global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
 {
     constexpr int S = 256;
-    __shared__ long long part[4][S];
+    __shared__ long long part[NW][S];
     const int tid = threadIdx.x;
-    if (weights_job_run(wj, tid)) return;   // uniform over the work-group
+    if (NW == 4 && weights_job_run(wj, tid)) return;   // uniform over the work-group
     const int sc = tid & 63;   // 16-byte chunk: samples 4*sc .. 4*sc+3
-    const int row = tid >> 6;  // 0..3
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int logical = xcd_remap((int)blockIdx.x - wj.nblocks, (int)gridDim.x - wj.nblocks);
-    const int fb = logical % p.nfb;
-    const int hg = logical / p.nfb;
+    const int fo = logical % p.Fo;
+    const int hg = logical / p.Fo;
     if (hg >= p.nhg) return;
 
-    // One word squared is at most 4 * 128^2 = 2^16, so the int32 partials
-    // over one channel's antennas are exact for A < 2^15 (fbf_ib_plan_create
-    // checks it); each channel's partials are then added in int64.
+    // Rows (channel k, antenna a) of the output channel, antennas fastest; this
+    // wave's are [r, r1).  One word squared is at most 4 * 128^2 = 2^16, so
+    // int32 sums over kRun = 2^14 rows are exact; each run's are then added in
+    // int64.
+    constexpr int kRun = 1 << 14;
     long long s0 = 0, s1 = 0, s2 = 0, s3 = 0;
     const size_t row_bytes = (size_t)S * 4;
-    for (int k = 0; k < p.cpb / 4; ++k) {
-        int c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-        const int f = fb * p.cpb + row + 4 * k;
-        const int8_t* base = p.taftp + ((size_t)hg * p.A * p.F + f) * row_bytes + (size_t)sc * 16;
-        const size_t astride = (size_t)p.F * row_bytes;
-        int a = 0;
-        for (; a + 4 <= p.A; a += 4) {
-            int4 x[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const int4*>(base + (size_t)(a + u) * astride);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                c0 = sq4(x[u].x, c0);
-                c1 = sq4(x[u].y, c1);
-                c2 = sq4(x[u].z, c2);
-                c3 = sq4(x[u].w, c3);
-            }
+    const size_t astride = (size_t)p.F * row_bytes;
+    const int rows = p.fs * p.A;   // (1 KiB each: below 2^31)
+    const int per = (rows + NW - 1) / NW;
+    int r = min(wave * per, rows);
+    const int r1 = min(r + per, rows);
+    const int k0 = r / p.A;
+    int a = r - k0 * p.A;
+    const int8_t* row = p.taftp + ((size_t)hg * p.A * p.F + (size_t)fo * p.fs + k0) * row_bytes +
+                        (size_t)a * astride + (size_t)sc * 16;
+    auto next = [&]() {   // the current row, and on to the next
+        const int8_t* q = row;
+        row += astride;
+        if (++a == p.A) {
+            a = 0;
+            row += row_bytes - (size_t)p.A * astride;
         }
-        for (; a < p.A; ++a) {
-            const int4 x = *reinterpret_cast<const int4*>(base + (size_t)a * astride);
+        return q;
+    };
+    auto load = [](const int8_t* q) { return PAST ? load_stream(q) : *reinterpret_cast<const int4*>(q); };
+    while (r < r1) {
+        int c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+        const int n = min(r1 - r, kRun);
+        auto add = [&](int4 x) {
             c0 = sq4(x.x, c0);
             c1 = sq4(x.y, c1);
             c2 = sq4(x.z, c2);
             c3 = sq4(x.w, c3);
+        };
+        int i = 0;
+        for (; i + 4 <= n; i += 4) {
+            int4 x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = load(next());
+#pragma unroll
+            for (int u = 0; u < 4; ++u) add(x[u]);
         }
+        for (; i < n; ++i) add(load(next()));
         s0 += c0;
         s1 += c1;
         s2 += c2;
         s3 += c3;
+        r += n;
     }
 
     // tscrunch: per-sample sums s0..s3 cover samples 4*sc + {0..3}.
@@ -91,34 +112,39 @@ __global__ __launch_bounds__(256) void ib_k(IbArgs p, WeightsJob wj)
     if (p.ts >= 4) {
         long long v = s0 + s1 + s2 + s3;
         for (int m = 1; m < p.ts / 4; m <<= 1) v += __shfl_xor(v, m, 64);
-        if ((sc % (p.ts / 4)) == 0) part[row][sc / (p.ts / 4)] = v;
+        if ((sc % (p.ts / 4)) == 0) part[wave][sc / (p.ts / 4)] = v;
     } else if (p.ts == 2) {
-        part[row][2 * sc] = s0 + s1;
-        part[row][2 * sc + 1] = s2 + s3;
+        part[wave][2 * sc] = s0 + s1;
+        part[wave][2 * sc + 1] = s2 + s3;
     } else {
-        part[row][4 * sc] = s0;
-        part[row][4 * sc + 1] = s1;
-        part[row][4 * sc + 2] = s2;
-        part[row][4 * sc + 3] = s3;
+        part[wave][4 * sc] = s0;
+        part[wave][4 * sc + 1] = s1;
+        part[wave][4 * sc + 2] = s2;
+        part[wave][4 * sc + 3] = s3;
     }
     __syncthreads();
 
-    // fscrunch: rows belonging to one output channel are summed.
-    const int rows_per_fo = p.fs >= 4 ? 4 : p.fs;
-    const int nfo_blk = 4 / rows_per_fo;
-    for (int idx = tid; idx < nwin * nfo_blk; idx += 256) {
-        const int fl = idx / nwin;
-        const int w = idx - fl * nwin;
+    // The waves' sums of a window.
+    if (tid < nwin) {
         long long v = 0;
-        for (int r = 0; r < rows_per_fo; ++r) v += part[fl * rows_per_fo + r][w];
-        const int fo = (fb * p.cpb) / p.fs + fl;
-        const size_t t = (size_t)hg * nwin + w;
+#pragma unroll
+        for (int r = 0; r < NW; ++r) v += part[r][tid];
+        const size_t t = (size_t)hg * nwin + tid;
         if (MODE == IB_POWER) {
             static_cast<double*>(p.out)[t * p.Fo + fo] = (double)v;
         } else {
             static_cast<int8_t*>(p.out)[t * p.Fo + fo] = quantise((double)v, p.offsets[fo], p.scales[fo], p.quant);
         }
     }
+}
+
+template <int MODE>
+void launch_ib(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool wide, bool past, hipStream_t s)
+{
+    if (wide)
+        past ? ib_k<MODE, 16, true><<<grid, 1024, 0, s>>>(a, wj) : ib_k<MODE, 16, false><<<grid, 1024, 0, s>>>(a, wj);
+    else
+        past ? ib_k<MODE, 4, true><<<grid, 256, 0, s>>>(a, wj) : ib_k<MODE, 4, false><<<grid, 256, 0, s>>>(a, wj);
 }
 
 }  // namespace
@@ -237,15 +263,19 @@ static int ib_run(fbf_ib_plan* plan, int mode, const void* taftp, size_t taftp_b
     a.ts = d.tscrunch;
     a.fs = d.fscrunch;
     a.quant = d.quant_mode;
-    a.cpb = d.fscrunch > 4 ? d.fscrunch : 4;
-    a.nfb = d.nchans / a.cpb;
-    const long long nblocks = nhg * a.nfb + wj.nblocks;
+    const long long work = nhg * Fo;
+    const long long nblocks = work + wj.nblocks;
     FBF_REQUIRE(nblocks < (1ll << 31), FBF_ERR_UNSUPPORTED, "fbf_ib: grid too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // 16 waves share the rows of a small block's few work-groups, at least two
+    // each (the weights job is made of work-groups of 4).
+    const bool wide = work < 1024 && (long long)d.nantennas * d.fscrunch >= 32 && wj.nblocks == 0;
+    const bool past = taftp_bytes >= ((size_t)16 << 20);   // (smaller blocks may be in the cache)
+    const dim3 grid((unsigned)nblocks);
     if (mode == IB_INT8)
-        ib_k<IB_INT8><<<dim3((unsigned)nblocks), 256, 0, s>>>(a, wj);
+        launch_ib<IB_INT8>(a, wj, grid, wide, past, s);
     else
-        ib_k<IB_POWER><<<dim3((unsigned)nblocks), 256, 0, s>>>(a, wj);
+        launch_ib<IB_POWER>(a, wj, grid, wide, past, s);
     FBF_LAUNCH_CHECK("ib_k");
     return FBF_OK;
 }

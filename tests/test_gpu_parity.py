@@ -701,3 +701,41 @@ def test_cb_antennas_in_fours_bit_exact(gpu, oracle, variant, F, T, A, B, ts, fs
     d_o.fill(0x5A)
     plan.beamform_subarray(_dev(capi, blk.reshape(-1)), A + a0, a0, d_w, d_o)
     np.testing.assert_array_equal(d_o.download(), ref)
+
+
+@pytest.mark.parametrize("A,F,nhg,ts,fs", [
+    (5, 260, 4, 1, 1),       # four waves, fewer antennas than a run each
+    (3, 8, 2, 256, 2),       # 16 waves, most of them without antennas
+    (91, 4, 3, 2, 4),        # 16 waves, a short last run
+    (70, 352, 3, 16, 1),     # four waves of 18, 18, 18 and 16 antennas
+])
+def test_ib_antenna_runs_bit_exact(gpu, oracle, A, F, nhg, ts, fs):
+    """The incoherent beam's antennas shared out over 4 and 16 waves."""
+    capi = gpu
+    taftp = gaussian_int8(6300 + A, nhg * A * F * 256 * 4, 40.0, clip=False)
+    _, _, ibo, ibs = oracle.power_levels(40.0, 24.0, A, ts, fs, A, ts, fs)
+    off, sc = np.full(F // fs, ibo, np.float32), np.full(F // fs, ibs, np.float32)
+    plan = capi.IbPlan(A, F, ts, fs, off, sc)
+    d_in = _dev(capi, taftp)
+    p_ref = oracle.ib_power(taftp, F, ts, fs, nhg, A)
+    d_p, d_tf = capi.DeviceBuffer(p_ref.size * 8), capi.DeviceBuffer(plan.output_bytes(taftp.nbytes))
+    plan.power(d_in, d_p)
+    plan.beamform(d_in, d_tf)
+    np.testing.assert_array_equal(d_p.download(np.float64), p_ref.reshape(-1))
+    np.testing.assert_array_equal(d_tf.download(), oracle.ib_tf(p_ref, off, sc).reshape(-1))
+
+
+@pytest.mark.parametrize("A,used,a0,F,nhg,S", [
+    (20, 13, 3, 5, 2, 256), (70, 63, 7, 3, 1, 256),   # vectors across columns, 128-column tiles
+    (130, 127, 1, 3, 1, 256), (20, 13, 3, 5, 3, 32),  # and 64-column tiles
+    (150, 131, 2, 2, 1, 64), (140, 130, 5, 2, 1, 32), # two tiles of antennas: single ones and pairs
+    (70, 68, 1, 3, 2, 96), (70, 1, 69, 3, 2, 64),
+])
+def test_split_transpose_tile_shapes_bit_exact(gpu, oracle, A, used, a0, F, nhg, S):
+    capi = gpu
+    taftp = gaussian_int8(6400 + used + S, nhg * A * F * S * 4, 40.0)
+    d_out = capi.DeviceBuffer(nhg * used * F * S * 4)
+    d_out.fill(0x5A)
+    capi.split_transpose(_dev(capi, taftp), d_out, A, used, a0, F, nsamples_per_heap=S)
+    np.testing.assert_array_equal(d_out.download(),
+                                  oracle.split_transpose(taftp, nhg, A, used, a0, F, nsamples_per_heap=S))
