@@ -6,9 +6,15 @@
 // MI355X design: for one (heap group, channel) the input is A_used rows of
 // 2*S complex samples (1 KiB each for S = 256) at a stride of F KiB, and the
 // output is one contiguous [2*S][A_used] block.  A 256-thread block moves a
-// 64-antenna x 64-(sample,pol) tile: 16-byte coalesced row loads into LDS,
-// then each thread gathers U antennas of one (sample, pol) and writes them as
-// one 2*U-byte vector, so the output side is fully coalesced too.
+// tile of 64 antennas x 128 (sample, pol) or 128 x 64: 16-byte coalesced row
+// loads into LDS, then each thread gathers 8 consecutive elements of the
+// output block and writes them as one 16-byte vector, across columns where
+// the antennas are no multiple of 4 (the tile holds them all; multiples of 4
+// take 8-byte vectors), so the output side is coalesced for any antennas.  HBM-bound.  The stores are
+// nontemporal: the block written is as large as the one read, and leaves the
+// cache to it.  44 of 64 antennas, 64 channels, 12 heaps (69 MB moved):
+// 13.8 us with cached stores from 64-column tiles, 13.1 us now; 13 of
+// 17 antennas, 83 channels, 39 heaps: 36.9 us with 2-byte stores, 14.7 us now.
 //
 // A launch can also generate the block's beamforming weights: its first
 // work-groups run the weights generator (weights_run) and leave, and the
@@ -20,9 +26,8 @@
 namespace fbf {
 namespace {
 
-constexpr int kTileA = 64;    // antennas per LDS tile
-constexpr int kTileSP = 64;   // (sample, pol) elements per LDS tile
-constexpr int kPad = 2;       // int16 padding per LDS row (row stride 132 B)
+constexpr int kIbSamples = 32;   // samples whose windows a tile is sure to hold whole
+constexpr int kPad = 2;          // int16 padding per LDS row (an odd number of dwords)
 
 template <int U>
 struct VecOf;
@@ -30,6 +35,22 @@ template <> struct VecOf<8> { using T = int4; };
 template <> struct VecOf<4> { using T = int2; };
 template <> struct VecOf<2> { using T = int; };
 template <> struct VecOf<1> { using T = int16_t; };
+
+__device__ __forceinline__ void store_stream(int4 v, int16_t* dst)
+{
+    typedef int v4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(v4{v.x, v.y, v.z, v.w}, reinterpret_cast<v4*>(dst));
+}
+__device__ __forceinline__ void store_stream(int2 v, int16_t* dst)
+{
+    typedef int v2 __attribute__((ext_vector_type(2)));
+    __builtin_nontemporal_store(v2{v.x, v.y}, reinterpret_cast<v2*>(dst));
+}
+__device__ __forceinline__ void store_stream(int v, int16_t* dst)
+{
+    __builtin_nontemporal_store(v, reinterpret_cast<int*>(dst));
+}
+__device__ __forceinline__ void store_stream(int16_t v, int16_t* dst) { __builtin_nontemporal_store(v, dst); }
 
 // Incoherent beam computed from the same tiles (all antennas of the block):
 // output [sample_out][channel] int8, tscrunch dividing the tile's 32 samples,
@@ -41,24 +62,31 @@ struct IbTile {
     int tscrunch, quant;
 };
 
-template <int U, bool IB>
+// SP: columns of the tile (its antennas are 8192 / SP).  U > 0: vectors of U
+// antennas of one column (U divides used_nantennas); U = 0: 16-byte vectors
+// of the whole output block, all antennas in one tile; `inv` is then
+// ceil(2^32 / used_nantennas).
+template <int U, int SP, bool IB>
 __global__ __launch_bounds__(256) void split_transpose_k(
     const int16_t* __restrict__ in, int16_t* __restrict__ out,
     int nheap_groups, int total_nantennas, int used_nantennas, int start_antenna,
-    int nchans, int sp_per_heap, int n_sp_tiles, IbTile ib, WeightsJob wj)
+    int nchans, int sp_per_heap, int n_sp_tiles, uint32_t inv, IbTile ib, WeightsJob wj)
 {
-    __shared__ int16_t tile[kTileA][kTileSP + kPad];
-    __shared__ int ibsum[4][kTileSP / 2];
+    constexpr int kTileA = 8192 / SP;
+    constexpr int TPR = SP / 8;         // threads per row
+    constexpr int RPP = 256 / TPR;      // rows per pass
+    __shared__ int16_t tile[kTileA][SP + kPad];
+    __shared__ int ibsum[4][SP / 2];
     const int tid = threadIdx.x;
     if (weights_job_run(wj, tid)) return;   // uniform over the work-group
-    const int logical = xcd_remap((int)blockIdx.x - wj.nblocks, (int)gridDim.x - wj.nblocks);
+    const int logical = (int)blockIdx.x - wj.nblocks;
     const int spt = logical % n_sp_tiles;
     const int rest = logical / n_sp_tiles;
     const int hg = rest % nheap_groups;
     const int f = rest / nheap_groups;
     if (f >= nchans) return;
 
-    const size_t out_block = ((size_t)f * nheap_groups + hg) * sp_per_heap + (size_t)spt * kTileSP;
+    const size_t out_block = ((size_t)f * nheap_groups + hg) * sp_per_heap + (size_t)spt * SP;
     // Incoherent beam: a 16-byte row load holds 4 samples x 2 pols of one
     // antenna, and one sdot4 of a 4-byte word with itself is the power of
     // both pols of a sample.  This thread sums its 4 samples over the rows it
@@ -69,65 +97,90 @@ __global__ __launch_bounds__(256) void split_transpose_k(
 
     for (int ab = 0; ab < used_nantennas; ab += kTileA) {
         const int na = min(kTileA, used_nantennas - ab);
-        // 64 rows x 64 int16 = 8 threads of 16 B per row, 32 rows per pass.
+        const int col = (tid % TPR) * 8;
+        int4 v[kTileA / RPP];
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-            const int r = pass * 32 + (tid >> 3);
-            const int col = (tid & 7) * 8;
+        for (int pass = 0; pass < kTileA / RPP; ++pass) {
+            const int r = pass * RPP + tid / TPR;
             if (r < na) {
                 const size_t row = ((size_t)hg * total_nantennas + start_antenna + ab + r) * nchans + f;
-                const int4 v = *reinterpret_cast<const int4*>(in + row * sp_per_heap + (size_t)spt * kTileSP + col);
+                v[pass] = *reinterpret_cast<const int4*>(in + row * sp_per_heap + (size_t)spt * SP + col);
+            }
+        }
+#pragma unroll
+        for (int pass = 0; pass < kTileA / RPP; ++pass) {
+            const int r = pass * RPP + tid / TPR;
+            if (r < na) {
                 if (IB) {
-                    ibacc[0] = __builtin_amdgcn_sdot4(v.x, v.x, ibacc[0], false);
-                    ibacc[1] = __builtin_amdgcn_sdot4(v.y, v.y, ibacc[1], false);
-                    ibacc[2] = __builtin_amdgcn_sdot4(v.z, v.z, ibacc[2], false);
-                    ibacc[3] = __builtin_amdgcn_sdot4(v.w, v.w, ibacc[3], false);
+                    ibacc[0] = __builtin_amdgcn_sdot4(v[pass].x, v[pass].x, ibacc[0], false);
+                    ibacc[1] = __builtin_amdgcn_sdot4(v[pass].y, v[pass].y, ibacc[1], false);
+                    ibacc[2] = __builtin_amdgcn_sdot4(v[pass].z, v[pass].z, ibacc[2], false);
+                    ibacc[3] = __builtin_amdgcn_sdot4(v[pass].w, v[pass].w, ibacc[3], false);
                 }
                 uint32_t* dst = reinterpret_cast<uint32_t*>(&tile[r][col]);
-                dst[0] = (uint32_t)v.x;
-                dst[1] = (uint32_t)v.y;
-                dst[2] = (uint32_t)v.z;
-                dst[3] = (uint32_t)v.w;
+                dst[0] = (uint32_t)v[pass].x;
+                dst[1] = (uint32_t)v[pass].y;
+                dst[2] = (uint32_t)v[pass].z;
+                dst[3] = (uint32_t)v[pass].w;
             }
         }
         __syncthreads();
-        const int units = na / U;
-        for (int idx = tid; idx < kTileSP * units; idx += 256) {
-            const int sp = idx / units;
-            const int u = idx - sp * units;
-            union {
-                typename VecOf<U>::T v;
-                int16_t e[U];
-            } pack;
+        if constexpr (U > 0) {
+            const int units = na / U;
+            for (int idx = tid; idx < SP * units; idx += 256) {
+                const int sp = idx / units;
+                const int u = idx - sp * units;
+                union {
+                    typename VecOf<U>::T v;
+                    int16_t e[U];
+                } pack;
 #pragma unroll
-            for (int i = 0; i < U; ++i) pack.e[i] = tile[u * U + i][sp];
-            int16_t* dst = out + (out_block + sp) * used_nantennas + ab + u * U;
-            *reinterpret_cast<typename VecOf<U>::T*>(dst) = pack.v;
+                for (int i = 0; i < U; ++i) pack.e[i] = tile[u * U + i][sp];
+                store_stream(pack.v, out + (out_block + sp) * used_nantennas + ab + u * U);
+            }
+        } else {
+            // SP is a multiple of 8, so the block is whole 16-byte vectors
+            // and starts at one.
+            for (int idx = tid; idx < SP / 8 * used_nantennas; idx += 256) {
+                int sp = (int)__umulhi((uint32_t)idx * 8u, inv);
+                int a = idx * 8 - sp * used_nantennas;
+                union {
+                    int4 v;
+                    int16_t e[8];
+                } pack;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    pack.e[i] = tile[a][sp];
+                    if (++a == used_nantennas) {
+                        a = 0;
+                        ++sp;
+                    }
+                }
+                store_stream(pack.v, out + out_block * used_nantennas + (size_t)idx * 8);
+            }
         }
         __syncthreads();
     }
     if (IB) {
-        // Lanes with the same tid % 8 hold the same 4 samples for different
-        // rows: sum over the 8 of them in the wave, then over the 4 waves.
+        // Lanes with the same tid % TPR hold the same 4 samples for different
+        // rows: sum over them in the wave, then over the 4 waves.
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            ibacc[q] += __shfl_xor(ibacc[q], 8);
-            ibacc[q] += __shfl_xor(ibacc[q], 16);
-            ibacc[q] += __shfl_xor(ibacc[q], 32);
-        }
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int m = TPR; m < 64; m <<= 1) ibacc[q] += __shfl_xor(ibacc[q], m);
         const int lane = tid & 63;
-        if (lane < 8) {
+        if (lane < TPR) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) ibsum[tid >> 6][lane * 4 + q] = ibacc[q];
         }
         __syncthreads();
-        // 32 samples per tile -> 32 / tscrunch outputs.
-        const int nout = (kTileSP / 2) / ib.tscrunch;
+        // SP / 2 samples per tile -> SP / 2 / tscrunch outputs.
+        const int nout = (SP / 2) / ib.tscrunch;
         if (tid < nout) {
             long long P = 0;
             for (int c = tid * ib.tscrunch; c < (tid + 1) * ib.tscrunch; ++c)
                 P += (long long)ibsum[0][c] + ibsum[1][c] + ibsum[2][c] + ibsum[3][c];
-            const long long t0 = ((long long)hg * sp_per_heap + (long long)spt * kTileSP) / 2;
+            const long long t0 = ((long long)hg * sp_per_heap + (long long)spt * SP) / 2;
             const long long to = t0 / ib.tscrunch + tid;
             ib.out[to * nchans + f] = quantise((double)P, ib.offsets[f], ib.scales[f], ib.quant);
         }
@@ -141,41 +194,50 @@ using namespace fbf;
 
 namespace {
 
-template <bool IB>
+template <int SP, bool IB>
 int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna,
                 int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream)
 {
     const int sp_per_heap = 2 * nsamples_per_heap;
-    const int n_sp_tiles = sp_per_heap / kTileSP;
+    const int n_sp_tiles = sp_per_heap / SP;
     const size_t nblocks = (size_t)nchans * nhg * n_sp_tiles + (size_t)wj.nblocks;
     FBF_REQUIRE(nblocks < (1ull << 31), FBF_ERR_UNSUPPORTED, "fbf_split_transpose: grid too large");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const auto* in = static_cast<const int16_t*>(taftp);
-    auto* out = static_cast<int16_t*>(ftpa);
-    dim3 grid((unsigned)nblocks), block(256);
-    if (used_nantennas % 8 == 0)
-        split_transpose_k<8, IB><<<grid, block, 0, s>>>(in, out, nhg, total_nantennas, used_nantennas,
-                                                         start_antenna, nchans, sp_per_heap, n_sp_tiles, ib, wj);
-    else if (used_nantennas % 4 == 0)
-        split_transpose_k<4, IB><<<grid, block, 0, s>>>(in, out, nhg, total_nantennas, used_nantennas,
-                                                         start_antenna, nchans, sp_per_heap, n_sp_tiles, ib, wj);
-    else if (used_nantennas % 2 == 0)
-        split_transpose_k<2, IB><<<grid, block, 0, s>>>(in, out, nhg, total_nantennas, used_nantennas,
-                                                         start_antenna, nchans, sp_per_heap, n_sp_tiles, ib, wj);
-    else
-        split_transpose_k<1, IB><<<grid, block, 0, s>>>(in, out, nhg, total_nantennas, used_nantennas,
-                                                         start_antenna, nchans, sp_per_heap, n_sp_tiles, ib, wj);
+    // Vectors of 8 antennas where they divide; else, while one tile holds
+    // every antenna, 16-byte vectors across columns; else what divides.
+    const uint32_t inv = (uint32_t)(((1ull << 32) + used_nantennas - 1) / used_nantennas);
+    const auto kernel = used_nantennas % 8 == 0       ? split_transpose_k<8, SP, IB>
+                        : used_nantennas % 4 == 0     ? split_transpose_k<4, SP, IB>
+                        : used_nantennas == 1         ? split_transpose_k<1, SP, IB>
+                        : used_nantennas <= 8192 / SP ? split_transpose_k<0, SP, IB>
+                        : used_nantennas % 2 == 0        ? split_transpose_k<2, SP, IB>
+                                                         : split_transpose_k<1, SP, IB>;
+    kernel<<<dim3((unsigned)nblocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const int16_t*>(taftp), static_cast<int16_t*>(ftpa), nhg, total_nantennas, used_nantennas,
+        start_antenna, nchans, sp_per_heap, n_sp_tiles, inv, ib, wj);
     FBF_LAUNCH_CHECK("split_transpose_k");
     return FBF_OK;
+}
+
+template <bool IB>
+int st_launch_sp(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna,
+                 int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream)
+{
+    // Tiles of 128 columns where 64 antennas hold a subset and they divide a
+    // heap, else of 64 columns and 128 antennas.
+    if (used_nantennas <= 64 && nsamples_per_heap % 64 == 0)
+        return st_launch_t<128, IB>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
+                                    nsamples_per_heap, nhg, ib, wj, stream);
+    return st_launch_t<64, IB>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
+                               nsamples_per_heap, nhg, ib, wj, stream);
 }
 
 int st_launch(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna, int nchans,
               int nsamples_per_heap, int nhg, IbTile ib, fbf_stream_t stream, WeightsJob wj = WeightsJob{})
 {
     if (ib.out)
-        return st_launch_t<true>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
+        return st_launch_sp<true>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
                                  nsamples_per_heap, nhg, ib, wj, stream);
-    return st_launch_t<false>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
+    return st_launch_sp<false>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
                               nsamples_per_heap, nhg, ib, wj, stream);
 }
 
@@ -224,7 +286,7 @@ static int st_ib_params(const void* taftp, size_t taftp_bytes, const void* ftpa,
     if (st) return st;
     FBF_REQUIRE(ibp.nchans == nchans && ibp.nsamples_per_heap == nsamples_per_heap, FBF_ERR_ARG,
                 "fbf_split_transpose_ib: incoherent-beam plan geometry differs from the block's");
-    FBF_REQUIRE(ibp.fscrunch == 1 && ibp.tscrunch > 0 && (kTileSP / 2) % ibp.tscrunch == 0, FBF_ERR_UNSUPPORTED,
+    FBF_REQUIRE(ibp.fscrunch == 1 && ibp.tscrunch > 0 && kIbSamples % ibp.tscrunch == 0, FBF_ERR_UNSUPPORTED,
                 "fbf_split_transpose_ib: needs fscrunch 1 and a tscrunch dividing 32");
     const int A = ibp.nantennas;
     FBF_REQUIRE(nsamples_per_heap > 0 && nsamples_per_heap % 32 == 0, FBF_ERR_UNSUPPORTED,
