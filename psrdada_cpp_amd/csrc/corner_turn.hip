@@ -6,10 +6,15 @@
 //                       (meerkat/tools/src/feng_to_dada.cu:54-80)
 //
 // Both are, per batch, the transpose of an R x C matrix of E-byte elements.
-// corner_turn_k stages a T x T tile of elements through LDS so that global
-// reads are whole input rows (T elements of one row, contiguous) and global
-// writes whole output rows, moving 16-, 4- or 1-byte units.  HBM-bound:
-// every byte is read once and written once.
+// corner_turn_k stages a TR x TC tile of elements through LDS so that global
+// reads are runs of input rows (TC elements, contiguous) and global writes
+// runs of output rows, moving 16-, 4- or 1-byte units.  HBM-bound: every byte
+// is read once and written once.  A block of 16 MiB or more is stored past the
+// cache, which leaves the cache to what is read, and one of 128 MiB or more
+// is read past it too (64 beams, 128 channels, 64 samples, 32 bands, 10 groups,
+// 336 MB moved: 65.7 us all cached, 61.5 us with the stores past the cache,
+// 56.0 us with both; 16 heaps of 4096 channels, 134 MB moved: 25.6, 20.0 and
+// 23.8 us).
 #include "fbf_internal.hpp"
 
 #include <climits>
@@ -25,20 +30,62 @@ struct CtArgs {
     long long out_s1, out_s2;
     int R, C;                      // input rows and columns (elements)
     int EU;                        // units per element
-    int T;                         // tile edge (elements)
+    int TR, TC;                    // tile rows and columns (elements)
     int tiles_r, tiles_c;
-    int sh_ru, sh_eu;              // log2(T * EU), log2(EU) (when powers of two)
+    int sh_ru, sh_eu;              // square tiles: log2(TC * EU), log2(EU) (when powers of two)
+    uint32_t inv_eu;               // ceil(2^32 / EU)
+    bool load_past, store_past;    // the block is read, and written, past the cache
 };
 
-// Tile row pitch in units: T * EU + 1, so that the transposed reads of the
+// A store past the cache where `past` says so (units of 16 and 4 bytes; a
+// wave's 64 single bytes leave half a line for a later store).
+template <typename U>
+__device__ __forceinline__ void store_unit(U v, U* p, bool past)
+{
+    if constexpr (sizeof(U) == 16) {
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+        if (past)
+            __builtin_nontemporal_store(v4u{v.x, v.y, v.z, v.w}, reinterpret_cast<v4u*>(p));
+        else
+            *p = v;
+    } else if constexpr (sizeof(U) == 4) {
+        if (past)
+            __builtin_nontemporal_store(v, p);
+        else
+            *p = v;
+    } else {
+        *p = v;
+    }
+}
+
+// 16-byte loads of a block too large for the cache go past it (`past`).
+__device__ __forceinline__ uint4 load_unit(const uint4* p, bool past)
+{
+    if (past) {
+        const int4 v = load_stream(p);
+        return uint4{(uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w};
+    }
+    return *p;
+}
+template <typename U>
+__device__ __forceinline__ U load_unit(const U* p, bool)
+{
+    return *p;
+}
+
+// Tile row pitch in units: TC * EU + 1, so that the transposed reads of the
 // write phase (threads stepping down the tile rows) fall in distinct banks.
+// POW2: square tiles with TC * EU and EU powers of two take shifts where the
+// tile is full; else a wave takes rows, its lanes the units of a row, and the
+// write phase splits a unit index into (row, unit of the element) with one
+// multiplication.
 template <typename U, bool POW2>
 __global__ __launch_bounds__(256) void corner_turn_k(CtArgs a)
 {
     extern __shared__ __align__(16) uint8_t ct_lds[];
     U* tile = reinterpret_cast<U*>(ct_lds);
     const int EU = a.EU;
-    const int pitch = a.T * EU + 1;
+    const int pitch = a.TC * EU + 1;
     long long bid = blockIdx.x;
     const int tc = (int)(bid % a.tiles_c);
     bid /= a.tiles_c;
@@ -48,39 +95,48 @@ __global__ __launch_bounds__(256) void corner_turn_k(CtArgs a)
     const long long i1 = bid / a.n2;
     const U* in = reinterpret_cast<const U*>(a.in + i1 * a.in_s1 + i2 * a.in_s2);
     U* out = reinterpret_cast<U*>(a.out + i1 * a.out_s1 + i2 * a.out_s2);
-    const int r0 = tr * a.T, c0 = tc * a.T;
-    const int nr = min(a.T, a.R - r0), nc = min(a.T, a.C - c0);
+    const int r0 = tr * a.TR, c0 = tc * a.TC;
+    const int nr = min(a.TR, a.R - r0), nc = min(a.TC, a.C - c0);
     const size_t in_row = (size_t)a.C * EU, out_row = (size_t)a.R * EU;
     const U* src = in + (size_t)r0 * in_row + (size_t)c0 * EU;
     U* dst = out + (size_t)c0 * out_row + (size_t)r0 * EU;
 
-    if (POW2 && nr == a.T && nc == a.T) {
-        // Full tile, T * EU and EU powers of two: shifts instead of divisions.
-        const int n = a.T << a.sh_ru;
+    if (POW2 && nr == a.TR && nc == a.TC) {
+        // Full tile, TC * EU and EU powers of two: shifts instead of divisions.
+        const int n = a.TR << a.sh_ru;
         const int mu = (1 << a.sh_ru) - 1, me = EU - 1;
         for (int i = threadIdx.x; i < n; i += 256) {
             const int r = i >> a.sh_ru, k = i & mu;
-            tile[r * pitch + k] = src[(size_t)r * in_row + k];
+            tile[r * pitch + k] = load_unit(src + (size_t)r * in_row + k, a.load_past);
         }
         __syncthreads();
         for (int i = threadIdx.x; i < n; i += 256) {
             const int c = i >> a.sh_ru, k = i & mu;
             const int r = k >> a.sh_eu, e = k & me;
-            dst[(size_t)c * out_row + k] = tile[r * pitch + c * EU + e];
+            store_unit(tile[r * pitch + c * EU + e], dst + (size_t)c * out_row + k, a.store_past);
         }
-    } else {
-        const int ru = nc * EU;
-        for (int i = threadIdx.x; i < nr * ru; i += 256) {
-            const int r = i / ru, k = i - r * ru;
-            tile[r * pitch + k] = src[(size_t)r * in_row + k];
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int ru = nc * EU;
+    for (int r = wave; r < nr; r += 16) {   // up to four rows' loads in flight
+        for (int k = lane; k < ru; k += 64) {
+            U v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r + 4 * j < nr) v[j] = load_unit(src + (size_t)(r + 4 * j) * in_row + k, a.load_past);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (r + 4 * j < nr) tile[(r + 4 * j) * pitch + k] = v[j];
         }
-        __syncthreads();
-        const int ou = nr * EU;
-        for (int i = threadIdx.x; i < nc * ou; i += 256) {
-            const int c = i / ou, k = i - c * ou;
-            const int r = k / EU, e = k - r * EU;
-            dst[(size_t)c * out_row + k] = tile[r * pitch + c * EU + e];
-        }
+    }
+    __syncthreads();
+    const int ou = nr * EU;
+    for (int k = lane; k < ou; k += 64) {
+        const int r = EU == 1 ? k : (int)__umulhi((uint32_t)k, a.inv_eu);
+        const U* t = tile + r * pitch + (k - r * EU);
+        for (int c = wave; c < nc; c += 4) store_unit(t[c * EU], dst + (size_t)c * out_row + k, a.store_past);
     }
 }
 
@@ -112,7 +168,7 @@ __global__ __launch_bounds__(256) void corner_turn_w4_k(CtArgs a)
         for (int j = 0; j < 4; ++j) {
             const int i = threadIdx.x + 256 * j;
             const int r = i >> 4, c = (i & 15) << 2;
-            const uint4 v = *reinterpret_cast<const uint4*>(src + (size_t)r * a.C + c);
+            const uint4 v = load_unit(reinterpret_cast<const uint4*>(src + (size_t)r * a.C + c), a.load_past);
             uint32_t* l = tile + r * P + c;
             l[0] = v.x;
             l[1] = v.y;
@@ -129,7 +185,7 @@ __global__ __launch_bounds__(256) void corner_turn_w4_k(CtArgs a)
             v.y = tile[(r + 1) * P + c];
             v.z = tile[(r + 2) * P + c];
             v.w = tile[(r + 3) * P + c];
-            *reinterpret_cast<uint4*>(dst + (size_t)c * a.R + r) = v;
+            store_unit(v, reinterpret_cast<uint4*>(dst + (size_t)c * a.R + r), a.store_past);
         }
     } else {
         for (int i = threadIdx.x; i < nr * nc; i += 256) {
@@ -152,13 +208,17 @@ inline int ilog2_exact(long long v)
     return s;
 }
 
-// Largest tile edge (power of two, at most 64) whose rows hold at most 64
-// units and whose tile fits the LDS budget.
+// Tile: square, the edge the largest power of two up to 64 whose rows hold
+// at most 1 KiB within the LDS budget; where the matrix has fewer rows than
+// that, all of them and as many more columns.  Rows of 64 units left 1- and
+// 4-byte units with tiles of one or two elements (23 channels, 92 samples, 44
+// bands, 72 beams and groups, 13 MB moved: 75 us, 13.2 us now).
 constexpr size_t kCtLdsMax = 32 * 1024;
+constexpr size_t kCtRow = 1024;
 
-inline size_t ct_tile_bytes(int T, int EU, size_t U)
+inline size_t ct_tile_bytes(int TR, int TC, int EU, size_t U)
 {
-    return (size_t)T * ((size_t)T * EU + 1) * U;
+    return (size_t)TR * ((size_t)TC * EU + 1) * U;
 }
 
 template <typename U>
@@ -166,18 +226,28 @@ int ct_launch_u(CtArgs a, long long n1, int E, hipStream_t s)
 {
     a.EU = E / (int)sizeof(U);
     int T = 64;
-    while (T > 1 && ((long long)T * a.EU > 64 || ct_tile_bytes(T, a.EU, sizeof(U)) > kCtLdsMax)) T >>= 1;
-    a.T = T;
-    const size_t shm = ct_tile_bytes(T, a.EU, sizeof(U));
-    FBF_REQUIRE(shm <= kCtLdsMax, FBF_ERR_UNSUPPORTED, "corner turn: element too large (at most 32 KiB - 16 B)");
-    a.tiles_r = (a.R + T - 1) / T;
-    a.tiles_c = (a.C + T - 1) / T;
+    while (T > 1 && ((size_t)T * E > kCtRow || ct_tile_bytes(T, T, a.EU, sizeof(U)) > kCtLdsMax)) T >>= 1;
+    auto tiles = [&](int tr, int tc) { return n1 * a.n2 * ((a.R + tr - 1) / tr) * ((a.C + tc - 1) / tc); };
+    // A small block takes smaller tiles, down to 256-byte rows, to fill the chip.
+    while (T > 1 && (size_t)T * E >= 512 && tiles(T, T) < 512) T >>= 1;
+    a.TR = a.TC = T;
+    if (a.R < T) {
+        a.TR = a.R;
+        for (int tc = T * T / a.R; tc > T && a.TC == T; tc -= T)
+            if (ct_tile_bytes(a.TR, tc, a.EU, sizeof(U)) <= kCtLdsMax && tiles(a.TR, tc) >= 512) a.TC = tc;
+    }
+    const size_t shm = ct_tile_bytes(a.TR, a.TC, a.EU, sizeof(U));
+    FBF_REQUIRE(ct_tile_bytes(1, 1, a.EU, sizeof(U)) <= kCtLdsMax, FBF_ERR_UNSUPPORTED,
+                "corner turn: element too large (at most 32 KiB - 16 B)");
+    a.tiles_r = (a.R + a.TR - 1) / a.TR;
+    a.tiles_c = (a.C + a.TC - 1) / a.TC;
     const long long nblocks = n1 * a.n2 * a.tiles_r * a.tiles_c;
     if (nblocks == 0) return FBF_OK;
     FBF_REQUIRE(nblocks < INT_MAX, FBF_ERR_UNSUPPORTED, "corner turn: too many tiles for one launch");
     a.sh_ru = ilog2_exact((long long)T * a.EU);
     a.sh_eu = ilog2_exact(a.EU);
-    const bool pow2 = a.sh_ru >= 0 && a.sh_eu >= 0;
+    a.inv_eu = (uint32_t)(((1ull << 32) + a.EU - 1) / a.EU);   // (0 for EU = 1, unused)
+    const bool pow2 = a.TR == T && a.sh_ru >= 0 && a.sh_eu >= 0;
     if (pow2)
         corner_turn_k<U, true><<<dim3((unsigned)nblocks), 256, shm, s>>>(a);
     else
@@ -189,12 +259,15 @@ int ct_launch_u(CtArgs a, long long n1, int E, hipStream_t s)
 // 16-byte units when every element and base is 16-byte aligned, else 4, else 1.
 int ct_launch(CtArgs a, long long n1, int E, hipStream_t s)
 {
+    const long long bytes = n1 * a.n2 * a.R * a.C * E;
+    a.load_past = bytes >= (128ll << 20);
+    a.store_past = bytes >= (16ll << 20);
     const uintptr_t al = reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out) |
                          (uintptr_t)a.in_s1 | (uintptr_t)a.in_s2 | (uintptr_t)a.out_s1 | (uintptr_t)a.out_s2;
     if (E == 4 && ((al | (uintptr_t)a.R * 4 | (uintptr_t)a.C * 4) & 15) == 0) {
         // word transposes with 16-byte global accesses (rows 16-byte aligned)
         a.EU = 1;
-        a.T = 64;
+        a.TR = a.TC = 64;
         a.tiles_r = (a.R + 63) / 64;
         a.tiles_c = (a.C + 63) / 64;
         const long long nblocks = n1 * a.n2 * a.tiles_r * a.tiles_c;

@@ -77,3 +77,23 @@ def test_feng_to_dada_rejects_bad_sizes(gpu):
         capi.call("fbf_feng_to_dada", d.ptr, capi.DeviceBuffer(d.nbytes).ptr, d.nbytes - 4, 32, None)
     with pytest.raises(RuntimeError, match="distinct"):
         capi.feng_to_dada(d, d, 32)
+
+
+@pytest.mark.parametrize("C,S,F,B,G,b0,nb", [
+    (23, 92, 44, 3, 2, 1, 2),        # bytes, odd elements, partial tiles both ways
+    (1, 300, 7, 2, 1, 0, 2),         # single bytes, fewer bands than a tile has rows
+    (148, 70, 41, 2, 2, 0, 2),       # 4-byte units, 37 to an element
+    (4, 289, 54, 2, 3, 0, 1),        # one 4-byte unit, rows of no 16-byte multiple
+    (48, 133, 5, 7, 2, 2, 5),        # 16-byte units, three to an element, few bands
+    (256, 64, 32, 33, 1, 0, 33),     # 16 MiB and more: stored past the cache
+    (36, 512, 64, 15, 1, 0, 15),     # the same in 4-byte units
+])
+def test_tuse_transpose_tile_shapes_bit_exact(gpu, C, S, F, B, G, b0, nb):
+    """Tile shapes by unit size, bands and block size against numpy."""
+    capi = gpu
+    rng = np.random.default_rng(C + S + F)
+    x = rng.integers(-128, 128, (G, B, F, S, C), dtype=np.int8)
+    d_out = capi.DeviceBuffer(G * nb * F * S * C)
+    capi.tuse_transpose(_dev(capi, x), d_out, C, S, F, B, G, beam0=b0, nbeams_out=nb)
+    ref = np.ascontiguousarray(x[:, b0:b0 + nb].transpose(1, 0, 3, 2, 4))
+    np.testing.assert_array_equal(d_out.download(), ref.reshape(-1))
