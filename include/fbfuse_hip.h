@@ -198,9 +198,9 @@ int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_block, size_t b
  * with fbf_cb_beamform, calls with one plan on different streams must not
  * overlap (they share the plan's buffers).  The automatic variant stages the
  * block itself with 128 beams per wave up to 64 antennas (32 or 64 for at
- * most so many beams) and with 64 above; a subset of at most 48 antennas with
- * at most 96 beams, and more than 64 antennas with at most 32, are
- * split-transposed. */
+ * most so many beams) and with 64 above; of blocks of at most 4096 channels x
+ * samples, a subset of at most 48 antennas with at most 96 beams, and more
+ * than 64 antennas with at most 32, are split-transposed. */
 int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes,
                           int nantennas_total, int start_antenna, int nsamples_per_heap,
                           const void* fba_weights, size_t weights_bytes,
@@ -277,9 +277,9 @@ int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void
 /* *fused = 1 when fbf_cb_ib_beamform_taftp forms the incoherent beam inside
  * the coherent kernel: fscrunch 1, the block staged by that kernel (every
  * automatic pick; 128 beams per wave, or 64 above 64 antennas) and an
- * incoherent-beam plan of the same antennas, channels and heap size (up to
- * 48 antennas with at most 96 beams one of fscrunch 1).  No counterpart in
- * the reference. */
+ * incoherent-beam plan of the same antennas, channels and heap size (of
+ * fscrunch 1 for at most 4096 channels x samples of up to 48 antennas and 96
+ * beams).  No counterpart in the reference. */
 int fbf_cb_ib_fused(const fbf_cb_plan* plan, const fbf_ib_plan* ib_plan, int nsamples_per_heap,
                     long long nsamples, int* fused);
 

@@ -865,25 +865,9 @@ inline int cb_tr_nslot(int rt, int W)
 // step outweighs the MFMA work.
 constexpr bool tr_four_waves(int rt, int ksteps) { return rt == 8 || (rt == 4 && ksteps > 4); }
 
-// Beam groups per four-wave work-group: 4 / fs, or fewer (and as many more
-// time slots) where that many would leave waves without beams.  Fewer beam
-// groups stage each tile for fewer waves, so they have to win a tenth, and
-// over more than four K steps the ring holds two time slots at most.
+// Fewest beam groups per four-wave work-group: over more than four K steps the
+// ring holds two time slots at most.
 constexpr int tr_nwb_min(int ksteps) { return ksteps > 4 ? 2 : 1; }
-
-inline int tr_nwb(int rt, int ksteps, int fs, int B)
-{
-    const int groups = (B + 16 * rt - 1) / (16 * rt);
-    int best = 4 / fs, cost = (groups + best - 1) / best * best;   // wave slots taken
-    for (int n = best / 2; n >= tr_nwb_min(ksteps); n /= 2) {
-        const int c = (groups + n - 1) / n * n;
-        if (10 * c <= 9 * cost) {
-            best = n;
-            cost = c;
-        }
-    }
-    return best;
-}
 
 // Time slots per work-group.
 constexpr int tr_nts(int rt, int ksteps, int nslot, int fs, int nwb)
@@ -934,22 +918,45 @@ inline int device_cu_count()
 // round wherever it fills the slots; 192 units on 512 slots (40 antennas, 768
 // beams, 64 channels) left a quarter of them empty: 185 us in one round, 165 us
 // in three (8192 samples, tscrunch 16).
-inline long long tr_groups_per_unit(long long units, long long slots, int passes, int nts, int ntp)
+struct TrRounds {
+    long long per_unit;   // work-groups per (channel group, beam group)
+    long long cost;       // tile steps in a row
+};
+
+inline TrRounds tr_rounds(long long units, long long slots, int passes, int nts, int ntp)
 {
     constexpr int kStart = 5;
     const long long most = (passes + nts - 1) / nts;
-    long long best = 1, best_cost = 0;
+    TrRounds best{1, 0};
     for (int round = 1; round <= 8; ++round) {   // the most work-groups of each number of rounds
         long long n = round * slots / units;
         n = n < 1 ? 1 : n > most ? most : n;
         const long long np = (passes + n * nts - 1) / (n * nts);   // passes per slot
         const long long groups = (passes + np * nts - 1) / (np * nts);
         const long long cost = (units * groups + slots - 1) / slots * (np * ntp + kStart);
-        if (best_cost == 0 || cost < best_cost) {
+        if (best.cost == 0 || cost < best.cost) best = {n, cost};
+        if (n == most) break;
+    }
+    return best;
+}
+
+// Beam groups per four-wave work-group: 4 / fs, or fewer (and as many more
+// time slots) where that takes fewer tile steps in a row (more beam groups
+// would leave waves without beams).  Fewer beam groups stage each tile for
+// fewer waves, so they have to win a tenth.
+inline int tr_nwb(int rt, int ksteps, int fs, const CbTrArgs& a, int passes)
+{
+    const long long slots = (long long)tr_wgs(rt, ksteps) * device_cu_count();
+    int best = 4 / fs;
+    long long best_cost = 0;
+    for (int n = best; n >= tr_nwb_min(ksteps); n /= 2) {
+        const int beams = 16 * rt * n;
+        const long long units = (long long)a.p.Fo * ((a.p.B + beams - 1) / beams);
+        const long long cost = tr_rounds(units, slots, passes, 4 / (fs * n), a.ntp).cost;
+        if (best_cost == 0 || 10 * cost <= 9 * best_cost) {
             best = n;
             best_cost = cost;
         }
-        if (n == most) break;
     }
     return best;
 }
@@ -971,7 +978,7 @@ hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
         occ = o;
     }
     const long long units = (long long)a.p.Fo * a.n_bgroups;
-    const long long per_unit = tr_groups_per_unit(units, (long long)occ * device_cu_count(), passes, NTS, a.ntp);
+    const long long per_unit = tr_rounds(units, (long long)occ * device_cu_count(), passes, NTS, a.ntp).per_unit;
     a.npasses = (int)((passes + per_unit * NTS - 1) / (per_unit * NTS));
     a.n_tgroups = (int)((passes + (long long)a.npasses * NTS - 1) / ((long long)a.npasses * NTS));
     const long long nblocks = units * a.n_tgroups;
@@ -1005,7 +1012,7 @@ template <int RT, int KSTEPS, int SPT, int NSLOT, int FS>
 hipError_t launch_tr_k(const CbTrArgs& a, int passes, hipStream_t s)
 {
     if constexpr (tr_four_waves(RT, KSTEPS)) {
-        const int nwb = tr_nwb(RT, KSTEPS, FS, a.p.B);
+        const int nwb = tr_nwb(RT, KSTEPS, FS, a, passes);
         if constexpr (FS <= 2 && tr_nwb_min(KSTEPS) == 1)
             if (nwb == 1) return launch_tr_kn<RT, KSTEPS, SPT, NSLOT, FS, 1>(a, passes, s);
         if constexpr (FS == 1)

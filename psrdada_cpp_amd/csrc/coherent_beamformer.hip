@@ -229,7 +229,9 @@ __global__ __launch_bounds__(256) void tbtf_k(TbtfArgs a, IbFinishJob job, Weigh
             v.y = l[1];
             v.z = l[2];
             v.w = l[3];
-            *reinterpret_cast<uint4*>(out + b * brow + (size_t)t * a.Fo + 16 * w) = v;
+            typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(v4u{v.x, v.y, v.z, v.w},
+                                        reinterpret_cast<v4u*>(out + b * brow + (size_t)t * a.Fo + 16 * w));
         }
     } else if ((a.Fo & 3) == 0) {
         const int nw = fv >> 2;
@@ -834,9 +836,12 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 // 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
 // of 32 or 64 beams for so few took 8.6 and 33.7 us where 128-beam waves took
 // 10.8 and 41.0.
-// On their own (kTaftpAlone), a subset of at most 48 antennas with at most 96
-// beams and more than 64 antennas with at most 32 keep the split-transpose,
-// as fbf_cb_taftp_direct has always answered for them.
+// Blocks of at most kTaftpSmall channels x samples keep the split-transpose
+// where fbf_cb_taftp_direct has always answered so: at most 96 beams of up to
+// 48 antennas (unless both beams of the whole block are formed), at most 32 of
+// more than 64 on their own.
+constexpr long long kTaftpSmall = 4096;
+
 enum TaftpUse {
     kTaftpAlone,     // fbf_cb_beamform_taftp
     kTaftpOnePass,   // with the incoherent beam of the whole block
@@ -849,7 +854,7 @@ static TaftpForm cb_taftp_form(const fbf_cb_plan* plan, long long T, int nantenn
     const TaftpForm none{0, false};
     const CbVariant v = cb_pick_variant(d, plan->variant, MODE_INT8, T);
     const int ksteps = (2 * d.nantennas + 31) / 32;
-    if (plan->variant <= 0 && use != kTaftpBatch) {
+    if (plan->variant <= 0 && use != kTaftpBatch && (long long)d.nchans * T <= kTaftpSmall) {
         if (ksteps > 4 && d.nbeams <= 32 && use == kTaftpAlone) return none;
         const bool whole = d.fscrunch == 1 && nantennas_total == d.nantennas;
         if ((ksteps <= 3 || (ksteps == 4 && d.fscrunch > 1)) && d.nbeams <= 96 && !whole) return none;
@@ -949,15 +954,18 @@ extern "C" int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_
 // coherent beamformer: the block staged by four-wave work-groups (every
 // automatic form at fscrunch 1; 128 beams per wave, or 64 above 64 antennas),
 // and an incoherent-beam plan of the same block (antennas, channels, heap
-// size).  Up to 48 antennas with at most 96 beams an incoherent beam of several
-// channels keeps its own pass, as fbf_cb_ib_fused has always answered.
+// size).  In a small block (kTaftpSmall) of up to 48 antennas and 96 beams an
+// incoherent beam of several channels keeps its own pass, as fbf_cb_ib_fused
+// has always answered.
 static bool cb_ib_fused(const fbf_cb_plan* plan, const IbFuseParams& ibp, long long T, int S)
 {
     const fbf_cb_desc& d = plan->d;
     const TaftpForm form = cb_taftp_form(plan, T, d.nantennas, kTaftpOnePass);
     const int ksteps = (2 * d.nantennas + 31) / 32;
     if (form.rt == 0 || d.fscrunch != 1 || !(form.few || tr_four_waves(form.rt, ksteps))) return false;
-    if (ksteps <= 3 && d.nbeams <= 96 && ibp.fscrunch > 1 && plan->variant <= 0) return false;
+    if ((long long)d.nchans * T <= kTaftpSmall && ksteps <= 3 && d.nbeams <= 96 && ibp.fscrunch > 1 &&
+        plan->variant <= 0)
+        return false;
     return cb_taftp_stages(plan, T, d.nantennas, S) && ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
            ibp.nsamples_per_heap == S;
 }
