@@ -146,9 +146,9 @@ int fbf_cb_plan_destroy(fbf_cb_plan* plan);
 int fbf_cb_plan_set_variant(fbf_cb_plan* plan, int variant);
 int fbf_cb_variant_count(int* count);
 int fbf_cb_output_bytes(const fbf_cb_plan* plan, size_t ftpa_bytes, size_t* tbtf_bytes);
-/* FTPA + FBA -> int8 TBTF.  The int8 beams pass through a staging buffer
- * ([Fo][To][B], the size of the output) that the plan owns and grows on
- * demand, so calls with one plan on different streams must not overlap, and
+/* FTPA + FBA -> int8 TBTF.  The int8 beams pass (but for small blocks of few
+ * beams) through a staging buffer ([Fo][To][B], the size of the output) that
+ * the plan owns and grows on demand, so calls with one plan on different streams must not overlap, and
  * a stream that is being captured needs fbf_cb_plan_reserve first. */
 int fbf_cb_beamform(fbf_cb_plan* plan, const void* ftpa, size_t ftpa_bytes,
                     const void* fba_weights, size_t weights_bytes,

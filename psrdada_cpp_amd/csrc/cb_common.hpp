@@ -50,6 +50,13 @@ struct CbTrArgs {
     // antennas and both pols split over columns 2j, 2j + 1 (its pols) of
     // both halves (ib_finish_run adds the four).
     int* ibp;
+    // The few-beam kernel of a small block (cb_tbtf_direct): the outputs go
+    // straight to TBTF at `tbtf` (else null), the incoherent beam of `ib`
+    // (ib.out null: none, or partials) to its output, and the first
+    // weights.nblocks work-groups generate weights.
+    int8_t* tbtf;
+    IbFinishJob ib;
+    WeightsJob weights;
 };
 
 struct CbWsArgs {
@@ -199,8 +206,9 @@ __device__ __forceinline__ bool wave_any(bool x)
 // weight (CoherentBeamformer.cu:150-155); the power is exact in int64 and the
 // quantiser is the exact one.  The path of waves (or work-groups) whose
 // weights hold a wi = -128; consecutive threads take consecutive beams, so a
-// wave's voltage reads are one broadcast column.
-template <int MODE>
+// wave's voltage reads are one broadcast column.  TBTF: the int8 output goes to
+// TBTF instead ([To/ohs][B][ohs][Fo]).
+template <int MODE, bool TBTF = false>
 __device__ __forceinline__ void cb_exact_outputs(const CbArgs& p, int fo, int b0, int nb, long long w0,
                                                  long long w1, int t, int nt)
 {
@@ -250,7 +258,13 @@ __device__ __forceinline__ void cb_exact_outputs(const CbArgs& p, int fo, int b0
         }
         const size_t o = ((size_t)fo * p.nsamples_out + (size_t)w) * p.B + b;
         if (MODE == MODE_POWER) static_cast<double*>(p.out)[o] = (double)P;
-        if (MODE == MODE_INT8) static_cast<int8_t*>(p.out)[o] = quantise((double)P, off, sc, p.quant);
+        if constexpr (TBTF) {
+            const long long heap = w / p.ohs;
+            const size_t ot = ((size_t)(heap * p.B + b) * p.ohs + (size_t)(w - heap * p.ohs)) * p.Fo + fo;
+            static_cast<int8_t*>(p.out)[ot] = quantise((double)P, off, sc, p.quant);
+        } else if (MODE == MODE_INT8) {
+            static_cast<int8_t*>(p.out)[o] = quantise((double)P, off, sc, p.quant);
+        }
     }
 }
 

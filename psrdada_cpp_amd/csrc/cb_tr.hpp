@@ -106,6 +106,28 @@ __device__ __forceinline__ void cb_exact_ib_partials(const CbArgs& p, int* ibp, 
     }
 }
 
+// The same work-groups' incoherent-beam outputs where the kernel writes them
+// itself (windows within a tile): one window per thread.
+__device__ __forceinline__ void cb_exact_ib_outputs(const CbArgs& p, const IbFinishJob& ib, int f, int t0, int t1,
+                                                 int tid, int nt)
+{
+    const size_t astep = (size_t)p.F * p.S * 4;
+    const int per_tile = 16 / ib.ts;
+    for (int i = tid; i < (t1 - t0) * per_tile; i += nt) {
+        const long long w = (long long)t0 * per_tile + i;
+        int sum = 0;
+        for (int j = 0; j < ib.ts; ++j) {
+            const long long t = w * ib.ts + j;
+            const int8_t* v = p.ftpa + (((size_t)(t / p.S) * p.Atot + p.a0) * p.F + f) * p.S * 4 + (size_t)(t % p.S) * 4;
+            for (int a = 0; a < p.A; ++a) {
+                const int x = *reinterpret_cast<const int*>(v + a * astep);
+                sum = __builtin_amdgcn_sdot4(x, x, sum, false);
+            }
+        }
+        ib.out[w * p.F + f] = quantise((double)sum, ib.offsets[f], ib.scales[f], ib.quant);
+    }
+}
+
 // The 16-byte A operands of one step's K slices (8 antennas x char2 of one
 // column each) from an LDS tile laid out [antenna][32 columns] int16, 64
 // bytes a row: two ds_read_b64_tr_b16 of 4 antenna rows each per slice.
@@ -196,10 +218,12 @@ __device__ __forceinline__ void tr_operands(const int8_t* src, v4i (&a)[KSTEPS])
 // wave (every K slice): per lane the power of its column over the 8 * KSTEPS
 // antennas of its row half, each word (two antennas' re, im) squared with
 // v_dot4, antenna groups of 4 past A left out (they re-read antenna 0); the
-// 64 lanes store their sums as the tile's [2 halves][32 columns] record.
+// 64 lanes store their sums as the tile's [2 halves][32 columns] record
+// (ib_tile), or add them up over each window's columns (at most 128 antennas
+// x 16 samples x 2 pols x 2^15 < 2^31) and store the window's quantised output
+// (ib_tile_outputs).
 template <int KSTEPS>
-__device__ __forceinline__ void ib_tile(const v4i (&a)[KSTEPS], int* ibp, int ntiles, int A, int f, int tile,
-                                        int lane)
+__device__ __forceinline__ int ib_columns(const v4i (&a)[KSTEPS], int A, int lane)
 {
     int v = 0;
     if (A == 16 * KSTEPS) {   // uniform: no padded rows, one dot chain
@@ -218,7 +242,47 @@ __device__ __forceinline__ void ib_tile(const v4i (&a)[KSTEPS], int* ibp, int nt
                 v += 8 * (h * KSTEPS + s) + 2 * q < A ? t : 0;
             }
     }
+    return v;
+}
+
+template <int KSTEPS>
+__device__ __forceinline__ void ib_tile(const v4i (&a)[KSTEPS], int* ibp, int ntiles, int A, int f, int tile,
+                                        int lane)
+{
+    const int v = ib_columns<KSTEPS>(a, A, lane);
     if (tile < ntiles) ibp[((size_t)f * ntiles + tile) * 64 + lane] = v;
+}
+
+// v plus its value in the lane that the data-parallel-primitive control names.
+template <int CTRL>
+__device__ __forceinline__ int add_dpp(int v)
+{
+    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+
+// `off` and `sc` are the channel's levels, read before the tile loop by scalar
+// loads.  The sums over a window's 2 ts columns and both halves stay in the
+// VALU (four DPP steps and two lane swaps).  With the sums through LDS and the
+// levels read per tile, the block of 16 antennas, 16 channels, 2048 spectra
+// and 32 beams took 8.2 us against 6.9; keeping the sums for one quantisation
+// of all tiles gained nothing more.
+template <int KSTEPS>
+__device__ __forceinline__ void ib_tile_outputs(const v4i (&a)[KSTEPS], const IbFinishJob& ib, float off, float sc,
+                                                int ntiles, int A, int F, int f, int tile, int lane)
+{
+    int v = ib_columns<KSTEPS>(a, A, lane);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    v = add_dpp<0xB1>((int)(h[0] + h[1]));     // quad_perm [1, 0, 3, 2]
+    if (ib.ts >= 2) v = add_dpp<0x4E>(v);      // quad_perm [2, 3, 0, 1]
+    if (ib.ts >= 4) v = add_dpp<0x141>(v);     // row_half_mirror
+    if (ib.ts >= 8) v = add_dpp<0x140>(v);     // row_mirror
+    if (ib.ts >= 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+        v = (int)(r[0] + r[1]);
+    }
+    if (tile < ntiles && lane < 32 && (lane & (2 * ib.ts - 1)) == 0)
+        ib.out[((long long)tile * (16 / ib.ts) + lane / (2 * ib.ts)) * F + f] =
+            quantise((double)v, off, sc, ib.quant);
 }
 
 // a + b' where lanes below 32 keep a and take b' = (a of lane + 32), and
@@ -414,8 +478,16 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     constexpr bool SHARE = FS > 1 && RV % FS == 0;
     constexpr int NV = SHARE ? VALS / FS : VALS;   // values a wave quantises
     static_assert(!IBF || (TA && FS == 1), "incoherent-beam partials");
+    // One beam group of 32 or 64 beams in all: the form that may write its
+    // outputs itself (CbTrArgs::tbtf).
+    constexpr bool FEW = RT <= 4 && NWB == 1 && FS == 1;
     extern __shared__ __align__(16) int8_t lds[];
     const CbArgs& p = ta.p;
+    int wjobs = 0;
+    if constexpr (FEW) {
+        if (weights_job_run(ta.weights, threadIdx.x)) return;   // uniform over the work-group
+        wjobs = ta.weights.nblocks;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -429,7 +501,7 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     const int wc = (wv - tsl * WPS) % FS;         // channel of the fscrunch group
     const int wb = (wv - tsl * WPS) / FS;         // beam group within the work-group
 
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int logical = xcd_remap((int)blockIdx.x - wjobs, (int)gridDim.x - wjobs);
     const int bgroup = logical % ta.n_bgroups;
     const int rest = logical / ta.n_bgroups;
     const int tgroup = rest % ta.n_tgroups;
@@ -624,6 +696,24 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
         if (any) {
             wait_vm_lgkm0<0>();   // the staging loads land before LDS is released
             const int tend = (tgroup + 1) * NTS * slot_tiles;
+            if constexpr (FEW) {
+                if (ta.tbtf) {
+                    CbArgs pt = p;
+                    pt.out = ta.tbtf;
+                    cb_exact_outputs<MODE_INT8, true>(pt, fo, 0, p.B, (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
+                                                      (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps,
+                                                      tid, (int)blockDim.x);
+                    if constexpr (IBF) {
+                        if (ta.ib.out)
+                            cb_exact_ib_outputs(p, ta.ib, fo, tgroup * NTS * slot_tiles,
+                                                tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
+                        else
+                            cb_exact_ib_partials(p, ta.ibp, ta.ntiles, fo, tgroup * NTS * slot_tiles,
+                                                 tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
+                    }
+                    return;
+                }
+            }
             cb_exact_outputs<MODE_INT8>(p, fo, bgroup * NWB * 16 * RT, NWB * 16 * RT,
                                         (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
                                         (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps, tid,
@@ -643,6 +733,10 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     const bool q_thr = thr_applies(q_off, q_sc);
     const bool q_f32 = q_thr && thr_f32_applies(q_off, q_sc);
     const QuantConst qz = quant_const(q_off, q_sc);
+    const bool ib_out = FEW && IBF && ta.ib.out;   // the incoherent beam's outputs are written here
+    typedef const __attribute__((address_space(4))) float* scalar_ptr;
+    const float ib_off = ib_out ? ((scalar_ptr)ta.ib.offsets)[fo] : 0.0f;
+    const float ib_sc = ib_out ? ((scalar_ptr)ta.ib.scales)[fo] : 1.0f;
     if (tid < kThr) thr[tid] = thr_v;
     if (tid + NTHR < kThr) thr[tid + NTHR] = thr_v2;
     const long long* const thr_mid = thr + 128;
@@ -678,6 +772,20 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
         } else {
 #pragma unroll
             for (int v = 0; v < NV; ++v) q[v] = quantise((double)t[v], q_off, q_sc, p.quant);
+        }
+        if constexpr (FEW) {
+            if (ta.tbtf) {   // [To/ohs][B][ohs][Fo], below 2^31 bytes
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const int row = w0 + (RT == 2 ? 2 * v + h : v % NSLOT);
+                    const int b = b_lane + (RT == 2 ? 0 : 64 * (v / NSLOT));
+                    if (!wave_active || row >= nout || b >= p.B) continue;
+                    const unsigned heap = (unsigned)row / (unsigned)p.ohs;
+                    const unsigned in_heap = (unsigned)row - heap * p.ohs;
+                    global_ptr(ta.tbtf)[((heap * p.B + b) * p.ohs + in_heap) * p.Fo + fo] = (int8_t)q[v];
+                }
+                return;
+            }
         }
         // Every beam of the wave and every window of the pass in range (the
         // usual case, uniform over the wave): the four rows' bases are
@@ -774,8 +882,13 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
                     }
                     if (live) detect_step<RT, KSTEPS, SPT, NSLOT>(a, w, pw, g);
                     if constexpr (IBF) {
-                        if (ib_now) ib_tile<KSTEPS>(a, ta.ibp, ta.ntiles, p.A, fo, tile0 + pass * ta.ntp + g * ta.tps + x,
-                                                    lane);
+                        const int tile = tile0 + pass * ta.ntp + g * ta.tps + x;
+                        if (ib_out) {
+                            if (ib_now)
+                                ib_tile_outputs<KSTEPS>(a, ta.ib, ib_off, ib_sc, ta.ntiles, p.A, p.F, fo, tile, lane);
+                        } else if (ib_now) {
+                            ib_tile<KSTEPS>(a, ta.ibp, ta.ntiles, p.A, fo, tile, lane);
+                        }
                     }
                 }
                 rs = rs + 1 == NB ? 0 : rs + 1;
@@ -981,7 +1094,7 @@ hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
     const long long per_unit = tr_rounds(units, (long long)occ * device_cu_count(), passes, NTS, a.ntp).per_unit;
     a.npasses = (int)((passes + per_unit * NTS - 1) / (per_unit * NTS));
     a.n_tgroups = (int)((passes + (long long)a.npasses * NTS - 1) / ((long long)a.npasses * NTS));
-    const long long nblocks = units * a.n_tgroups;
+    const long long nblocks = units * a.n_tgroups + a.weights.nblocks;
     if (nblocks <= 0 || nblocks >= (1ll << 31)) return hipErrorInvalidConfiguration;
     kernel<<<dim3((unsigned)nblocks), NTHR, shm, s>>>(a);
     return hipGetLastError();

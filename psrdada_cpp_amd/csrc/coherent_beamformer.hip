@@ -9,9 +9,10 @@
 // The int8 output leaves the beamformer kernel as [Fo][To][B] (beams
 // contiguous: each work-group writes whole 64-byte runs) and a second kernel
 // (tbtf_k) moves it to TBTF [To/ohs][B][ohs][Fo].  Writing TBTF directly from
-// the beamformer scatters single bytes 1 channel apart across work-groups
-// (one work-group owns one channel), which the memory system turns into
-// 32-byte partial writes: 32x the output size in HBM writes.
+// the beamformer (done for small blocks only, cb_tbtf_direct) scatters single
+// bytes 1 channel apart across work-groups (one work-group owns one channel),
+// which the memory system turns into 32-byte partial writes: 32x the output
+// size in HBM writes.
 //
 // MI355X design.  Per channel the contraction is a real GEMM
 //   C[2B x T*P] = W'[2B x 2A] * V'[2A x T*P]
@@ -503,7 +504,7 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
 // earlier picks (us; antennas / beams / channels / samples / tscrunch):
 // 16/256/64/8192/16 40.6 against 44.7, 48/512/64/8192/16 111 against 128,
 // 40/768/64/8192/4 250 against 272, 8/64/64/8192/16 16.4 against 17.4,
-// 16/32/16/2048/16 8.3 against 9.4.  fscrunch 2 and 4: 128 beams per wave
+// 16/32/16/2048/16 8.3 against 9.4 (5.4 in one launch, cb_tbtf_direct).  fscrunch 2 and 4: 128 beams per wave
 // above 96 beams, or where the forms with several time slots per work-group
 // end (two K steps of four channels); 44/1024/64/8192/16 at fscrunch 4 took
 // 205 against 348 of the LDS-staged kernel, 44/64 32 against 50, but 24/64 26.7
@@ -585,6 +586,44 @@ struct TailJobs {
     WeightsJob weights;
 };
 
+struct Span {
+    const void* p;
+    size_t n;
+};
+
+static bool spans_overlap(const Span& a, const Span& b)
+{
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a.p), y = reinterpret_cast<uintptr_t>(b.p);
+    return a.n && b.n && x < y + b.n && y < x + a.n;
+}
+
+// Whether the few-beam kernel of a block writes TBTF itself, with the tail's
+// jobs in its own launch (CbTrArgs::tbtf): outputs of at most kTbtfDirect
+// bytes, none of them over the kernel's inputs (next weights written over the
+// block's, say: those are read until the launch ends), and an incoherent beam
+// of this block alone in windows within a tile.
+//
+// Such blocks are launches and latency: the reorder's launch costs more than
+// its scattered bytes.  One launch against two (us; antennas / beams /
+// channels / heaps, output size): both beams and the next weights 16/32/16/8,
+// 64 KiB 7.0 against 9.5, 48/64/64/4, 256 KiB 10.6 against 12.9, 48/64/64/8,
+// 512 KiB 13.9 against 15.0, but 48/64/64/16, 1 MiB 20.8 against 20.5; the
+// coherent beams alone 5.3 against 8.9, 8.7 against 11.2, 11.3 against 13.4, and
+// 2 MiB 33.7 against 30.7.
+constexpr size_t kTbtfDirect = 1 << 19;
+
+static bool cb_tbtf_direct(const Span& volts, const Span& weights, const Span& out, const TailJobs& tail)
+{
+    auto clear = [&](const Span& o) { return !spans_overlap(o, volts) && !spans_overlap(o, weights); };
+    if (out.n > kTbtfDirect || !clear(out)) return false;
+    const IbFinishJob& ib = tail.ib;
+    if (ib.nblocks && (ib.nparts != 1 || ib.fs != 1 || ib.ts > 16 ||
+                       !clear(Span{ib.out, (size_t)ib.nwin * ib.Fo})))
+        return false;
+    const WeightsLaunch& w = tail.weights.w;
+    return !tail.weights.nblocks || clear(Span{w.weights, (size_t)2 * w.F * w.nd});
+}
+
 // Validates and launches one coherent-beam kernel over T samples of voltage
 // columns that are `vstride` bytes apart, the beamformer's antennas starting
 // `voff` bytes into each column; or, with `tv`, over the TAFTP block `ftpa`
@@ -625,20 +664,22 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
                 FBF_ERR_ARG, "fbf_cb: buffers must be 16-byte aligned");
     if (T == 0) return FBF_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const CbVariant var =
+        tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_variant(d, plan->variant, mode, T);
+    const size_t vbytes = tv ? (size_t)4 * tv->Atot * d.nchans * T : (size_t)2 * vstride * d.nchans * T;
+    const bool direct = var.few && !plan->t_before && !plan->t_after &&
+                        cb_tbtf_direct(Span{ftpa, vbytes}, Span{fba, wbytes}, Span{out, expect}, tail);
     void* kout = out;
     if (mode == MODE_INT8) {
         if (workspace) {
             FBF_REQUIRE(workspace_bytes >= expect && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
                         FBF_ERR_SIZE, "fbf_cb: workspace too small or not 16-byte aligned");
             kout = workspace;
-        } else {
+        } else if (!direct) {
             const int st = cb_staging(plan, expect, s, &kout);
             if (st) return st;
         }
     }
-
-    const CbVariant var =
-        tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_variant(d, plan->variant, mode, T);
     // The timing events (fbf_cb_plan_set_timing), around the coherent kernel only.
     auto mark = [&](hipEvent_t ev) { return ev ? hipEventRecord(ev, s) : hipSuccess; };
     if (var.ws) {
@@ -708,6 +749,11 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
             ta.lgtph = __builtin_ctz((unsigned)(tv->S / 16));
             ta.ibp = tv->ibp;
         }
+        if (direct) {
+            ta.tbtf = static_cast<int8_t*>(out);
+            ta.ib = tail.ib;
+            ta.weights = tail.weights;
+        }
         const int rt = var.rows;
         const int W = 2 * d.tscrunch;
         const int spt = W >= 32 ? 1 : 32 / W;
@@ -726,6 +772,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
                                     : cb_launch_tr8_fs(ta, d.fscrunch, W, ksteps, passes, s);
         if (e == hipSuccess) e = mark(plan->t_after);
         if (e != hipSuccess) return hip_status(e, "cb_tr_k launch");
+        if (direct) return FBF_OK;
         e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
                                   plan->ohs),
                         s, tail.ib, tail.weights);
@@ -832,8 +879,9 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 //
 // Staging the block itself was the faster at every size measured.  Blocks of
 // both beams, direct against split-transposed (us; antennas / beams / channels
-// / heaps, tscrunch 16): 16/32/16/8 8.6 against 17.1, 48/64/64/8 13.0 against
-// 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
+// / heaps, tscrunch 16; the reorder in a launch of its own, which the first two
+// now do without, cb_tbtf_direct): 16/32/16/8 8.6 against 17.1, 48/64/64/8 13.0
+// against 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
 // of 32 or 64 beams for so few took 8.6 and 33.7 us where 128-beam waves took
 // 10.8 and 41.0.
 // Blocks of at most kTaftpSmall channels x samples keep the split-transpose

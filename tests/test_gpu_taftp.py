@@ -441,3 +441,62 @@ def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs, va
     np.testing.assert_array_equal(d_o.download(), ref)
     np.testing.assert_array_equal(d_tf.download(), ib_ref.reshape(-1))
     np.testing.assert_array_equal(d_w.download(), d_next.download())
+
+
+@pytest.mark.parametrize("A,F,nhg,B,ts,ohs,ib_ts,over,m128", [
+    (16, 16, 8, 32, 16, 128, 16, "", False),     # one output heap
+    (40, 4, 3, 24, 4, 16, 1, "", False),         # many output heaps, unused beams, a window per sample
+    (60, 12, 2, 64, 16, 4, 2, "", False),        # 64 beams per wave, antennas in fours
+    (64, 4, 3, 40, 64, 3, 8, "", False),         # windows over four tiles
+    (20, 8, 2, 8, 8, 32, 4, "", True),           # a weight of -128: the exact path
+    (16, 64, 8, 64, 16, 128, 16, "", False),     # the largest outputs written directly (512 KiB)
+    (16, 64, 9, 64, 16, 16, 16, "", False),      # just above
+    (16, 16, 2, 32, 16, 16, 32, "", False),      # windows longer than a tile: partials
+    (16, 16, 2, 32, 16, 32, 16, "weights", False),   # next weights over this block's
+    (16, 16, 2, 32, 4, 16, 16, "block", False),  # beams over the block
+])
+def test_small_block_outputs_in_one_launch(gpu, oracle, A, F, nhg, B, ts, ohs, ib_ts, over, m128):
+    """Small blocks of few beams, whose kernel writes TBTF, the incoherent beam
+    and the next weights itself (unless its outputs lie over its inputs or are
+    too large): TAFTP and FTPA entry points against the oracle."""
+    capi = gpu
+    S = 256
+    T = nhg * S
+    taftp = gaussian_int8(3600 + A + B, nhg * A * F * S * 4, 16.0)
+    off, sc = _levels(oracle, A, ts, 1, F)
+    _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, A, ts, 1, A, ib_ts, 1)
+    ioff, isc = np.full(F, ibo, np.float32), np.full(F, ibs, np.float32)
+    w = unit_weights(3601 + A, F * B * A).reshape(F, B, A, 2).copy()
+    if m128:
+        w[1, 3, 5, 1] = -128
+    w = w.reshape(-1)
+    ftpa = oracle.split_transpose(taftp, nhg, A, A, 0, F)
+    ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, ohs)
+    ib_ref = oracle.ib_tf(oracle.ib_power(taftp, F, ib_ts, 1, nhg, A), ioff, isc)
+    wp = capi.WeightsPlan(A, B, F, capi.channel_frequencies_f64(1284e6, 856e6, F))
+    delays = np.stack([capi.synth_uniform_f32(3602, -1e-9, 1e-9, B * A),
+                       capi.synth_uniform_f32(3603, -1e-6, 1e-6, B * A)], axis=1)
+    d_d, d_gen = _dev(capi, delays.reshape(-1)), capi.DeviceBuffer(F * B * A * 2)
+    wp.generate(d_d, 8.25, d_gen)
+    plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=ohs)
+    ib = capi.IbPlan(A, F, ib_ts, 1, ioff, isc)
+    d_t, d_w, d_f = _dev(capi, taftp), _dev(capi, w), _dev(capi, ftpa)
+    d_o, d_tf = capi.DeviceBuffer(F * (T // ts) * B), capi.DeviceBuffer(ib.output_bytes(d_t.nbytes))
+
+    for call in (lambda: plan.beamform_taftp(d_t, d_w, d_o), lambda: plan.beamform(d_f, d_w, d_o)):
+        d_o.fill(0x5A)
+        call()
+        np.testing.assert_array_equal(d_o.download(), ref)
+
+    d_next = d_w if over == "weights" else capi.DeviceBuffer(d_gen.nbytes)
+    d_out = d_t if over == "block" else d_o
+    d_tf.fill(0x5A)
+    plan.ib_beamform_taftp_next(ib, d_t, d_w, _View(d_out.ptr, d_o.nbytes), d_tf, wp, d_d, 8.25, d_next)
+    np.testing.assert_array_equal(d_out.download(count=ref.size), ref)
+    np.testing.assert_array_equal(d_tf.download(), ib_ref.reshape(-1))
+    np.testing.assert_array_equal(d_next.download(), d_gen.download())
+
+
+class _View:
+    def __init__(self, ptr, nbytes):
+        self.ptr, self.nbytes = ptr, nbytes
