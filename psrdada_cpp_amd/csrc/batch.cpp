@@ -349,19 +349,21 @@ static int batch_enqueue_direct(fbf_batch* b, const void* taftp, size_t taftp_by
     }
     int* const part = static_cast<int*>(b->ibp);
     const size_t step = (size_t)4 * b->F * T;   // ints per subarray
+    IbFinishJob job{};
+    if (partials) {
+        st = ib_finish_job(b->ib, part, n, T, outputs[n], ob, &job);
+        if (st) return st;
+    }
+    std::vector<TbtfArgs> reorders(n);
     for (int i = 0; i < n; ++i) {
-        IbFinishJob job{};
-        if (partials && i == n - 1) {
-            st = ib_finish_job(b->ib, part, n, T, outputs[n], ob, &job);
-            if (st) return st;
-        }
         size_t wb = 0;
         fbf_batch_weights_bytes(b, i, &wb);
         st = cb_batch_beamform(b->plans[i], taftp, T, b->A, b->subs[i].start_antenna, b->S, weights[i], wb, outputs[i],
-                               sub_out_bytes(b, b->subs[i]), stream, partials ? part + i * step : nullptr, job);
+                               sub_out_bytes(b, b->subs[i]), stream, partials ? part + i * step : nullptr,
+                               &reorders[i]);
         if (st) return st;
     }
-    return FBF_OK;
+    return cb_batch_reorder(reorders.data(), n, job, stream);
 }
 
 // Enqueues one block in turn on `stream`: incoherent beam (when not fused),

@@ -38,6 +38,7 @@
 // A <= 128) and handed to the quantiser as a double, like the oracle.
 #include "cb_tr.hpp"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
@@ -90,29 +91,9 @@ constexpr int kTrBeams = 128;
 constexpr int kTrMaxChans = 64;
 constexpr int kTrLdsBudget = 40 * 1024;
 
-struct TbtfArgs {
-    const int8_t* src;
-    int8_t* dst;
-    long long To;
-    int B, Fo, ohs;
-    int tt, ft, bp, tp;           // tile samples / channels, LDS pitches (dwords)
-    int n_ttiles, n_ftiles, n_btiles;
-};
-
-// The first wj.nblocks work-groups generate weights (the next block's,
-// weights_job_run), the next job.nblocks finish the incoherent beam from the
-// coherent kernel's partials (ib_finish_run), both beside the reorder; the
-// rest reorder, numbered from 0.
-__global__ __launch_bounds__(256) void tbtf_k(TbtfArgs a, IbFinishJob job, WeightsJob wj)
+// Tile bid of one reorder.
+__device__ __forceinline__ void tbtf_tile(const TbtfArgs& a, long long bid, int8_t* tr_lds)
 {
-    extern __shared__ __align__(16) int8_t tr_lds[];
-    if (weights_job_run(wj, threadIdx.x)) return;   // uniform over the work-group
-    const int b1 = (int)blockIdx.x - wj.nblocks;
-    if (b1 < job.nblocks) {
-        ib_finish_run(job, (long long)b1 * 256 + threadIdx.x);
-        return;
-    }
-    long long bid = (long long)b1 - job.nblocks;
     const int bt = (int)(bid % a.n_btiles);
     bid /= a.n_btiles;
     const int ftile = (int)(bid % a.n_ftiles);
@@ -258,6 +239,51 @@ __global__ __launch_bounds__(256) void tbtf_k(TbtfArgs a, IbFinishJob job, Weigh
     }
 }
 
+// The first wj.nblocks work-groups generate weights (the next block's,
+// weights_job_run), the next job.nblocks finish the incoherent beam from the
+// coherent kernel's partials (ib_finish_run), both beside the reorder; the
+// rest reorder, numbered from 0.
+__global__ __launch_bounds__(256) void tbtf_k(TbtfArgs a, IbFinishJob job, WeightsJob wj)
+{
+    extern __shared__ __align__(16) int8_t tr_lds[];
+    if (weights_job_run(wj, threadIdx.x)) return;   // uniform over the work-group
+    const int b1 = (int)blockIdx.x - wj.nblocks;
+    if (b1 < job.nblocks) {
+        ib_finish_run(job, (long long)b1 * 256 + threadIdx.x);
+        return;
+    }
+    tbtf_tile(a, (long long)b1 - job.nblocks, tr_lds);
+}
+
+// The reorders of up to kTbtfJobs subarrays of a batch in one launch (after
+// the incoherent beam's finish): each by itself fills the chip for a few
+// microseconds at most, and starts and drains alone.  Subarrays of 40, 16 and 8
+// antennas (768, 256, 64 beams, 64 channels, 8192 samples) took 253.8 us with a
+// launch for each and 247.3 us with one; 8, 16, 8, 32 antennas (72, 112, 16, 32
+// beams, 44 channels, 2304 samples) 64.5 and 52.0 us.
+constexpr int kTbtfJobs = 8;
+
+struct TbtfJobs {
+    TbtfArgs a[kTbtfJobs];
+    int first[kTbtfJobs];   // first work-group of each
+    int n;
+};
+
+__global__ __launch_bounds__(256) void tbtf_jobs_k(TbtfJobs jobs, IbFinishJob job)
+{
+    extern __shared__ __align__(16) int8_t tr_lds[];
+    const int b1 = (int)blockIdx.x;
+    if (b1 < job.nblocks) {
+        ib_finish_run(job, (long long)b1 * 256 + threadIdx.x);
+        return;
+    }
+    const int b = b1 - job.nblocks;
+    int k = jobs.n - 1;
+    while (k > 0 && b < jobs.first[k]) --k;
+    const TbtfArgs a = jobs.a[k];
+    tbtf_tile(a, b - jobs.first[k], tr_lds);
+}
+
 // Tile shape and grid for tbtf_k.
 TbtfArgs tbtf_args(const int8_t* src, int8_t* dst, long long To, int B, int Fo, int ohs)
 {
@@ -287,11 +313,11 @@ TbtfArgs tbtf_args(const int8_t* src, int8_t* dst, long long To, int B, int Fo, 
     return a;
 }
 
-hipError_t launch_tbtf(const TbtfArgs& a, hipStream_t s, const IbFinishJob& job = IbFinishJob{},
-                       const WeightsJob& wj = WeightsJob{})
+long long tbtf_blocks(const TbtfArgs& a) { return a.To / a.ohs * a.n_ttiles * a.n_ftiles * a.n_btiles; }
+
+hipError_t launch_tbtf(const TbtfArgs& a, hipStream_t s, const IbFinishJob& job, const WeightsJob& wj)
 {
-    const long long heaps = a.To / a.ohs;
-    const long long nblocks = heaps * a.n_ttiles * a.n_ftiles * a.n_btiles + job.nblocks + wj.nblocks;
+    const long long nblocks = tbtf_blocks(a) + job.nblocks + wj.nblocks;
     if (nblocks <= 0) return hipSuccess;
     if (nblocks >= (1ll << 31)) return hipErrorInvalidConfiguration;
     const size_t shm = (size_t)a.tt * a.tp * 4;
@@ -584,7 +610,15 @@ struct TaftpView {
 struct TailJobs {
     IbFinishJob ib;
     WeightsJob weights;
+    TbtfArgs* defer = nullptr;   // leave the reorder's arguments here instead of launching it
 };
+
+static hipError_t cb_reorder(const TbtfArgs& a, hipStream_t s, const TailJobs& tail)
+{
+    if (!tail.defer) return launch_tbtf(a, s, tail.ib, tail.weights);
+    *tail.defer = a;
+    return hipSuccess;
+}
 
 struct Span {
     const void* p;
@@ -714,9 +748,8 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         if (e == hipSuccess) e = cb_launch_ws(wa, W, ksteps, s);
         if (e == hipSuccess) e = mark(plan->t_after);
         if (e != hipSuccess) return hip_status(e, "cb_ws_k launch");
-        e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
-                                  plan->ohs),
-                        s, tail.ib, tail.weights);
+        e = cb_reorder(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo, plan->ohs), s,
+                   tail);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
         return FBF_OK;
     }
@@ -773,9 +806,8 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
         if (e == hipSuccess) e = mark(plan->t_after);
         if (e != hipSuccess) return hip_status(e, "cb_tr_k launch");
         if (direct) return FBF_OK;
-        e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
-                                  plan->ohs),
-                        s, tail.ib, tail.weights);
+        e = cb_reorder(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo, plan->ohs), s,
+                   tail);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
         return FBF_OK;
     }
@@ -838,9 +870,8 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
     if (e == hipSuccess) e = mark(plan->t_after);
     if (e != hipSuccess) return hip_status(e, "cb_mfma_k launch");
     if (mode == MODE_INT8) {
-        e = launch_tbtf(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo,
-                                  plan->ohs),
-                        s, tail.ib, tail.weights);
+        e = cb_reorder(tbtf_args(static_cast<const int8_t*>(kout), static_cast<int8_t*>(out), To, d.nbeams, Fo, plan->ohs), s,
+                   tail);
         if (e != hipSuccess) return hip_status(e, "tbtf_k launch");
     }
     return FBF_OK;
@@ -1082,7 +1113,7 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
         }
         const SplitIb sib{ib_plan, tf, tf_bytes};
         st = cb_taftp_run(plan, taftp, taftp_bytes, d.nantennas, 0, nsamples_per_heap, fba_weights, weights_bytes,
-                          tbtf, tbtf_bytes, stream, TailJobs{IbFinishJob{}, wj}, split_ib ? &sib : nullptr);
+                          tbtf, tbtf_bytes, stream, TailJobs{IbFinishJob{}, wj, nullptr}, split_ib ? &sib : nullptr);
         if (st || !next || T > 0) return st;
         return fbf_weights_generate(next->plan, next->delays, next->delays_bytes, next->epoch, next->weights,
                                     next->weights_bytes, nullptr, stream);
@@ -1105,7 +1136,7 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
     const TaftpView tv{nsamples_per_heap, d.nantennas, 0, cb_taftp_form(plan, T, d.nantennas, kTaftpOnePass),
                        static_cast<int*>(part)};
     return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
-                     stream, nullptr, 0, &tv, TailJobs{ibj, wj});
+                     stream, nullptr, 0, &tv, TailJobs{ibj, wj, nullptr});
 }
 
 std::pair<int, int> fbf::cb_plan_tuning(const fbf_cb_plan* plan) { return {plan->variant, plan->chunk}; }
@@ -1120,12 +1151,45 @@ bool fbf::cb_batch_stages(const fbf_cb_plan* plan, long long T, int nantennas_to
 
 int fbf::cb_batch_beamform(fbf_cb_plan* plan, const void* taftp, long long T, int nantennas_total, int start_antenna,
                            int S, const void* fba_weights, size_t weights_bytes, void* tbtf, size_t tbtf_bytes,
-                           hipStream_t s, int* partials, const IbFinishJob& ib)
+                           hipStream_t s, int* partials, TbtfArgs* reorder)
 {
+    *reorder = TbtfArgs{};
     const TaftpView tv{S, nantennas_total, start_antenna, cb_taftp_form(plan, T, nantennas_total, kTaftpBatch),
                        partials};
     return cb_launch(plan, MODE_INT8, taftp, T, 2 * plan->d.nantennas, 0, fba_weights, weights_bytes, tbtf,
-                     tbtf_bytes, s, nullptr, 0, &tv, TailJobs{ib, WeightsJob{}});
+                     tbtf_bytes, s, nullptr, 0, &tv, TailJobs{IbFinishJob{}, WeightsJob{}, reorder});
+}
+
+int fbf::cb_batch_reorder(const TbtfArgs* reorders, int n, const IbFinishJob& ib, hipStream_t s)
+{
+    TbtfJobs jobs{};
+    IbFinishJob job = ib;   // (in the first launch)
+    long long nblocks = 0;
+    size_t shm = 0;
+    auto flush = [&]() {
+        const long long all = nblocks + job.nblocks;
+        if (all == 0) return hipSuccess;
+        if (all >= (1ll << 31)) return hipErrorInvalidConfiguration;
+        tbtf_jobs_k<<<dim3((unsigned)all), 256, shm, s>>>(jobs, job);
+        jobs = TbtfJobs{};
+        job = IbFinishJob{};
+        nblocks = 0;
+        shm = 0;
+        return hipGetLastError();
+    };
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        const TbtfArgs& a = reorders[i];
+        if (!a.src) continue;   // (written by the coherent kernel itself)
+        const long long nb = tbtf_blocks(a);
+        if (jobs.n == kTbtfJobs || nblocks + nb + job.nblocks >= (1ll << 31)) e = flush();
+        jobs.a[jobs.n] = a;
+        jobs.first[jobs.n++] = (int)nblocks;
+        nblocks += nb;
+        shm = std::max(shm, (size_t)a.tt * a.tp * 4);
+    }
+    if (e == hipSuccess) e = flush();
+    return e == hipSuccess ? FBF_OK : hip_status(e, "tbtf_jobs_k launch");
 }
 
 extern "C" int fbf_cb_ib_beamform_taftp(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,

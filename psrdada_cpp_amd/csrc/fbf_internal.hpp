@@ -78,14 +78,26 @@ int ib_finish_job(const fbf_ib_plan* plan, const int* partials, int nparts, long
 // A coherent plan's kernel variant and chunk length.
 std::pair<int, int> cb_plan_tuning(const fbf_cb_plan* plan);
 
+// One reorder of staged beams to TBTF (tbtf_k).
+struct TbtfArgs {
+    const int8_t* src;
+    int8_t* dst;
+    long long To;
+    int B, Fo, ohs;
+    int tt, ft, bp, tp;           // tile samples / channels, LDS pitches (dwords)
+    int n_ttiles, n_ftiles, n_btiles;
+};
+
 // A batch's subarray beamformed from the TAFTP block itself: whether the
 // plan's kernel stages such a block (with `partials`: and leaves the
-// incoherent beam's partials of its antennas), and the call, whose reorder
-// launch also runs the `ib` job.
+// incoherent beam's partials of its antennas); the call, which leaves its
+// reorder in *reorder (src null: none is needed); and the reorders of the
+// batch's subarrays with the incoherent beam's finish.
 bool cb_batch_stages(const fbf_cb_plan* plan, long long T, int nantennas_total, int S, bool partials);
 int cb_batch_beamform(fbf_cb_plan* plan, const void* taftp, long long T, int nantennas_total, int start_antenna,
                       int S, const void* fba_weights, size_t weights_bytes, void* tbtf, size_t tbtf_bytes,
-                      hipStream_t s, int* partials, const IbFinishJob& ib);
+                      hipStream_t s, int* partials, TbtfArgs* reorder);
+int cb_batch_reorder(const TbtfArgs* reorders, int n, const IbFinishJob& ib, hipStream_t s);
 
 // Weights generation (weights.hip), shared by weights_k and by launches that
 // generate the weights beside other work.  A thread takes one (beam,

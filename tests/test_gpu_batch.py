@@ -123,6 +123,9 @@ def test_autotune_picks_a_variant_that_is_bit_exact(gpu, oracle):
     ([(0, 32, 128), (32, 32, 104)], 16, 2, (1, 1)),                # fscrunch 2 leaves no partials
     ([(0, 60, 40), (60, 4, 8)], 4, 1, (256, 1)),                   # antennas in fours
     ([(0, 56, 40), (56, 8, 8)], 24, 1, (16, 1)),                   # tscrunch 24: the split-transposed block
+    ([(8 * k, 8 - 4 * (k == 3), 72 + 8 * k) for k in range(8)] + [(28, 4, 24), (0, 8, 96)], 16, 1, (16, 1)),
+    # more reorders than one launch takes, one subarray that needs none, antennas shared by two
+    ([(8 * k, 8, 72) for k in range(5)] + [(40 + 4 * k, 4, 80) for k in range(6)], 4, 1, (64, 1)),   # likewise, partials
 ])
 def test_batch_straight_from_taftp(gpu, oracle, split, ts, fs, ib):
     """Subarrays in turn from the TAFTP block itself, and the batch's
