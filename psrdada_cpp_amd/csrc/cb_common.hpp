@@ -50,7 +50,7 @@ struct CbTrArgs {
     // antennas and both pols split over columns 2j, 2j + 1 (its pols) of
     // both halves (ib_finish_run adds the four).
     int* ibp;
-    // The few-beam kernel of a small block (cb_tbtf_direct): the outputs go
+    // The few-beam forms for a small block (cb_tbtf_direct): the outputs go
     // straight to TBTF at `tbtf` (else null), the incoherent beam of `ib`
     // (ib.out null: none, or partials) to its output, and the first
     // weights.nblocks work-groups generate weights.

@@ -441,10 +441,15 @@ struct TrRed {
     static constexpr int VALS = RT == 2 ? NSLOT / 2 : (RT / 4) * NSLOT;
 };
 
+// Forms of at most 64 beams per wave in four-wave work-groups.
+constexpr bool tr_writes_tbtf(int rt, int fs, int nw) { return rt <= 4 && fs == 1 && nw == 4; }
+
 // RT: beam tiles per wave (RT / 2 groups of 32 beams, a Re and an Im tile
 // each); SPT: windows per tile (1, 2, 4); NSLOT: windows
 // per pass held in registers; FS: fscrunch; NTS: time slots and NWB: beam
 // groups (of 16 RT beams) per work-group;
+// DT: the outputs go straight to TBTF (CbTrArgs::tbtf; an instance of its own:
+// as a branch it cost the 128-antenna kernel 5 %);
 // TA: the voltages are a TAFTP block (CbArgs::S > 0), staged straight into
 // [antenna][column] tiles and read with transposed LDS loads (tr_operands),
 // else FTPA columns; IBF (with TA, FS = 1, all antennas of the block): the
@@ -460,7 +465,7 @@ struct TrRed {
 // which leaves SIMDs with one wave at the end.  With 128 beams per wave
 // (two waves per SIMD) a work-group is four waves, two share a compute
 // unit, and they take turns at a raised wave priority instead.
-template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF>
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF, bool DT>
 __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(RT, KSTEPS) : 1) void cb_tr_k(CbTrArgs ta)
 {
     using St = TrStage<RT, FS, KSTEPS, NTS, NWB>;
@@ -478,13 +483,11 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     constexpr bool SHARE = FS > 1 && RV % FS == 0;
     constexpr int NV = SHARE ? VALS / FS : VALS;   // values a wave quantises
     static_assert(!IBF || (TA && FS == 1), "incoherent-beam partials");
-    // One beam group of 32 or 64 beams in all: the form that may write its
-    // outputs itself (CbTrArgs::tbtf).
-    constexpr bool FEW = RT <= 4 && NWB == 1 && FS == 1;
+    static_assert(!DT || tr_writes_tbtf(RT, FS, St::NW), "direct outputs");
     extern __shared__ __align__(16) int8_t lds[];
     const CbArgs& p = ta.p;
     int wjobs = 0;
-    if constexpr (FEW) {
+    if constexpr (DT) {
         if (weights_job_run(ta.weights, threadIdx.x)) return;   // uniform over the work-group
         wjobs = ta.weights.nblocks;
     }
@@ -696,30 +699,24 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
         if (any) {
             wait_vm_lgkm0<0>();   // the staging loads land before LDS is released
             const int tend = (tgroup + 1) * NTS * slot_tiles;
-            if constexpr (FEW) {
-                if (ta.tbtf) {
-                    CbArgs pt = p;
-                    pt.out = ta.tbtf;
-                    cb_exact_outputs<MODE_INT8, true>(pt, fo, 0, p.B, (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
-                                                      (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps,
-                                                      tid, (int)blockDim.x);
-                    if constexpr (IBF) {
-                        if (ta.ib.out)
-                            cb_exact_ib_outputs(p, ta.ib, fo, tgroup * NTS * slot_tiles,
-                                                tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
-                        else
-                            cb_exact_ib_partials(p, ta.ibp, ta.ntiles, fo, tgroup * NTS * slot_tiles,
-                                                 tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
-                    }
-                    return;
-                }
+            if constexpr (DT) {
+                CbArgs pt = p;
+                pt.out = ta.tbtf;
+                cb_exact_outputs<MODE_INT8, true>(pt, fo, bgroup * NWB * 16 * RT, NWB * 16 * RT,
+                                                  (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
+                                                  (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps, tid,
+                                                  (int)blockDim.x);
+            } else {
+                cb_exact_outputs<MODE_INT8>(p, fo, bgroup * NWB * 16 * RT, NWB * 16 * RT,
+                                            (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
+                                            (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps, tid,
+                                            (int)blockDim.x);
             }
-            cb_exact_outputs<MODE_INT8>(p, fo, bgroup * NWB * 16 * RT, NWB * 16 * RT,
-                                        (long long)tgroup * NTS * slot_tiles * SPT / ta.tps,
-                                        (long long)(tend < ta.ntiles ? tend : ta.ntiles) * SPT / ta.tps, tid,
-                                        (int)blockDim.x);
             if constexpr (IBF) {
-                if (bgroup == 0)
+                if (DT && bgroup == 0 && ta.ib.out)
+                    cb_exact_ib_outputs(p, ta.ib, fo, tgroup * NTS * slot_tiles, tend < ta.ntiles ? tend : ta.ntiles,
+                                        tid, (int)blockDim.x);
+                else if (bgroup == 0)
                     cb_exact_ib_partials(p, ta.ibp, ta.ntiles, fo, tgroup * NTS * slot_tiles,
                                          tend < ta.ntiles ? tend : ta.ntiles, tid, (int)blockDim.x);
             }
@@ -733,7 +730,7 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     const bool q_thr = thr_applies(q_off, q_sc);
     const bool q_f32 = q_thr && thr_f32_applies(q_off, q_sc);
     const QuantConst qz = quant_const(q_off, q_sc);
-    const bool ib_out = FEW && IBF && ta.ib.out;   // the incoherent beam's outputs are written here
+    const bool ib_out = DT && IBF && ta.ib.out;   // the incoherent beam's outputs are written here
     typedef const __attribute__((address_space(4))) float* scalar_ptr;
     const float ib_off = ib_out ? ((scalar_ptr)ta.ib.offsets)[fo] : 0.0f;
     const float ib_sc = ib_out ? ((scalar_ptr)ta.ib.scales)[fo] : 1.0f;
@@ -773,19 +770,17 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
 #pragma unroll
             for (int v = 0; v < NV; ++v) q[v] = quantise((double)t[v], q_off, q_sc, p.quant);
         }
-        if constexpr (FEW) {
-            if (ta.tbtf) {   // [To/ohs][B][ohs][Fo], below 2^31 bytes
+        if constexpr (DT) {   // [To/ohs][B][ohs][Fo], below 2^31 bytes
 #pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    const int row = w0 + (RT == 2 ? 2 * v + h : v % NSLOT);
-                    const int b = b_lane + (RT == 2 ? 0 : 64 * (v / NSLOT));
-                    if (!wave_active || row >= nout || b >= p.B) continue;
-                    const unsigned heap = (unsigned)row / (unsigned)p.ohs;
-                    const unsigned in_heap = (unsigned)row - heap * p.ohs;
-                    global_ptr(ta.tbtf)[((heap * p.B + b) * p.ohs + in_heap) * p.Fo + fo] = (int8_t)q[v];
-                }
-                return;
+            for (int v = 0; v < NV; ++v) {
+                const int row = w0 + (RT == 2 ? 2 * v + h : v % NSLOT);
+                const int b = b_lane + (RT == 2 ? 0 : 64 * (v / NSLOT));
+                if (!wave_active || row >= nout || b >= p.B) continue;
+                const unsigned heap = (unsigned)row / (unsigned)p.ohs;
+                const unsigned in_heap = (unsigned)row - heap * p.ohs;
+                global_ptr(ta.tbtf)[((heap * p.B + b) * p.ohs + in_heap) * p.Fo + fo] = (int8_t)q[v];
             }
+            return;
         }
         // Every beam of the wave and every window of the pass in range (the
         // usual case, uniform over the wave): the four rows' bases are
@@ -1074,11 +1069,14 @@ inline int tr_nwb(int rt, int ksteps, int fs, const CbTrArgs& a, int passes)
     return best;
 }
 
-template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF = false>
+template <int RT, int KSTEPS, int SPT, int NSLOT, int FS, int NTS, int NWB, bool TA, bool IBF = false, bool DT = false>
 hipError_t launch_tr_kt(CbTrArgs a, int passes, hipStream_t s)
 {
+    if constexpr (!DT && tr_writes_tbtf(RT, FS, NTS * NWB * FS))
+        if (a.tbtf) return launch_tr_kt<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, TA, IBF, true>(a, passes, s);
+    if (a.tbtf && !DT) return hipErrorInvalidValue;
     constexpr int NTHR = 64 * NTS * NWB * FS;
-    constexpr auto kernel = cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, TA, IBF>;
+    constexpr auto kernel = cb_tr_k<RT, KSTEPS, SPT, NSLOT, FS, NTS, NWB, TA, IBF, DT>;
     const size_t shm = cb_tr_shm(RT, FS, KSTEPS, TrRed<RT, NSLOT>::VALS, NTS, NWB);
     if (shm > 65536) return hipErrorInvalidConfiguration;
     constexpr int beams_per_wg = 16 * RT * NWB;

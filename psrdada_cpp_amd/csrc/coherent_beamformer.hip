@@ -631,7 +631,7 @@ static bool spans_overlap(const Span& a, const Span& b)
     return a.n && b.n && x < y + b.n && y < x + a.n;
 }
 
-// Whether the few-beam kernel of a block writes TBTF itself, with the tail's
+// Whether a few-beam form of the kernel writes TBTF itself, with the tail's
 // jobs in its own launch (CbTrArgs::tbtf): outputs of at most kTbtfDirect
 // bytes, none of them over the kernel's inputs (next weights written over the
 // block's, say: those are read until the launch ends), and an incoherent beam
@@ -643,15 +643,20 @@ static bool spans_overlap(const Span& a, const Span& b)
 // 64 KiB 7.0 against 9.5, 48/64/64/4, 256 KiB 10.6 against 12.9, 48/64/64/8,
 // 512 KiB 13.9 against 15.0, but 48/64/64/16, 1 MiB 20.8 against 20.5; the
 // coherent beams alone 5.3 against 8.9, 8.7 against 11.2, 11.3 against 13.4, and
-// 2 MiB 33.7 against 30.7.
+// 2 MiB 33.7 against 30.7.  Above 64 antennas the coherent beams alone 96/128/64/4,
+// 512 KiB 14.8 against 17.6, but with the incoherent beam, whose outputs a wave
+// with beams sums and quantises tile by tile, only up to 65536 channels x
+// samples: 72/16/64/4 14.3 against 14.8, 72/16/64/8 20.0 against 19.1.
 constexpr size_t kTbtfDirect = 1 << 19;
+constexpr long long kTbtfDirectIb = 1 << 16;
 
-static bool cb_tbtf_direct(const Span& volts, const Span& weights, const Span& out, const TailJobs& tail)
+static bool cb_tbtf_direct(int ksteps, const Span& volts, const Span& weights, const Span& out, const TailJobs& tail)
 {
     auto clear = [&](const Span& o) { return !spans_overlap(o, volts) && !spans_overlap(o, weights); };
     if (out.n > kTbtfDirect || !clear(out)) return false;
     const IbFinishJob& ib = tail.ib;
     if (ib.nblocks && (ib.nparts != 1 || ib.fs != 1 || ib.ts > 16 ||
+                       (ksteps > 4 && ib.nwin * ib.ts * ib.Fo > kTbtfDirectIb) ||
                        !clear(Span{ib.out, (size_t)ib.nwin * ib.Fo})))
         return false;
     const WeightsLaunch& w = tail.weights.w;
@@ -701,8 +706,10 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
     const CbVariant var =
         tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_variant(d, plan->variant, mode, T);
     const size_t vbytes = tv ? (size_t)4 * tv->Atot * d.nchans * T : (size_t)2 * vstride * d.nchans * T;
-    const bool direct = var.few && !plan->t_before && !plan->t_after &&
-                        cb_tbtf_direct(Span{ftpa, vbytes}, Span{fba, wbytes}, Span{out, expect}, tail);
+    const int wsteps = (2 * d.nantennas + 31) / 32;   // 32-byte K steps
+    const bool four_waves = var.few || (var.tr && !var.ws && var.rows == 4 && tr_four_waves(4, wsteps));
+    const bool direct = four_waves && mode == MODE_INT8 && d.fscrunch == 1 && !plan->t_before && !plan->t_after &&
+                        cb_tbtf_direct(wsteps, Span{ftpa, vbytes}, Span{fba, wbytes}, Span{out, expect}, tail);
     void* kout = out;
     if (mode == MODE_INT8) {
         if (workspace) {

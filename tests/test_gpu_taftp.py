@@ -451,6 +451,9 @@ def test_cb_ib_next_weights_split_transposed(gpu, oracle, A, B, ib_ts, ib_fs, va
     (20, 8, 2, 8, 8, 32, 4, "", True),           # a weight of -128: the exact path
     (16, 64, 8, 64, 16, 128, 16, "", False),     # the largest outputs written directly (512 KiB)
     (16, 64, 9, 64, 16, 16, 16, "", False),      # just above
+    (72, 8, 2, 136, 16, 16, 4, "", False),       # more than 64 antennas: beam groups, over five K steps
+    (128, 4, 2, 72, 4, 32, 16, "", False),
+    (100, 8, 2, 72, 32, 16, 8, "", True),
     (16, 16, 2, 32, 16, 16, 32, "", False),      # windows longer than a tile: partials
     (16, 16, 2, 32, 16, 32, 16, "weights", False),   # next weights over this block's
     (16, 16, 2, 32, 4, 16, 16, "block", False),  # beams over the block
