@@ -27,9 +27,11 @@ struct fbf_batch {
     std::vector<fbf_cb_plan*> plans;
     fbf_ib_plan* ib = nullptr;
     bool ib_fused = false;         // incoherent beam computed by the split-transpose pass
-    void* ftpa = nullptr;          // full-antenna FTPA workspace
+    // Full-antenna FTPA workspace; a block that is read straight from TAFTP
+    // leaves its incoherent-beam partials there instead.
+    void* ftpa = nullptr;
     size_t ftpa_bytes = 0;
-    void* ibp = nullptr;           // incoherent-beam partials of each subarray, where they share the antennas out
+    bool shares_antennas = false;  // each of the block's antennas in exactly one subarray
     std::vector<hipStream_t> streams;
     std::vector<hipEvent_t> join;
     hipEvent_t fork_ib = nullptr;   // block available: incoherent beam may start
@@ -80,7 +82,6 @@ static void batch_release(fbf_batch* b)
     for (auto* p : b->plans) fbf_cb_plan_destroy(p);
     if (b->ib) fbf_ib_plan_destroy(b->ib);
     if (b->ftpa) (void)hipFree(b->ftpa);
-    if (b->ibp) (void)hipFree(b->ibp);
     for (auto s : b->streams) (void)hipStreamDestroy(s);
     for (auto e : b->join) (void)hipEventDestroy(e);
     if (b->fork_ib) (void)hipEventDestroy(b->fork_ib);
@@ -131,6 +132,7 @@ extern "C" int fbf_batch_create(int total_nantennas, int nchans, int nsamples_pe
             return st;
         }
     }
+    b->shares_antennas = batch_shares_antennas(b);
     b->ftpa_bytes = (size_t)4 * total_nantennas * nchans * nsamples_per_heap * nheap_groups;
     hipError_t e = hipMalloc(&b->ftpa, b->ftpa_bytes);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->fork_ib, hipEventDisableTiming);
@@ -165,14 +167,6 @@ extern "C" int fbf_batch_enable_ib(fbf_batch* b, int tscrunch, int fscrunch, int
     fbf_ib_plan* p = nullptr;
     int st = fbf_ib_plan_create(&d, offsets, scales, &p);
     if (st) return st;
-    if (!b->ibp && batch_shares_antennas(b)) {
-        // (16 bytes per channel and sample for each subarray.)
-        const hipError_t e = hipMalloc(&b->ibp, (size_t)16 * b->F * b->nhg * b->S * b->subs.size());
-        if (e != hipSuccess) {
-            fbf_ib_plan_destroy(p);
-            return hip_status(e, "hipMalloc(incoherent-beam partials)");
-        }
-    }
     if (b->ib) fbf_ib_plan_destroy(b->ib);
     b->ib = p;
     b->ib_fused = fscrunch == 1 && tscrunch > 0 && 32 % tscrunch == 0 && b->S % 32 == 0;
@@ -342,12 +336,16 @@ static int batch_enqueue_direct(fbf_batch* b, const void* taftp, size_t taftp_by
         st = fbf_ib_output_bytes(b->ib, taftp_bytes, &ob);
         if (st) return st;
     }
-    const bool partials = b->ib && b->ibp && batch_direct(b, true);
+    // 16 bytes per channel and sample for each subarray: subarrays of at least
+    // four antennas that share the block's out leave room in its FTPA copy's
+    // place.
+    const bool partials = b->ib && b->shares_antennas && (size_t)16 * b->F * T * n <= b->ftpa_bytes &&
+                          batch_direct(b, true);
     if (b->ib && !partials) {
         st = fbf_ib_beamform(b->ib, taftp, taftp_bytes, outputs[n], ob, stream);
         if (st) return st;
     }
-    int* const part = static_cast<int*>(b->ibp);
+    int* const part = static_cast<int*>(b->ftpa);
     const size_t step = (size_t)4 * b->F * T;   // ints per subarray
     IbFinishJob job{};
     if (partials) {
