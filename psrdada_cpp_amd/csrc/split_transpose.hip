@@ -10,11 +10,13 @@
 // loads into LDS, then each thread gathers 8 consecutive elements of the
 // output block and writes them as one 16-byte vector, across columns where
 // the antennas are no multiple of 4 (the tile holds them all; multiples of 4
-// take 8-byte vectors), so the output side is coalesced for any antennas.  HBM-bound.  The stores are
-// nontemporal: the block written is as large as the one read, and leaves the
-// cache to it.  44 of 64 antennas, 64 channels, 12 heaps (69 MB moved):
-// 13.8 us with cached stores from 64-column tiles, 13.1 us now; 13 of
-// 17 antennas, 83 channels, 39 heaps: 36.9 us with 2-byte stores, 14.7 us now.
+// take 8-byte vectors), so the output side is coalesced for any antennas.
+// HBM-bound.  These stores are nontemporal: the block written is as large as the
+// one read, and leaves the cache to it.  44 of 64 antennas, 64 channels, 12
+// heaps (69 MB moved): 13.8 us with cached stores from 64-column tiles, 12.6 us
+// now; 13 of 17 antennas, 83 channels, 39 heaps: 36.9 us with 2-byte stores,
+// 14.7 us now.  Full tiles and large blocks keep to cached stores from 64 x 64
+// tiles (NEAR, st_near).
 //
 // A launch can also generate the block's beamforming weights: its first
 // work-groups run the weights generator (weights_run) and leave, and the
@@ -52,6 +54,15 @@ __device__ __forceinline__ void store_stream(int v, int16_t* dst)
 }
 __device__ __forceinline__ void store_stream(int16_t v, int16_t* dst) { __builtin_nontemporal_store(v, dst); }
 
+template <bool NEAR, typename V>
+__device__ __forceinline__ void store_out(V v, int16_t* dst)
+{
+    if constexpr (NEAR)
+        *reinterpret_cast<V*>(dst) = v;
+    else
+        store_stream(v, dst);
+}
+
 // Incoherent beam computed from the same tiles (all antennas of the block):
 // output [sample_out][channel] int8, tscrunch dividing the tile's 32 samples,
 // fscrunch 1 (IncoherentBeamformer.cu:10-69).
@@ -65,21 +76,23 @@ struct IbTile {
 // SP: columns of the tile (its antennas are 8192 / SP).  U > 0: vectors of U
 // antennas of one column (U divides used_nantennas); U = 0: 16-byte vectors
 // of the whole output block, all antennas in one tile; `inv` is then
-// ceil(2^32 / used_nantennas).
-template <int U, int SP, bool IB>
+// ceil(2^32 / used_nantennas).  NEAR: tiles of 64 antennas, neighbours on one
+// XCD, cached stores.
+template <int U, int SP, bool IB, bool NEAR>
 __global__ __launch_bounds__(256) void split_transpose_k(
     const int16_t* __restrict__ in, int16_t* __restrict__ out,
     int nheap_groups, int total_nantennas, int used_nantennas, int start_antenna,
     int nchans, int sp_per_heap, int n_sp_tiles, uint32_t inv, IbTile ib, WeightsJob wj)
 {
-    constexpr int kTileA = 8192 / SP;
+    constexpr int kTileA = NEAR ? 64 : 8192 / SP;
     constexpr int TPR = SP / 8;         // threads per row
     constexpr int RPP = 256 / TPR;      // rows per pass
     __shared__ int16_t tile[kTileA][SP + kPad];
     __shared__ int ibsum[4][SP / 2];
     const int tid = threadIdx.x;
     if (weights_job_run(wj, tid)) return;   // uniform over the work-group
-    const int logical = (int)blockIdx.x - wj.nblocks;
+    const int logical = NEAR ? xcd_remap((int)blockIdx.x - wj.nblocks, (int)gridDim.x - wj.nblocks)
+                             : (int)blockIdx.x - wj.nblocks;
     const int spt = logical % n_sp_tiles;
     const int rest = logical / n_sp_tiles;
     const int hg = rest % nheap_groups;
@@ -98,30 +111,40 @@ __global__ __launch_bounds__(256) void split_transpose_k(
     for (int ab = 0; ab < used_nantennas; ab += kTileA) {
         const int na = min(kTileA, used_nantennas - ab);
         const int col = (tid % TPR) * 8;
-        int4 v[kTileA / RPP];
-#pragma unroll
-        for (int pass = 0; pass < kTileA / RPP; ++pass) {
-            const int r = pass * RPP + tid / TPR;
-            if (r < na) {
-                const size_t row = ((size_t)hg * total_nantennas + start_antenna + ab + r) * nchans + f;
-                v[pass] = *reinterpret_cast<const int4*>(in + row * sp_per_heap + (size_t)spt * SP + col);
+        auto load = [&](int r) {
+            const size_t row = ((size_t)hg * total_nantennas + start_antenna + ab + r) * nchans + f;
+            return *reinterpret_cast<const int4*>(in + row * sp_per_heap + (size_t)spt * SP + col);
+        };
+        auto stage = [&](int r, const int4& v) {
+            if (IB) {
+                ibacc[0] = __builtin_amdgcn_sdot4(v.x, v.x, ibacc[0], false);
+                ibacc[1] = __builtin_amdgcn_sdot4(v.y, v.y, ibacc[1], false);
+                ibacc[2] = __builtin_amdgcn_sdot4(v.z, v.z, ibacc[2], false);
+                ibacc[3] = __builtin_amdgcn_sdot4(v.w, v.w, ibacc[3], false);
             }
-        }
+            uint32_t* dst = reinterpret_cast<uint32_t*>(&tile[r][col]);
+            dst[0] = (uint32_t)v.x;
+            dst[1] = (uint32_t)v.y;
+            dst[2] = (uint32_t)v.z;
+            dst[3] = (uint32_t)v.w;
+        };
+        if constexpr (NEAR) {
 #pragma unroll
-        for (int pass = 0; pass < kTileA / RPP; ++pass) {
-            const int r = pass * RPP + tid / TPR;
-            if (r < na) {
-                if (IB) {
-                    ibacc[0] = __builtin_amdgcn_sdot4(v[pass].x, v[pass].x, ibacc[0], false);
-                    ibacc[1] = __builtin_amdgcn_sdot4(v[pass].y, v[pass].y, ibacc[1], false);
-                    ibacc[2] = __builtin_amdgcn_sdot4(v[pass].z, v[pass].z, ibacc[2], false);
-                    ibacc[3] = __builtin_amdgcn_sdot4(v[pass].w, v[pass].w, ibacc[3], false);
-                }
-                uint32_t* dst = reinterpret_cast<uint32_t*>(&tile[r][col]);
-                dst[0] = (uint32_t)v[pass].x;
-                dst[1] = (uint32_t)v[pass].y;
-                dst[2] = (uint32_t)v[pass].z;
-                dst[3] = (uint32_t)v[pass].w;
+            for (int pass = 0; pass < kTileA / RPP; ++pass) {
+                const int r = pass * RPP + tid / TPR;
+                if (r < na) stage(r, load(r));
+            }
+        } else {
+            int4 v[kTileA / RPP];
+#pragma unroll
+            for (int pass = 0; pass < kTileA / RPP; ++pass) {
+                const int r = pass * RPP + tid / TPR;
+                if (r < na) v[pass] = load(r);
+            }
+#pragma unroll
+            for (int pass = 0; pass < kTileA / RPP; ++pass) {
+                const int r = pass * RPP + tid / TPR;
+                if (r < na) stage(r, v[pass]);
             }
         }
         __syncthreads();
@@ -136,7 +159,7 @@ __global__ __launch_bounds__(256) void split_transpose_k(
                 } pack;
 #pragma unroll
                 for (int i = 0; i < U; ++i) pack.e[i] = tile[u * U + i][sp];
-                store_stream(pack.v, out + (out_block + sp) * used_nantennas + ab + u * U);
+                store_out<NEAR>(pack.v, out + (out_block + sp) * used_nantennas + ab + u * U);
             }
         } else {
             // SP is a multiple of 8, so the block is whole 16-byte vectors
@@ -156,7 +179,7 @@ __global__ __launch_bounds__(256) void split_transpose_k(
                         ++sp;
                     }
                 }
-                store_stream(pack.v, out + out_block * used_nantennas + (size_t)idx * 8);
+                store_out<NEAR>(pack.v, out + out_block * used_nantennas + (size_t)idx * 8);
             }
         }
         __syncthreads();
@@ -194,7 +217,7 @@ using namespace fbf;
 
 namespace {
 
-template <int SP, bool IB>
+template <int SP, bool IB, bool NEAR = false>
 int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna,
                 int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream)
 {
@@ -205,12 +228,17 @@ int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nan
     // Vectors of 8 antennas where they divide; else, while one tile holds
     // every antenna, 16-byte vectors across columns; else what divides.
     const uint32_t inv = (uint32_t)(((1ull << 32) + used_nantennas - 1) / used_nantennas);
-    const auto kernel = used_nantennas % 8 == 0       ? split_transpose_k<8, SP, IB>
-                        : used_nantennas % 4 == 0     ? split_transpose_k<4, SP, IB>
-                        : used_nantennas == 1         ? split_transpose_k<1, SP, IB>
-                        : used_nantennas <= 8192 / SP ? split_transpose_k<0, SP, IB>
-                        : used_nantennas % 2 == 0        ? split_transpose_k<2, SP, IB>
-                                                         : split_transpose_k<1, SP, IB>;
+    const auto kernel = [&] {
+        if constexpr (NEAR)
+            return used_nantennas % 8 == 0 ? split_transpose_k<8, SP, IB, true> : split_transpose_k<4, SP, IB, true>;
+        else
+            return used_nantennas % 8 == 0       ? split_transpose_k<8, SP, IB, false>
+                   : used_nantennas % 4 == 0     ? split_transpose_k<4, SP, IB, false>
+                   : used_nantennas == 1         ? split_transpose_k<1, SP, IB, false>
+                   : used_nantennas <= 8192 / SP ? split_transpose_k<0, SP, IB, false>
+                   : used_nantennas % 2 == 0     ? split_transpose_k<2, SP, IB, false>
+                                                 : split_transpose_k<1, SP, IB, false>;
+    }();
     kernel<<<dim3((unsigned)nblocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const int16_t*>(taftp), static_cast<int16_t*>(ftpa), nhg, total_nantennas, used_nantennas,
         start_antenna, nchans, sp_per_heap, n_sp_tiles, inv, ib, wj);
@@ -218,10 +246,32 @@ int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nan
     return FBF_OK;
 }
 
+// Whether a block takes 64 x 64 tiles with cached stores: antennas in fours
+// (others need their vectors across columns) that fill such tiles, and copies
+// that outgrow the cache.  us, these tiles against 64 x 128 with nontemporal
+// stores (antennas / channels / heaps of 256 samples; with the incoherent beam
+// in brackets): 64/64/32 46 against 61 (46, 66), 64/64/12 16.2 against 17.0,
+// 56/64/32 41 against 45 (42, 46), 128/64/32 116 against 128 (116, 125), 60/64/32
+// 46 against 49, 40/64/48 (252 MB moved) 43 against 48; but 40/64/32 (168 MB) 31
+// against 25 (37, 28), and with the incoherent beam 40/64/48 53 against 49.
+bool st_near(bool ib, int used_nantennas, size_t moved)
+{
+    // (Columns of whole 64-byte lines, 32 antennas, gain from the cache sooner:
+    // 32/64/32, 128 MiB, 21.5 against 22.9; 32/64/16 11.6 against 11.4.)
+    const size_t near_bytes = (size_t)(used_nantennas % 32 == 0 ? 128 : 192) << 20;
+    if (used_nantennas % 4 != 0) return false;
+    if (used_nantennas > 64) return true;
+    if (used_nantennas >= 56 && used_nantennas % 8 == 0) return true;
+    return moved >= near_bytes && (!ib || used_nantennas >= 56);
+}
+
 template <bool IB>
 int st_launch_sp(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna,
                  int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream)
 {
+    if (st_near(IB, used_nantennas, (size_t)8 * used_nantennas * nchans * nsamples_per_heap * nhg))
+        return st_launch_t<64, IB, true>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
+                                         nsamples_per_heap, nhg, ib, wj, stream);
     // Tiles of 128 columns where 64 antennas hold a subset and they divide a
     // heap, else of 64 columns and 128 antennas.
     if (used_nantennas <= 64 && nsamples_per_heap % 64 == 0)

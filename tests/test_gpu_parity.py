@@ -730,6 +730,8 @@ def test_ib_antenna_runs_bit_exact(gpu, oracle, A, F, nhg, ts, fs):
     (130, 127, 1, 3, 1, 256), (20, 13, 3, 5, 3, 32),  # and 64-column tiles
     (150, 131, 2, 2, 1, 64), (140, 130, 5, 2, 1, 32), # two tiles of antennas: single ones and pairs
     (70, 68, 1, 3, 2, 96), (70, 1, 69, 3, 2, 64),
+    (60, 56, 3, 3, 2, 32), (150, 136, 9, 2, 2, 64),   # cached stores from 64 x 64 tiles, a ragged last one
+    (130, 100, 5, 9, 3, 96),
 ])
 def test_split_transpose_tile_shapes_bit_exact(gpu, oracle, A, used, a0, F, nhg, S):
     capi = gpu
@@ -739,3 +741,19 @@ def test_split_transpose_tile_shapes_bit_exact(gpu, oracle, A, used, a0, F, nhg,
     capi.split_transpose(_dev(capi, taftp), d_out, A, used, a0, F, nsamples_per_heap=S)
     np.testing.assert_array_equal(d_out.download(),
                                   oracle.split_transpose(taftp, nhg, A, used, a0, F, nsamples_per_heap=S))
+
+
+@pytest.mark.parametrize("A,F,nhg,ts", [(56, 4, 2, 32), (100, 12, 1, 4), (136, 4, 2, 1), (44, 8, 2, 16)])
+def test_split_transpose_ib_tile_shapes_bit_exact(gpu, oracle, A, F, nhg, ts):
+    """The incoherent beam in the split-transpose's pass: tiles of 64 x 64 over
+    one, two and three runs of antennas, and of 64 x 128."""
+    capi = gpu
+    taftp = gaussian_int8(6500 + A, nhg * A * F * 256 * 4, 40.0)
+    _, _, ibo, ibs = oracle.power_levels(40.0, 24.0, A, ts, 1, A, ts, 1)
+    off, sc = np.full(F, ibo, np.float32), np.full(F, ibs, np.float32)
+    plan = capi.IbPlan(A, F, ts, 1, off, sc)
+    d_out, d_tf = capi.DeviceBuffer(taftp.size), capi.DeviceBuffer(plan.output_bytes(taftp.nbytes))
+    capi.split_transpose_ib(_dev(capi, taftp), d_out, F, plan, d_tf)
+    np.testing.assert_array_equal(d_out.download(), oracle.split_transpose(taftp, nhg, A, A, 0, F))
+    ib_ref = oracle.ib_tf(oracle.ib_power(taftp, F, ts, 1, nhg, A), off, sc)
+    np.testing.assert_array_equal(d_tf.download(), ib_ref.reshape(-1))
