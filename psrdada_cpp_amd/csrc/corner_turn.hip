@@ -133,6 +133,18 @@ __global__ __launch_bounds__(256) void corner_turn_k(CtArgs a)
     }
     __syncthreads();
     const int ou = nr * EU;
+    if (ou <= 16) {
+        // Few rows: a wave of the loop below would be nearly empty.  1 channel,
+        // 300 samples, 2 bands, 100 beams, 4 groups: 10.2 us through it, 4.5
+        // here; 64, 512, 1, 256, 4 (34 MB): 23.3 and 13.3; but 26 units (13, 64,
+        // 2, 500, 4) 9.6 and 10.1.
+        for (int i = threadIdx.x; i < nc * ou; i += 256) {
+            const int c = (int)((uint32_t)i / (uint32_t)ou), k = i - c * ou;
+            const int r = EU == 1 ? k : (int)__umulhi((uint32_t)k, a.inv_eu);
+            store_unit(tile[r * pitch + c * EU + k - r * EU], dst + (size_t)c * out_row + k, a.store_past);
+        }
+        return;
+    }
     for (int k = lane; k < ou; k += 64) {
         const int r = EU == 1 ? k : (int)__umulhi((uint32_t)k, a.inv_eu);
         const U* t = tile + r * pitch + (k - r * EU);

@@ -87,6 +87,9 @@ def test_feng_to_dada_rejects_bad_sizes(gpu):
     (48, 133, 5, 7, 2, 2, 5),        # 16-byte units, three to an element, few bands
     (256, 64, 32, 33, 1, 0, 33),     # 16 MiB and more: stored past the cache
     (36, 512, 64, 15, 1, 0, 15),     # the same in 4-byte units
+    (64, 100, 1, 6, 3, 1, 5),        # one band: rows of four units
+    (1, 300, 2, 5, 4, 0, 5),         # two bands of single bytes
+    (5, 77, 3, 4, 2, 0, 4), (17, 33, 1, 3, 2, 0, 3),   # 15 and 17 units
 ])
 def test_tuse_transpose_tile_shapes_bit_exact(gpu, C, S, F, B, G, b0, nb):
     """Tile shapes by unit size, bands and block size against numpy."""
