@@ -41,8 +41,9 @@ __device__ __forceinline__ int sq4(int x, int acc)
 }
 
 // NW waves per work-group: 4, or 16 where the grid is small; PAST: the block
-// is read past the cache (ib_run).
-template <int MODE, int NW, bool PAST>
+// is read past the cache (ib_run); ONE: a wave per output channel, NW of them
+// to a work-group, instead of the waves sharing one's rows out.
+template <int MODE, int NW, bool PAST, bool ONE>
 __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
 {
     constexpr int S = 256;
@@ -52,8 +53,9 @@ __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
     const int sc = tid & 63;   // 16-byte chunk: samples 4*sc .. 4*sc+3
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int logical = xcd_remap((int)blockIdx.x - wj.nblocks, (int)gridDim.x - wj.nblocks);
-    const int fo = logical % p.Fo;
-    const int hg = logical / p.Fo;
+    const int groups = ONE ? (p.Fo + NW - 1) / NW : p.Fo;
+    const int fo = ONE ? logical % groups * NW + wave : logical % groups;
+    const int hg = logical / groups;
     if (hg >= p.nhg) return;
 
     // Rows (channel k, antenna a) of the output channel, antennas fastest; this
@@ -64,9 +66,9 @@ __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
     long long s0 = 0, s1 = 0, s2 = 0, s3 = 0;
     const size_t row_bytes = (size_t)S * 4;
     const size_t astride = (size_t)p.F * row_bytes;
-    const int rows = p.fs * p.A;   // (1 KiB each: below 2^31)
-    const int per = (rows + NW - 1) / NW;
-    int r = min(wave * per, rows);
+    const int rows = ONE && fo >= p.Fo ? 0 : p.fs * p.A;   // (1 KiB each: below 2^31)
+    const int per = ONE ? rows : (rows + NW - 1) / NW;
+    int r = ONE ? 0 : min(wave * per, rows);
     const int r1 = min(r + per, rows);
     const int k0 = r / p.A;
     int a = r - k0 * p.A;
@@ -125,11 +127,15 @@ __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
     __syncthreads();
 
     // The waves' sums of a window.
-    if (tid < nwin) {
+    for (int w = ONE ? sc : tid; w < nwin && fo < p.Fo; w += ONE ? 64 : 64 * NW) {
         long long v = 0;
+        if constexpr (ONE) {
+            v = part[wave][w];
+        } else {
 #pragma unroll
-        for (int r = 0; r < NW; ++r) v += part[r][tid];
-        const size_t t = (size_t)hg * nwin + tid;
+            for (int r = 0; r < NW; ++r) v += part[r][w];
+        }
+        const size_t t = (size_t)hg * nwin + w;
         if (MODE == IB_POWER) {
             static_cast<double*>(p.out)[t * p.Fo + fo] = (double)v;
         } else {
@@ -139,12 +145,17 @@ __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
 }
 
 template <int MODE>
-void launch_ib(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool wide, bool past, hipStream_t s)
+void launch_ib(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool one, bool wide, bool past, hipStream_t s)
 {
-    if (wide)
-        past ? ib_k<MODE, 16, true><<<grid, 1024, 0, s>>>(a, wj) : ib_k<MODE, 16, false><<<grid, 1024, 0, s>>>(a, wj);
+    if (one)
+        past ? ib_k<MODE, 4, true, true><<<grid, 256, 0, s>>>(a, wj)
+             : ib_k<MODE, 4, false, true><<<grid, 256, 0, s>>>(a, wj);
+    else if (wide)
+        past ? ib_k<MODE, 16, true, false><<<grid, 1024, 0, s>>>(a, wj)
+             : ib_k<MODE, 16, false, false><<<grid, 1024, 0, s>>>(a, wj);
     else
-        past ? ib_k<MODE, 4, true><<<grid, 256, 0, s>>>(a, wj) : ib_k<MODE, 4, false><<<grid, 256, 0, s>>>(a, wj);
+        past ? ib_k<MODE, 4, true, false><<<grid, 256, 0, s>>>(a, wj)
+             : ib_k<MODE, 4, false, false><<<grid, 256, 0, s>>>(a, wj);
 }
 
 }  // namespace
@@ -263,19 +274,24 @@ static int ib_run(fbf_ib_plan* plan, int mode, const void* taftp, size_t taftp_b
     a.ts = d.tscrunch;
     a.fs = d.fscrunch;
     a.quant = d.quant_mode;
-    const long long work = nhg * Fo;
+    // A wave per output channel where there are few rows and many outputs:
+    // one row or two to a wave left mostly the sums over the waves (us, shared
+    // out against a wave each; antennas / channels / heaps, tscrunch 16:
+    // 4/128/48 10.3 against 6.1, 8/64/32 5.7 against 4.8, 12/64/32 6.4 against 5.8).
+    const bool one = (long long)d.nantennas * d.fscrunch <= 12 && nhg * Fo >= 1024;
+    const long long work = one ? nhg * ((Fo + 3) / 4) : nhg * Fo;
     const long long nblocks = work + wj.nblocks;
     FBF_REQUIRE(nblocks < (1ll << 31), FBF_ERR_UNSUPPORTED, "fbf_ib: grid too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
     // 16 waves share the rows of a small block's few work-groups, at least two
     // each (the weights job is made of work-groups of 4).
-    const bool wide = work < 1024 && (long long)d.nantennas * d.fscrunch >= 32 && wj.nblocks == 0;
+    const bool wide = !one && work < 1024 && (long long)d.nantennas * d.fscrunch >= 32 && wj.nblocks == 0;
     const bool past = taftp_bytes >= ((size_t)16 << 20);   // (smaller blocks may be in the cache)
     const dim3 grid((unsigned)nblocks);
     if (mode == IB_INT8)
-        launch_ib<IB_INT8>(a, wj, grid, wide, past, s);
+        launch_ib<IB_INT8>(a, wj, grid, one, wide, past, s);
     else
-        launch_ib<IB_POWER>(a, wj, grid, wide, past, s);
+        launch_ib<IB_POWER>(a, wj, grid, one, wide, past, s);
     FBF_LAUNCH_CHECK("ib_k");
     return FBF_OK;
 }

@@ -704,7 +704,9 @@ def test_cb_antennas_in_fours_bit_exact(gpu, oracle, variant, F, T, A, B, ts, fs
 
 
 @pytest.mark.parametrize("A,F,nhg,ts,fs", [
-    (5, 260, 4, 1, 1),       # four waves, fewer antennas than a run each
+    (5, 260, 4, 1, 1),       # a wave per output channel
+    (3, 1032, 4, 16, 4),     # the same, a group short of output channels
+    (13, 260, 4, 1, 1),      # four waves share an output channel's rows
     (3, 8, 2, 256, 2),       # 16 waves, most of them without antennas
     (91, 4, 3, 2, 4),        # 16 waves, a short last run
     (70, 352, 3, 16, 1),     # four waves of 18, 18, 18 and 16 antennas
