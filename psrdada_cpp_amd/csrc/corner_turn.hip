@@ -17,6 +17,8 @@
 // 23.8 us).
 #include "fbf_internal.hpp"
 
+#include <algorithm>
+
 #include <climits>
 
 namespace fbf {
@@ -34,6 +36,7 @@ struct CtArgs {
     int tiles_r, tiles_c;
     int sh_ru, sh_eu;              // square tiles: log2(TC * EU), log2(EU) (when powers of two)
     uint32_t inv_eu;               // ceil(2^32 / EU)
+    uint32_t inv_ou;               // ceil(2^32 / (TR * EU)): the units of a full tile's output row
     bool load_past, store_past;    // the block is read, and written, past the cache
 };
 
@@ -120,26 +123,39 @@ __global__ __launch_bounds__(256) void corner_turn_k(CtArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int ru = nc * EU;
-    for (int r = wave; r < nr; r += 16) {   // up to four rows' loads in flight
-        for (int k = lane; k < ru; k += 64) {
-            U v[4];
+    if (ru < 64 && nr * ru <= 256) {
+        // A matrix of few units: all of it at once (8 channels, 22 samples, 3
+        // bands, 412 beams, 6 groups: 6.4 us through the loop below, 5.1 so).
+        const int r = (int)threadIdx.x / ru, k = (int)threadIdx.x - r * ru;
+        if (r < nr) tile[r * pitch + k] = load_unit(src + (size_t)r * in_row + k, a.load_past);
+    } else if (nr < 4) {
+        // A wave per row would leave some without one: 64 channels, 512
+        // samples, 1 band, 256 beams, 4 groups (34 MB) 17.8 us so, 12.4 here.
+        for (int r = 0; r < nr; ++r)
+            for (int k = threadIdx.x; k < ru; k += 256)
+                tile[r * pitch + k] = load_unit(src + (size_t)r * in_row + k, a.load_past);
+    } else {
+        for (int r = wave; r < nr; r += 16) {   // up to four rows' loads in flight
+            for (int k = lane; k < ru; k += 64) {
+                U v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (r + 4 * j < nr) v[j] = load_unit(src + (size_t)(r + 4 * j) * in_row + k, a.load_past);
+                for (int j = 0; j < 4; ++j)
+                    if (r + 4 * j < nr) v[j] = load_unit(src + (size_t)(r + 4 * j) * in_row + k, a.load_past);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (r + 4 * j < nr) tile[(r + 4 * j) * pitch + k] = v[j];
+                for (int j = 0; j < 4; ++j)
+                    if (r + 4 * j < nr) tile[(r + 4 * j) * pitch + k] = v[j];
+            }
         }
     }
     __syncthreads();
     const int ou = nr * EU;
-    if (ou <= 16) {
+    if (ou <= 16 && nr == a.TR) {
         // Few rows: a wave of the loop below would be nearly empty.  1 channel,
         // 300 samples, 2 bands, 100 beams, 4 groups: 10.2 us through it, 4.5
-        // here; 64, 512, 1, 256, 4 (34 MB): 23.3 and 13.3; but 26 units (13, 64,
+        // here; but 26 units (13, 64,
         // 2, 500, 4) 9.6 and 10.1.
         for (int i = threadIdx.x; i < nc * ou; i += 256) {
-            const int c = (int)((uint32_t)i / (uint32_t)ou), k = i - c * ou;
+            const int c = ou == 1 ? i : (int)__umulhi((uint32_t)i, a.inv_ou), k = i - c * ou;
             const int r = EU == 1 ? k : (int)__umulhi((uint32_t)k, a.inv_eu);
             store_unit(tile[r * pitch + c * EU + k - r * EU], dst + (size_t)c * out_row + k, a.store_past);
         }
@@ -176,16 +192,29 @@ __global__ __launch_bounds__(256) void corner_turn_w4_k(CtArgs a)
     const uint32_t* src = in + (size_t)r0 * a.C + c0;
     uint32_t* dst = out + (size_t)c0 * a.R + r0;
     if (nr == T && nc == T) {
+        // One uniform branch around all four loads: a branch for each kept them
+        // from being in flight together (64 channels, 146 heaps 4.9 us, 4.5
+        // so).
+        uint4 v[4];
+        auto load = [&](bool past) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = threadIdx.x + 256 * j;
+                v[j] = load_unit(reinterpret_cast<const uint4*>(src + (size_t)(i >> 4) * a.C + ((i & 15) << 2)), past);
+            }
+        };
+        if (a.load_past)
+            load(true);
+        else
+            load(false);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int i = threadIdx.x + 256 * j;
-            const int r = i >> 4, c = (i & 15) << 2;
-            const uint4 v = load_unit(reinterpret_cast<const uint4*>(src + (size_t)r * a.C + c), a.load_past);
-            uint32_t* l = tile + r * P + c;
-            l[0] = v.x;
-            l[1] = v.y;
-            l[2] = v.z;
-            l[3] = v.w;
+            uint32_t* l = tile + (i >> 4) * P + ((i & 15) << 2);
+            l[0] = v[j].x;
+            l[1] = v[j].y;
+            l[2] = v[j].z;
+            l[3] = v[j].w;
         }
         __syncthreads();
 #pragma unroll
@@ -245,7 +274,7 @@ int ct_launch_u(CtArgs a, long long n1, int E, hipStream_t s)
     a.TR = a.TC = T;
     if (a.R < T) {
         a.TR = a.R;
-        for (int tc = T * T / a.R; tc > T && a.TC == T; tc -= T)
+        for (int tc = std::min(T * T / a.R, (a.C + T - 1) / T * T); tc > T && a.TC == T; tc -= T)
             if (ct_tile_bytes(a.TR, tc, a.EU, sizeof(U)) <= kCtLdsMax && tiles(a.TR, tc) >= 512) a.TC = tc;
     }
     const size_t shm = ct_tile_bytes(a.TR, a.TC, a.EU, sizeof(U));
@@ -259,6 +288,8 @@ int ct_launch_u(CtArgs a, long long n1, int E, hipStream_t s)
     a.sh_ru = ilog2_exact((long long)T * a.EU);
     a.sh_eu = ilog2_exact(a.EU);
     a.inv_eu = (uint32_t)(((1ull << 32) + a.EU - 1) / a.EU);   // (0 for EU = 1, unused)
+    const unsigned long long row = (unsigned long long)a.TR * a.EU;   // exact below 2^16 units
+    a.inv_ou = (uint32_t)(((1ull << 32) + row - 1) / row);
     const bool pow2 = a.TR == T && a.sh_ru >= 0 && a.sh_eu >= 0;
     if (pow2)
         corner_turn_k<U, true><<<dim3((unsigned)nblocks), 256, shm, s>>>(a);

@@ -90,6 +90,7 @@ def test_feng_to_dada_rejects_bad_sizes(gpu):
     (64, 100, 1, 6, 3, 1, 5),        # one band: rows of four units
     (1, 300, 2, 5, 4, 0, 5),         # two bands of single bytes
     (5, 77, 3, 4, 2, 0, 4), (17, 33, 1, 3, 2, 0, 3),   # 15 and 17 units
+    (8, 22, 3, 7, 2, 0, 7), (4, 63, 4, 3, 1, 0, 3), (4, 64, 4, 3, 1, 0, 3),   # whole matrices of few units
 ])
 def test_tuse_transpose_tile_shapes_bit_exact(gpu, C, S, F, B, G, b0, nb):
     """Tile shapes by unit size, bands and block size against numpy."""
