@@ -531,17 +531,33 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     // 32, so a lane's Re and Im outputs belong to one beam and its power
     // sums in-lane.
     v4i w[RT][KSTEPS];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
+    auto load_weights = [&](int g, auto al16) {
         const int b = beam_base + 32 * g + c;
         const bool bvalid = b < p.B;
         const int8_t* wcol = p.fba + ((size_t)f * p.B + (bvalid ? b : p.B - 1)) * K;
-        if (K & 15) {   // antennas a multiple of 4 only: rows of 8-byte alignment
 #pragma unroll
-            for (int s = 0; s < KSTEPS; ++s) w[2 * g][s] = load_wslice<false>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+        for (int s = 0; s < KSTEPS; ++s)
+            w[2 * g][s] = load_wslice<decltype(al16)::value>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+    };
+    // Antennas a multiple of 4 only: rows of 8-byte alignment.  One uniform
+    // branch around all groups' loads: with one for each group they waited for
+    // one another, 0.7 to 1.2 us of a launch.  (The larger work-groups have 128
+    // VGPRs a wave and spill two of them that way.)
+    if constexpr (St::NW == 4) {
+        if (K & 15) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) load_weights(g, std::false_type{});
         } else {
 #pragma unroll
-            for (int s = 0; s < KSTEPS; ++s) w[2 * g][s] = load_wslice<true>(wcol, 16 * (h * KSTEPS + s), K, bvalid);
+            for (int g = 0; g < NG; ++g) load_weights(g, std::true_type{});
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (K & 15)
+                load_weights(g, std::false_type{});
+            else
+                load_weights(g, std::true_type{});
         }
     }
 
