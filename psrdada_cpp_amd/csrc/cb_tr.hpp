@@ -3,6 +3,7 @@
 #pragma once
 
 #include "cb_common.hpp"
+#include "cb_stage.hpp"
 
 namespace fbf {
 namespace {
@@ -470,7 +471,6 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
 {
     using St = TrStage<RT, FS, KSTEPS, NTS, NWB>;
     constexpr int KPAD = 32 * KSTEPS;
-    constexpr int PR = 2 * KSTEPS;                 // 16-byte pieces per LDS column
     constexpr int VALS = TrRed<RT, NSLOT>::VALS;
     constexpr int NB = St::NB;
     constexpr int NG = RT / 2;                     // groups of 32 beams per wave
@@ -562,16 +562,11 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
     }
 
     // Staging.  A wave's 16-byte load lands at LDS offset 16 * lane of a
-    // 1 KiB run.  FTPA: the bank swizzle is chosen on the global side:
-    // physical piece pp of column col holds K piece (pp + rot(col)) % PR with
-    // rot(col) = col * KPAD / 256.  K pieces past the column (k >= K) re-read
-    // piece 0: the weights there are zero.  Where K % 16 == 8 the last piece
-    // runs 8 bytes into the next column (zero weights again), and past the
-    // block's end in its very last column: there the load starts 8 bytes
-    // early (`early`) and the operand is moved down (`tail_s`).  TAFTP: a tile is 16 * KSTEPS
-    // antenna rows of 64 bytes (its 32 columns, contiguous in TAFTP), and a
-    // load fills 16 rows, 4 lanes a row; rows past A re-read antenna 0.
-    const int kpieces = (K + 15) / 16;
+    // 1 KiB run.  FTPA: staged_load says which 16 bytes that is; where it
+    // starts early, the operand is moved down (`tail_s`).  TAFTP: a tile is
+    // 16 * KSTEPS antenna rows of 64 bytes (its 32 columns, contiguous in
+    // TAFTP), and a load fills 16 rows, 4 lanes a row; rows past A re-read
+    // antenna 0.
     // LDS: the channel's thresholds first (at address 0, so that a
     // threshold read takes the table's offset as its immediate), then the
     // ring, the dummy run and the fscrunch reduction.
@@ -602,14 +597,10 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
                 cbase[m] = p.ftpa + (size_t)(fo * FS + ti % FS) * p.S * 4;
                 goff[m] = (uint32_t)(p.a0 + an) * (uint32_t)(p.F * p.S * 4) + 16 * (lane & 3);
             } else {
-                const int rem = (u - ti * KSTEPS) * 1024 + lane * 16;
-                const int col = rem / KPAD;
-                const int pp = (rem - col * KPAD) >> 4;
-                const int j = (pp + ((col * KPAD) >> 8)) % PR;
-                const int jj = j < kpieces ? j : 0;
+                const StagedLoad ld = staged_load((u - ti * KSTEPS) * 1024 + lane * 16, KPAD, K, p.vstride);
                 cbase[m] = p.ftpa + (size_t)(fo * FS + ti % FS) * TP * p.vstride + p.voff;
-                goff[m] = (uint32_t)(col * p.vstride + 16 * jj);
-                early[m] = (K & 15) && fo * FS + ti % FS == p.F - 1 && col == 31 && jj == kpieces - 1 ? 8 : 0;
+                goff[m] = (uint32_t)ld.offset;
+                early[m] = fo * FS + ti % FS == p.F - 1 ? ld.early : 0;
             }
             gtile[m] = (tgroup * NTS + ti / FS) * slot_tiles;
             ldst[m] = u * 1024;
@@ -669,16 +660,15 @@ __global__ __launch_bounds__(64 * NTS * NWB * FS, NTS * NWB * FS == 4 ? tr_wgs(R
         for (int s = 0; s < KSTEPS; ++s)
             aoff[s] = (tsl * FS + wc) * KSTEPS * 1024 + (8 * (h * KSTEPS + s) + rr) * 64 + 32 * gh + 8 * xx;
     } else {
-        const int rot = (c * KPAD) >> 8;
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s)
-            aoff[s] = ((tsl * FS + wc) * 32 + c) * KPAD + 16 * ((h * KSTEPS + s - rot + 32 * PR) % PR);
+            aoff[s] = (tsl * FS + wc) * 32 * KPAD + staged_piece(c, h * KSTEPS + s, KPAD);
     }
 
     // The block's last tile (FTPA, K % 16 == 8) and the slice of this lane's
     // operands that was loaded 8 bytes early there.
     const int tail_tile = !TA && (K & 15) && f == p.F - 1 ? ta.ntiles - 1 : -1;
-    const int tail_s = c == 31 ? K / 16 - h * KSTEPS : -1;
+    const int tail_s = c == 31 ? staged_tail_piece(K) - h * KSTEPS : -1;
 
     const bool wave_active = beam_base < p.B;
 #pragma unroll

@@ -60,7 +60,6 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
 {
     using St = WsStage<KSTEPS>;
     constexpr int KPAD = St::KPAD;
-    constexpr int PR = 2 * KSTEPS;
     constexpr int NB = St::NB;
     constexpr int RT = 4, NG = 2;
     static_assert(NSLOT % SPT == 0, "slots");
@@ -126,31 +125,21 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
     }
 
     const size_t TP = (size_t)2 * p.nsamples;
-    const int kpieces = (K + 15) / 16;
     const int chunk_tiles = wa.ct;
 
-    // This lane's part of a tile load m: column and K piece (swizzled as in
-    // cb_tr_k: physical piece pp of column col holds K piece
-    // (pp + col * KPAD / 256) % PR; pieces past K re-read piece 0, whose
-    // weights there are zero; the block's last piece is loaded 8 bytes early
-    // where K % 16 == 8).
+    // This lane's part of a tile load m (staged_load), and the offsets of its K
+    // pieces.
     int goff[St::LPT];
     int early[St::LPT];
 #pragma unroll
     for (int m = 0; m < St::LPT; ++m) {
-        const int off = m * 1024 + lane * 16;
-        const int col = off / KPAD;
-        const int pp = (off - col * KPAD) >> 4;
-        const int j = (pp + ((col * KPAD) >> 8)) % PR;
-        goff[m] = col * p.vstride + 16 * (j < kpieces ? j : 0);
-        early[m] = !AL16 && col == 31 && j == kpieces - 1 ? 8 : 0;
+        const StagedLoad ld = staged_load(m * 1024 + lane * 16, KPAD, K, p.vstride);
+        goff[m] = ld.offset;
+        early[m] = ld.early;
     }
     int aoff[KSTEPS];
-    {
-        const int rot = (c * KPAD) >> 8;
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) aoff[s] = c * KPAD + 16 * ((h * KSTEPS + s - rot + 32 * PR) % PR);
-    }
+    for (int s = 0; s < KSTEPS; ++s) aoff[s] = staged_piece(c, h * KSTEPS + s, KPAD);
 
     // Chunk descriptors: (local unit << 24) | chunk, or -1 once every unit
     // of the work-group is dry.
@@ -272,7 +261,7 @@ __global__ __launch_bounds__(64 * kWsWaves) void cb_ws_k(CbWsArgs wa)
                     if (!AL16 && fo == p.F - 1 && ctile0 + pc + g * wa.tps + x == wa.ntiles - 1) {
 #pragma unroll
                         for (int s = 0; s < KSTEPS; ++s)
-                            if (c == 31 && h * KSTEPS + s == K / 16) a[s] = v4i{a[s].z, a[s].w, a[s].z, a[s].w};
+                            if (c == 31 && h * KSTEPS + s == staged_tail_piece(K)) a[s] = v4i{a[s].z, a[s].w, a[s].z, a[s].w};
                     }
                     wait_vm_lgkm0<63>();
                     // The slot is free again: refill it NB positions ahead.
