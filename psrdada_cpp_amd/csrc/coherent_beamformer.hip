@@ -376,6 +376,18 @@ static int cb_grow(void** buf, size_t* have, size_t bytes, hipStream_t s, void**
     return FBF_OK;
 }
 
+// Whether a call wants more of a buffer than there is while its stream is
+// being captured, which leaves cb_grow only its error.
+static int cb_cannot_grow(size_t have, size_t bytes, hipStream_t s, bool* out)
+{
+    *out = false;
+    if (have >= bytes) return FBF_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    FBF_HIP_TRY(hipStreamIsCapturing(s, &cs));
+    *out = cs != hipStreamCaptureStatusNone;
+    return FBF_OK;
+}
+
 static int cb_staging(fbf_cb_plan* plan, size_t bytes, hipStream_t s, void** out)
 {
     return cb_grow(&plan->staging, &plan->staging_bytes, bytes, s, out);
@@ -716,9 +728,19 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
             FBF_REQUIRE(workspace_bytes >= expect && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
                         FBF_ERR_SIZE, "fbf_cb: workspace too small or not 16-byte aligned");
             kout = workspace;
-        } else if (!direct) {
-            const int st = cb_staging(plan, expect, s, &kout);
-            if (st) return st;
+        } else {
+            // Also where the kernel writes TBTF itself (at most kTbtfDirect
+            // bytes): the plan's next call on such a block may be captured and
+            // need it (beams over its inputs, timing events).
+            bool skip = false;
+            if (direct) {
+                const int st = cb_cannot_grow(plan->staging_bytes, expect, s, &skip);
+                if (st) return st;
+            }
+            if (!skip) {
+                const int st = cb_staging(plan, expect, s, &kout);
+                if (st) return st;
+            }
         }
     }
     // The timing events (fbf_cb_plan_set_timing), around the coherent kernel only.

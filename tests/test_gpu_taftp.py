@@ -503,3 +503,72 @@ def test_small_block_outputs_in_one_launch(gpu, oracle, A, F, nhg, B, ts, ohs, i
 class _View:
     def __init__(self, ptr, nbytes):
         self.ptr, self.nbytes = ptr, nbytes
+
+
+def _captured(capi, stream, call):
+    """The call captured into an executable graph; returns its launcher."""
+    import ctypes as C
+    hip = capi.lib()   # (finds the HIP runtime's functions through its dependencies)
+    graph, execg = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream.handle, 1) == 0
+    try:
+        call()
+    finally:
+        e = hip.hipStreamEndCapture(stream.handle, C.byref(graph))
+    assert e == 0 and hip.hipGraphInstantiate(C.byref(execg), graph, None, None, C.c_size_t(0)) == 0
+    return lambda: hip.hipGraphLaunch(execg, stream.handle)
+
+
+@pytest.mark.parametrize("warm,captured,Atot,A,a0,F,nhg,nhg_warm,B,ts", [
+    ("ftpa", "ftpa over the block", 16, 16, 0, 4, 2, 2, 32, 4),   # first in one launch, then staged
+])
+def test_calls_captured_after_other_calls(gpu, oracle, warm, captured, Atot, A, a0, F, nhg, nhg_warm, B, ts):
+    """A call that is captured uses the scratch that other calls of its plan
+    have left: one call runs eagerly, another is captured on a block of at most
+    that size and replayed on new voltages, against the oracle."""
+    capi = gpu
+    S = 256
+    off, sc = _levels(oracle, A, ts, 1, F)
+    _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, 8, ts, 1, Atot, 16, 1)
+    ioff, isc = np.full(F, ibo, np.float32), np.full(F, ibs, np.float32)
+    plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=S // ts)
+    ib = capi.IbPlan(Atot, F, 16, 1, ioff, isc)
+    w = unit_weights(3800 + A, F * B * A)
+    d_w = _dev(capi, w)
+    s = capi.Stream()
+
+    def call(name, d_t, d_o, d_tf):
+        if name == "both":
+            plan.ib_beamform_taftp(ib, d_t, d_w, d_o, d_tf, stream=s)
+        elif name == "taftp":
+            plan.beamform_taftp(d_t, d_w, d_o, nantennas_total=Atot, start_antenna=a0, stream=s)
+        else:
+            plan.beamform(d_t, d_w, d_o, stream=s)
+
+    def buffers(n):
+        return (capi.DeviceBuffer(n * Atot * F * S * 4), capi.DeviceBuffer(F * (n * S // ts) * B),
+                capi.DeviceBuffer(F * n * 16))
+
+    bufs = buffers(nhg_warm)
+    bufs[0].fill(1, s)
+    call(warm, *bufs)
+    s.sync()
+    d_t, d_o, d_tf = buffers(nhg)
+    d_out = _View(d_t.ptr, d_o.nbytes) if captured.endswith("block") else d_o
+    replay = _captured(capi, s, lambda: call(captured.split()[0], d_t, d_out, d_tf))
+    T = nhg * S
+    for rep in range(3):
+        taftp = gaussian_int8(3801 + rep, nhg * Atot * F * S * 4, 16.0)
+        ftpa = oracle.split_transpose(taftp, nhg, Atot, A, a0, F)
+        d_t.upload(ftpa if captured.startswith("ftpa") else taftp, s)
+        d_o.fill(0x5A, s)
+        d_tf.fill(0x5A, s)
+        s.sync()
+        assert replay() == 0
+        s.sync()
+        ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, S // ts)
+        got = (d_t if captured.endswith("block") else d_o).download(count=ref.size)
+        np.testing.assert_array_equal(got, ref, err_msg=f"replay {rep}")
+        if captured == "both":
+            np.testing.assert_array_equal(d_tf.download(),
+                                          oracle.ib_tf(oracle.ib_power(taftp, F, 16, 1, nhg, Atot), ioff, isc))
