@@ -993,6 +993,24 @@ static bool cb_taftp_direct(const fbf_cb_plan* plan, long long T, int nantennas_
     return cb_taftp_form(plan, T, nantennas_total, kTaftpAlone).rt > 0 && cb_taftp_stages(plan, T, nantennas_total, S);
 }
 
+// The form in which a call on the block stages it (rt 0: split-transposed).  A
+// block that would be split-transposed under capture, without the FTPA buffer
+// that needs, is staged where its geometry allows it: calls of other sizes or
+// of both beams, which size no FTPA buffer, may have been the plan's first.
+static int cb_taftp_takes(const fbf_cb_plan* plan, long long T, int nantennas_total, int S, hipStream_t s,
+                          TaftpForm* form)
+{
+    *form = TaftpForm{0, false};
+    if (!cb_taftp_stages(plan, T, nantennas_total, S)) return FBF_OK;
+    *form = cb_taftp_form(plan, T, nantennas_total, kTaftpAlone);
+    if (form->rt > 0) return FBF_OK;
+    bool fixed = false;
+    const int st = cb_cannot_grow(plan->ftpa_bytes, (size_t)4 * plan->d.nantennas * plan->d.nchans * T, s, &fixed);
+    if (st) return st;
+    if (fixed) *form = cb_taftp_form(plan, T, nantennas_total, kTaftpBatch);
+    return FBF_OK;
+}
+
 // The incoherent beam of the block formed in the split-transpose's pass.
 struct SplitIb {
     fbf_ib_plan* plan;
@@ -1020,9 +1038,11 @@ static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes
     const long long T = (long long)(taftp_bytes / hg_bytes) * nsamples_per_heap;
     FBF_REQUIRE((reinterpret_cast<uintptr_t>(taftp) & 15) == 0, FBF_ERR_ARG,
                 "fbf_cb_beamform_taftp: buffers must be 16-byte aligned");
-    if (T == 0 || cb_taftp_direct(plan, T, nantennas_total, nsamples_per_heap)) {
-        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna,
-                           cb_taftp_form(plan, T, nantennas_total, kTaftpAlone), nullptr};
+    TaftpForm form{0, false};
+    int st = cb_taftp_takes(plan, T, nantennas_total, nsamples_per_heap, static_cast<hipStream_t>(stream), &form);
+    if (st) return st;
+    if (T == 0 || form.rt > 0) {
+        const TaftpView tv{nsamples_per_heap, nantennas_total, start_antenna, form, nullptr};
         return cb_launch(plan, MODE_INT8, taftp, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf,
                          tbtf_bytes, stream, nullptr, 0, T ? &tv : nullptr, tail);
     }
@@ -1033,7 +1053,7 @@ static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes
                 "fbf_cb_beamform_taftp: weights size " + std::to_string(weights_bytes) + " != expected " +
                     std::to_string((size_t)2 * d.nchans * d.nbeams * d.nantennas));
     size_t expect = 0;
-    int st = fbf_cb_output_bytes(plan, fbytes, &expect);
+    st = fbf_cb_output_bytes(plan, fbytes, &expect);
     if (st) return st;
     FBF_REQUIRE(tbtf_bytes == expect && (T / d.tscrunch) % plan->ohs == 0, FBF_ERR_SIZE,
                 "fbf_cb_beamform_taftp: output size " + std::to_string(tbtf_bytes) + " != expected " +
@@ -1119,15 +1139,28 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
                     "fbf_cb_ib_beamform_taftp_next: too many weights work-groups");
         wj.nblocks = (int)(wj.w.gx * wj.w.gy);
     }
-    if (T == 0 || !cb_ib_fused(plan, ibp, T, nsamples_per_heap)) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    bool fused = T > 0 && cb_ib_fused(plan, ibp, T, nsamples_per_heap);
+    const size_t part_bytes = (size_t)d.nchans * T * 4 * sizeof(int);
+    if (fused) {
+        // Under capture without the partials' buffer (the coherent beams alone
+        // were the plan's first call, say) the incoherent beam runs on its own.
+        bool fixed = false;
+        st = cb_cannot_grow(plan->ibp_bytes, part_bytes, s, &fixed);
+        if (st) return st;
+        fused = !fixed;
+    }
+    if (!fused) {
         // The incoherent beam comes out of the split-transpose's pass where
         // there is one and the plan's scrunch allows it (one read of the
         // block and one launch less: a block of 16 antennas, 16 channels,
         // 2048 spectra and 32 beams, which is launches and latency, took
         // 21.4 us in five launches and takes 17.2 us in three); else it runs
         // first.
-        const bool split_ib = T > 0 && !cb_taftp_direct(plan, T, d.nantennas, nsamples_per_heap) &&
-                              ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
+        TaftpForm form{0, false};
+        st = cb_taftp_takes(plan, T, d.nantennas, nsamples_per_heap, s, &form);
+        if (st) return st;
+        const bool split_ib = T > 0 && form.rt == 0 && ibp.nantennas == d.nantennas && ibp.nchans == d.nchans &&
                               ibp.nsamples_per_heap == nsamples_per_heap && split_ib_applies(ibp);
         if (split_ib) {
             size_t tf_expect = 0;
@@ -1156,8 +1189,7 @@ static int cb_ib_run(fbf_cb_plan* plan, fbf_ib_plan* ib_plan, const void* taftp,
     FBF_REQUIRE((reinterpret_cast<uintptr_t>(taftp) & 15) == 0, FBF_ERR_ARG,
                 "fbf_cb_ib_beamform_taftp: buffers must be 16-byte aligned");
     void* part = nullptr;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    st = cb_grow(&plan->ibp, &plan->ibp_bytes, (size_t)d.nchans * T * 4 * sizeof(int), s, &part);
+    st = cb_grow(&plan->ibp, &plan->ibp_bytes, part_bytes, s, &part);
     if (st) return st;
     IbFinishJob ibj{};
     st = ib_finish_job(ib_plan, static_cast<const int*>(part), 1, T, tf, tf_bytes, &ibj);

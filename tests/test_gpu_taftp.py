@@ -521,6 +521,11 @@ def _captured(capi, stream, call):
 
 @pytest.mark.parametrize("warm,captured,Atot,A,a0,F,nhg,nhg_warm,B,ts", [
     ("ftpa", "ftpa over the block", 16, 16, 0, 4, 2, 2, 32, 4),   # first in one launch, then staged
+    ("taftp", "both", 40, 40, 0, 4, 2, 2, 136, 16),               # the incoherent beam on its own
+    ("taftp", "both", 16, 16, 0, 16, 3, 3, 32, 16),
+    ("both", "taftp", 72, 72, 0, 4, 4, 4, 16, 16),                # small blocks that are split-transposed
+    ("taftp", "taftp", 24, 16, 5, 4, 2, 6, 40, 16),               # after a larger block that was not
+    ("taftp", "both", 44, 44, 0, 4, 2, 6, 64, 8),
 ])
 def test_calls_captured_after_other_calls(gpu, oracle, warm, captured, Atot, A, a0, F, nhg, nhg_warm, B, ts):
     """A call that is captured uses the scratch that other calls of its plan
