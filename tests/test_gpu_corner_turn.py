@@ -101,3 +101,41 @@ def test_tuse_transpose_tile_shapes_bit_exact(gpu, C, S, F, B, G, b0, nb):
     capi.tuse_transpose(_dev(capi, x), d_out, C, S, F, B, G, beam0=b0, nbeams_out=nb)
     ref = np.ascontiguousarray(x[:, b0:b0 + nb].transpose(1, 0, 3, 2, 4))
     np.testing.assert_array_equal(d_out.download(), ref.reshape(-1))
+
+
+@pytest.mark.parametrize("C,S,F,B,G", [
+    (7, 900, 40, 2, 1), (3, 64, 64, 8, 4),     # few tiles: shrunk to two units a thread
+    (5, 7, 5, 300, 3),                         # a matrix smaller than a tile
+    (13, 37, 41, 3, 2),                        # steps: a tile's last rows and columns in bytes
+    (36, 50, 17, 4, 3),                        # the same in 4-byte units, nine to an element
+    (1, 4000, 2, 40, 20),                      # rows: output rows of two bytes
+    (20, 530, 33, 2, 40),                      # rows: the last tile holds one row
+    (52, 166, 2, 30, 15),                      # rows: fewer than a work-group has waves
+    (64, 61, 9, 3, 2), (48, 61, 9, 3, 2),      # 16-byte units, shifts and multiplications, partial tiles
+    (512, 9, 5, 3, 2),                         # two elements a tile row
+    (112, 77, 19, 30, 2),                      # 8 MiB and more: past the cache, no power of two
+    (4, 4, 4, 3, 2), (4, 68, 60, 3, 2), (4, 260, 132, 2, 3),   # word tiles: partial rows and columns
+    (4, 1024, 96, 24, 1),                      # word tiles of whole lines past the cache, partial rows
+    (4, 1024, 100, 24, 1),                     # and cached, rows of no whole lines
+])
+def test_tuse_transpose_every_walk_bit_exact(gpu, C, S, F, B, G):
+    """Each way a tile is walked, at its edges, against numpy."""
+    capi = gpu
+    rng = np.random.default_rng(C + S + F + 1)
+    x = rng.integers(-128, 128, (G, B, F, S, C), dtype=np.int8)
+    d_out = capi.DeviceBuffer(G * B * F * S * C)
+    capi.tuse_transpose(_dev(capi, x), d_out, C, S, F, B, G)
+    ref = np.ascontiguousarray(x.transpose(1, 0, 3, 2, 4))
+    np.testing.assert_array_equal(d_out.download(), ref.reshape(-1))
+
+
+@pytest.mark.parametrize("C,n", [(96, 200), (193, 100), (1056, 16), (1024, 140)])
+def test_feng_to_dada_large_blocks_bit_exact(gpu, C, n):
+    """F-engine blocks of 16 MiB and more (a partial tile of 32 channels, odd
+    channels, 33 lines to a row) and one of 140 MiB."""
+    capi = gpu
+    rng = np.random.default_rng(C)
+    x = rng.integers(0, 1 << 32, (n, C, 256), dtype=np.uint32)
+    d_out = capi.DeviceBuffer(x.nbytes)
+    capi.feng_to_dada(_dev(capi, x), d_out, C)
+    np.testing.assert_array_equal(d_out.download(np.uint32), x.transpose(0, 2, 1).reshape(-1))
