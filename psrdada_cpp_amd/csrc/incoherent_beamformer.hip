@@ -12,9 +12,9 @@
 // antenna) out in contiguous runs, and each reads whole 1 KiB (channel, antenna) rows as
 // 16-byte vectors (4 samples x 2 pols a lane) and squares with v_dot4_i32_i8
 // (exact int32).  tscrunch is reduced in-lane and across lanes with shuffles,
-// the waves' sums through LDS, in int64 (exact).  Blocks of 16 MiB or more are
-// read past the cache (once), and work-groups that follow each other in a heap
-// group stay on one XCD.  64 antennas, 64 channels, 32 heaps, fscrunch 2:
+// the waves' sums through LDS, in int64 (exact).  Blocks that the cache is not
+// likely to hold are read past it, and work-groups that follow each other in a
+// heap group stay on one XCD.  64 antennas, 64 channels, 32 heaps, fscrunch 2:
 // 26.0 us with cached loads and a wave to each of four channels, 21.5 us now
 // (6.2 TB/s).
 //
@@ -40,7 +40,7 @@ __device__ __forceinline__ int sq4(int x, int acc)
     return __builtin_amdgcn_sdot4(x, x, acc, false);
 }
 
-// NW waves per work-group: 4, or 16 where the grid is small; PAST: the block
+// NW waves per work-group: 4, 8 or 16 (ib_waves); PAST: the block
 // is read past the cache (ib_run); ONE: a wave per output channel, NW of them
 // to a work-group, instead of the waves sharing one's rows out.
 template <int MODE, int NW, bool PAST, bool ONE>
@@ -144,18 +144,43 @@ __global__ __launch_bounds__(64 * NW) void ib_k(IbArgs p, WeightsJob wj)
     }
 }
 
+// Waves that share the rows of a work-group (`work` of them), on blocks in turn
+// (us; antennas / channels / heaps / fscrunch):
+//                      work  rows     4     8    16
+//   120/16/4/1          64   120    6.5   4.8   4.2   16 where few work-groups
+//   64/40/4/8           20   512   14.2   8.5   7.8   have many rows;
+//   40/40/30/4         300   160    9.2   9.7   9.8   4 where few compute units
+//   64/40/30/4         300   256   13.1  14.1  13.9   would have two work-groups
+//   68/56/39/4         546   272   26.1  27.8  27.4   and the others one, longer
+//                                                     so past the cache;
+//   24/64/60/1        3840    24   16.0  17.5  26.1   4 where rows are few;
+//   40/16/60/1         960    40    8.0   7.7   8.9   else 8
+//   96/64/12/1         768    96   12.8  12.4  13.1
+inline int ib_waves(long long work, long long rows, bool past)
+{
+    if (rows >= 112 && work <= 96) return 16;
+    if (rows < 16 || (rows < 32 && work >= 1024)) return 4;
+    return work > 256 && work < (past ? 1024 : 384) ? 4 : 8;
+}
+
+template <int MODE, int NW, bool ONE>
+void launch_ib_nw(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool past, hipStream_t s)
+{
+    past ? ib_k<MODE, NW, true, ONE><<<grid, 64 * NW, 0, s>>>(a, wj)
+         : ib_k<MODE, NW, false, ONE><<<grid, 64 * NW, 0, s>>>(a, wj);
+}
+
 template <int MODE>
-void launch_ib(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool one, bool wide, bool past, hipStream_t s)
+void launch_ib(const IbArgs& a, const WeightsJob& wj, dim3 grid, bool one, int waves, bool past, hipStream_t s)
 {
     if (one)
-        past ? ib_k<MODE, 4, true, true><<<grid, 256, 0, s>>>(a, wj)
-             : ib_k<MODE, 4, false, true><<<grid, 256, 0, s>>>(a, wj);
-    else if (wide)
-        past ? ib_k<MODE, 16, true, false><<<grid, 1024, 0, s>>>(a, wj)
-             : ib_k<MODE, 16, false, false><<<grid, 1024, 0, s>>>(a, wj);
+        launch_ib_nw<MODE, 4, true>(a, wj, grid, past, s);
+    else if (waves == 16)
+        launch_ib_nw<MODE, 16, false>(a, wj, grid, past, s);
+    else if (waves == 8)
+        launch_ib_nw<MODE, 8, false>(a, wj, grid, past, s);
     else
-        past ? ib_k<MODE, 4, true, false><<<grid, 256, 0, s>>>(a, wj)
-             : ib_k<MODE, 4, false, false><<<grid, 256, 0, s>>>(a, wj);
+        launch_ib_nw<MODE, 4, false>(a, wj, grid, past, s);
 }
 
 }  // namespace
@@ -283,15 +308,17 @@ static int ib_run(fbf_ib_plan* plan, int mode, const void* taftp, size_t taftp_b
     const long long nblocks = work + wj.nblocks;
     FBF_REQUIRE(nblocks < (1ll << 31), FBF_ERR_UNSUPPORTED, "fbf_ib: grid too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // 16 waves share the rows of a small block's few work-groups, at least two
-    // each (the weights job is made of work-groups of 4).
-    const bool wide = !one && work < 1024 && (long long)d.nantennas * d.fscrunch >= 32 && wj.nblocks == 0;
-    const bool past = taftp_bytes >= ((size_t)16 << 20);   // (smaller blocks may be in the cache)
+    // Past the cache (256 MiB) from 96 MiB: with three blocks in turn smaller
+    // ones are read from it (us, cached and past; 64 antennas, 40 channels, 30
+    // heaps, fscrunch 4, 75 MiB 13.1 and 15.1; 96/40/30, 112 MiB 22.0 and 19.3).
+    const bool past = taftp_bytes >= ((size_t)96 << 20);
+    // (The weights job is made of work-groups of 4 waves.)
+    const int waves = wj.nblocks ? 4 : ib_waves(work, (long long)d.nantennas * d.fscrunch, past);
     const dim3 grid((unsigned)nblocks);
     if (mode == IB_INT8)
-        launch_ib<IB_INT8>(a, wj, grid, one, wide, past, s);
+        launch_ib<IB_INT8>(a, wj, grid, one, waves, past, s);
     else
-        launch_ib<IB_POWER>(a, wj, grid, one, wide, past, s);
+        launch_ib<IB_POWER>(a, wj, grid, one, waves, past, s);
     FBF_LAUNCH_CHECK("ib_k");
     return FBF_OK;
 }

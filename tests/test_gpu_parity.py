@@ -759,3 +759,33 @@ def test_split_transpose_ib_tile_shapes_bit_exact(gpu, oracle, A, F, nhg, ts):
     np.testing.assert_array_equal(d_out.download(), oracle.split_transpose(taftp, nhg, A, A, 0, F))
     ib_ref = oracle.ib_tf(oracle.ib_power(taftp, F, ts, 1, nhg, A), off, sc)
     np.testing.assert_array_equal(d_tf.download(), ib_ref.reshape(-1))
+
+
+@pytest.mark.parametrize("A,F,nhg,ts,fs", [
+    (15, 8, 2, 16, 1),         # four waves: rows below 16
+    (16, 8, 2, 1, 1),          # eight waves of two rows
+    (28, 64, 16, 64, 1),       # four waves: 1024 work-groups of few rows
+    (13, 12, 3, 4, 4),         # eight waves of 7 rows, the last with 3
+    (113, 4, 5, 256, 1),       # sixteen waves of 8 rows, the last without any
+    (20, 60, 18, 16, 4),       # 270 work-groups: four waves
+    (20, 96, 16, 16, 4),       # 384: eight
+    (64, 64, 24, 16, 1),       # 96 MiB: past the cache, eight waves
+    (96, 40, 26, 2, 4),        # past the cache, four waves of 96 rows
+    (8, 128, 100, 16, 1),      # past the cache, a wave per output channel
+])
+def test_ib_waves_bit_exact(gpu, oracle, A, F, nhg, ts, fs):
+    """The incoherent beam by waves to a work-group, cached and past the cache,
+    against the oracle: int8 and power output."""
+    capi = gpu
+    taftp = np.random.default_rng(7200 + A).integers(-128, 128, nhg * A * F * 256 * 4, dtype=np.int8)
+    Fo = F // fs
+    p_ref = oracle.ib_power(taftp, F, ts, fs, nhg, A)
+    off = np.full(Fo, float(np.median(p_ref)), np.float32)
+    sc = np.full(Fo, max(1.0, float(np.std(p_ref)) / 40.0), np.float32)
+    plan = capi.IbPlan(A, F, ts, fs, off, sc)
+    d_t = _dev(capi, taftp)
+    d_o, d_p = capi.DeviceBuffer(p_ref.size), capi.DeviceBuffer(p_ref.size * 8)
+    plan.beamform(d_t, d_o)
+    np.testing.assert_array_equal(d_o.download(), oracle.ib_tf(p_ref, off, sc).reshape(-1))
+    plan.power(d_t, d_p)
+    np.testing.assert_array_equal(d_p.download(np.float64), p_ref.reshape(-1))
