@@ -375,13 +375,13 @@ static int batch_enqueue_serial(fbf_batch* b, const void* taftp, size_t taftp_by
         size_t ob = 0;
         st = fbf_ib_output_bytes(b->ib, taftp_bytes, &ob);
         if (st) return st;
-        st = b->ib_fused ? fbf_split_transpose_ib(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->F, b->S, b->ib,
-                                                  outputs[n], ob, stream)
+        st = b->ib_fused ? split_transpose_ib_read_next(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->F, b->S, b->ib,
+                                                        outputs[n], ob, stream)
                          : fbf_ib_beamform(b->ib, taftp, taftp_bytes, outputs[n], ob, stream);
         if (st) return st;
     }
     if (!b->ib || !b->ib_fused) {
-        st = fbf_split_transpose(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->A, b->A, 0, b->F, b->S, stream);
+        st = split_transpose_read_next(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->A, b->A, 0, b->F, b->S, stream);
         if (st) return st;
     }
     for (int i = 0; i < n; ++i) {
@@ -413,8 +413,8 @@ static int batch_enqueue(fbf_batch* b, const void* taftp, size_t taftp_bytes, co
         st = fbf_ib_output_bytes(b->ib, taftp_bytes, &ob);
         if (st) return st;
         if (b->ib_fused) {
-            st = fbf_split_transpose_ib(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->F, b->S, b->ib, outputs[n],
-                                        ob, stream);
+            st = split_transpose_ib_read_next(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->F, b->S, b->ib, outputs[n],
+                                              ob, stream);
             if (st) return st;
         } else {
             ib_branch = true;
@@ -427,7 +427,7 @@ static int batch_enqueue(fbf_batch* b, const void* taftp, size_t taftp_bytes, co
         }
     }
     if (!b->ib || !b->ib_fused) {
-        st = fbf_split_transpose(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->A, b->A, 0, b->F, b->S, stream);
+        st = split_transpose_read_next(taftp, taftp_bytes, b->ftpa, b->ftpa_bytes, b->A, b->A, 0, b->F, b->S, stream);
         if (st) return st;
     }
     FBF_HIP_TRY(hipEventRecord(b->fork_cb, stream));

@@ -1061,10 +1061,10 @@ static int cb_taftp_run(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes
     void* ftpa = nullptr;
     st = cb_grow(&plan->ftpa, &plan->ftpa_bytes, fbytes, static_cast<hipStream_t>(stream), &ftpa);
     if (st) return st;
-    st = split_ib ? fbf_split_transpose_ib(taftp, taftp_bytes, ftpa, fbytes, d.nchans, nsamples_per_heap,
-                                           split_ib->plan, split_ib->tf, split_ib->tf_bytes, stream)
-                  : fbf_split_transpose(taftp, taftp_bytes, ftpa, fbytes, nantennas_total, d.nantennas,
-                                        start_antenna, d.nchans, nsamples_per_heap, stream);
+    st = split_ib ? split_transpose_ib_read_next(taftp, taftp_bytes, ftpa, fbytes, d.nchans, nsamples_per_heap,
+                                                 split_ib->plan, split_ib->tf, split_ib->tf_bytes, stream)
+                  : split_transpose_read_next(taftp, taftp_bytes, ftpa, fbytes, nantennas_total, d.nantennas,
+                                              start_antenna, d.nchans, nsamples_per_heap, stream);
     if (st) return st;
     return cb_launch(plan, MODE_INT8, ftpa, T, 2 * d.nantennas, 0, fba_weights, weights_bytes, tbtf, tbtf_bytes,
                      stream, nullptr, 0, nullptr, tail);

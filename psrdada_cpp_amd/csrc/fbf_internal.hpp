@@ -56,6 +56,15 @@ inline bool split_ib_applies(const IbFuseParams& p)
 {
     return p.fscrunch == 1 && p.tscrunch > 0 && 32 % p.tscrunch == 0 && p.nsamples_per_heap % 32 == 0;
 }
+// fbf_split_transpose and fbf_split_transpose_ib of a copy that the coherent
+// beamformer reads in the next launch (st_near).
+int split_transpose_read_next(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
+                              int total_nantennas, int used_nantennas, int start_antenna, int nchans,
+                              int nsamples_per_heap, fbf_stream_t stream);
+int split_transpose_ib_read_next(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes, int nchans,
+                                 int nsamples_per_heap, fbf_ib_plan* ib_plan, void* tf, size_t tf_bytes,
+                                 fbf_stream_t stream);
+
 // The incoherent beam from the partials that the coherent beamformer left
 // ([F][T / 16][2 halves][32 columns] int32; sample j of a tile is the sum of
 // columns 2j, 2j + 1 of both halves), int8 TF of T samples with the IB

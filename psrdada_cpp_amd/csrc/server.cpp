@@ -185,10 +185,10 @@ int enqueue_block(fbf_server* s, Request* r)
     off += align_up(f.cb_bytes);
     void* ib_dev = mem + off;
     const bool fused = f.ib && f.d.ib_fscrunch == 1 && 32 % f.d.ib_tscrunch == 0;
-    int e = fused ? fbf_split_transpose_ib(input, f.block_bytes, ftpa, f.block_bytes, f.d.nchans,
-                                           f.d.nsamples_per_heap, f.ib, ib_dev, f.ib_bytes, st)
-                  : fbf_split_transpose(input, f.block_bytes, ftpa, f.block_bytes, f.d.nantennas, f.d.nantennas, 0,
-                                        f.d.nchans, f.d.nsamples_per_heap, st);
+    int e = fused ? split_transpose_ib_read_next(input, f.block_bytes, ftpa, f.block_bytes, f.d.nchans,
+                                                 f.d.nsamples_per_heap, f.ib, ib_dev, f.ib_bytes, st)
+                  : split_transpose_read_next(input, f.block_bytes, ftpa, f.block_bytes, f.d.nantennas,
+                                              f.d.nantennas, 0, f.d.nchans, f.d.nsamples_per_heap, st);
     if (e) return e;
     e = fbf_cb_beamform_ws(f.cb, ftpa, f.block_bytes, f.weights[r->wbuf], f.weights_bytes, cb_dev, f.cb_bytes,
                            cb_stage, f.cb_bytes, st);

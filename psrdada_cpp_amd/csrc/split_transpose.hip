@@ -254,7 +254,16 @@ int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nan
 // 56/64/32 41 against 45 (42, 46), 128/64/32 116 against 128 (116, 125), 60/64/32
 // 46 against 49, 40/64/48 (252 MB moved) 43 against 48; but 40/64/32 (168 MB) 31
 // against 25 (37, 28), and with the incoherent beam 40/64/48 53 against 49.
-bool st_near(bool ib, int used_nantennas, size_t moved)
+//
+// A copy that the next launch reads (`read_next`: the library's own calls) takes
+// them too from 24 antennas, and smaller copies sooner: the coherent kernel
+// finds its channels in the L2 of its XCD.  Both launches, us, cached 64 x 64
+// tiles against the others (antennas / channels / heaps, 64 beams): 32/64/8 17.1
+// against 24.6, 24/64/16 25.8 and 30.0, 16/64/8 15.0 and 16.2, 48/16/8 10.4 and
+// 12.2; but 8/64/32 33.0 and 28.0, 12/64/8 with the incoherent beam 18.4 and 17.2.
+// With the incoherent beam small copies are launches and latency either way:
+// 52/16/1 5.0 against 5.9, but 16/64/8 10.3 and 7.4.
+bool st_near(bool ib, int used_nantennas, size_t moved, bool read_next)
 {
     // (Columns of whole 64-byte lines, 32 antennas, gain from the cache sooner:
     // 32/64/32, 128 MiB, 21.5 against 22.9; 32/64/16 11.6 against 11.4.)
@@ -262,14 +271,18 @@ bool st_near(bool ib, int used_nantennas, size_t moved)
     if (used_nantennas % 4 != 0) return false;
     if (used_nantennas > 64) return true;
     if (used_nantennas >= 56 && used_nantennas % 8 == 0) return true;
+    const size_t copy_mib = (moved / 2) >> 20;
+    if (read_next && (used_nantennas >= 24 || copy_mib < 2 || (used_nantennas >= 16 && copy_mib < 16))) return true;
+    if (ib && used_nantennas >= 20 && copy_mib < 4) return true;
     return moved >= near_bytes && (!ib || used_nantennas >= 56);
 }
 
 template <bool IB>
 int st_launch_sp(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna,
-                 int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream)
+                 int nchans, int nsamples_per_heap, int nhg, IbTile ib, WeightsJob wj, fbf_stream_t stream,
+                 bool read_next)
 {
-    if (st_near(IB, used_nantennas, (size_t)8 * used_nantennas * nchans * nsamples_per_heap * nhg))
+    if (st_near(IB, used_nantennas, (size_t)8 * used_nantennas * nchans * nsamples_per_heap * nhg, read_next))
         return st_launch_t<64, IB, true>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
                                          nsamples_per_heap, nhg, ib, wj, stream);
     // Tiles of 128 columns where 64 antennas hold a subset and they divide a
@@ -282,21 +295,19 @@ int st_launch_sp(const void* taftp, void* ftpa, int total_nantennas, int used_na
 }
 
 int st_launch(const void* taftp, void* ftpa, int total_nantennas, int used_nantennas, int start_antenna, int nchans,
-              int nsamples_per_heap, int nhg, IbTile ib, fbf_stream_t stream, WeightsJob wj = WeightsJob{})
+              int nsamples_per_heap, int nhg, IbTile ib, fbf_stream_t stream, bool read_next,
+              WeightsJob wj = WeightsJob{})
 {
     if (ib.out)
         return st_launch_sp<true>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
-                                 nsamples_per_heap, nhg, ib, wj, stream);
+                                 nsamples_per_heap, nhg, ib, wj, stream, read_next);
     return st_launch_sp<false>(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans,
-                              nsamples_per_heap, nhg, ib, wj, stream);
+                              nsamples_per_heap, nhg, ib, wj, stream, read_next);
 }
 
-}  // namespace
-
-extern "C" int fbf_split_transpose(const void* taftp, size_t taftp_bytes, void* ftpa,
-                                   size_t ftpa_bytes, int total_nantennas, int used_nantennas,
-                                   int start_antenna, int nchans, int nsamples_per_heap,
-                                   fbf_stream_t stream)
+int st_run(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes, int total_nantennas,
+           int used_nantennas, int start_antenna, int nchans, int nsamples_per_heap, fbf_stream_t stream,
+           bool read_next)
 {
     FBF_REQUIRE(taftp && ftpa, FBF_ERR_ARG, "fbf_split_transpose: null buffer");
     FBF_REQUIRE(total_nantennas > 0 && used_nantennas > 0 && start_antenna >= 0 &&
@@ -321,12 +332,12 @@ extern "C" int fbf_split_transpose(const void* taftp, size_t taftp_bytes, void* 
     FBF_REQUIRE(nhg < (1u << 20), FBF_ERR_UNSUPPORTED, "fbf_split_transpose: too many heap groups");
 
     return st_launch(taftp, ftpa, total_nantennas, used_nantennas, start_antenna, nchans, nsamples_per_heap,
-                     (int)nhg, IbTile{nullptr, nullptr, nullptr, 1, 0}, stream);
+                     (int)nhg, IbTile{nullptr, nullptr, nullptr, 1, 0}, stream, read_next);
 }
 
 // Checks a fused split-transpose + incoherent-beam call and returns the
 // launch arguments.
-static int st_ib_params(const void* taftp, size_t taftp_bytes, const void* ftpa, size_t ftpa_bytes, int nchans,
+int st_ib_params(const void* taftp, size_t taftp_bytes, const void* ftpa, size_t ftpa_bytes, int nchans,
                         int nsamples_per_heap, const fbf_ib_plan* ib_plan, void* tf, size_t tf_bytes, int* nhg_out,
                         int* nantennas, IbTile* tile)
 {
@@ -358,9 +369,9 @@ static int st_ib_params(const void* taftp, size_t taftp_bytes, const void* ftpa,
     return FBF_OK;
 }
 
-extern "C" int fbf_split_transpose_ib(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
-                                      int nchans, int nsamples_per_heap, fbf_ib_plan* ib_plan, void* tf,
-                                      size_t tf_bytes, fbf_stream_t stream)
+int st_ib_run(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes, int nchans,
+              int nsamples_per_heap, fbf_ib_plan* ib_plan, void* tf, size_t tf_bytes, fbf_stream_t stream,
+              bool read_next)
 {
     int nhg = 0, A = 0;
     IbTile ib{};
@@ -368,7 +379,42 @@ extern "C" int fbf_split_transpose_ib(const void* taftp, size_t taftp_bytes, voi
                                 tf_bytes, &nhg, &A, &ib);
     if (st) return st;
     if (nhg == 0) return FBF_OK;
-    return st_launch(taftp, ftpa, A, A, 0, nchans, nsamples_per_heap, nhg, ib, stream);
+    return st_launch(taftp, ftpa, A, A, 0, nchans, nsamples_per_heap, nhg, ib, stream, read_next);
+}
+
+}  // namespace
+
+extern "C" int fbf_split_transpose(const void* taftp, size_t taftp_bytes, void* ftpa,
+                                   size_t ftpa_bytes, int total_nantennas, int used_nantennas,
+                                   int start_antenna, int nchans, int nsamples_per_heap,
+                                   fbf_stream_t stream)
+{
+    return st_run(taftp, taftp_bytes, ftpa, ftpa_bytes, total_nantennas, used_nantennas, start_antenna, nchans,
+                  nsamples_per_heap, stream, false);
+}
+
+int fbf::split_transpose_read_next(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
+                                   int total_nantennas, int used_nantennas, int start_antenna, int nchans,
+                                   int nsamples_per_heap, fbf_stream_t stream)
+{
+    return st_run(taftp, taftp_bytes, ftpa, ftpa_bytes, total_nantennas, used_nantennas, start_antenna, nchans,
+                  nsamples_per_heap, stream, true);
+}
+
+extern "C" int fbf_split_transpose_ib(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
+                                      int nchans, int nsamples_per_heap, fbf_ib_plan* ib_plan, void* tf,
+                                      size_t tf_bytes, fbf_stream_t stream)
+{
+    return st_ib_run(taftp, taftp_bytes, ftpa, ftpa_bytes, nchans, nsamples_per_heap, ib_plan, tf, tf_bytes, stream,
+                     false);
+}
+
+int fbf::split_transpose_ib_read_next(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
+                                      int nchans, int nsamples_per_heap, fbf_ib_plan* ib_plan, void* tf,
+                                      size_t tf_bytes, fbf_stream_t stream)
+{
+    return st_ib_run(taftp, taftp_bytes, ftpa, ftpa_bytes, nchans, nsamples_per_heap, ib_plan, tf, tf_bytes, stream,
+                     true);
 }
 
 extern "C" int fbf_split_transpose_ib_weights(const void* taftp, size_t taftp_bytes, void* ftpa, size_t ftpa_bytes,
@@ -392,5 +438,5 @@ extern "C" int fbf_split_transpose_ib_weights(const void* taftp, size_t taftp_by
     wj.nblocks = (int)(wj.w.gx * wj.w.gy);
     if (nhg == 0) return fbf_weights_generate(weights_plan, delays, delays_bytes, epoch, weights, weights_bytes,
                                               nullptr, stream);
-    return st_launch(taftp, ftpa, A, A, 0, nchans, nsamples_per_heap, nhg, ib, stream, wj);
+    return st_launch(taftp, ftpa, A, A, 0, nchans, nsamples_per_heap, nhg, ib, stream, false, wj);
 }

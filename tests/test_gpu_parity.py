@@ -789,3 +789,28 @@ def test_ib_waves_bit_exact(gpu, oracle, A, F, nhg, ts, fs):
     np.testing.assert_array_equal(d_o.download(), oracle.ib_tf(p_ref, off, sc).reshape(-1))
     plan.power(d_t, d_p)
     np.testing.assert_array_equal(d_p.download(np.float64), p_ref.reshape(-1))
+
+
+@pytest.mark.parametrize("Atot,A,a0,F,nhg", [
+    (20, 16, 3, 64, 15), (20, 16, 3, 64, 16),   # 15 and 16 MiB copies: either side of the line
+    (28, 24, 1, 16, 3),                         # from 24 antennas, whatever the size
+    (12, 8, 4, 64, 3), (12, 8, 4, 64, 4),       # 1.5 and 2 MiB
+])
+def test_split_transpose_of_taftp_calls(gpu, oracle, Atot, A, a0, F, nhg):
+    """The tiles of the library's own split-transposes, which the coherent
+    kernel reads next: a TAFTP call of a plan that stages no TAFTP (variant 10)
+    against the oracle."""
+    capi = gpu
+    B, ts, T = 8, 64, nhg * 256
+    taftp = gaussian_int8(7300 + A + nhg, nhg * Atot * F * 256 * 4, 16.0)
+    w = unit_weights(7301, F * B * A)
+    off, sc = _levels(oracle, A, ts, 1, F)
+    plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=4)
+    plan.set_variant(10)
+    assert not plan.taftp_direct(Atot, T, 256)
+    d_o = capi.DeviceBuffer(F * (T // ts) * B)
+    d_o.fill(0x5A)
+    plan.beamform_taftp(_dev(capi, taftp), _dev(capi, w), d_o, nantennas_total=Atot, start_antenna=a0)
+    ftpa = oracle.split_transpose(taftp, nhg, Atot, A, a0, F)
+    np.testing.assert_array_equal(d_o.download(),
+                                  oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, 4))
