@@ -197,8 +197,8 @@ int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_block, size_t b
  * that the plan owns (grown on demand, as the staging buffer) first.  As
  * with fbf_cb_beamform, calls with one plan on different streams must not
  * overlap (they share the plan's buffers).  The automatic variant stages the
- * block itself with 128 beams per wave up to 64 antennas (32 or 64 for at
- * most so many beams) and with 64 above; of blocks of at most 4096 channels x
+ * block itself with 128 beams per wave up to 64 antennas (32 or 64 for few
+ * beams or a small block) and with 64 above; of blocks of at most 4096 channels x
  * samples, a subset of at most 48 antennas with at most 96 beams, and more
  * than 64 antennas with at most 32, are split-transposed. */
 int fbf_cb_beamform_taftp(fbf_cb_plan* plan, const void* taftp, size_t taftp_bytes,

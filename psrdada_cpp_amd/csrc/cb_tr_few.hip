@@ -1,6 +1,6 @@
-// Instances of the transposed kernel (cb_tr_k) for at most 64 beams of up to 64
-// antennas: one wave of 32 or 64 beams per time slot, four
-// time slots to a work-group.
+// Instances of the transposed kernel (cb_tr_k) for few beams or small blocks of
+// up to 64 antennas: one wave of 32 or 64 beams per time slot, four time slots to
+// a work-group (cb_few_rows).
 #include "cb_tr.hpp"
 
 namespace fbf {

@@ -501,7 +501,7 @@ struct CbVariant {
     bool lds;        // voltage tile staged through LDS and shared by the work-group
     bool tr;         // transposed tiles (cb_tr_k): voltages as the A operand
     bool ws;         // transposed tiles with wave-private staging (cb_ws_k)
-    bool few = false;   // transposed: one wave per time slot, for at most 64 beams (cb_tr_few.hip)
+    bool few = false;   // transposed: one beam group, four time slots to a work-group (cb_tr_few.hip)
 };
 static const CbVariant kCbVariants[] = {
     {0, 0, false, false, false},   // auto
@@ -534,25 +534,56 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
            cb_ws_supported(d.nantennas, d.tscrunch, d.fscrunch);
 }
 
+// Whether the few-beam form (cb_tr_few.hip: waves of 16 rt beams, four time slots
+// to a work-group) runs all its waves in `rounds` rounds of one pass each.
+//
+// A pass is two windows or more in a row, whatever else of the chip is idle, and
+// a wave of 128 beams takes twice as long over it as one of 64.  So small blocks
+// take waves of 64 beams, and where the windows are long and there is room even
+// for those waves of 32 (us; 128, 64 and 32 beams a wave, and the wave-private
+// kernel from FTPA; antennas / beams / channels / samples / tscrunch, TAFTP
+// marked t): 48/96/4/1024/256 t 33.8, 24.3, 20.2; 16/96/4/1024/64 12.6, 7.1,
+// 6.1, 10.7; 48/96/16/2048/128 20.5, 13.4, 11.0, 15.0; 40/256/16/2048/16 14.4,
+// 10.4, -, 14.0; but with 32 beams 56/208/8/256/8 7.4 against 6.1, and in four
+// rounds of 64 40/512/64/4096/128 64.0 against 52.2 with 128.
+static bool cb_few_fit(const fbf_cb_desc& d, long long T, int rt, int rounds)
+{
+    const int W = 2 * d.tscrunch;
+    const int spt = W >= 32 ? 1 : 32 / W, tps = W >= 32 ? W / 32 : 1;
+    const long long ntp = (long long)(cb_tr_nslot(rt, W) / spt) * tps;
+    const long long passes = (2 * T / 32 + ntp - 1) / ntp;
+    const long long groups = (long long)d.nchans * ((d.nbeams + 16 * rt - 1) / (16 * rt)) * ((passes + 3) / 4);
+    return groups <= (long long)rounds * tr_wgs(rt, 1) * device_cu_count();
+}
+
+// Beam tiles of the few-beam form for a block, 0: it takes another form.
+static int cb_few_rows(const fbf_cb_desc& d, long long T)
+{
+    if (d.nbeams <= 32 || (d.tscrunch >= 32 && cb_few_fit(d, T, 2, 1))) return 2;
+    return d.nbeams <= 64 || cb_few_fit(d, T, 4, 2) ? 4 : 0;
+}
+
 // Automatic choice from FTPA: the transposed kernel, up to 64 antennas with
-// 128 beams per wave or with 32 or 64 for so few beams, above with 64 (32 for
-// at most 32: a 64-beam wave would be half empty); the LDS-staged kernel for
-// the rest (tscrunch below 4 or no power of two, fscrunch above 4, also int32
-// sums and power output).  Measured against the wave-private kernel and the
-// earlier picks (us; antennas / beams / channels / samples / tscrunch):
-// 16/256/64/8192/16 40.6 against 44.7, 48/512/64/8192/16 111 against 128,
-// 40/768/64/8192/4 250 against 272, 8/64/64/8192/16 16.4 against 17.4,
-// 16/32/16/2048/16 8.3 against 9.4 (5.4 in one launch, cb_tbtf_direct).  fscrunch 2 and 4: 128 beams per wave
-// above 96 beams, or where the forms with several time slots per work-group
-// end (two K steps of four channels); 44/1024/64/8192/16 at fscrunch 4 took
-// 205 against 348 of the LDS-staged kernel, 44/64 32 against 50, but 24/64 26.7
-// against 24.5 with 32 beams per wave.
+// 128 beams per wave or with 32 or 64 for few beams and small blocks
+// (cb_few_rows), above with 64 (32 for at most 32: a 64-beam wave would be half
+// empty); the LDS-staged kernel for the rest (tscrunch below 4 or no power of
+// two, fscrunch above 4, also int32 sums and power output).  Measured against the
+// wave-private kernel and the earlier picks (us; antennas / beams / channels /
+// samples / tscrunch): 16/256/64/8192/16 40.6 against 44.7, 48/512/64/8192/16 111
+// against 128, 40/768/64/8192/4 250 against 272, 8/64/64/8192/16 16.4 against
+// 17.4, 16/32/16/2048/16 8.3 against 9.4 (5.4 in one launch, cb_tbtf_direct); but
+// 8/768/64/8192/128, whose units fill the rounds of the grid to 87 %, 92 against
+// 85.  fscrunch 2 and 4: 128 beams per wave above 96 beams, or where the forms
+// with several time slots per work-group end (two K steps of four channels);
+// 44/1024/64/8192/16 at fscrunch 4 took 205 against 348 of the LDS-staged kernel,
+// 44/64 32 against 50, but 24/64 26.7 against 24.5 with 32 beams per wave.
 static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, long long T)
 {
     if (variant <= 0) {
         const int ksteps = (2 * d.nantennas + 31) / 32;
         const bool tr8 = cb_tr_applies(d, 8, mode, T);
-        if (tr8 && d.fscrunch == 1 && d.nbeams <= 64) return {32, d.nbeams <= 32 ? 2 : 4, true, true, false, true};
+        const int few = tr8 && d.fscrunch == 1 ? cb_few_rows(d, T) : 0;
+        if (few) return {32, few, true, true, false, true};
         if (tr8 && (d.fscrunch == 1 || d.nbeams > 96 || d.fscrunch * ksteps > 8)) return kCbVariants[kCbVariantTr8];
         if ((ksteps <= 4 || d.nbeams > 32) && cb_tr_applies(d, 4, mode, T)) return kCbVariants[kCbVariantTr4];
         if (cb_tr_applies(d, 2, mode, T)) return kCbVariants[kCbVariantTr2];
@@ -934,8 +965,8 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 
 // The kernel that stages a TAFTP block itself for the plan's coherent beams
 // (rt 0: none, the block is split-transposed): the plan's variant, or when
-// that is automatic 128 beams per wave up to 64 antennas and 64 beams per
-// wave above, with 32 or 64 per wave where at most so many are asked for.
+// that is automatic 128 beams per wave up to 64 antennas (32 or 64 for few beams
+// and small blocks, cb_few_rows) and 64 beams per wave above.
 //
 // Staging the block itself was the faster at every size measured.  Blocks of
 // both beams, direct against split-transposed (us; antennas / beams / channels

@@ -577,3 +577,36 @@ def test_calls_captured_after_other_calls(gpu, oracle, warm, captured, Atot, A, 
         if captured == "both":
             np.testing.assert_array_equal(d_tf.download(),
                                           oracle.ib_tf(oracle.ib_power(taftp, F, 16, 1, nhg, Atot), ioff, isc))
+
+
+@pytest.mark.parametrize("A,F,nhg,B,ts,ib_ts,m128", [
+    (48, 4, 4, 96, 256, 16, False),    # long windows, waves of 32 beams in three groups
+    (60, 4, 3, 136, 64, 256, False),   # five groups of 32, the last with 8
+    (16, 4, 2, 72, 32, 1, True),       # a weight of -128
+    (20, 8, 2, 136, 16, 16, False),    # waves of 64 beams in three groups
+    (40, 4, 1, 96, 4, 4, True),
+    (12, 64, 4, 192, 16, 16, False),   # the most that run in two rounds
+    (12, 64, 4, 200, 16, 16, False),   # just above: 128 beams
+    (12, 64, 8, 192, 32, 16, False),   # 32 beams would not fit in one round: 64
+])
+def test_small_blocks_of_narrow_waves(gpu, oracle, A, F, nhg, B, ts, ib_ts, m128):
+    """Small blocks of more than 64 beams on waves of 32 and 64: both beams from
+    TAFTP, a subset of a wider block and FTPA, against the oracle."""
+    capi = gpu
+    w = unit_weights(3901 + A, F * B * A).reshape(F, B, A, 2).copy()
+    if m128:
+        w[1, B - 1, 5, 1] = -128
+    w = w.reshape(-1)
+    _check_cb_ib(capi, oracle, A, F, nhg, B, ts, ib_ts, 1, 256, 0, True, 3900 + A, weights=w)
+    T = nhg * 256
+    off, sc = _levels(oracle, A, ts, 1, F)
+    plan = capi.CbPlan(A, B, F, ts, 1, off, sc, nsamples_per_heap_out=T // ts)
+    taftp = gaussian_int8(3902 + A, nhg * (A + 8) * F * 256 * 4, 16.0)
+    ftpa = oracle.split_transpose(taftp, nhg, A + 8, A, 3, F)
+    ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, T // ts)
+    d_w, d_o = _dev(capi, w), capi.DeviceBuffer(ref.size)
+    for call in (lambda: plan.beamform_taftp(_dev(capi, taftp), d_w, d_o, nantennas_total=A + 8, start_antenna=3),
+                 lambda: plan.beamform(_dev(capi, ftpa), d_w, d_o)):
+        d_o.fill(0x5A)
+        call()
+        np.testing.assert_array_equal(d_o.download(), ref)
