@@ -534,6 +534,17 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
            cb_ws_supported(d.nantennas, d.tscrunch, d.fscrunch);
 }
 
+// Work-groups of the transposed kernel with waves of 16 rt beams, `beams` beams
+// and `slots` time slots to a work-group and one pass on every slot.
+static long long cb_groups(const fbf_cb_desc& d, long long T, int rt, int beams, int slots)
+{
+    const int W = 2 * d.tscrunch;
+    const int spt = W >= 32 ? 1 : 32 / W, tps = W >= 32 ? W / 32 : 1;
+    const long long ntp = (long long)(cb_tr_nslot(rt, W) / spt) * tps;
+    const long long passes = (2 * T / 32 + ntp - 1) / ntp;
+    return (long long)(d.nchans / d.fscrunch) * ((d.nbeams + beams - 1) / beams) * ((passes + slots - 1) / slots);
+}
+
 // Whether the few-beam form (cb_tr_few.hip: waves of 16 rt beams, four time slots
 // to a work-group) runs all its waves in `rounds` rounds of one pass each.
 //
@@ -548,12 +559,7 @@ static bool cb_ws_applies(const fbf_cb_desc& d, int mode, long long T)
 // rounds of 64 40/512/64/4096/128 64.0 against 52.2 with 128.
 static bool cb_few_fit(const fbf_cb_desc& d, long long T, int rt, int rounds)
 {
-    const int W = 2 * d.tscrunch;
-    const int spt = W >= 32 ? 1 : 32 / W, tps = W >= 32 ? W / 32 : 1;
-    const long long ntp = (long long)(cb_tr_nslot(rt, W) / spt) * tps;
-    const long long passes = (2 * T / 32 + ntp - 1) / ntp;
-    const long long groups = (long long)d.nchans * ((d.nbeams + 16 * rt - 1) / (16 * rt)) * ((passes + 3) / 4);
-    return groups <= (long long)rounds * tr_wgs(rt, 1) * device_cu_count();
+    return cb_groups(d, T, rt, 16 * rt, 4) <= (long long)rounds * tr_wgs(rt, 1) * device_cu_count();
 }
 
 // Beam tiles of the few-beam form for a block, 0: it takes another form.
@@ -576,7 +582,8 @@ static int cb_few_rows(const fbf_cb_desc& d, long long T)
 // 85.  fscrunch 2 and 4: 128 beams per wave above 96 beams, or where the forms
 // with several time slots per work-group end (two K steps of four channels);
 // 44/1024/64/8192/16 at fscrunch 4 took 205 against 348 of the LDS-staged kernel,
-// 44/64 32 against 50, but 24/64 26.7 against 24.5 with 32 beams per wave.
+// 44/64 32 against 50, but 24/64 26.7 against 24.5 with 32 beams per wave.  Small
+// blocks of them in FTPA: cb_pick_ftpa.
 static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, long long T)
 {
     if (variant <= 0) {
@@ -593,6 +600,29 @@ static CbVariant cb_pick_variant(const fbf_cb_desc& d, int variant, int mode, lo
     if (v.ws && !cb_ws_applies(d, mode, T)) return cb_pick_variant(d, 0, mode, T);
     if (v.tr && !v.ws && !cb_tr_applies(d, v.rows, mode, T)) return kCbVariants[kCbVariantLds];
     return v;
+}
+
+// The kernel of a block in FTPA.  As cb_pick_variant, but automatic blocks with
+// channels summed over and more than 96 beams take waves of 32 beams where the
+// kernel has them (three time slots to a work-group: of eight K slices over the
+// summed channels, which 44 to 64 antennas at fscrunch 2 and 20 to 32 at 4 have,
+// and windows of 32 columns or more) and one round of one pass each holds the
+// block.
+//
+// With 128 beams a wave, such a block is a few waves that each take four times
+// as long over a pass (us, 32 beams against 128; antennas / beams / channels /
+// samples / tscrunch / fscrunch): 64/264/6/1024/256/2 26.0 against 35.6,
+// 52/512/4/256/128/2 16.2 against 22.3, 64/304/16/1024/128/2 20.5 against 24.0,
+// 56/256/4/3072/32/2 13.2 against 14.3, 20/400/8/1536/256/4 25.9 against 28.8; but
+// in two rounds 32/232/24/4096/128/4 31.0 against 25.2.  From TAFTP only 128
+// beams a wave stage the block, and the split-transpose costs what the narrow
+// waves give: 64/136/6/2048/64/2 18.3 staged, 21.0 split.
+static CbVariant cb_pick_ftpa(const fbf_cb_desc& d, int variant, int mode, long long T)
+{
+    if (variant <= 0 && d.fscrunch > 1 && d.nbeams > 96 && cb_tr_applies(d, 2, mode, T) &&
+        cb_groups(d, T, 2, 128 / d.fscrunch, 3) <= device_cu_count())
+        return kCbVariants[kCbVariantTr2];
+    return cb_pick_variant(d, variant, mode, T);
 }
 
 extern "C" int fbf_cb_variant_count(int* count)
@@ -747,7 +777,7 @@ static int cb_launch(fbf_cb_plan* plan, int mode, const void* ftpa, long long T,
     if (T == 0) return FBF_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const CbVariant var =
-        tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_variant(d, plan->variant, mode, T);
+        tv ? CbVariant{32, tv->form.rt, true, true, false, tv->form.few} : cb_pick_ftpa(d, plan->variant, mode, T);
     const size_t vbytes = tv ? (size_t)4 * tv->Atot * d.nchans * T : (size_t)2 * vstride * d.nchans * T;
     const int wsteps = (2 * d.nantennas + 31) / 32;   // 32-byte K steps
     const bool four_waves = var.few || (var.tr && !var.ws && var.rows == 4 && tr_four_waves(4, wsteps));
@@ -1470,7 +1500,7 @@ extern "C" int fbf_cb_autotune(fbf_cb_plan* plan, long long nsamples, int reps, 
     // choice.  It is reported as the variant of its kernel.
     const bool keep_auto = auto_ms <= 1.01f * bms;
     if (keep_auto) {
-        const CbVariant v = cb_pick_variant(d, 0, MODE_INT8, nsamples);
+        const CbVariant v = cb_pick_ftpa(d, 0, MODE_INT8, nsamples);
         bv = !v.tr ? kCbVariantLds : v.rows == 2 ? kCbVariantTr2 : v.rows == 4 ? kCbVariantTr4 : kCbVariantTr8;
         bc = 0;
         bms = auto_ms;

@@ -610,3 +610,37 @@ def test_small_blocks_of_narrow_waves(gpu, oracle, A, F, nhg, B, ts, ib_ts, m128
         d_o.fill(0x5A)
         call()
         np.testing.assert_array_equal(d_o.download(), ref)
+
+
+@pytest.mark.parametrize("A,B,F,T,ts,fs,m128", [
+    (64, 104, 2, 64, 32, 2, False),       # two windows, a ragged beam group
+    (64, 264, 6, 512, 256, 2, True),      # one pass of long windows, a weight of -128
+    (44, 168, 4, 768, 16, 2, False),      # 4 antennas past a multiple of 8
+    (52, 104, 2, 4352, 16, 2, False),     # passes over six groups, the last with two
+    (20, 400, 8, 256, 64, 4, False),      # four channels to a sum
+    (32, 136, 4, 128, 128, 4, True),      # one window
+    (28, 1032, 4, 1344, 16, 4, False),    # 33 x 7 work-groups, one round
+    (28, 1032, 4, 1360, 16, 4, False),    # 33 x 8, more than one: 128 beams a wave
+    (64, 1024, 32, 96, 16, 2, False),     # 16 x 16 = 256 work-groups
+    (64, 1032, 32, 96, 16, 2, False),     # 16 x 17: 128 beams a wave
+])
+def test_small_blocks_of_summed_channels(gpu, oracle, A, B, F, T, ts, fs, m128):
+    """Small blocks with channels summed over and more than 96 beams (32 beams per
+    wave, three time slots to a work-group) in FTPA and as a subarray of a wider
+    FTPA block, 4 antennas in, against the oracle."""
+    capi = gpu
+    w = unit_weights(4101 + A, F * B * A).reshape(F, B, A, 2).copy()
+    if m128:
+        w[1, B - 1, 5, 1] = -128
+    w = w.reshape(-1)
+    off, sc = _levels(oracle, A, ts, fs, F)
+    plan = capi.CbPlan(A, B, F, ts, fs, off, sc, nsamples_per_heap_out=T // ts)
+    wide = gaussian_int8(4102 + A, F * T * 2 * (A + 8) * 2, 16.0).reshape(F, 2 * T, A + 8, 2)
+    ftpa = np.ascontiguousarray(wide[:, :, 4:4 + A]).reshape(-1)
+    ref = oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, fs), off, sc, T // ts)
+    d_w, d_o = _dev(capi, w), capi.DeviceBuffer(ref.size)
+    for call in (lambda: plan.beamform(_dev(capi, ftpa), d_w, d_o),
+                 lambda: plan.beamform_subarray(_dev(capi, wide.reshape(-1)), A + 8, 4, d_w, d_o)):
+        d_o.fill(0x5A)
+        call()
+        np.testing.assert_array_equal(d_o.download(), ref)
