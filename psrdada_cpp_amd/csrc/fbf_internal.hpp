@@ -126,10 +126,11 @@ int weights_launch_params(const fbf_weights_plan* plan, const void* delays, size
                           void* weights, size_t weights_bytes, WeightsLaunch* out);
 
 // phase = (rate * t + offset) * f in FP64 (contraction off, the oracle's
-// order), the whole-cycle part removed, then FP32 sincospif of the reduced
-// phase and both components rounded to the nearest integer, ties to even.
+// order), the whole-cycle part removed, then 127 times the FP32 cosine and sine
+// of the reduced phase, rounded to the nearest integer, ties to even: the bytes
+// that sincospif gives.
 //
-// The generator is bound by VALU issue, two thirds of it sincospif.  The
+// The generator was bound by VALU issue, two thirds of it sincospif.  The
 // hardware's v_sin_f32 / v_cos_f32 take a phase in cycles, and over every
 // float in [-1/2, 1/2] 127 times either is within 1.9e-5 of 127 times
 // sincospif's value (all 2 * 0x3f000001 of them compared on gfx950).  So where

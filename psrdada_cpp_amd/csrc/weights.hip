@@ -10,12 +10,14 @@
 // MI355X design: the phase argument is formed in FP64 -- the only FP64 step --
 // because f * tau reaches thousands of cycles at GHz x microseconds and FP32
 // would leave ~1e-3 rad of error.  The whole-cycle part is removed in FP64
-// (phase - rint(phase), exact), the reduced argument in [-1/2, 1/2] goes to
-// FP32 sincospif (HIP's device math library), then rounds to the nearest
-// integer, ties to even, as __float2int_rn does in WeightsManager.cu:70-71.
+// (phase - rint(phase), exact), the reduced argument in [-1/2, 1/2] goes to the
+// hardware's FP32 sine and cosine of cycles, or to sincospif (HIP's device math
+// library) where those are too near a half-integer to tell its rounding
+// (weights_run), then rounds to the nearest integer, ties to even, as
+// __float2int_rn does in WeightsManager.cu:70-71.
 // A thread takes one (beam, antenna) over a run of kWChans channels: the
 // delay model is read and tau formed once, and each channel costs one FP64
-// product, the reduction, sincospif and the rounding.  Antennas are fastest
+// product, the reduction, a sine, a cosine and the rounding.  Antennas are fastest
 // across lanes, so the delay reads and each channel's weight writes are
 // coalesced; the grid's y dimension runs over the channel runs.
 #include "fbf_internal.hpp"

@@ -814,3 +814,32 @@ def test_split_transpose_of_taftp_calls(gpu, oracle, Atot, A, a0, F, nhg):
     ftpa = oracle.split_transpose(taftp, nhg, Atot, A, a0, F)
     np.testing.assert_array_equal(d_o.download(),
                                   oracle.cb_tbtf(oracle.cb_power(ftpa, w, F, T, A, B, ts, 1), off, sc, 4))
+
+
+@pytest.mark.parametrize("exponent", range(-11, 0))
+def test_weights_of_every_reduced_phase(gpu, exponent):
+    """Every float of the binades that make up [2^-12, 1/2) cycles, either sign, as
+    the reduced phase (rate 0, 1 Hz): each component whose FP64 value lies
+    further than 3e-5 from a half-integer (sincospif's bound at amplitude 127)
+    equals its rounding, though the hardware's sine and cosine are rounded up to
+    1e-4 from one.  Smaller phases are below a fifth of a unit."""
+    capi = gpu
+    n = 1 << 23
+    x = (np.arange(n, dtype=np.uint32) + np.uint32((126 + exponent) << 23)).view(np.float32)
+    assert x[0] == np.float32(2.0 ** (exponent - 1)) and x[-1] < 2.0 ** exponent
+    plan = capi.WeightsPlan(1, n, 1, np.ones(1))
+    d_w = capi.DeviceBuffer(2 * n)
+    wide = 2 * np.pi * x.astype(np.float64)
+    refs = []
+    for fn in (np.cos, np.sin):
+        v = 127.0 * fn(wide)
+        refs.append((np.rint(v).astype(np.int8), np.abs(np.abs(v - np.floor(v)) - 0.5) > 3e-5))
+    assert min(ok.mean() for _, ok in refs) > 0.99
+    for sign in (1, -1):
+        d = np.zeros((n, 2), np.float32)
+        d[:, 1] = sign * x
+        plan.generate(_dev(capi, d.reshape(-1)), 0.0, d_w)
+        w = d_w.download(np.int8).reshape(n, 2)
+        for k, (r, ok) in enumerate(refs):
+            r = sign * r if k else r
+            np.testing.assert_array_equal(w[ok, k], r[ok], err_msg="cos sin".split()[k])
