@@ -662,8 +662,6 @@ extern "C" int fbf_cb_output_bytes(const fbf_cb_plan* plan, size_t ftpa_bytes, s
     return FBF_OK;
 }
 
-// A TAFTP block read directly by the coherent beamformer: S samples per
-// heap, Atot antennas, the beamformer's antennas from antenna a0.
 // The transposed kernel that stages a TAFTP block itself: RT beam tiles (16
 // RT beams) per wave, 0 where none does; `few` as in CbVariant.
 struct TaftpForm {
@@ -671,6 +669,8 @@ struct TaftpForm {
     bool few;
 };
 
+// A TAFTP block read directly by the coherent beamformer: S samples per
+// heap, Atot antennas, the beamformer's antennas from antenna a0.
 struct TaftpView {
     int S, Atot, a0;
     TaftpForm form;   // the kernel (cb_taftp_form)
@@ -1005,10 +1005,13 @@ extern "C" int fbf_cb_beamform_subarray(fbf_cb_plan* plan, const void* ftpa_bloc
 // against 27.8, 64/64/64/32 33.7 against 79.5, 128/32/64/8 22.9 against 45.0.  Waves
 // of 32 or 64 beams for so few took 8.6 and 33.7 us where 128-beam waves took
 // 10.8 and 41.0.
-// Blocks of at most kTaftpSmall channels x samples keep the split-transpose
-// where fbf_cb_taftp_direct has always answered so: at most 96 beams of up to
-// 48 antennas (unless both beams of the whole block are formed), at most 32 of
-// more than 64 on their own.
+// Not for speed, blocks of at most kTaftpSmall channels x samples are
+// split-transposed where fbf_cb_taftp_direct and fbf_cb_ib_fused tell callers,
+// who choose their calls and reserve their buffers by it, that they are: at most
+// 96 beams of up to 48 antennas (unless both beams of the whole block are
+// formed), at most 32 of more than 64 on their own.  It costs one launch of the
+// small ones (16 of 64 antennas, 32 beams, 4 channels, 4 heaps 7.9 us) and much
+// above 64 antennas (96/32/4/4 23.5 us, 6.4 staged; 128/32/2/1 16.4 and 6.9).
 constexpr long long kTaftpSmall = 4096;
 
 enum TaftpUse {
