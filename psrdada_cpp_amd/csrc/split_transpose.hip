@@ -230,7 +230,9 @@ int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nan
     const uint32_t inv = (uint32_t)(((1ull << 32) + used_nantennas - 1) / used_nantennas);
     const auto kernel = [&] {
         if constexpr (NEAR)
-            return used_nantennas % 8 == 0 ? split_transpose_k<8, SP, IB, true> : split_transpose_k<4, SP, IB, true>;
+            return used_nantennas % 8 == 0   ? split_transpose_k<8, SP, IB, true>
+                   : used_nantennas % 4 == 0 ? split_transpose_k<4, SP, IB, true>
+                                             : split_transpose_k<0, SP, IB, true>;
         else
             return used_nantennas % 8 == 0       ? split_transpose_k<8, SP, IB, false>
                    : used_nantennas % 4 == 0     ? split_transpose_k<4, SP, IB, false>
@@ -246,14 +248,19 @@ int st_launch_t(const void* taftp, void* ftpa, int total_nantennas, int used_nan
     return FBF_OK;
 }
 
-// Whether a block takes 64 x 64 tiles with cached stores: antennas in fours
-// (others need their vectors across columns) that fill such tiles, and copies
-// that outgrow the cache.  us, these tiles against 64 x 128 with nontemporal
-// stores (antennas / channels / heaps of 256 samples; with the incoherent beam
-// in brackets): 64/64/32 46 against 61 (46, 66), 64/64/12 16.2 against 17.0,
-// 56/64/32 41 against 45 (42, 46), 128/64/32 116 against 128 (116, 125), 60/64/32
-// 46 against 49, 40/64/48 (252 MB moved) 43 against 48; but 40/64/32 (168 MB) 31
-// against 25 (37, 28), and with the incoherent beam 40/64/48 53 against 49.
+// Whether a block takes 64 x 64 tiles with cached stores: antennas that fill such
+// tiles, and copies that outgrow the cache.  us, these tiles against 64 x 128 with
+// nontemporal stores (antennas / channels / heaps of 256 samples; with the
+// incoherent beam in brackets): 64/64/32 46 against 61 (46, 66), 64/64/12 16.2
+// against 17.0, 56/64/32 41 against 45 (42, 46), 128/64/32 116 against 128 (116,
+// 125), 60/64/32 46 against 49, 40/64/48 (252 MB moved) 43 against 48; but
+// 40/64/32 (168 MB) 31 against 25 (37, 28), and with the incoherent beam 40/64/48
+// 53 against 49.  Antennas not in fours, whose vectors run across columns, where one tile
+// holds them and the copy outgrows the cache without being far beyond it:
+// 62/64/32 45.7 against 53.0 (46.5, 53.6), 62/64/40 59.0 against 64.4 (60.0, 65.5),
+// 58/64/28 37.0 against 40.3, 50/64/32 38.2 against 41.0 (42.9, 42.4); but 62/64/20
+// 30.4 against 27.2 (32.0, 29.1), 62/64/52 84.7 against 82.4, 58/64/46 with the
+// incoherent beam 68.5 against 65.7, 46/64/32 35.2 against 35.4 (41.5, 37.1).
 //
 // A copy that the next launch reads (`read_next`: the library's own calls) takes
 // them too from 24 antennas, and smaller copies sooner: the coherent kernel
@@ -268,7 +275,9 @@ bool st_near(bool ib, int used_nantennas, size_t moved, bool read_next)
     // (Columns of whole 64-byte lines, 32 antennas, gain from the cache sooner:
     // 32/64/32, 128 MiB, 21.5 against 22.9; 32/64/16 11.6 against 11.4.)
     const size_t near_bytes = (size_t)(used_nantennas % 32 == 0 ? 128 : 192) << 20;
-    if (used_nantennas % 4 != 0) return false;
+    if (used_nantennas % 4 != 0)
+        return used_nantennas >= (ib ? 54 : 48) && used_nantennas < 64 && moved >= near_bytes &&
+               moved < (size_t)320 << 20;
     if (used_nantennas > 64) return true;
     if (used_nantennas >= 56 && used_nantennas % 8 == 0) return true;
     const size_t copy_mib = (moved / 2) >> 20;

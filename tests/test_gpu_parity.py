@@ -843,3 +843,29 @@ def test_weights_of_every_reduced_phase(gpu, exponent):
         for k, (r, ok) in enumerate(refs):
             r = sign * r if k else r
             np.testing.assert_array_equal(w[ok, k], r[ok], err_msg="cos sin".split()[k])
+
+
+@pytest.mark.parametrize("A,F,nhg,ts", [
+    (62, 4, 1, 16), (63, 4, 3, 32),          # small: 128-column tiles
+    (50, 64, 30, 16), (54, 64, 28, 8),       # 188 and 189 MiB moved
+    (50, 64, 31, 16), (54, 64, 29, 8),       # 194 and 196 MiB: 64 x 64 tiles, the first not with the incoherent beam
+    (63, 64, 40, 32), (63, 64, 41, 16),      # 315 and 323 MiB
+])
+def test_split_transpose_of_antennas_not_in_fours(gpu, oracle, A, F, nhg, ts):
+    """Vectors across columns from either form of the tiles, without the incoherent
+    beam and with it, against the oracle."""
+    capi = gpu
+    taftp = gaussian_int8(7400 + A + nhg, nhg * A * F * 256 * 4, 16.0)
+    ref = oracle.split_transpose(taftp, nhg, A, A, 0, F)
+    _, _, ibo, ibs = oracle.power_levels(16.0, 24.0, A, 16, 1, A, ts, 1)
+    off, sc = np.full(F, ibo, np.float32), np.full(F, ibs, np.float32)
+    plan = capi.IbPlan(A, F, ts, 1, off, sc)
+    d_in, d_out = _dev(capi, taftp), capi.DeviceBuffer(taftp.nbytes)
+    d_tf = capi.DeviceBuffer(plan.output_bytes(taftp.nbytes))
+    d_out.fill(0x5A)
+    capi.split_transpose(d_in, d_out, A, A, 0, F)
+    np.testing.assert_array_equal(d_out.download(), ref)
+    d_out.fill(0x5A)
+    capi.split_transpose_ib(d_in, d_out, F, plan, d_tf)
+    np.testing.assert_array_equal(d_out.download(), ref)
+    np.testing.assert_array_equal(d_tf.download(), oracle.ib_tf(oracle.ib_power(taftp, F, ts, 1, nhg, A), off, sc))
